@@ -136,10 +136,11 @@ def draw(rng):
                     compute=rng.choice(["native", "bf16"]))
     while case["batch"] > 1 and not _fits(case):
         case["batch"] -= 1
-    while not _fits(case):   # one element is still too much: fewer channels
-        for key in ("cin", "cout", "channels", "patch"):
-            if key in case and case[key] > 4:
-                case[key] = case[key] * 3 // 4
+    while not _fits(case):   # one element is still too much: a smaller picture or mesh
+        if path == "ico":
+            case["level"] -= 1
+        else:
+            case["height"], case["width"] = case["height"] * 3 // 4, case["width"] * 3 // 4
     return case
 
 
