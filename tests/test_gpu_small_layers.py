@@ -1,0 +1,104 @@
+"""Layers over images of at most four channels: the sizes at which the windowed kernels can go
+wrong.  Rows that end inside a wave's 32 pixels, grids with fewer rows than a workgroup has
+waves, more batch elements than a window space holds, kernel sizes on both sides of a lane
+half's sample group, output channels on both sides of a 32-row block, maps that fit no window,
+point weights, and values that must not be touched under a zero weight.
+
+Tolerances: forward sums at most 4 * 25 products (1e-5); gradients add over batch and pixels in an
+order of their own (1e-4), as for the other float32 convolution kernels.
+"""
+import numpy as np
+import pytest
+import torch
+
+import workloads
+from conftest import relerr
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from _spherical_distortion_ext import _ops
+    return _ops
+
+
+def _t(a):
+    return None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def _check(ops, oracle, B, Cin, Cout, m, wts, H, W, interp, seed):
+    rng = np.random.default_rng(seed)
+    K = m.shape[2]
+    x = rng.standard_normal((B, Cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((Cout, Cin, K)) / np.sqrt(Cin * K)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    g = rng.standard_normal((B, Cout) + m.shape[:2]).astype(np.float32)
+    y = ops.mapped_conv_forward(_t(x), _t(m), _t(wts), _t(w), _t(b), K, interp)
+    assert relerr(y.cpu().numpy(),
+                  oracle.mapped_conv_forward(x, m, w, b, K, interp, wts)) <= 1e-5
+    grads = ops.mapped_conv_backward(_t(g), _t(m), _t(wts), _t(x), _t(w), _t(b), K, interp)
+    for got, want in zip(grads, oracle.mapped_conv_backward(g, m, x, w, b, K, interp, wts)):
+        assert relerr(got.cpu().numpy(), want) <= 1e-4
+
+
+def _near(rng, OH, OW, K, spread, wild, stride=1):
+    """Samples within `spread` of their pixel, a share `wild` of them anywhere, some outside."""
+    ys, xs = np.meshgrid(np.arange(OH) * stride, np.arange(OW) * stride, indexing="ij")
+    c = np.stack([xs, ys], -1)[:, :, None, :] + rng.uniform(-spread, spread, (OH, OW, K, 2))
+    far = rng.uniform(-3, 1.1 * stride * max(OH, OW), (OH, OW, K, 2))
+    return np.where(rng.random((OH, OW, K, 1)) < wild, far, c).astype(np.float32)
+
+
+@pytest.mark.parametrize("interp", [0, 1, 2])
+@pytest.mark.parametrize("B,Cin,Cout,OH,OW,K", [
+    (1, 1, 8, 3, 31, 9),      # fewer rows than waves, no full piece, one pixel row block
+    (2, 3, 17, 5, 33, 10),    # one pixel in a second piece; the largest single sample group
+    (9, 3, 32, 40, 64, 9),    # four waves a workgroup; more batch elements than fit at once
+    (3, 4, 33, 37, 70, 11),   # a second 32-row block; the smallest of three sample groups
+    (1, 2, 65, 1, 130, 1),    # one row, one sample, a second channel chunk
+    (2, 4, 128, 9, 40, 25),
+])
+def test_edges_of_pieces_groups_and_blocks(ops, oracle, B, Cin, Cout, OH, OW, K, interp):
+    rng = np.random.default_rng(OH * OW + K)
+    m = _near(rng, OH, OW, K, 1.6, 0.0)
+    _check(ops, oracle, B, Cin, Cout, m, None, OH, OW, interp, 3)
+
+
+@pytest.mark.parametrize("interp", [0, 1, 2])
+def test_tiles_that_fit_no_window(ops, oracle, interp):
+    rng = np.random.default_rng(5)
+    m = _near(rng, 48, 96, 9, 1.6, 0.3)
+    # (coordinates that no integer holds are left out: converting them is undefined in C++, and
+    # the oracle's result for them with it)
+    m[1, 2, 3] = [1e6, -1e6]
+    _check(ops, oracle, 4, 3, 24, m, None, 48, 96, 1 if interp == 2 else interp, 4)
+    # a spherical kernel: the rows next to the poles span the image, tiles cross the wrap seam
+    m = workloads.gnomonic_kernel_map(64, 128)
+    _check(ops, oracle, 4, 3, 24, m, None, 64, 128, interp, 5)
+    m = workloads.gnomonic_kernel_map(65, 130, stride=2)
+    _check(ops, oracle, 2, 4, 40, m, None, 65, 130, interp, 6)
+
+
+def test_point_weights(ops, oracle):
+    m, wts = workloads.four_nearest_weighted(workloads.gnomonic_kernel_map(40, 80), 40, 80)
+    _check(ops, oracle, 3, 3, 20, m, wts, 40, 80, 2, 7)
+
+
+def test_zero_weight_taps_are_not_read(ops):
+    """Integer coordinates put weight on one tap; infinite and missing values all round it must
+    not reach the sums."""
+    H, W, K, Cout = 32, 64, 9, 24
+    ys, xs = np.meshgrid(np.arange(H) // 2 * 2, np.arange(W) // 2 * 2, indexing="ij")
+    m = np.broadcast_to(np.stack([xs, ys], -1)[:, :, None, :], (H, W, K, 2)).astype(np.float32)
+    x = np.full((4, 3, H, W), np.inf, np.float32)
+    x[:, :, 1::2] = np.nan
+    x[:, :, ::2, ::2] = 1.0
+    w = np.ones((Cout, 3, K), np.float32)
+    g = np.ones((4, Cout, H, W), np.float32)
+    b = np.zeros(Cout, np.float32)
+    y = ops.mapped_conv_forward(_t(x), _t(m), None, _t(w), _t(b), K, 1)
+    assert torch.equal(y, torch.full_like(y, 3.0 * K))
+    _, gw, _ = ops.mapped_conv_backward(_t(g), _t(m), None, _t(x), _t(w), _t(b), K, 1)
+    assert torch.equal(gw, torch.full_like(gw, 4.0 * H * W))
