@@ -583,6 +583,21 @@ int sdk_mapped_conv_backward_planned(const void* grad_output, const void* sample
     int64_t batch, int64_t in_channels, int64_t height, int64_t width, int64_t out_channels,
     int64_t out_height, int64_t out_width, int64_t kernel_size, int32_t num_interp_pts, int32_t
     interp, int32_t dtype, int32_t compute, sdk_stream_t stream);
+/* The gradients of a layer that are wanted, of the three that sdk_mapped_conv_backward forms:
+ * grad_input may be NULL, and so may grad_weight and grad_bias together.  plan: a kept plan, or
+ * NULL (plan_bytes 0). */
+int sdk_mapped_conv_backward_select(const void* grad_output, const void* sample_map, const void*
+    interp_weights, const void* input, const void* weight, void* grad_input, void* grad_weight,
+    void* grad_bias, void* workspace, size_t workspace_bytes, void* plan, size_t plan_bytes,
+    int64_t batch, int64_t in_channels, int64_t height, int64_t width, int64_t out_channels,
+    int64_t out_height, int64_t out_width, int64_t kernel_size, int32_t num_interp_pts, int32_t
+    interp, int32_t dtype, int32_t compute, sdk_stream_t stream);
+int sdk_mapped_transposed_conv_backward_select(const void* grad_output, const void* sample_map,
+    const void* interp_weights, const void* input, const void* weight, void* grad_input, void*
+    grad_weight, void* grad_bias, void* workspace, size_t workspace_bytes, void* plan, size_t
+    plan_bytes, int64_t batch, int64_t in_channels, int64_t in_height, int64_t in_width, int64_t
+    out_channels, int64_t out_height, int64_t out_width, int64_t kernel_size, int32_t
+    num_interp_pts, int32_t interp, int32_t dtype, int32_t compute, sdk_stream_t stream);
 int sdk_mapped_transposed_conv_forward_planned(const void* input, const void* sample_map, const
     void* interp_weights, const void* weight, const void* bias, void* output, void* workspace,
     size_t workspace_bytes, void* plan, size_t plan_bytes, int64_t batch, int64_t in_channels,

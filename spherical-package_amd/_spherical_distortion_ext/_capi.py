@@ -57,6 +57,9 @@ SIGNATURES = {
     "sdk_mapped_transposed_conv_forward_planned": [_vp] * 7 + [_sz, _vp, _sz] + _CONV_DIMS,
     "sdk_mapped_transposed_conv_backward_input_planned": [_vp] * 6 + [_sz, _vp, _sz] + _CONV_DIMS,
     "sdk_mapped_transposed_conv_backward_weight_planned": [_vp] * 6 + [_sz, _vp, _sz] + _CONV_DIMS,
+    # gradients that are not wanted passed as NULL (the plan may be NULL too)
+    "sdk_mapped_conv_backward_select": [_vp] * 9 + [_sz, _vp, _sz] + _CONV_DIMS,
+    "sdk_mapped_transposed_conv_backward_select": [_vp] * 9 + [_sz, _vp, _sz] + _CONV_DIMS,
     "sdk_mapped_conv_plan_build": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
     # plans of the scatter direction
     "sdk_resample_to_map_plan_build": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],

@@ -670,6 +670,33 @@ def mapped_transposed_conv_backward(grad_output, sample_map, interp_weights, x, 
     return gi, gw, gb
 
 
+def mapped_conv_backward_select(grad_output, sample_map, interp_weights, x, weight, kernel_size,
+                                interp, transposed, need_input, need_params):
+    """(grad_input or None, grad_weight or None, grad_bias or None) of a (transposed) mapped
+    convolution: what mapped_conv_backward returns, without the gradients nobody asks for."""
+    grad_output = grad_output.contiguous()
+    _check(grad_output, grad_output=grad_output, input=x, sample_map=sample_map,
+           interp_weights=interp_weights, weight=weight)
+    P = _npts(sample_map, interp_weights, 4)
+    B, Cin, Cout, K = _conv_dims(x.shape, weight, sample_map, kernel_size, transposed)
+    IH, IW = x.shape[2:]
+    OH, OW = grad_output.shape[2:]
+    gi = torch.empty_like(x) if need_input else None
+    gw = torch.empty_like(weight) if need_params else None
+    gb = torch.empty((Cout,), dtype=x.dtype, device=x.device) if need_params else None
+    img, grid = ((OH, OW), (IH, IW)) if transposed else ((IH, IW), (OH, OW))
+    name = ("sdk_mapped_transposed_conv_backward_select" if transposed
+            else "sdk_mapped_conv_backward_select")
+    with torch.cuda.device(x.device):
+        ws, nws = _workspace(x, B, Cin, Cout, *img, *grid, K, P, int(interp))
+        plan, nplan = _conv_plan(x, sample_map, interp_weights, *img, K, P, int(interp))
+        _capi.call(name, _ptr(grad_output), _ptr(sample_map), _ptr(interp_weights), _ptr(x),
+                   _ptr(weight), _ptr(gi), _ptr(gw), _ptr(gb), _ptr(ws), nws, _ptr(plan), nplan,
+                   B, Cin, IH, IW, Cout, OH, OW, K, P, int(interp), _DTYPES[x.dtype],
+                   _current_mode(), _stream(x))
+    return gi, gw, gb
+
+
 # --------------------------------------------------------------------------- UV resample
 def _uv_dims(quad_idx, tex_uv):
     if quad_idx.dtype != torch.int64 or quad_idx.dim() != 2:
@@ -884,6 +911,10 @@ _SCHEMAS = (
      "(Tensor grad_output, Tensor sample_map, Tensor? interp_weights, Tensor x, Tensor weight,"
      " Tensor bias, int kernel_size, int interp) -> (Tensor, Tensor, Tensor)",
      mapped_transposed_conv_backward),
+    ("mapped_conv_backward_select",
+     "(Tensor grad_output, Tensor sample_map, Tensor? interp_weights, Tensor x, Tensor weight,"
+     " int kernel_size, int interp, bool transposed, bool need_input, bool need_params)"
+     " -> (Tensor, Tensor, Tensor)", mapped_conv_backward_select),
 )
 
 def _load_native():
@@ -902,6 +933,7 @@ def _load_native():
     for name in ("sdk_torch_set_default_mode", "sdk_torch_set_plan_cache",
                  "sdk_torch_set_unpool_workspace"):
         getattr(lib, name).restype = None
+    lib.sdk_torch_native_select.restype = ctypes.c_char_p
     return lib, frozenset(lib.sdk_torch_native_ops().decode().split(","))
 
 
@@ -909,8 +941,11 @@ _library = torch.library.Library(_NS, "DEF")
 for _name, _schema, _fn in _SCHEMAS:
     _library.define(_name + _schema)
 _native, _NATIVE_OPS = _load_native()
+# the operator the compiled layer implements beside those of the reference's extension modules
+_NATIVE_SELECT = frozenset() if _native is None else \
+    frozenset([_native.sdk_torch_native_select().decode()])
 for _name, _schema, _fn in _SCHEMAS:
-    if _name not in _NATIVE_OPS:
+    if _name not in _NATIVE_OPS | _NATIVE_SELECT:
         _library.impl(_name, _fn, "CUDA")
 
 
@@ -919,5 +954,5 @@ for _name, _schema, _fn in _SCHEMAS:
 # that callers of this module and callers of torch.ops.sdk_mapped_ops run the same code.
 ops = getattr(torch.ops, _NS)
 PYTHON_IMPL = {_name: _fn for _name, _schema, _fn in _SCHEMAS}
-for _name in _NATIVE_OPS:
+for _name in _NATIVE_OPS | _NATIVE_SELECT:
     globals()[_name] = getattr(ops, _name)

@@ -343,10 +343,12 @@ static int impl_mapped_conv_backward(const void* grad_output, const void* sample
                              int64_t in_channels, int64_t height, int64_t width,
                              int64_t out_channels, int64_t out_height, int64_t out_width,
                              int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
-                             int32_t dtype, int32_t compute, sdk_stream_t stream, PlanArg plan) {
+                             int32_t dtype, int32_t compute, sdk_stream_t stream, PlanArg plan,
+                             bool select = false) {
   const char* what = "mapped_conv_backward";
-  SDK_REQUIRE(grad_output && sample_map && input && weight && grad_input && grad_weight &&
-                  grad_bias,
+  SDK_REQUIRE(grad_output && sample_map && input && weight &&
+                  (select ? (grad_weight != nullptr) == (grad_bias != nullptr)
+                          : grad_input && grad_weight && grad_bias),
               "%s: NULL pointer", what);
   SDK_REQUIRE(out_height >= 1 && out_width >= 1, "%s: bad output size", what);
   const int64_t M = out_height * out_width;
@@ -360,11 +362,12 @@ static int impl_mapped_conv_backward(const void* grad_output, const void* sample
   SharedPlan shared;   // the tap plan of the map is built once for both contractions
   // A layer with at most four image channels runs three small kernels, each adding into a
   // target that has to start from zero: the three targets are cleared by one launch.
-  if (dtype == SDK_F32 && compute != SDK_COMPUTE_UNFUSED && batch > 0 && fused_supported(g) &&
-      small_conv_supported(g) && small_wgrad_supported(g) &&
+  if (grad_weight != nullptr && dtype == SDK_F32 && compute != SDK_COMPUTE_UNFUSED && batch > 0 &&
+      fused_supported(g) && small_conv_supported(g) && small_wgrad_supported(g) &&
       !side_worth(batch, out_channels, M, dtype)) {
     rc = zero_fill3(grad_bias, sizeof(float) * (size_t)out_channels, grad_input,
-                    sizeof(float) * (size_t)batch * in_channels * height * width, grad_weight,
+                    grad_input ? sizeof(float) * (size_t)batch * in_channels * height * width : 0,
+                    grad_weight,
                     sizeof(float) * (size_t)out_channels * in_channels * kernel_size,
                     (hipStream_t)stream);
     if (rc) return rc;
@@ -372,17 +375,17 @@ static int impl_mapped_conv_backward(const void* grad_output, const void* sample
     shared.bias_sum = static_cast<float*>(grad_bias);   // summed by the weight-gradient kernel
   }
   hipEvent_t joined = nullptr;
-  if (!shared.cleared)
+  if (!shared.cleared && grad_bias != nullptr)
     rc = fork_side((hipStream_t)stream, &joined, side_worth(batch, out_channels, M, dtype),
                    [&](hipStream_t s) {
       return bias_grad(grad_output, grad_bias, batch, out_channels, M, dtype, s,
                        s != (hipStream_t)stream);
     });
-  if (rc == SDK_OK)
+  if (rc == SDK_OK && grad_input != nullptr)
     rc = run(what, GEMM_SCATTER, g, dtype, compute, grad_output, sample_map, interp_weights,
              weight, nullptr, grad_input, workspace, workspace_bytes, (hipStream_t)stream, &shared,
              plan);
-  if (rc == SDK_OK)
+  if (rc == SDK_OK && grad_weight != nullptr)
     rc = run(what, GATHER_WGRAD, g, dtype, compute, grad_output, sample_map, interp_weights, input,
              nullptr, grad_weight, workspace, workspace_bytes, (hipStream_t)stream, &shared, plan);
   // (joined also after an error: the caller's stream must not run ahead of the side stream)
@@ -400,9 +403,11 @@ static int impl_mapped_transposed_conv_backward(const void* grad_output, const v
                                         int64_t out_height, int64_t out_width,
                                         int64_t kernel_size, int32_t num_interp_pts,
                                         int32_t interp, int32_t dtype, int32_t compute,
-                                        sdk_stream_t stream, PlanArg plan) {
+                                        sdk_stream_t stream, PlanArg plan, bool select = false) {
   const char* what = "mapped_transposed_conv_backward";
-  SDK_REQUIRE(grad_output && grad_bias, "%s: NULL pointer", what);
+  SDK_REQUIRE(grad_output && (select ? (grad_weight != nullptr) == (grad_bias != nullptr)
+                                     : grad_bias != nullptr),
+              "%s: NULL pointer", what);
   SDK_REQUIRE(out_height >= 1 && out_width >= 1 && out_height * out_width < ((int64_t)1 << 31),
               "%s: bad output size", what);
   SDK_REQUIRE(in_height >= 1 && in_width >= 1, "%s: bad input size", what);
@@ -418,18 +423,19 @@ static int impl_mapped_transposed_conv_backward(const void* grad_output, const v
     if (rc) return rc;
   }
   hipEvent_t joined = nullptr;
-  rc = fork_side((hipStream_t)stream, &joined,
-                     side_worth(batch, out_channels, out_height * out_width, dtype),
-                     [&](hipStream_t s) {
-    return bias_grad(grad_output, grad_bias, batch, out_channels, out_height * out_width, dtype, s,
-                     s != (hipStream_t)stream);
-  });
-  if (rc == SDK_OK)
+  if (!select || grad_bias != nullptr)
+    rc = fork_side((hipStream_t)stream, &joined,
+                   side_worth(batch, out_channels, out_height * out_width, dtype),
+                   [&](hipStream_t s) {
+      return bias_grad(grad_output, grad_bias, batch, out_channels, out_height * out_width, dtype,
+                       s, s != (hipStream_t)stream);
+    });
+  if (rc == SDK_OK && (!select || grad_input != nullptr))
     rc = impl_mapped_transposed_conv_backward_input(
         grad_output, sample_map, interp_weights, weight, grad_input, workspace, workspace_bytes,
         batch, in_channels, in_height, in_width, out_channels, out_height, out_width,
         kernel_size, num_interp_pts, interp, dtype, compute, stream, plan);
-  if (rc == SDK_OK)
+  if (rc == SDK_OK && (!select || grad_weight != nullptr))
     rc = impl_mapped_transposed_conv_backward_weight(
         grad_output, sample_map, interp_weights, input, grad_weight, workspace, workspace_bytes,
         batch, in_channels, in_height, in_width, out_channels, out_height, out_width, kernel_size,
@@ -693,6 +699,41 @@ int sdk_mapped_transposed_conv_backward_planned(const void* grad_output, const v
   pa.buffer = plan;
   pa.bytes = plan_bytes;
   return impl_mapped_transposed_conv_backward(grad_output, sample_map, interp_weights, input, weight, grad_input, grad_weight, grad_bias, workspace, workspace_bytes, batch, in_channels, in_height, in_width, out_channels, out_height, out_width, kernel_size, num_interp_pts, interp, dtype, compute, stream, pa);
+}
+
+int sdk_mapped_conv_backward_select(const void* grad_output, const void* sample_map,
+                                    const void* interp_weights, const void* input,
+                                    const void* weight, void* grad_input, void* grad_weight,
+                                    void* grad_bias, void* workspace, size_t workspace_bytes,
+                                    void* plan, size_t plan_bytes, int64_t batch,
+                                    int64_t in_channels, int64_t height, int64_t width,
+                                    int64_t out_channels, int64_t out_height, int64_t out_width,
+                                    int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
+                                    int32_t dtype, int32_t compute, sdk_stream_t stream) {
+  PlanArg pa;
+  pa.buffer = plan;
+  pa.bytes = plan_bytes;
+  return impl_mapped_conv_backward(grad_output, sample_map, interp_weights, input, weight,
+                                   grad_input, grad_weight, grad_bias, workspace, workspace_bytes,
+                                   batch, in_channels, height, width, out_channels, out_height,
+                                   out_width, kernel_size, num_interp_pts, interp, dtype, compute,
+                                   stream, pa, true);
+}
+
+int sdk_mapped_transposed_conv_backward_select(
+    const void* grad_output, const void* sample_map, const void* interp_weights, const void* input,
+    const void* weight, void* grad_input, void* grad_weight, void* grad_bias, void* workspace,
+    size_t workspace_bytes, void* plan, size_t plan_bytes, int64_t batch, int64_t in_channels,
+    int64_t in_height, int64_t in_width, int64_t out_channels, int64_t out_height,
+    int64_t out_width, int64_t kernel_size, int32_t num_interp_pts, int32_t interp, int32_t dtype,
+    int32_t compute, sdk_stream_t stream) {
+  PlanArg pa;
+  pa.buffer = plan;
+  pa.bytes = plan_bytes;
+  return impl_mapped_transposed_conv_backward(
+      grad_output, sample_map, interp_weights, input, weight, grad_input, grad_weight, grad_bias,
+      workspace, workspace_bytes, batch, in_channels, in_height, in_width, out_channels, out_height,
+      out_width, kernel_size, num_interp_pts, interp, dtype, compute, stream, pa, true);
 }
 
 }  // extern "C"

@@ -621,6 +621,45 @@ std::tuple<Tensor, Tensor, Tensor> mapped_transposed_conv_backward(
   return {gi, gw, gb};
 }
 
+// The gradients that are wanted, undefined tensors for the others (what the plain backward
+// operators return, without the work nobody asks for).
+std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward_select(
+    const Tensor& grad_output, const Tensor& map, const OptTensor& wts, const Tensor& x,
+    const Tensor& weight, int64_t kernel_size, int64_t interp, bool transposed, bool need_input,
+    bool need_params) {
+  const Tensor g = grad_output.contiguous();
+  check_first(g);
+  check_one(g, "input", x);
+  check_one(g, "sample_map", map);
+  check_opt(g, "interp_weights", wts);
+  check_one(g, "weight", weight);
+  const int64_t P = npts(map, wts, 4);
+  const ConvDims d = conv_dims(x, weight, map, kernel_size, transposed);
+  TORCH_CHECK(g.dim() == 4, "grad_output must be [B, C, OH, OW]");
+  const int64_t IH = x.size(2), IW = x.size(3), OH = g.size(2), OW = g.size(3);
+  const int64_t img_h = transposed ? OH : IH, img_w = transposed ? OW : IW;
+  Tensor gi, gw, gb;
+  if (need_input) gi = at::empty_like(x);
+  if (need_params) {
+    gw = at::empty_like(weight);
+    gb = at::empty({d.Cout}, x.options());
+  }
+  c10::DeviceGuard guard(x.device());
+  hipStream_t s = stream_of(x);
+  size_t nws = 0;
+  Tensor ws = workspace(x, d, img_h, img_w, map.size(0), map.size(1), P, interp, &nws);
+  PlanRef plan = conv_plan(x, map, wts, img_h, img_w, d.K, P, interp, s);
+  const auto ptr = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
+  const auto call = transposed ? sdk_mapped_transposed_conv_backward_select
+                               : sdk_mapped_conv_backward_select;
+  const int rc =
+      call(g.data_ptr(), map.data_ptr(), cptr(wts), x.data_ptr(), weight.data_ptr(), ptr(gi),
+           ptr(gw), ptr(gb), ptr(ws), nws, plan.ptr(), plan.nbytes, d.B, d.Cin, IH, IW, d.Cout, OH,
+           OW, d.K, (int32_t)P, (int32_t)interp, dtype_code(x), current_mode(), s);
+  if (rc != 0) fail_call("sdk_mapped_conv_backward_select", rc);
+  return {gi, gw, gb};
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(sdk_mapped_ops, CUDA, m) {
@@ -635,6 +674,7 @@ TORCH_LIBRARY_IMPL(sdk_mapped_ops, CUDA, m) {
   m.impl("mapped_conv_backward", &mapped_conv_backward);
   m.impl("mapped_transposed_conv_forward", &mapped_transposed_conv_forward);
   m.impl("mapped_transposed_conv_backward", &mapped_transposed_conv_backward);
+  m.impl("mapped_conv_backward_select", &mapped_conv_backward_select);
 }
 
 // Controls, called from Python (ctypes): the compute mode (process default and per-thread
@@ -645,6 +685,7 @@ const char* sdk_torch_native_ops(void) {
          "mapped_max_unpool,mapped_avg_pool,mapped_avg_unpool,mapped_conv_forward,"
          "mapped_conv_backward,mapped_transposed_conv_forward,mapped_transposed_conv_backward";
 }
+const char* sdk_torch_native_select(void) { return "mapped_conv_backward_select"; }
 void sdk_torch_set_default_mode(int mode) { g_default_mode = mode; }
 // mode < 0 removes the override; returns the previous override (-1: none)
 int sdk_torch_set_thread_mode(int mode) {

@@ -24,6 +24,17 @@ from _spherical_distortion_ext._ops import conv_compute, get_conv_compute, ops a
 from ..layer_utils import InterpolationType, check_args, check_input_map_shape
 
 
+def _wanted_conv_grads(ctx, grad_output, sample_map, interp_weights, input, weight, transposed):
+    """(grad_input, grad_weight, grad_bias), None where the graph has no use for it: the image
+    of a first layer, the parameters of a frozen one.  (The reference forms all three,
+    layers/functional/mapped_convolution.py:39-61.)"""
+    need_input, need_weight, need_bias = ctx.needs_input_grad[:3]
+    gi, gw, gb = _sdk_ops.mapped_conv_backward_select(
+        grad_output, sample_map, interp_weights, input, weight, ctx.kernel_size, int(ctx.interp),
+        transposed, need_input, need_weight or need_bias)
+    return gi, gw if need_weight else None, gb if need_bias else None
+
+
 class MappedConvolutionFunction(torch.autograd.Function):
     """layers/functional/mapped_convolution.py:14-61."""
 
@@ -43,6 +54,9 @@ class MappedConvolutionFunction(torch.autograd.Function):
     def backward(ctx, grad_output):
         input, weight, bias, sample_map, interp_weights = ctx.saved_tensors
         with conv_compute(ctx.compute):
+            if not all(ctx.needs_input_grad[:3]):
+                return _wanted_conv_grads(ctx, grad_output, sample_map, interp_weights, input,
+                                          weight, False) + (None,) * 4
             if interp_weights is None:
                 grads = _mapped_conv.mapped_conv_backward(grad_output, sample_map, input, weight,
                                                           bias, ctx.kernel_size, ctx.interp)
@@ -76,6 +90,9 @@ class MappedTransposedConvolutionFunction(torch.autograd.Function):
     def backward(ctx, grad_output):
         input, sample_map, weight, bias, interp_weights = ctx.saved_tensors
         with conv_compute(ctx.compute):
+            if not all(ctx.needs_input_grad[:3]):
+                return _wanted_conv_grads(ctx, grad_output, sample_map, interp_weights, input,
+                                          weight, True) + (None,) * 6
             if interp_weights is None:
                 grads = _mapped_transposed_conv.mapped_transposed_conv_backward(
                     grad_output, sample_map, input, weight, bias, ctx.kernel_size, ctx.interp)
@@ -101,6 +118,7 @@ class MappedMaxPoolFunction(torch.autograd.Function):
             pooled, idx_mask = _weighted_mapped_max_pool.weighted_mapped_max_pool(
                 input, sample_map, interp_weights, kernel_size, interp)
         ctx.mark_non_differentiable(idx_mask)
+        ctx.set_materialize_grads(False)   # no gradient of zeros for the indices
         ctx.save_for_backward(idx_mask, sample_map, interp_weights)
         ctx.in_hw = (int(input.shape[2]), int(input.shape[3]))
         ctx.kernel_size = int(kernel_size)
@@ -109,6 +127,8 @@ class MappedMaxPoolFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, idx_mask_grad=None):
+        if grad_output is None:
+            return None, None, None, None, None
         idx_mask, sample_map, interp_weights = ctx.saved_tensors
         grad_output = grad_output.contiguous()
         if interp_weights is None:
