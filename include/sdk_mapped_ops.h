@@ -559,6 +559,29 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
                                int64_t map_height, int64_t map_width, int64_t kernel_size,
                                int32_t num_interp_pts, int32_t interp, int32_t dtype,
                                sdk_stream_t stream);
+/* Small calls run as an im2col, matrix products and a col2im instead of the tile kernels and
+ * read only the inverted map of a plan, the forward of a convolution and the backward of a
+ * transposed one not even that:
+ *
+ *   sdk_mapped_conv_by_columns(...)           1 when a call of these sizes does (transposed: of a
+ *                                             transposed convolution), 0 otherwise
+ *   sdk_mapped_conv_plan_build_columns(...)   fills, of a plan buffer of full size, the part
+ *                                             such calls read; for no other call
+ *   sdk_mapped_conv_columns_enable(0 / 1)     turns the route off / on for the calling thread
+ *                                             (to measure or test the tile kernels at small
+ *                                             sizes); returns the previous value.  Workspace
+ *                                             queries and calls must see the same value. */
+int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_channels,
+                               int64_t image_height, int64_t image_width, int64_t map_height,
+                               int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
+                               int32_t interp, int32_t dtype, int32_t compute,
+                               int32_t transposed);
+int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
+                                       void* plan, size_t plan_bytes, int64_t image_height,
+                                       int64_t image_width, int64_t map_height, int64_t map_width,
+                                       int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
+                                       int32_t dtype, sdk_stream_t stream);
+int sdk_mapped_conv_columns_enable(int32_t enabled);
 int sdk_mapped_conv_forward_planned(const void* input, const void* sample_map, const void*
     interp_weights, const void* weight, const void* bias, void* output, void* workspace, size_t
     workspace_bytes, void* plan, size_t plan_bytes, int64_t batch, int64_t in_channels, int64_t

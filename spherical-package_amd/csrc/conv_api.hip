@@ -481,6 +481,44 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
                            (hipStream_t)stream);
 }
 
+int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_channels,
+                               int64_t image_height, int64_t image_width, int64_t map_height,
+                               int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
+                               int32_t interp, int32_t dtype, int32_t compute,
+                               int32_t transposed) {
+  if (dtype != SDK_F32 || compute == SDK_COMPUTE_UNFUSED || kernel_size < 1 || map_height < 1 ||
+      map_width < 1 || image_height < 1 || image_width < 1 || num_interp_pts < 0 ||
+      map_height * map_width >= ((int64_t)1 << 31) || image_height * image_width >= ((int64_t)1 << 31))
+    return 0;
+  ConvGeom g{batch, (int)(transposed ? out_channels : in_channels), (int)image_height,
+             (int)image_width, (int)(transposed ? in_channels : out_channels),
+             (int)(map_height * map_width), (int)kernel_size, num_interp_pts, interp,
+             (int)map_width};
+  return fused_supported(g) && plan_supported(g) && columns_first(g) ? 1 : 0;
+}
+
+int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
+                                       void* plan, size_t plan_bytes, int64_t image_height,
+                                       int64_t image_width, int64_t map_height, int64_t map_width,
+                                       int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
+                                       int32_t dtype, sdk_stream_t stream) {
+  const char* what = "mapped_conv_plan_build_columns";
+  SDK_REQUIRE(sample_map && plan, "%s: NULL pointer", what);
+  SDK_REQUIRE(num_interp_pts >= 0 && (num_interp_pts == 0 || interp_weights),
+              "%s: weighted map needs interp_weights", what);
+  const size_t need = sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width,
+                                                 kernel_size, num_interp_pts, interp, dtype);
+  if (need == 0)
+    return fail(SDK_ERR_UNSUPPORTED, "%s: no plan for this geometry (ask sdk_mapped_conv_plan_bytes)",
+                what);
+  if (plan_bytes < need)
+    return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, plan_bytes);
+  ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
+             (int)kernel_size, num_interp_pts, interp, (int)map_width};
+  return build_cached_columns_plan(g, (const float*)sample_map, (const float*)interp_weights, plan,
+                                   (hipStream_t)stream);
+}
+
 int sdk_mapped_conv_forward(const void* input, const void* sample_map, const void* interp_weights,
                             const void* weight, const void* bias, void* output, void* workspace,
                             size_t workspace_bytes, int64_t batch, int64_t in_channels,

@@ -1,0 +1,644 @@
+// Mapped convolution with the column matrix in memory, for calls so small that the fused
+// kernels cannot fill the GPU.
+//
+// The fused kernels (conv_window_gemm.hip, conv_window_wgrad.hip) own 128-pixel tiles and walk
+// all samples and channels of a tile in one workgroup: at 6 x 25 x 50 output pixels that is a
+// few dozen workgroups on 256 CUs, each a serial chain of hundreds of dependent LDS and memory
+// steps, once per class of tiles.  The same work cut into an im2col, a matrix product and a
+// col2im (the reference's own order, ext_modules/src/cpp/mapped_convolution_layer.cpp:8-60)
+// has thousands of independent pieces per launch, and the column matrix, a few tens of MB,
+// stays in the 256 MB memory-side cache between the launch that writes it and the one that
+// reads it.  No tap plan is needed either: the map is read once per sample.
+// (Measured: 96 -> 160 channels, 6 x 50 x 100, stride 2, split, forward + backward 907 -> 180 us;
+// 64 -> 64 channels on a map not seen before, 1 x 128 x 256, forward 368 -> 62 us, of which 265
+// were its plan.)
+//
+// Everything is channels-last and padded with zeros to a multiple of eight channels, so that
+// every access of these kernels is an aligned 16-byte one:
+//   rows   img[b][c][u] -> [b][u][c]            (channels_last_kernel)
+//   col    [b][m][k][c], row length R = K * Cgp (columns_kernel)
+//   W      [n][k][c] or [k][c][n]               (columns_weight_kernel)
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "conv_columns.hpp"
+#include "conv_product.hpp"
+#include "sdk_host.hpp"
+#include "sdk_mfma.hpp"
+#include "sdk_taps.hpp"
+
+namespace sdk {
+namespace {
+
+constexpr int kClThreads = 256;
+typedef float vec4 __attribute__((ext_vector_type(4)));
+
+int pad8(int c) { return (c + 7) & ~7; }
+
+// dst[b][n][c] = src[b][c][n], c padded to Cp8 with zeros.  grid (tiles of 64 n, tiles of 32 c,
+// batch): the tile goes through LDS, reads run along n, writes along c.
+__global__ __launch_bounds__(kClThreads) void channels_last_kernel(
+    const float* __restrict__ src, float* __restrict__ dst, int C, int Cp8, int N) {
+  __shared__ float tile[32][65];
+  const int n0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
+  const float* s = src + (size_t)blockIdx.z * C * N;
+  float* d = dst + (size_t)blockIdx.z * N * Cp8;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = c0 + w + 4 * i, n = n0 + lane;
+    tile[w + 4 * i][lane] = (c < C && n < N) ? s[(size_t)c * N + n] : 0.0f;
+  }
+  __syncthreads();
+  // 64 n x 8 channel quads
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int item = threadIdx.x + kClThreads * i;
+    const int n = item >> 3, q = item & 7;
+    if (n0 + n < N && c0 + 4 * q < Cp8) {
+      vec4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile[4 * q + e][n];
+      *reinterpret_cast<vec4*>(d + (size_t)(n0 + n) * Cp8 + c0 + 4 * q) = v;
+    }
+  }
+}
+
+// REDUCTION_N = false: W[n][k][c]; true: W[k][c][n].  c and n padded to multiples of eight.
+template <bool REDUCTION_N>
+__global__ __launch_bounds__(kClThreads) void columns_weight_kernel(
+    const float* __restrict__ Wm, float* __restrict__ dst, int Cg, int Cgp, int K, int Cp,
+    int Cpp, int total) {
+  const int e = blockIdx.x * kClThreads + threadIdx.x;
+  if (e >= total) return;
+  int n, k, c;
+  if constexpr (REDUCTION_N) {
+    n = e % Cpp;
+    const int q = e / Cpp;
+    c = q % Cgp;
+    k = q / Cgp;
+  } else {
+    c = e % Cgp;
+    const int q = e / Cgp;
+    k = q % K;
+    n = q / K;
+  }
+  dst[e] = (c < Cg && n < Cp) ? Wm[((size_t)n * Cg + c) * K + k] : 0.0f;
+}
+
+// col[b][m][k][:] = the blended image rows of sample (m, k).  A workgroup owns 64 consecutive
+// samples of one batch element: their taps are worked out once into LDS (zero-weight and
+// outside taps dropped), then a thread takes four channels of a sample.
+// SLOTS: most taps of a sample the LDS lists hold (the points of a weighted sample times four).
+constexpr int kClSamples = 64;
+template <int INTERP, bool WEIGHTED, int SLOTS>
+__global__ __launch_bounds__(kClThreads) void columns_kernel(
+    const float* __restrict__ rows, const float* __restrict__ map, const float* __restrict__ wts,
+    float* __restrict__ col, int samples, int P, int H, int W, int C4) {
+  __shared__ int s_n[kClSamples];
+  __shared__ int s_off[SLOTS][kClSamples];
+  __shared__ float s_co[SLOTS][kClSamples];
+  const int s0 = blockIdx.x * kClSamples;
+  if (threadIdx.x < kClSamples) {
+    const int s = s0 + threadIdx.x;
+    int n = 0;
+    if (s < samples) {
+      PointTaps<float, INTERP> t;
+      const int q = WEIGHTED ? P : 1;
+      for (int p = 0; p < q; ++p) {
+        const size_t at = (size_t)s * q + p;
+        t.set(map[2 * at], map[2 * at + 1], H, W);
+        const float wt = WEIGHTED ? wts[at] : 1.0f;
+#pragma unroll
+        for (int i = 0; i < PointTaps<float, INTERP>::N; ++i) {
+          const float c = WEIGHTED ? t.w[i] * wt : t.w[i];
+          if (t.off[i] >= 0 && c != 0.0f && n < SLOTS) {
+            s_off[n][threadIdx.x] = t.off[i];
+            s_co[n][threadIdx.x] = c;
+            ++n;
+          }
+        }
+      }
+    }
+    s_n[threadIdx.x] = n;
+  }
+  __syncthreads();
+  const vec4* r = reinterpret_cast<const vec4*>(rows) + (size_t)blockIdx.y * H * W * C4;
+  vec4* out = reinterpret_cast<vec4*>(col) + ((size_t)blockIdx.y * samples + s0) * C4;
+  const int items = min(kClSamples, samples - s0) * C4;
+  for (int it = threadIdx.x; it < items; it += kClThreads) {
+    const int s = it / C4, c = it - s * C4;
+    const int n = s_n[s];
+    vec4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n; i0 += 4) {
+      vec4 v[4];
+      float w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = min(i0 + i, n - 1);
+        w[i] = s_co[j][s];
+        v[i] = r[(size_t)s_off[j][s] * C4 + c];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i0 + i < n) acc += w[i] * v[i];
+    }
+    out[it] = acc;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The products.  A workgroup of four waves makes a (64 WM) x (64 WN) tile of C, each wave a
+// quarter of 32 WM x 32 WN; the reduction goes through LDS in steps of 32, double-buffered, the
+// values of the step after next requested from memory before the current step's MFMAs (a step
+// of a 64 x 64 tile is 0.1 to 0.4 us of matrix work, a read from beyond the L2 takes longer).  LDS rows hold 32
+// reduction elements and are 36 floats apart (16-byte reads of 32 consecutive rows then use
+// all banks evenly); a lane reads eight consecutive reduction elements of its row, which are a
+// bf16 operand once converted, or the operands of eight fp32 MFMAs (whose two reduction
+// indices may be any pair, as long as both operands agree).
+//   TN = false: C[i][n] = sum_r A[i][r] B[n][r] + bias[i]    (both operands run along r)
+//   TN = true:  C[i][n] = sum_r A[r][i] B[r][n], r in the split's range (a thread transposes
+//               4 x 4 blocks in registers on the way to LDS)
+// Leading dimensions and the reduction length (TN: the rows' lengths) are multiples of eight.
+// ---------------------------------------------------------------------------
+constexpr int kGk = 32;
+constexpr int kGld = 36;
+
+struct GemmArgs {
+  const float *A, *B;
+  float* C;
+  const float* bias;
+  int rows_a, rows_b;       // tiles past them read the last row and store nothing
+  int red;                  // reduction length
+  int lda, ldb;
+  size_t ldc;
+  size_t batch_b, batch_c;  // strides of grid.y (TN: batch_c of the split)
+  int split;                // TN: reduction elements of one split (grid.y)
+  int tiles_a, tiles_b;
+};
+
+template <int MM, int WM, int WN, bool TN>
+__global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
+  constexpr int BM = 64 * WM, BN = 64 * WN;
+  constexpr int LA = BM / 32, LB = BN / 32;   // 16-byte pieces per thread and step
+  __shared__ __attribute__((aligned(16))) float As[2][BM * kGld];
+  __shared__ __attribute__((aligned(16))) float Bs[2][BN * kGld];
+  __shared__ float s_bias[BM];
+  // consecutive slots of one XCD share the tile of the larger operand (workgroup ids go
+  // round-robin over the 8 XCDs)
+  const int total = g.tiles_a * g.tiles_b;
+  const int slot = (blockIdx.x & 7) * ((total + 7) / 8) + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= (total + 7) / 8 || slot >= total) return;
+  const int ta = slot % g.tiles_a, tb = slot / g.tiles_a;
+  const int i0 = ta * BM, n0 = tb * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 31, h = lane >> 5;
+  const int wr = (wave >> 1) * 32 * WM, wc = (wave & 1) * 32 * WN;
+  const float* B = TN ? g.B : g.B + (size_t)blockIdx.y * g.batch_b;
+  float* C = g.C + (size_t)blockIdx.y * g.batch_c;
+  const int r_begin = TN ? (int)blockIdx.y * g.split : 0;
+  const int r_end = TN ? min(r_begin + g.split, g.red) : g.red;
+
+  const int kb = tid & 7, rb = tid >> 3;   // reduction quad, row (TN: quad of columns)
+  vec4 ra[2][LA], rbv[2][LB];   // two steps in flight
+  const vec4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](int r0, vec4 (&ga)[LA], vec4 (&gb)[LB]) {
+    // (every read is made, from a clamped address, and what lies past the end becomes zero on
+    // the way to LDS: a test around a read costs a branch and a wait for it)
+    if constexpr (!TN) {
+      const int r = min(r0 + 4 * kb, g.red - 4);
+#pragma unroll
+      for (int i = 0; i < LA; ++i)
+        ga[i] = *reinterpret_cast<const vec4*>(g.A + (size_t)min(i0 + rb + 32 * i, g.rows_a - 1) * g.lda + r);
+#pragma unroll
+      for (int i = 0; i < LB; ++i)
+        gb[i] = *reinterpret_cast<const vec4*>(B + (size_t)min(n0 + rb + 32 * i, g.rows_b - 1) * g.ldb + r);
+    } else {
+      // blocks of four reduction rows x four columns: threads 0..127 take A's, the others B's
+      static_assert(!TN || (WM == 1 && WN == 1), "64 x 64 tiles only");
+      const bool is_a = tid < 128;
+      const int ld = is_a ? g.lda : g.ldb;
+      const float* src = (is_a ? g.A : B) + min((is_a ? i0 : n0) + 4 * (rb & 15), ld - 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const vec4 v = *reinterpret_cast<const vec4*>(src + (size_t)min(r0 + 4 * kb + e, g.red - 1) * ld);
+        if (e < 2) ga[e] = v;
+        else gb[e - 2] = v;
+      }
+    }
+  };
+  auto stash = [&](int buf, int r0, const vec4 (&ga)[LA], const vec4 (&gb)[LB]) {
+    if constexpr (!TN) {
+      const bool on = r0 + 4 * kb < r_end;
+#pragma unroll
+      for (int i = 0; i < LA; ++i)
+        *reinterpret_cast<vec4*>(&As[buf][(rb + 32 * i) * kGld + 4 * kb]) = on ? ga[i] : zero;
+#pragma unroll
+      for (int i = 0; i < LB; ++i)
+        *reinterpret_cast<vec4*>(&Bs[buf][(rb + 32 * i) * kGld + 4 * kb]) = on ? gb[i] : zero;
+    } else {
+      float* dst = (tid < 128 ? As[buf] : Bs[buf]) + 4 * (rb & 15) * kGld + 4 * kb;
+      const int r = r0 + 4 * kb;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const vec4 v = {r < r_end ? ga[0][e] : 0.0f, r + 1 < r_end ? ga[1][e] : 0.0f,
+                        r + 2 < r_end ? gb[0][e] : 0.0f, r + 3 < r_end ? gb[1][e] : 0.0f};
+        *reinterpret_cast<vec4*>(dst + e * kGld) = v;
+      }
+    }
+  };
+
+  for (int i = tid; i < BM; i += kClThreads)
+    s_bias[i] = !TN && g.bias != nullptr ? g.bias[min(i0 + i, g.rows_a - 1)] : 0.0f;
+
+  floatx16 acc[WM][WN];
+#pragma unroll
+  for (int a = 0; a < WM; ++a)
+#pragma unroll
+    for (int b = 0; b < WN; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+
+  auto load8 = [&](const float* p, float (&f)[8]) {
+    const vec4 lo = *reinterpret_cast<const vec4*>(p), hi = *reinterpret_cast<const vec4*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[e] = lo[e];
+      f[4 + e] = hi[e];
+    }
+  };
+
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < kGk / 16; ++s) {
+      float fa[WM][8], fb[WN][8];
+#pragma unroll
+      for (int a = 0; a < WM; ++a)
+        load8(&As[buf][(wr + 32 * a + j) * kGld + 16 * s + 8 * h], fa[a]);
+#pragma unroll
+      for (int b = 0; b < WN; ++b)
+        load8(&Bs[buf][(wc + 32 * b + j) * kGld + 16 * s + 8 * h], fb[b]);
+      if constexpr (MM == kMmF32) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int a = 0; a < WM; ++a)
+#pragma unroll
+            for (int b = 0; b < WN; ++b)
+              acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][e], fb[b][e], acc[a][b], 0, 0, 0);
+      } else if constexpr (MM == kMmBf16) {
+        Bf16Frag pa[WM], pb[WN];
+#pragma unroll
+        for (int a = 0; a < WM; ++a) pa[a] = pack_bf16x8(fa[a]);
+#pragma unroll
+        for (int b = 0; b < WN; ++b) pb[b] = pack_bf16x8(fb[b]);
+#pragma unroll
+        for (int a = 0; a < WM; ++a)
+#pragma unroll
+          for (int b = 0; b < WN; ++b) acc[a][b] = mfma_bf16(pa[a], pb[b], acc[a][b]);
+      } else {
+        Bf16Split pa[WM], pb[WN];
+#pragma unroll
+        for (int a = 0; a < WM; ++a) pa[a] = split_bf16x8(fa[a]);
+#pragma unroll
+        for (int b = 0; b < WN; ++b) pb[b] = split_bf16x8(fb[b]);
+#pragma unroll
+        for (int a = 0; a < WM; ++a)
+#pragma unroll
+          for (int b = 0; b < WN; ++b) acc[a][b] = mfma_split(pa[a], pb[b], acc[a][b]);
+      }
+    }
+  };
+
+  // step t: registers t & 1 hold its values until they go to LDS buffer t & 1, one step ahead
+  // of the MFMAs; step t + 2 is requested right after
+  const int steps = (r_end - r_begin + kGk - 1) / kGk;
+  fetch(r_begin, ra[0], rbv[0]);
+  fetch(r_begin + kGk, ra[1], rbv[1]);
+  stash(0, r_begin, ra[0], rbv[0]);
+  __syncthreads();
+  // (the scheduling barriers keep the requests in front of the MFMAs and the waits for older
+  // ones behind them; left alone the compiler sinks the requests to their uses)
+  for (int t = 0; t < steps; t += 2) {
+    const int r0 = r_begin + t * kGk;
+    fetch(r0 + 2 * kGk, ra[0], rbv[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    stash(1, r0 + kGk, ra[1], rbv[1]);
+    __syncthreads();
+    fetch(r0 + 3 * kGk, ra[1], rbv[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);   // (a step past the end multiplies zeros)
+    __builtin_amdgcn_sched_barrier(0);
+    stash(0, r0 + 2 * kGk, ra[0], rbv[0]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < WM; ++a)
+#pragma unroll
+    for (int b = 0; b < WN; ++b) {
+      const int n = n0 + wc + 32 * b + j;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int i = i0 + wr + 32 * a + 8 * (v >> 2) + 4 * h + (v & 3);
+        if (i < g.rows_a && n < g.rows_b)
+          C[(size_t)i * g.ldc + n] = acc[a][b][v] + s_bias[i - i0];
+      }
+    }
+}
+
+// gW[i][c][k] = sum over the splits of partial[split][i][k][c].
+__global__ __launch_bounds__(kClThreads) void columns_wgrad_sum_kernel(
+    const float* __restrict__ partial, float* __restrict__ gW, int splits, size_t split_stride,
+    int Cg, int Cgp, int K, int total) {
+  const int e = blockIdx.x * kClThreads + threadIdx.x;   // (i, k, c), c fastest
+  if (e >= total) return;
+  const int c = e % Cgp, q = e / Cgp, k = q % K, i = q / K;
+  if (c >= Cg) return;
+  float sum = 0.f;
+  for (int s = 0; s < splits; s += 8) {
+    float v[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) v[x] = partial[(size_t)min(s + x, splits - 1) * split_stride + e];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) sum += s + x < splits ? v[x] : 0.0f;
+  }
+  gW[((size_t)i * Cg + c) * K + k] = sum;
+}
+
+// img[b][c][u] = bias[c] + sum over the entries of u's list of coefficient * col[b][sample][c].
+// A workgroup owns 16 image elements x 64 channels of one batch element, a thread one element
+// and four channels: the 16 lanes of an element read an entry's 64 products as one run, four
+// entries in flight, and the sums leave through LDS as runs along the image.  grid (blocks of 16
+// elements, channel chunks, batch).
+constexpr int kClTargets = 16;
+__global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
+    const float* __restrict__ col, const int* __restrict__ offset, const int* __restrict__ src,
+    const float* __restrict__ co, const float* __restrict__ bias, float* __restrict__ img, int Cg,
+    int C4, int HW, int samples) {
+  __shared__ float tile[64][kClTargets + 1];
+  const int q = threadIdx.x & 15, t = threadIdx.x >> 4;
+  const int u0 = blockIdx.x * kClTargets, c0 = blockIdx.y * 64;
+  const vec4* col_b = reinterpret_cast<const vec4*>(col) + (size_t)blockIdx.z * samples * C4 +
+                      min(c0 / 4 + q, C4 - 1);
+  const int u = min(u0 + t, HW - 1);
+  const int beg = offset[u], end = offset[u + 1];
+  vec4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int e = beg; e < end; e += 8) {
+    vec4 v[8];
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at = min(e + i, end - 1);
+      w[i] = co[at];
+      v[i] = col_b[(size_t)src[at] * C4];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (e + i < end) acc += w[i] * v[i];
+  }
+#pragma unroll
+  for (int x = 0; x < 4; ++x) tile[4 * q + x][t] = acc[x];
+  __syncthreads();
+  float* img_b = img + (size_t)blockIdx.z * Cg * HW;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = (threadIdx.x >> 4) + 16 * i, n = threadIdx.x & 15;
+    if (c0 + c < Cg && u0 + n < HW)
+      img_b[(size_t)(c0 + c) * HW + u0 + n] = tile[c][n] + (bias != nullptr ? bias[c0 + c] : 0.0f);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Host side
+// ---------------------------------------------------------------------------
+size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+struct ColumnsLayout {
+  size_t pix_rows, img_rows, col, weights, partial, lists, total;
+  int splits, split_len;
+};
+
+size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(g.Cg); }
+
+ColumnsLayout columns_layout(const ConvGeom& g) {
+  const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp);
+  ColumnsLayout l;
+  size_t at = 0;
+  auto take = [&](size_t values) {
+    const size_t here = at;
+    at += up256(values * sizeof(float));
+    return here;
+  };
+  l.pix_rows = take((size_t)g.B * g.M * Cpp);
+  l.img_rows = take((size_t)g.B * g.H * g.W * Cgp);
+  l.col = take(column_values(g));
+  l.weights = take((size_t)g.K * Cgp * Cpp);
+  // the weight gradient's reduction (all pixels of the batch) in splits: about two
+  // workgroups per CU, at least 64 pixels each
+  const int64_t tiles = ceil_div(g.Cp, 64) * ceil_div((int64_t)g.K * Cgp, 64);
+  const int64_t pixels = g.B * (int64_t)g.M;
+  int64_t splits = std::max<int64_t>(1, std::min<int64_t>(ceil_div(512, tiles), ceil_div(pixels, 64)));
+  l.split_len = (int)(ceil_div(ceil_div(pixels, splits), kGk) * kGk);
+  l.splits = (int)ceil_div(pixels, l.split_len);
+  l.partial = take((size_t)l.splits * g.Cp * g.K * Cgp);
+  l.lists = at;
+  l.total = at + up256(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp));
+  return l;
+}
+
+int to_rows(const float* src, float* dst, int64_t B, int C, int64_t N, hipStream_t stream) {
+  const dim3 grid((unsigned)ceil_div(N, 64), (unsigned)ceil_div(pad8(C), 32), (unsigned)B);
+  launch(channels_last_kernel, grid, dim3(kClThreads), stream, src, dst, C, pad8(C), (int)N);
+  SDK_LAUNCH_CHECK("mapped_conv(channels last)");
+  return SDK_OK;
+}
+
+int make_columns(const ConvGeom& g, const float* rows, const float* map, const float* wts,
+                 float* col, hipStream_t stream) {
+  const int samples = g.M * g.K;
+  const dim3 grid((unsigned)ceil_div(samples, kClSamples), (unsigned)g.B);
+  const int C4 = pad8(g.Cg) / 4;
+  SDK_DISPATCH_INTERP(g.interp, g.P,
+                      (launch((columns_kernel<INTERP, WEIGHTED, WEIGHTED ? 32 : 4>), grid,
+                              dim3(kClThreads), stream, rows, map, wts, col, samples, g.P, g.H,
+                              g.W, C4)));
+  SDK_LAUNCH_CHECK("mapped_conv(columns)");
+  return SDK_OK;
+}
+
+template <bool TN>
+int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
+  a.tiles_a = (int)ceil_div(a.rows_a, 64);
+  a.tiles_b = (int)ceil_div(a.rows_b, 64);
+  const int64_t total = (int64_t)a.tiles_a * a.tiles_b;
+  const dim3 grid((unsigned)((total + 7) / 8 * 8), (unsigned)batches);
+  if (mm == kMmBf16)
+    launch((columns_gemm_kernel<kMmBf16, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
+  else if (mm == kMmSplit)
+    launch((columns_gemm_kernel<kMmSplit, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
+  else
+    launch((columns_gemm_kernel<kMmF32, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
+  SDK_LAUNCH_CHECK("mapped_conv(columns product)");
+  return SDK_OK;
+}
+
+// Column matrices of at most this many bytes take the route.  Measured against the fused kernels,
+// forward + backward of one layer on a kept plan, 3 x 3 kernels (before -> columns):
+//   25 MB  6 x 50 x 100, stride 2, 96 -> 160, split   899 -> 190 us
+//   36 MB  2 x 64 x 128, 64 -> 64, float32            327 -> 160 us
+//   72 MB  1 x 128 x 256, 64 -> 64, float32 / bf16    347 -> 235 / 271 -> 195 us
+//   84 MB  3 x 45 x 91, 200 -> 37, split              570 -> 275 us
+//  144 MB  8 x 64 x 128, 64 -> 128, float32 / bf16    621 -> 585 / 396 -> 470 us: no gain left, the
+//          tiles fill the GPU by then
+// Nearest taps cost the fused kernels least, their line lies lower: 4 x 128 x 256, 32 -> 32
+// (144 MB) 250 -> 380 us.
+constexpr size_t kColumnsBytes = (size_t)100 << 20, kColumnsNearestBytes = (size_t)36 << 20;
+size_t column_limit(const ConvGeom& g) {
+  return g.interp == 0 && g.P == 0 ? kColumnsNearestBytes : kColumnsBytes;
+}
+
+thread_local bool t_columns = true;
+
+}  // namespace
+
+bool columns_map(const ConvGeom& g) {
+  return g.M >= 1 && g.K >= 1 && (int64_t)g.M * g.K <= ((int64_t)1 << 20) && pts(g.P) <= 8 &&
+         col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp) != 0;
+}
+
+bool columns_route(const ConvGeom& g) {
+  const size_t limit = column_limit(g);
+  return t_columns && g.B >= 1 && g.B <= 65535 && g.Cg >= 5 && columns_map(g) &&
+         column_values(g) * sizeof(float) <= limit &&
+         (size_t)g.B * g.H * g.W * pad8(g.Cg) * sizeof(float) <= 2 * limit &&
+         (size_t)g.B * g.M * pad8(g.Cp) * sizeof(float) <= 2 * limit &&
+         (size_t)pad8(g.Cp) * g.K * pad8(g.Cg) < ((size_t)1 << 31);
+}
+
+size_t columns_workspace_bytes(const ConvGeom& g) {
+  return columns_route(g) ? columns_layout(g).total : 0;
+}
+
+int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float* map,
+                        const float* wts, const float* Wm, const float* bias, float* pix,
+                        void* workspace, hipStream_t stream) {
+  const ColumnsLayout l = columns_layout(g);
+  char* ws = static_cast<char*>(workspace);
+  float* rows = reinterpret_cast<float*>(ws + l.img_rows);
+  float* col = reinterpret_cast<float*>(ws + l.col);
+  float* w = reinterpret_cast<float*>(ws + l.weights);
+  const int Cgp = pad8(g.Cg), R = g.K * Cgp;
+  int rc = to_rows(img, rows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
+  if (rc) return rc;
+  rc = make_columns(g, rows, map, wts, col, stream);
+  if (rc) return rc;
+  const int total = g.Cp * R;
+  launch(columns_weight_kernel<false>, dim3((unsigned)ceil_div(total, kClThreads)),
+         dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, g.Cp, total);
+  SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
+  GemmArgs a{};
+  a.A = w;
+  a.B = col;
+  a.C = pix;
+  a.bias = bias;
+  a.rows_a = g.Cp;
+  a.rows_b = g.M;
+  a.red = R;
+  a.lda = a.ldb = R;
+  a.ldc = (size_t)g.M;
+  a.batch_b = (size_t)g.M * R;
+  a.batch_c = (size_t)g.Cp * g.M;
+  return gemm<false>(mm, a, g.B, stream);
+}
+
+int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const float* map,
+                         const float* wts, const float* Wm, const float* bias, float* img,
+                         void* workspace, hipStream_t stream, const void* lists) {
+  const ColumnsLayout l = columns_layout(g);
+  char* ws = static_cast<char*>(workspace);
+  float* rows = reinterpret_cast<float*>(ws + l.pix_rows);
+  float* col = reinterpret_cast<float*>(ws + l.col);
+  float* w = reinterpret_cast<float*>(ws + l.weights);
+  const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp), R = g.K * Cgp;
+  int rc = SDK_OK;
+  if (lists == nullptr) {
+    rc = col2im_lists_build(map, wts, ws + l.lists, g.H, g.W, g.M, g.K, g.P, g.interp, stream);
+    if (rc) return rc;
+    lists = ws + l.lists;
+  }
+  rc = to_rows(pix, rows, g.B, g.Cp, g.M, stream);
+  if (rc) return rc;
+  const int total = R * Cpp;
+  launch(columns_weight_kernel<true>, dim3((unsigned)ceil_div(total, kClThreads)),
+         dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, Cpp, total);
+  SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
+  // all pixels of the batch are the rows of one product
+  GemmArgs a{};
+  a.A = rows;
+  a.B = w;
+  a.C = col;
+  a.rows_a = (int)(g.B * g.M);
+  a.rows_b = R;
+  a.red = Cpp;
+  a.lda = a.ldb = Cpp;
+  a.ldc = (size_t)R;
+  rc = gemm<false>(mm, a, 1, stream);
+  if (rc) return rc;
+  const Col2imView v = col2im_lists_view(lists, g.H, g.W, g.M, g.K, g.P, g.interp);
+  const int HW = g.H * g.W;
+  launch(columns_col2im_kernel,
+         dim3((unsigned)ceil_div(HW, kClTargets), (unsigned)ceil_div(g.Cg, 64), (unsigned)g.B),
+         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, img, g.Cg,
+         Cgp / 4, HW, g.M * g.K);
+  SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
+  return SDK_OK;
+}
+
+int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
+                         const float* wts, const float* img, float* gW, void* workspace,
+                         hipStream_t stream, bool pix_ready) {
+  const ColumnsLayout l = columns_layout(g);
+  char* ws = static_cast<char*>(workspace);
+  float* prows = reinterpret_cast<float*>(ws + l.pix_rows);
+  float* irows = reinterpret_cast<float*>(ws + l.img_rows);
+  float* col = reinterpret_cast<float*>(ws + l.col);
+  float* partial = reinterpret_cast<float*>(ws + l.partial);
+  const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp), R = g.K * Cgp;
+  int rc = SDK_OK;
+  if (!pix_ready) rc = to_rows(pix, prows, g.B, g.Cp, g.M, stream);
+  if (rc) return rc;
+  rc = to_rows(img, irows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
+  if (rc) return rc;
+  rc = make_columns(g, irows, map, wts, col, stream);
+  if (rc) return rc;
+  GemmArgs a{};
+  a.A = prows;
+  a.B = col;
+  a.C = partial;
+  a.rows_a = g.Cp;
+  a.rows_b = R;
+  a.red = (int)(g.B * g.M);
+  a.lda = Cpp;
+  a.ldb = R;
+  a.ldc = (size_t)R;
+  a.batch_c = (size_t)g.Cp * R;
+  a.split = l.split_len;
+  rc = gemm<true>(mm, a, l.splits, stream);
+  if (rc) return rc;
+  const int total = g.Cp * R;
+  launch(columns_wgrad_sum_kernel, dim3((unsigned)ceil_div(total, kClThreads)), dim3(kClThreads),
+         stream, (const float*)partial, gW, l.splits, a.batch_c, g.Cg, Cgp, g.K, total);
+  SDK_LAUNCH_CHECK("mapped_conv(columns sums)");
+  return SDK_OK;
+}
+
+}  // namespace sdk
+
+extern "C" int sdk_mapped_conv_columns_enable(int32_t enabled) {
+  const int before = sdk::t_columns ? 1 : 0;
+  sdk::t_columns = enabled != 0;
+  return before;
+}

@@ -25,6 +25,7 @@
 // MFMA 32x32x2 f32 register layout used below (wave64, lane l):
 //   A operand: A[i = l % 32][k = l / 32]        B operand: B[k = l / 32][j = l % 32]
 //   D, 16 registers v: D[i = 8*(v/4) + 4*(l/32) + v%4][j = l % 32]
+#include "conv_columns.hpp"
 #include "conv_fused.hpp"
 #include "conv_small.hpp"
 #include "conv_product.hpp"
@@ -693,6 +694,10 @@ bool fused_supported(const ConvGeom& g) {
   return true;
 }
 
+bool columns_first(const ConvGeom& g) {
+  return !small_conv_supported(g) && !product_route(g) && columns_route(g);
+}
+
 static bool inverse_candidate(const ConvGeom& g);
 static size_t inverse_bytes(const ConvGeom& g);
 static bool scatter_tries_inverse(const ConvGeom& g);
@@ -729,6 +734,8 @@ static GatherLayout gather_layout(const ConvGeom& g) {
 static bool gather_from_window(const ConvGeom& g) { return window_gemm_supported(g); }
 
 size_t fused_workspace_bytes(const ConvGeom& g) {
+  if (columns_first(g))
+    return columns_workspace_bytes(g);
   const int CpP = round_up(g.Cp, 128), CgP = round_up(g.Cg, 128);
   size_t need = std::max((size_t)g.K * CpP * CgP * sizeof(float), staged_workspace_bytes(g));
   if (gather_from_window(g)) need = std::max(need, gather_layout(g).total);
@@ -848,6 +855,8 @@ int fused_gather_gemm(const ConvGeom& g, int compute, const float* img, const fl
   // images of a few channels: the packed kernel (a 32-channel chunk would be mostly padding)
   if (small_conv_supported(g)) return small_forward(g, img, map, wts, Wm, bias, pix, stream);
   const int mm = matrix_mode(compute);
+  if (columns_first(g))
+    return columns_gather_gemm(g, mm, img, map, wts, Wm, bias, pix, workspace, stream);
   const int slots = slots_for(g);
   const bool narrow = g.Cp <= 64;
   const int TN = narrow ? 64 : 128, TM = narrow ? 256 : 128;
@@ -1158,6 +1167,14 @@ int fused_gemm_scatter(const ConvGeom& g, int compute, const float* pix, const f
     return product_gemm_scatter(g, pix, map, wts, Wm, bias, img, workspace, stream,
                                 cached != nullptr ? cached->col2im_lists : nullptr);
   }
+  if (columns_first(g)) {
+    if (shared != nullptr) {
+      shared->valid = false;
+      shared->pix_rows = true;
+    }
+    return columns_gemm_scatter(g, matrix_mode(compute), pix, map, wts, Wm, bias, img, workspace,
+                                stream, cached != nullptr ? cached->col2im_lists : nullptr);
+  }
   const bool planned_fb = planned_scatter_supported(g);
   const int* generic_gate = nullptr;   // gate of the atomic scatter kernel at the end
   bool filled = false;
@@ -1290,6 +1307,9 @@ int fused_gather_wgrad(const ConvGeom& g, int compute, const float* pix, const f
                        const float* wts, const float* img, float* gW, float* workspace,
                        hipStream_t stream, const SharedPlan* shared, const CachedPlan* cached) {
   const bool bf16 = compute == SDK_COMPUTE_BF16;
+  if (g.B > 0 && !small_wgrad_supported(g) && columns_first(g))
+    return columns_gather_wgrad(g, matrix_mode(compute), pix, map, wts, img, gW, workspace, stream,
+                                shared != nullptr && shared->pix_rows);
   const bool cleared = shared != nullptr && shared->cleared && small_wgrad_supported(g);
   int rc = cleared ? SDK_OK : zero_fill(gW, sizeof(float) * (size_t)g.Cp * g.Cg * g.K, stream);
   if (rc) return rc;
@@ -1356,8 +1376,8 @@ CachedLayout cached_layout(const ConvGeom& g) {
                   (int64_t)g.H * g.W * g.K < ((int64_t)1 << 31);
   l.inverse_lists = l.inverse + (l.has_inverse ? up(inverse_plan_bytes(g)) : 0);
   l.col2im = l.inverse_lists + (l.has_inverse ? up(tile_lists_bytes(inverse_geom(g))) : 0);
-  // the inverted map of the product route (conv_product.hpp), where the map may take it
-  l.has_col2im = product_route_map(g);
+  // the inverted map of the product and columns routes, where the map may take one of them
+  l.has_col2im = product_route_map(g) || columns_map(g);
   l.total = l.col2im + (l.has_col2im ? up(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp)) : 0);
   return l;
 }
@@ -1405,6 +1425,14 @@ int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, voi
     if (rc) return rc;
   }
   return SDK_OK;
+}
+
+int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
+                              hipStream_t stream) {
+  const CachedLayout l = cached_layout(g);
+  if (!l.has_col2im) return SDK_OK;
+  return col2im_lists_build(map, wts, static_cast<char*>(buffer) + l.col2im, g.H, g.W, g.M, g.K,
+                            g.P, g.interp, stream);
 }
 
 }  // namespace sdk

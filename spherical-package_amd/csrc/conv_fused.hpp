@@ -18,6 +18,8 @@ struct SharedPlan {
   // ... and wants the bias gradient (the sum of the weight gradient's pixel-side operand over
   // batch and pixels) from the weight-gradient kernel, into this cleared buffer.
   float* bias_sum = nullptr;
+  // The workspace holds the channels-last pixel-side tensor the columns route's scatter left.
+  bool pix_rows = false;
 };
 
 // Everything the fused kernels derive from the sample map alone, built once into a
@@ -29,14 +31,20 @@ struct CachedPlan {
   bool has_inverse = false;
   InversePlan inverse;
   TileLists inverse_lists;
-  const void* col2im_lists = nullptr;   // the inverted map of the product route, where kept
+  const void* col2im_lists = nullptr;   // the inverted map of the product and columns routes, where kept
 };
 // g: only H, W, M, OW, K, P and interp matter.  0 bytes: no plan for this geometry.
 size_t cached_plan_bytes(const ConvGeom& g);
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                       hipStream_t stream);
+// The part of the same buffer that calls of the columns route (conv_columns.hpp) read.
+int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
+                              hipStream_t stream);
 // Pointers into a buffer build_cached_plan filled for the same geometry.
 void load_cached_plan(const ConvGeom& g, void* buffer, CachedPlan* out);
+
+// Calls every contraction of which runs as columns and products (conv_columns.hpp).
+bool columns_first(const ConvGeom& g);
 
 // True when the fused kernels cover this geometry.
 bool fused_supported(const ConvGeom& g);

@@ -30,6 +30,12 @@ int product_gemm_scatter(const ConvGeom& g, const float* pix, const float* map, 
 size_t col2im_lists_bytes(int H, int W, int M, int K, int P, int interp);   // 0: too large
 int col2im_lists_build(const float* map, const float* wts, void* lists, int H, int W, int M,
                        int K, int P, int interp, hipStream_t stream);
+// The entries of image element u: (src[e], co[e]) for offset[u] <= e < offset[u + 1].
+struct Col2imView {
+  const int *offset, *src;
+  const float* co;
+};
+Col2imView col2im_lists_view(const void* lists, int H, int W, int M, int K, int P, int interp);
 int col2im_from_lists(const float* col, const float* bias, float* img, const void* lists,
                       int64_t planes, int channels, int H, int W, int M, int K, int P, int interp,
                       hipStream_t stream);

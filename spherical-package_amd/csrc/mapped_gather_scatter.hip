@@ -2081,6 +2081,11 @@ size_t col2im_lists_bytes(int H, int W, int M, int K, int P, int interp) {
   return col2im_lists_at(nullptr, H, W, M, K, P, interp).bytes;
 }
 
+Col2imView col2im_lists_view(const void* lists, int H, int W, int M, int K, int P, int interp) {
+  const Col2imLists l = col2im_lists_at(const_cast<void*>(lists), H, W, M, K, P, interp);
+  return Col2imView{l.offset, l.src, l.co};
+}
+
 int col2im_lists_build(const float* map, const float* wts, void* lists, int H, int W, int M,
                        int K, int P, int interp, hipStream_t stream) {
   const Col2imLists l = col2im_lists_at(lists, H, W, M, K, P, interp);

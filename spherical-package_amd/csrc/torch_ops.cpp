@@ -66,7 +66,7 @@ bool tensor_key(const OptTensor& t, TensorKey* k) {
   return true;
 }
 
-enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3 };
+enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kConvColumns = 4 };
 
 struct Key {
   int kind = 0, device = 0, dtype = 0;
@@ -85,6 +85,7 @@ struct Entry {
   c10::Storage keep_map, keep_wts;   // an address cannot be reused while its entry lives
   hipStream_t stream = nullptr;      // last user: a call on another stream is ordered behind it
   int complete = 0;
+  bool built = false;   // false: the buffer is there, nothing has needed its contents yet
 };
 std::list<Entry> g_cache;   // most recently used last
 
@@ -170,10 +171,11 @@ Tensor bytes_on(const Tensor& ref, size_t n) {
 }
 
 // The kept plan of `key`, or one built by `build` (which returns the plan's size, 0 for none,
-// and fills the buffer it is handed on `stream`).
+// and fills the buffer it is handed on `stream`).  needed: false for a call that reads nothing of
+// the plan; its entry is made, and filled by the first call that does.
 template <typename Size, typename Build>
 PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor& wts,
-                 hipStream_t stream, Size size, Build build) {
+                 hipStream_t stream, Size size, Build build, bool needed = true) {
   PlanRef out;
   if (!g_cache_enabled) return out;
   if (!tensor_key(map, &key.map) || !tensor_key(wts, &key.wts)) return out;
@@ -182,8 +184,13 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
     if (it->key == key) {
       g_cache.splice(g_cache.end(), g_cache, it);   // most recently used
       Entry& e = g_cache.back();
+      if (!e.built && (!needed || capturing(stream))) return out;
       order_behind(stream, e.stream);
       e.stream = stream;
+      if (!e.built) {
+        e.complete = build(e.plan.data_ptr(), e.nbytes);
+        e.built = true;
+      }
       out.plan = e.plan;
       out.nbytes = e.nbytes;
       out.complete = e.complete;
@@ -197,24 +204,37 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
   e.key = key;
   e.plan = bytes_on(ref, n);
   e.nbytes = n;
-  e.complete = build(e.plan.data_ptr(), n);
+  if (needed) e.complete = build(e.plan.data_ptr(), n);
+  e.built = needed;
   e.keep_map = map.storage();
   if (wts.has_value() && wts->defined()) e.keep_wts = wts->storage();
   e.stream = stream;
   while (g_cache.size() >= g_cache_max) g_cache.pop_front();
   g_cache.push_back(std::move(e));
+  if (!needed) return out;
   out.plan = g_cache.back().plan;
   out.nbytes = n;
   out.complete = g_cache.back().complete;
   return out;
 }
 
-PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, int64_t img_h,
-                  int64_t img_w, int64_t K, int64_t P, int64_t interp, hipStream_t stream) {
+struct ConvDims {
+  int64_t B, Cin, Cout, K;
+};
+
+// The plan of a (transposed) convolution call.  scatter: the call splats into the image (the
+// backward of a convolution, the forward of a transposed one); of the calls that run as columns
+// and products only those read a plan, and only the part with the inverted map.
+PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, const ConvDims& d,
+                  int64_t img_h, int64_t img_w, int64_t P, int64_t interp, bool transposed,
+                  bool scatter, hipStream_t stream) {
   if (ref.scalar_type() != at::kFloat) return PlanRef();
-  const int64_t MH = map.size(0), MW = map.size(1);
+  const int64_t MH = map.size(0), MW = map.size(1), K = d.K;
+  const bool columns =
+      sdk_mapped_conv_by_columns(d.B, d.Cin, d.Cout, img_h, img_w, MH, MW, K, (int32_t)P,
+                                 (int32_t)interp, SDK_F32, current_mode(), transposed ? 1 : 0) == 1;
   Key key;
-  key.kind = kConv;
+  key.kind = columns ? kConvColumns : kConv;
   key.device = ref.device().index();
   key.a = img_h;
   key.b = img_w;
@@ -225,10 +245,15 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, in
       key, ref, map, wts, stream,
       [&] { return sdk_mapped_conv_plan_bytes(img_h, img_w, MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32); },
       [&](void* buf, size_t n) {
-        SDK_CALL(sdk_mapped_conv_plan_build, map.data_ptr(), cptr(wts), buf, n, img_h, img_w, MH,
-                 MW, K, (int32_t)P, (int32_t)interp, SDK_F32, stream);
+        if (columns)
+          SDK_CALL(sdk_mapped_conv_plan_build_columns, map.data_ptr(), cptr(wts), buf, n, img_h,
+                   img_w, MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32, stream);
+        else
+          SDK_CALL(sdk_mapped_conv_plan_build, map.data_ptr(), cptr(wts), buf, n, img_h, img_w, MH,
+                   MW, K, (int32_t)P, (int32_t)interp, SDK_F32, stream);
         return 0;
-      });
+      },
+      !columns || scatter);
 }
 
 PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptTensor& wts,
@@ -455,9 +480,6 @@ Tensor mapped_avg_unpool(const Tensor& g, const Tensor& map, const OptTensor& wt
 }
 
 // ----------------------------------------------------------------------------- convolution
-struct ConvDims {
-  int64_t B, Cin, Cout, K;
-};
 ConvDims conv_dims(const Tensor& x, const Tensor& weight, const Tensor& map, int64_t kernel_size,
                    bool transposed) {
   TORCH_CHECK(x.dim() == 4 && weight.dim() == 3 && map.dim() >= 4, "bad tensor ranks");
@@ -498,7 +520,7 @@ Tensor mapped_conv_forward(const Tensor& x, const Tensor& map, const OptTensor& 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, H, W, d.K, P, interp, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -536,7 +558,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward(const Tensor& grad_outpu
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, H, W, d.K, P, interp, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -570,7 +592,7 @@ Tensor mapped_transposed_conv_forward(const Tensor& x, const Tensor& map, const 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, out_h, out_w, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, out_h, out_w, d.K, P, interp, s);
+  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -606,7 +628,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_transposed_conv_backward(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, OH, OW, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, OH, OW, d.K, P, interp, s);
+  PlanRef plan = conv_plan(x, map, wts, d, OH, OW, P, interp, true, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -648,7 +670,8 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward_select(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, img_h, img_w, map.size(0), map.size(1), P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, img_h, img_w, d.K, P, interp, s);
+  PlanRef plan = conv_plan(x, map, wts, d, img_h, img_w, P, interp, transposed,
+                           !transposed && need_input, s);
   const auto ptr = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
   const auto call = transposed ? sdk_mapped_transposed_conv_backward_select
                                : sdk_mapped_conv_backward_select;

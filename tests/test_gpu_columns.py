@@ -1,0 +1,132 @@
+"""Small convolution calls as columns and matrix products (csrc/conv_columns.hip) against the
+oracle in float64 accumulation, and the tile kernels at the same sizes.
+
+The tile kernels are reached at small sizes by turning the route off for the thread
+(sdk_mapped_conv_columns_enable); the plan tests then run on them.
+"""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_conv_plans as plans
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import _spherical_distortion_ext._ops as o
+    return o
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from oracle import oracle as o
+    return o
+
+
+@pytest.fixture
+def tile_kernels(ops):
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    before = lib.sdk_mapped_conv_columns_enable(0)
+    yield
+    lib.sdk_mapped_conv_columns_enable(before)
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", plans.CASES, ids=lambda t: "x".join(map(str, t)))
+def test_tile_kernels_at_small_sizes(ops, oracle, tile_kernels, tc, mode):
+    plans.test_planned_calls_match_plain_calls_and_the_oracle(ops, oracle, tc, mode)
+
+
+# (batch, Cin, Cout, H, W, OH, OW, K, P, interp): one tile and one over its edges (64 x 64 tiles,
+# reduction steps of 32, splits of the pixels), widths that are no multiple of eight, one pixel,
+# one sample, the most points a weighted sample may have on the route
+SIZES = [
+    (1, 5, 1, 1, 1, 1, 1, 1, 0, 0),
+    (1, 8, 64, 8, 8, 8, 8, 4, 0, 1),
+    (2, 9, 65, 9, 15, 5, 13, 9, 0, 1),
+    (1, 64, 7, 16, 20, 8, 8, 1, 0, 2),
+    (3, 33, 40, 12, 25, 6, 11, 25, 0, 1),
+    (2, 7, 130, 10, 18, 13, 20, 9, 0, 2),
+    (1, 12, 17, 10, 14, 10, 14, 3, 8, 1),
+    (2, 16, 24, 11, 13, 9, 10, 7, 2, 0),
+    (5, 40, 72, 20, 31, 10, 16, 9, 0, 0),
+]
+
+
+def _arrays(tc):
+    B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
+    rng = np.random.default_rng(sum(tc))
+    shape = (OH, OW, K) + ((P,) if P else ())
+    ys = rng.uniform(-2, H + 1, shape)      # some samples outside the image
+    xs = rng.uniform(-2, W + 1, shape)
+    ys[0, 0, 0], xs[0, 0, 0] = -9, -9       # ... one with no tap in it
+    m = np.stack([xs, ys], -1).astype(np.float32)
+    iw = rng.uniform(0.1, 1, shape).astype(np.float32) if P else None
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    return (m, iw, f(B, Cin, H, W), f(Cout, Cin, K), f(Cout), f(B, Cout, OH, OW), f(Cin))
+
+
+def _rel(a, b):
+    d = np.linalg.norm(np.asarray(a, np.float64) - b)
+    return d / max(np.linalg.norm(np.asarray(b, np.float64)), 1e-30)
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
+def test_columns_route_matches_the_oracle(ops, oracle, tc, mode):
+    from _spherical_distortion_ext import _capi
+    B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
+    for transposed in (0, 1) if Cout >= 5 else (0,):   # (nearest up-sampling layers: products)
+        taken = _capi.load().sdk_mapped_conv_by_columns(
+            B, Cout if transposed else Cin, Cin if transposed else Cout, H, W, OH, OW, K, P,
+            interp, _capi.SDK_F32, 0, transposed)
+        assert taken == 1 or (interp == 0 and P == 0)
+    m, iw, x, w, b, g, bt = _arrays(tc)
+    t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(t(x), t(m), t(iw), t(w), t(b), K, interp)
+        gi, gw, gb = ops.ops.mapped_conv_backward(t(g), t(m), t(iw), t(x), t(w), t(b), K, interp)
+        yt = ops.ops.mapped_transposed_conv_forward(t(g), t(m), t(iw), t(w), t(bt), H, W, K, interp)
+    # float32: sums of at most Cin * K (or pixels) terms, random signs: eps * sqrt(n) < 5e-6;
+    # bf16 operands: 2^-9 each, so 2^-8 of the norm at most
+    tol = 4e-3 if mode == "bf16" else 5e-6
+    assert _rel(y.cpu().numpy(), oracle.mapped_conv_forward(x, m, w, b, K, interp, iw)) <= tol
+    wi, ww, wb = oracle.mapped_conv_backward(g, m, x, w, b, K, interp, iw)
+    for have, want in ((gi, wi), (gw, ww), (gb, wb)):
+        assert _rel(have.cpu().numpy(), want) <= tol
+    want = oracle.mapped_transposed_conv_forward(g, m, w, bt, H, W, K, interp, iw)
+    assert _rel(yt.cpu().numpy(), want) <= tol
+
+
+def test_the_inverted_map_is_built_by_the_first_backward(ops):
+    """A forward makes the map's cache entry and builds nothing; results do not depend on which
+    call comes first, and a replayed capture whose entry is not built gives the eager result."""
+    m, iw, x, w, b, g, _ = _arrays((2, 16, 24, 11, 13, 9, 10, 9, 0, 1))
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    tx, tw, tb, tg, K = t(x), t(w), t(b), t(g), 9
+    args = lambda tm: (tg, tm, None, tx, tw, tb, K, 1)  # noqa: E731
+    want = [o.cpu() for o in ops.ops.mapped_conv_backward(*args(t(m)))]
+    tm = t(m)
+    before = ops.plan_cache_size()
+    ops.ops.mapped_conv_forward(tx, tm, None, tw, tb, K, 1)
+    after = ops.plan_cache_size()
+    assert after - before in (0, 1)        # (0: the cache was full and dropped another)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        outs = [torch.empty_like(o, device=DEV) for o in want]
+        with torch.cuda.graph(graph, stream=side):
+            for o, r in zip(outs, ops.ops.mapped_conv_backward(*args(tm))):
+                o.copy_(r)
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = ops.ops.mapped_conv_backward(*args(tm))
+        for o, e, r in zip(outs, eager, want):
+            assert torch.equal(o.cpu(), r) and torch.equal(e.cpu(), r)
