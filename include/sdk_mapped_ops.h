@@ -715,6 +715,26 @@ int sdk_mapped_avg_unpool_planned(const void* grad_output, const void* sample_ma
                                   int64_t out_height, int64_t out_width, int64_t kernel_size,
                                   int32_t num_interp_pts, int32_t interp, int32_t dtype,
                                   sdk_stream_t stream);
+/* Average unpooling of blended or weighted samples (float32) as a gather: per image element the
+ * pooled pixels that sample it, with the sum of their coefficients, built once per map into
+ * caller-owned memory of sdk_mapped_avg_unpool_lists_bytes (0: no lists for this geometry, use
+ * the entry points above), 256-byte aligned, only read by sdk_mapped_avg_unpool_from_lists.
+ * Sums in a fixed order, no atomics, and no map whose shape it cannot take.  (Adjoint of
+ * ext_modules/include/common/mapped_avg_pool.h:42-68, :107-140.) */
+size_t sdk_mapped_avg_unpool_lists_bytes(int64_t height, int64_t width, int64_t out_height,
+                                         int64_t out_width, int64_t kernel_size,
+                                         int32_t num_interp_pts, int32_t interp, int32_t dtype);
+int sdk_mapped_avg_unpool_lists_build(const void* sample_map, const void* interp_weights,
+                                      void* lists, size_t lists_bytes, int64_t height,
+                                      int64_t width, int64_t out_height, int64_t out_width,
+                                      int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
+                                      int32_t dtype, sdk_stream_t stream);
+int sdk_mapped_avg_unpool_from_lists(const void* grad_output, void* grad_input, const void* lists,
+                                     size_t lists_bytes, int64_t batch, int64_t channels,
+                                     int64_t height, int64_t width, int64_t out_height,
+                                     int64_t out_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype,
+                                     sdk_stream_t stream);
 int sdk_mapped_max_unpool_plan_build(const void* sample_map, void* plan, size_t plan_bytes,
                                      int64_t height, int64_t width, int64_t out_height,
                                      int64_t out_width, int64_t kernel_size,

@@ -69,6 +69,8 @@ SIGNATURES = {
     "sdk_resample_plan_complete": [_vp, _sz, _vp, _vp],
     "sdk_resample_to_map_planned": [_vp] * 6 + [_sz, _i32, _i32, ctypes.c_double] + [_i64] * 6
                                    + [_i32] * 3 + [_vp],
+    "sdk_mapped_avg_unpool_lists_build": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
+    "sdk_mapped_avg_unpool_from_lists": [_vp] * 3 + [_sz] + [_i64] * 7 + [_i32] * 3 + [_vp],
     "sdk_mapped_avg_unpool_planned": [_vp] * 5 + [_sz, _i32] + [_i64] * 7 + [_i32] * 3 + [_vp],
     "sdk_mapped_max_unpool_plan_build": [_vp, _vp, _sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
     "sdk_mapped_max_unpool_planned": [_vp] * 6 + [_sz] + [_i64] * 7 + [_i32] * 3 + [_vp],
@@ -112,6 +114,8 @@ def load():
     lib.sdk_voting_resample_workspace_bytes.argtypes = [_i64] * 4
     lib.sdk_voting_resample_workspace_bytes.restype = _sz
     lib.sdk_mapped_conv_plan_bytes.argtypes = [_i64] * 5 + [_i32] * 3
+    lib.sdk_mapped_avg_unpool_lists_bytes.restype = _sz
+    lib.sdk_mapped_avg_unpool_lists_bytes.argtypes = [_i64] * 5 + [_i32] * 3
     lib.sdk_mapped_conv_plan_bytes.restype = _sz
     _lib = lib
     return lib

@@ -267,7 +267,8 @@ def _scatter_plan(kind, ref, sample_map, interp_weights, out_h, out_w, K, P, int
     kind "resample" / "avg_unpool": the inverted map (sdk_resample_to_map_plan_build; K = 1 for
     a resampling map), complete = 1 when every target's list holds all its sources, checked
     once after the build (not under stream capture, where the check's synchronisation is not
-    allowed).  kind "max_unpool": the tile windows (sdk_mapped_max_unpool_plan_build), complete = 1
+    allowed).  kind "avg_unpool_lists": the merged lists (sdk_mapped_avg_unpool_lists_build), for
+    the geometries that have them.  kind "max_unpool": the tile windows (sdk_mapped_max_unpool_plan_build), complete = 1
     when the row-band kernel does every call on the plan (sdk_mapped_max_unpool_plan_bands)."""
     if not _plan_cache_enabled:
         return None, 0, 0
@@ -283,15 +284,25 @@ def _scatter_plan(kind, ref, sample_map, interp_weights, out_h, out_w, K, P, int
     if torch.cuda.is_current_stream_capturing():
         return None, 0, 0
     lib = _capi.load()
-    query = ("sdk_mapped_max_unpool_workspace_bytes" if kind == "max_unpool"
-             else "sdk_resample_to_map_workspace_bytes")
-    n = getattr(lib, query)(int(out_h), int(out_w), dt)
+    if kind == "avg_unpool_lists":
+        n = lib.sdk_mapped_avg_unpool_lists_bytes(int(out_h), int(out_w), int(sample_map.shape[0]),
+                                                  int(sample_map.shape[1]), int(K), int(P),
+                                                  int(interp), dt)
+    else:
+        query = ("sdk_mapped_max_unpool_workspace_bytes" if kind == "max_unpool"
+                 else "sdk_resample_to_map_workspace_bytes")
+        n = getattr(lib, query)(int(out_h), int(out_w), dt)
     if n == 0:
         return None, 0, 0
     plan = torch.empty(n, dtype=torch.uint8, device=ref.device)
     MH, MW = int(sample_map.shape[0]), int(sample_map.shape[1])
     complete = 0
-    if kind == "max_unpool":
+    if kind == "avg_unpool_lists":
+        _capi.call("sdk_mapped_avg_unpool_lists_build", _ptr(sample_map), _ptr(interp_weights),
+                   _ptr(plan), n, int(out_h), int(out_w), MH, MW, int(K), int(P), int(interp), dt,
+                   _stream(ref))
+        complete = 1
+    elif kind == "max_unpool":
         _capi.call("sdk_mapped_max_unpool_plan_build", _ptr(sample_map), _ptr(plan), n, int(out_h),
                    int(out_w), MH, MW, int(K), int(P), int(interp), dt, _stream(ref))
         flag = ctypes.c_int32(0)
@@ -529,6 +540,13 @@ def mapped_avg_unpool(grad_output, sample_map, interp_weights, in_h, in_w, kerne
     gin = torch.empty((B, C, int(in_h), int(in_w)), dtype=grad_output.dtype,
                       device=grad_output.device)
     with torch.cuda.device(grad_output.device):
+        plan, nplan, _ = _scatter_plan("avg_unpool_lists", grad_output, sample_map,
+                                       interp_weights, in_h, in_w, kernel_size, P, interp)
+        if plan is not None:
+            _capi.call("sdk_mapped_avg_unpool_from_lists", _ptr(grad_output), _ptr(gin), _ptr(plan),
+                       nplan, B, C, int(in_h), int(in_w), OH, OW, int(kernel_size), P, int(interp),
+                       _DTYPES[grad_output.dtype], _stream(grad_output))
+            return gin
         plan, nplan, complete = _scatter_plan("avg_unpool", grad_output, sample_map,
                                               interp_weights, in_h, in_w, kernel_size, P, interp)
         if plan is not None:

@@ -1940,32 +1940,83 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(const int* __restric
 }
 
 // Every element's entries sorted by source, then coefficient (the fill appends in the order
-// its atomics are served); selection sort in place, the lists are short.
+// its atomics are served).  A wave takes one element after another, a list of at most kSortLds
+// entries in LDS, by a bitonic network whose exchanges all ascend, so that any length will do
+// (pairs past the end are left out: what is not there counts as larger than everything).  A
+// longer list, of a map that sends hundreds of samples to one image element, is sorted in
+// memory by the whole workgroup.  (One thread per list, by selection: a list of 100 entries, a 5 x 5
+// kernel's, costs it 5000 steps, one of ten thousand seconds.)
+constexpr int kSortLds = 512;
+constexpr int kSortTargets = 16;   // elements of a workgroup
+
+__device__ __forceinline__ bool entry_less(int sa, float ca, int sb, float cb) {
+  return sa < sb || (sa == sb && ca < cb);
+}
+
 __global__ __launch_bounds__(kBlock) void col2im_sort_kernel(const int* __restrict__ offset,
                                                              int* __restrict__ src,
                                                              float* __restrict__ co, int HW) {
-  const int u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= HW) return;
-  const int beg = offset[u], end = offset[u + 1];
-  for (int i = beg; i + 1 < end; ++i) {
-    int best = i, bs = src[i];
-    float bc = co[i];
-    const int first_s = bs;
-    const float first_c = bc;
-    for (int j = i + 1; j < end; ++j) {
-      const int sj = src[j];
-      const float cj = co[j];
-      if (sj < bs || (sj == bs && cj < bc)) {
-        best = j;
-        bs = sj;
-        bc = cj;
-      }
+  constexpr int kWaves = kBlock / 64;
+  __shared__ int s_src[kWaves][kSortLds];
+  __shared__ float s_co[kWaves][kSortLds];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int u0 = blockIdx.x * kSortTargets;
+  // one wave alone touches its part of LDS, whose operations are served in order
+  volatile int* ls = s_src[wave];
+  volatile float* lc = s_co[wave];
+  for (int t = wave; t < kSortTargets && u0 + t < HW; t += kWaves) {
+    const int beg = offset[u0 + t], n = offset[u0 + t + 1] - beg;
+    if (n < 2 || n > kSortLds) continue;
+    for (int i = lane; i < n; i += 64) {
+      ls[i] = src[beg + i];
+      lc[i] = co[beg + i];
     }
-    if (best != i) {
-      src[best] = first_s;
-      co[best] = first_c;
-      src[i] = bs;
-      co[i] = bc;
+    for (int k = 2; k < 2 * n; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        __builtin_amdgcn_wave_barrier();
+        for (int i = lane; i < n; i += 64) {
+          const int o = j == (k >> 1) ? (i ^ (k - 1)) : (i ^ j);
+          if (o > i && o < n) {
+            const int si = ls[i], so = ls[o];
+            const float ci = lc[i], cj = lc[o];
+            if (entry_less(so, cj, si, ci)) {
+              ls[i] = so;
+              lc[i] = cj;
+              ls[o] = si;
+              lc[o] = ci;
+            }
+          }
+        }
+      }
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < n; i += 64) {
+      src[beg + i] = ls[i];
+      co[beg + i] = lc[i];
+    }
+  }
+  for (int t = 0; t < kSortTargets && u0 + t < HW; ++t) {
+    const int beg = offset[u0 + t], n = offset[u0 + t + 1] - beg;
+    if (n <= kSortLds) continue;   // (uniform)
+    int* s = src + beg;
+    float* c = co + beg;
+    for (int64_t k = 2; k < 2 * (int64_t)n; k <<= 1) {
+      for (int64_t j = k >> 1; j > 0; j >>= 1) {
+        for (int i = threadIdx.x; i < n; i += kBlock) {
+          const int64_t o = j == (k >> 1) ? (i ^ (k - 1)) : (i ^ j);
+          if (o > i && o < n) {
+            const int si = s[i], so = s[o];
+            const float ci = c[i], cj = c[o];
+            if (entry_less(so, cj, si, ci)) {
+              s[i] = so;
+              c[i] = cj;
+              s[o] = si;
+              c[o] = ci;
+            }
+          }
+        }
+        __syncthreads();
+      }
     }
   }
 }
@@ -2045,6 +2096,77 @@ __global__ __launch_bounds__(kBlock) void col2im_gather_kernel(
   }
 }
 
+// Entries of one image element that come from the same pooled pixel (neighbours in a sorted
+// list) become one with the sum of their coefficients; src then names the pooled pixel and
+// count[u] the entries left.
+__global__ __launch_bounds__(kBlock) void unpool_merge_kernel(const int* __restrict__ offset,
+                                                              int* __restrict__ src,
+                                                              float* __restrict__ co,
+                                                              int* __restrict__ count, int HW,
+                                                              int K) {
+  const int u = blockIdx.x * kBlock + threadIdx.x;
+  if (u >= HW) return;
+  const int beg = offset[u], end = offset[u + 1];
+  int at = beg - 1, cur = -1;
+  float sum = 0.0f;
+  for (int e = beg; e < end; ++e) {
+    const int m = src[e] / K;
+    const float c = co[e];
+    if (m != cur) {
+      if (at >= beg) co[at] = sum;
+      src[++at] = m;
+      cur = m;
+      sum = 0.0f;
+    }
+    sum += c;
+  }
+  if (at >= beg) co[at] = sum;
+  count[u] = at - beg + 1;
+}
+
+// Average unpooling of blended samples as a gather over the merged lists: a thread owns an image
+// element in PC planes, four entries in flight.  Neighbouring elements draw on the same few pooled
+// pixels, so the reads of a wave fall into few lines.  (The tile kernel adds K * 4 values per
+// pooled pixel and plane to LDS by compare-and-swap: 4 x 48 planes of 190 x 378 from 95 x 189,
+// 94 us; and a map whose windows it cannot hold, stride 1 at 256 x 512, went to atomics in
+// memory: 7.9 ms for 128 planes.)
+template <int PC>
+__global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
+    const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
+    const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
+    int M, int planes, float K) {
+  const int u = banded_pixel_block() * kBlock + threadIdx.x;
+  if (u >= HW) return;
+  const int plane0 = blockIdx.y * PC;
+  const int np = min(PC, planes - plane0);
+  const int beg = offset[u], n = count[u];
+  const float* g0 = gout + (size_t)plane0 * M;
+  float acc[PC];
+#pragma unroll
+  for (int j = 0; j < PC; ++j) acc[j] = 0.0f;
+  for (int e = 0; e < n; e += 4) {
+    int m[4];
+    float c[4], v[4][PC];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = beg + min(e + i, n - 1);
+      m[i] = src[at];
+      c[i] = co[at];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < PC; ++j) v[i][j] = g0[(size_t)(j < np ? j : 0) * M + m[i]];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < PC; ++j) acc[j] += e + i < n ? c[i] * v[i][j] : 0.0f;
+  }
+#pragma unroll
+  for (int j = 0; j < PC; ++j)
+    if (j < np) gin[(size_t)(plane0 + j) * HW + u] = acc[j] / K;
+}
+
 struct Col2imLists {
   int *count, *offset, *cursor, *sums, *src;
   float* co;
@@ -2106,9 +2228,41 @@ int col2im_lists_build(const float* map, const float* wts, void* lists, int H, i
   SDK_DISPATCH_INTERP(interp, P,
                       (launch((col2im_invert_kernel<INTERP, WEIGHTED, true>), grid, dim3(kBlock),
                               stream, map, wts, H, W, M, K, P, l.cursor, l.src, l.co)));
-  launch(col2im_sort_kernel, dim3((unsigned)ceil_div(HW, kBlock)), dim3(kBlock), stream,
+  launch(col2im_sort_kernel, dim3((unsigned)ceil_div(HW, kSortTargets)), dim3(kBlock), stream,
          (const int*)l.offset, l.src, l.co, HW);
   SDK_LAUNCH_CHECK("mapped_conv(inverted map)");
+  return SDK_OK;
+}
+
+// Lists of more than this are not kept (128 planes of 256 x 512, stride 1, bilinear: 38 MB).
+constexpr int64_t kUnpoolListsMost = (int64_t)256 << 20;
+
+static int build_unpool_lists(const float* map, const float* wts, void* lists, int H, int W, int M,
+                              int K, int P, int interp, hipStream_t stream) {
+  int rc = col2im_lists_build(map, wts, lists, H, W, M, K, P, interp, stream);
+  if (rc) return rc;
+  const Col2imLists l = col2im_lists_at(lists, H, W, M, K, P, interp);
+  launch(unpool_merge_kernel, dim3((unsigned)ceil_div((int64_t)H * W, kBlock)), dim3(kBlock), stream,
+         (const int*)l.offset, l.src, l.co, l.count, H * W, K);
+  SDK_LAUNCH_CHECK("mapped_avg_unpool(merged lists)");
+  return SDK_OK;
+}
+
+static int launch_unpool_lists(const float* gout, float* gin, const void* lists, int64_t planes,
+                               int H, int W, int M, int K, int P, int interp, hipStream_t stream) {
+  const Col2imLists l = col2im_lists_at(const_cast<void*>(lists), H, W, M, K, P, interp);
+  const int HW = H * W;
+#define UL(PCv)                                                                                \
+  launch(unpool_lists_kernel<PCv>, dim3(banded_grid_x(HW), (unsigned)ceil_div(planes, PCv)),   \
+         dim3(kBlock), stream, gout, (const int*)l.offset, (const int*)l.count,                \
+         (const int*)l.src, (const float*)l.co, gin, HW, M, (int)planes, (float)K)
+  // as many planes to a thread as still leave the GPU a few workgroups per CU
+  const int64_t blocks = ceil_div(HW, kBlock);
+  if (blocks * ceil_div(planes, 8) >= 1024) UL(8);
+  else if (blocks * ceil_div(planes, 4) >= 1024) UL(4);
+  else UL(2);
+#undef UL
+  SDK_LAUNCH_CHECK("mapped_avg_unpool(lists)");
   return SDK_OK;
 }
 
@@ -2736,6 +2890,67 @@ int sdk_mapped_avg_unpool_planned(const void* grad_output, const void* sample_ma
                                 (hipStream_t)stream, false, 0.0, (int)kernel_size, true,
                                 plan_complete, (int)out_width));
   return SDK_OK;
+}
+
+size_t sdk_mapped_avg_unpool_lists_bytes(int64_t height, int64_t width, int64_t out_height,
+                                         int64_t out_width, int64_t kernel_size,
+                                         int32_t num_interp_pts, int32_t interp, int32_t dtype) {
+  const bool blended = interp == 1 || interp == 2;
+  if (dtype != SDK_F32 || (!blended && num_interp_pts == 0) || height < 1 || width < 1 ||
+      out_height < 1 || out_width < 1 || kernel_size < 1 || num_interp_pts < 0 ||
+      height >= ((int64_t)1 << 31) || width >= ((int64_t)1 << 31) ||
+      out_height >= ((int64_t)1 << 31) || out_width >= ((int64_t)1 << 31) ||
+      kernel_size >= ((int64_t)1 << 24) || num_interp_pts >= (1 << 16))
+    return 0;
+  // (every product below is of factors checked to be small enough to form it)
+  if (height * width >= ((int64_t)1 << 31) - 1 || out_height * out_width >= ((int64_t)1 << 31))
+    return 0;
+  const int64_t M = out_height * out_width;
+  if (M * kernel_size >= ((int64_t)1 << 31) || M * kernel_size * pts(num_interp_pts) * (blended ? 4 : 1) * 8 > kUnpoolListsMost) return 0;
+  return col2im_lists_bytes((int)height, (int)width, (int)M, (int)kernel_size, num_interp_pts,
+                            interp);
+}
+
+int sdk_mapped_avg_unpool_lists_build(const void* sample_map, const void* interp_weights,
+                                      void* lists, size_t lists_bytes, int64_t height,
+                                      int64_t width, int64_t out_height, int64_t out_width,
+                                      int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
+                                      int32_t dtype, sdk_stream_t stream) {
+  const char* what = "mapped_avg_unpool_lists_build";
+  SDK_REQUIRE(sample_map && lists && (num_interp_pts == 0 || interp_weights), "%s: NULL pointer", what);
+  const size_t need = sdk_mapped_avg_unpool_lists_bytes(height, width, out_height, out_width,
+                                                        kernel_size, num_interp_pts, interp, dtype);
+  if (need == 0) return fail(SDK_ERR_UNSUPPORTED, "%s: no lists for this geometry", what);
+  if (lists_bytes < need)
+    return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, lists_bytes);
+  return build_unpool_lists((const float*)sample_map, (const float*)interp_weights, lists,
+                            (int)height, (int)width, (int)(out_height * out_width),
+                            (int)kernel_size, num_interp_pts, interp, (hipStream_t)stream);
+}
+
+int sdk_mapped_avg_unpool_from_lists(const void* grad_output, void* grad_input, const void* lists,
+                                     size_t lists_bytes, int64_t batch, int64_t channels,
+                                     int64_t height, int64_t width, int64_t out_height,
+                                     int64_t out_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype,
+                                     sdk_stream_t stream) {
+  const char* what = "mapped_avg_unpool_from_lists";
+  SDK_REQUIRE(lists, "%s: NULL pointer", what);
+  const size_t need = sdk_mapped_avg_unpool_lists_bytes(height, width, out_height, out_width,
+                                                        kernel_size, num_interp_pts, interp, dtype);
+  if (need == 0) return fail(SDK_ERR_UNSUPPORTED, "%s: no lists for this geometry", what);
+  if (lists_bytes < need)
+    return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, lists_bytes);
+  const int64_t M = out_height * out_width;
+  // (the map and its weights were read by the build; here they only have to be named)
+  int rc = check_mapped(grad_output, lists, lists, grad_input, batch, channels, height, width, M,
+                        kernel_size, num_interp_pts, what);
+  if (rc) return rc;
+  const int64_t planes = batch * channels;
+  if (planes == 0) return SDK_OK;
+  return launch_unpool_lists((const float*)grad_output, (float*)grad_input, lists, planes,
+                             (int)height, (int)width, (int)M, (int)kernel_size, num_interp_pts,
+                             interp, (hipStream_t)stream);
 }
 
 int sdk_mapped_max_unpool_plan_build(const void* sample_map, void* plan, size_t plan_bytes,

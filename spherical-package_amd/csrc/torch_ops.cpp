@@ -66,7 +66,8 @@ bool tensor_key(const OptTensor& t, TensorKey* k) {
   return true;
 }
 
-enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kConvColumns = 4 };
+enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kConvColumns = 4,
+            kAvgUnpoolLists = 5 };
 
 struct Key {
   int kind = 0, device = 0, dtype = 0;
@@ -273,10 +274,18 @@ PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptT
   return plan_for(
       key, ref, map, wts, stream,
       [&] {
+        if (kind == kAvgUnpoolLists)
+          return sdk_mapped_avg_unpool_lists_bytes(out_h, out_w, MH, MW, K, (int32_t)P,
+                                                   (int32_t)interp, dt);
         return kind == kMaxUnpool ? sdk_mapped_max_unpool_workspace_bytes(out_h, out_w, dt)
                                   : sdk_resample_to_map_workspace_bytes(out_h, out_w, dt);
       },
       [&](void* buf, size_t n) {
+        if (kind == kAvgUnpoolLists) {
+          SDK_CALL(sdk_mapped_avg_unpool_lists_build, map.data_ptr(), cptr(wts), buf, n, out_h,
+                   out_w, MH, MW, K, (int32_t)P, (int32_t)interp, dt, stream);
+          return 1;
+        }
         if (kind == kMaxUnpool) {
           SDK_CALL(sdk_mapped_max_unpool_plan_build, map.data_ptr(), buf, n, out_h, out_w, MH, MW,
                    K, (int32_t)P, (int32_t)interp, dt, stream);
@@ -463,6 +472,16 @@ Tensor mapped_avg_unpool(const Tensor& g, const Tensor& map, const OptTensor& wt
   Tensor gin = at::empty({B, C, in_h, in_w}, g.options());
   c10::DeviceGuard guard(g.device());
   hipStream_t s = stream_of(g);
+  if (sdk_mapped_avg_unpool_lists_bytes(in_h, in_w, OH, OW, kernel_size, (int32_t)P,
+                                        (int32_t)interp, dt) != 0) {
+    PlanRef lists = scatter_plan(kAvgUnpoolLists, g, map, wts, in_h, in_w, kernel_size, P, interp, s);
+    if (lists.plan.defined()) {
+      SDK_CALL(sdk_mapped_avg_unpool_from_lists, g.data_ptr(), gin.data_ptr(), lists.ptr(),
+               lists.nbytes, B, C, in_h, in_w, OH, OW, kernel_size, (int32_t)P, (int32_t)interp, dt,
+               s);
+      return gin;
+    }
+  }
   PlanRef plan = scatter_plan(kAvgUnpool, g, map, wts, in_h, in_w, kernel_size, P, interp, s);
   if (plan.plan.defined()) {
     SDK_CALL(sdk_mapped_avg_unpool_planned, g.data_ptr(), map.data_ptr(), cptr(wts), gin.data_ptr(),
