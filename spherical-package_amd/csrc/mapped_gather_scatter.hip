@@ -2632,6 +2632,14 @@ int sdk_mapped_max_pool(const void* input, const void* sample_map, const void* i
     SDK_LAUNCH_CHECK("mapped_max_pool");
     return SDK_OK;
   }
+  if (dtype == SDK_F32 && num_interp_pts == 0 && out_height < ((int64_t)1 << 24) &&
+      out_width < ((int64_t)1 << 24) &&
+      pool_blend_launch(false, (const float*)input, (const float*)sample_map, (float*)out, indices,
+                        planes, (int)height, (int)width, (int)out_height, (int)out_width,
+                        (int)kernel_size, interp, (hipStream_t)stream)) {
+    SDK_LAUNCH_CHECK("mapped_max_pool");
+    return SDK_OK;
+  }
   const dim3 grid(banded_grid_x(M), (unsigned)ceil_div(planes, kPC));
   SDK_DISPATCH_DTYPE(
       dtype,
@@ -2662,6 +2670,14 @@ int sdk_mapped_avg_pool(const void* input, const void* sample_map, const void* i
       pool_band_launch(true, (const float*)input, (const float*)sample_map, (float*)out, nullptr,
                        planes, (int)height, (int)width, (int)out_height, (int)out_width,
                        (int)kernel_size, (hipStream_t)stream)) {
+    SDK_LAUNCH_CHECK("mapped_avg_pool");
+    return SDK_OK;
+  }
+  if (dtype == SDK_F32 && num_interp_pts == 0 && out_height < ((int64_t)1 << 24) &&
+      out_width < ((int64_t)1 << 24) &&
+      pool_blend_launch(true, (const float*)input, (const float*)sample_map, (float*)out, nullptr,
+                        planes, (int)height, (int)width, (int)out_height, (int)out_width,
+                        (int)kernel_size, interp, (hipStream_t)stream)) {
     SDK_LAUNCH_CHECK("mapped_avg_pool");
     return SDK_OK;
   }

@@ -40,4 +40,11 @@ void unpool_band_launch(bool avg, const float* gout, const int64_t* idx, const f
                         float* gin, const int* table, const unsigned* taps, int* gate,
                         int64_t planes, int H, int W, int OH, int OW, int K, hipStream_t stream);
 
+// The pooling of pool_band_launch for blended samples (interp 1 or 2, unweighted; pool_blend.hip):
+// K = 4 or 9, pooled rows of at most 256 pixels, half a million results or more; false: not
+// launched.
+bool pool_blend_launch(bool avg, const float* in, const float* map, float* out, int64_t* idx,
+                       int64_t planes, int H, int W, int OH, int OW, int K, int interp,
+                       hipStream_t stream);
+
 }  // namespace sdk
