@@ -149,14 +149,15 @@ __global__ __launch_bounds__(kClThreads) void columns_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// The products.  A workgroup of four waves makes a (64 WM) x (64 WN) tile of C, each wave a
-// quarter of 32 WM x 32 WN; the reduction goes through LDS in steps of 32, double-buffered, the
-// values of the step after next requested from memory before the current step's MFMAs (a step
-// of a 64 x 64 tile is 0.1 to 0.4 us of matrix work, a read from beyond the L2 takes longer).  LDS rows hold 32
-// reduction elements and are 36 floats apart (16-byte reads of 32 consecutive rows then use
-// all banks evenly); a lane reads eight consecutive reduction elements of its row, which are a
-// bf16 operand once converted, or the operands of eight fp32 MFMAs (whose two reduction
-// indices may be any pair, as long as both operands agree).
+// The products.  Four waves make a 64 x 64 tile of C, 32 x 32 each (KS = 2: two such groups
+// share the reduction of one tile, alternate steps each, and add up at the end); the reduction
+// goes through LDS in steps of 32, double-buffered, the values of the step after next requested
+// from memory before the current step's MFMAs (a step is 0.1 to 0.4 us of matrix work, a read
+// from beyond the L2 takes longer).  LDS rows hold 32 reduction elements and are 36 floats apart
+// (16-byte reads of 32 consecutive rows then use all banks evenly); a lane reads eight
+// consecutive reduction elements of its row, which are a bf16 operand once converted, or the
+// operands of eight fp32 MFMAs (whose two reduction indices may be any pair, as long as both
+// operands agree).
 //   TN = false: C[i][n] = sum_r A[i][r] B[n][r] + bias[i]    (both operands run along r)
 //   TN = true:  C[i][n] = sum_r A[r][i] B[r][n], r in the split's range (a thread transposes
 //               4 x 4 blocks in registers on the way to LDS)
@@ -178,12 +179,11 @@ struct GemmArgs {
   int tiles_a, tiles_b;
 };
 
-template <int MM, int WM, int WN, bool TN>
-__global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
-  constexpr int BM = 64 * WM, BN = 64 * WN;
+template <int MM, bool TN, int KS>
+__global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs g) {
+  constexpr int BM = 64, BN = 64;
   constexpr int LA = BM / 32, LB = BN / 32;   // 16-byte pieces per thread and step
-  __shared__ __attribute__((aligned(16))) float As[2][BM * kGld];
-  __shared__ __attribute__((aligned(16))) float Bs[2][BN * kGld];
+  __shared__ __attribute__((aligned(16))) float lds[KS][2][(BM + BN) * kGld];
   __shared__ float s_bias[BM];
   // consecutive slots of one XCD share the tile of the larger operand (workgroup ids go
   // round-robin over the 8 XCDs)
@@ -192,9 +192,12 @@ __global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
   if ((int)(blockIdx.x >> 3) >= (total + 7) / 8 || slot >= total) return;
   const int ta = slot % g.tiles_a, tb = slot / g.tiles_a;
   const int i0 = ta * BM, n0 = tb * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kClThreads);
+  const int tid = threadIdx.x % kClThreads, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
-  const int wr = (wave >> 1) * 32 * WM, wc = (wave & 1) * 32 * WN;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  float* As[2] = {lds[group][0], lds[group][1]};
+  float* Bs[2] = {lds[group][0] + BM * kGld, lds[group][1] + BM * kGld};
   const float* B = TN ? g.B : g.B + (size_t)blockIdx.y * g.batch_b;
   float* C = g.C + (size_t)blockIdx.y * g.batch_c;
   const int r_begin = TN ? (int)blockIdx.y * g.split : 0;
@@ -216,7 +219,6 @@ __global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
         gb[i] = *reinterpret_cast<const vec4*>(B + (size_t)min(n0 + rb + 32 * i, g.rows_b - 1) * g.ldb + r);
     } else {
       // blocks of four reduction rows x four columns: threads 0..127 take A's, the others B's
-      static_assert(!TN || (WM == 1 && WN == 1), "64 x 64 tiles only");
       const bool is_a = tid < 128;
       const int ld = is_a ? g.lda : g.ldb;
       const float* src = (is_a ? g.A : B) + min((is_a ? i0 : n0) + 4 * (rb & 15), ld - 4);
@@ -249,16 +251,12 @@ __global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
     }
   };
 
-  for (int i = tid; i < BM; i += kClThreads)
-    s_bias[i] = !TN && g.bias != nullptr ? g.bias[min(i0 + i, g.rows_a - 1)] : 0.0f;
+  if (threadIdx.x < BM)
+    s_bias[threadIdx.x] = !TN && g.bias != nullptr ? g.bias[min(i0 + (int)threadIdx.x, g.rows_a - 1)] : 0.0f;
 
-  floatx16 acc[WM][WN];
+  floatx16 acc;
 #pragma unroll
-  for (int a = 0; a < WM; ++a)
-#pragma unroll
-    for (int b = 0; b < WN; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
 
   auto load8 = [&](const float* p, float (&f)[8]) {
     const vec4 lo = *reinterpret_cast<const vec4*>(p), hi = *reinterpret_cast<const vec4*>(p + 4);
@@ -272,81 +270,66 @@ __global__ __launch_bounds__(kClThreads) void columns_gemm_kernel(GemmArgs g) {
   auto multiply = [&](int buf) {
 #pragma unroll
     for (int s = 0; s < kGk / 16; ++s) {
-      float fa[WM][8], fb[WN][8];
-#pragma unroll
-      for (int a = 0; a < WM; ++a)
-        load8(&As[buf][(wr + 32 * a + j) * kGld + 16 * s + 8 * h], fa[a]);
-#pragma unroll
-      for (int b = 0; b < WN; ++b)
-        load8(&Bs[buf][(wc + 32 * b + j) * kGld + 16 * s + 8 * h], fb[b]);
+      float fa[8], fb[8];
+      load8(&As[buf][(wr + j) * kGld + 16 * s + 8 * h], fa);
+      load8(&Bs[buf][(wc + j) * kGld + 16 * s + 8 * h], fb);
       if constexpr (MM == kMmF32) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-#pragma unroll
-          for (int a = 0; a < WM; ++a)
-#pragma unroll
-            for (int b = 0; b < WN; ++b)
-              acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][e], fb[b][e], acc[a][b], 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
       } else if constexpr (MM == kMmBf16) {
-        Bf16Frag pa[WM], pb[WN];
-#pragma unroll
-        for (int a = 0; a < WM; ++a) pa[a] = pack_bf16x8(fa[a]);
-#pragma unroll
-        for (int b = 0; b < WN; ++b) pb[b] = pack_bf16x8(fb[b]);
-#pragma unroll
-        for (int a = 0; a < WM; ++a)
-#pragma unroll
-          for (int b = 0; b < WN; ++b) acc[a][b] = mfma_bf16(pa[a], pb[b], acc[a][b]);
+        acc = mfma_bf16(pack_bf16x8(fa), pack_bf16x8(fb), acc);
       } else {
-        Bf16Split pa[WM], pb[WN];
-#pragma unroll
-        for (int a = 0; a < WM; ++a) pa[a] = split_bf16x8(fa[a]);
-#pragma unroll
-        for (int b = 0; b < WN; ++b) pb[b] = split_bf16x8(fb[b]);
-#pragma unroll
-        for (int a = 0; a < WM; ++a)
-#pragma unroll
-          for (int b = 0; b < WN; ++b) acc[a][b] = mfma_split(pa[a], pb[b], acc[a][b]);
+        acc = mfma_split(split_bf16x8(fa), split_bf16x8(fb), acc);
       }
     }
   };
 
   // step t: registers t & 1 hold its values until they go to LDS buffer t & 1, one step ahead
-  // of the MFMAs; step t + 2 is requested right after
-  const int steps = (r_end - r_begin + kGk - 1) / kGk;
-  fetch(r_begin, ra[0], rbv[0]);
-  fetch(r_begin + kGk, ra[1], rbv[1]);
-  stash(0, r_begin, ra[0], rbv[0]);
+  // of the MFMAs; step t + 2 is requested right after.  With KS groups, group q's step t is the
+  // reduction's step KS t + q.
+  constexpr int kStep = KS * kGk;
+  const int steps = (r_end - r_begin + kStep - 1) / kStep;
+  const int r_first = r_begin + group * kGk;
+  fetch(r_first, ra[0], rbv[0]);
+  fetch(r_first + kStep, ra[1], rbv[1]);
+  stash(0, r_first, ra[0], rbv[0]);
   __syncthreads();
   // (the scheduling barriers keep the requests in front of the MFMAs and the waits for older
   // ones behind them; left alone the compiler sinks the requests to their uses)
   for (int t = 0; t < steps; t += 2) {
-    const int r0 = r_begin + t * kGk;
-    fetch(r0 + 2 * kGk, ra[0], rbv[0]);
+    const int r0 = r_first + t * kStep;
+    fetch(r0 + 2 * kStep, ra[0], rbv[0]);
     __builtin_amdgcn_sched_barrier(0);
     multiply(0);
     __builtin_amdgcn_sched_barrier(0);
-    stash(1, r0 + kGk, ra[1], rbv[1]);
+    stash(1, r0 + kStep, ra[1], rbv[1]);
     __syncthreads();
-    fetch(r0 + 3 * kGk, ra[1], rbv[1]);
+    fetch(r0 + 3 * kStep, ra[1], rbv[1]);
     __builtin_amdgcn_sched_barrier(0);
     multiply(1);   // (a step past the end multiplies zeros)
     __builtin_amdgcn_sched_barrier(0);
-    stash(0, r0 + 2 * kGk, ra[0], rbv[0]);
+    stash(0, r0 + 2 * kStep, ra[0], rbv[0]);
     __syncthreads();
   }
+  if constexpr (KS == 2) {
+    // the second group's sums join the first's through LDS, [register][thread]
+    float* sums = &lds[1][0][0];
+    if (group == 1) {
 #pragma unroll
-  for (int a = 0; a < WM; ++a)
-#pragma unroll
-    for (int b = 0; b < WN; ++b) {
-      const int n = n0 + wc + 32 * b + j;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int i = i0 + wr + 32 * a + 8 * (v >> 2) + 4 * h + (v & 3);
-        if (i < g.rows_a && n < g.rows_b)
-          C[(size_t)i * g.ldc + n] = acc[a][b][v] + s_bias[i - i0];
-      }
+      for (int v = 0; v < 16; ++v) sums[v * kClThreads + tid] = acc[v];
     }
+    __syncthreads();
+    if (group == 1) return;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] += sums[v * kClThreads + tid];
+  }
+  const int n = n0 + wc + j;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int i = wr + 8 * (v >> 2) + 4 * h + (v & 3);
+    if (i0 + i < g.rows_a && n < g.rows_b) C[(size_t)(i0 + i) * g.ldc + n] = acc[v] + s_bias[i];
+  }
 }
 
 // gW[i][c][k] = sum over the splits of partial[split][i][k][c].
@@ -475,12 +458,24 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
   a.tiles_b = (int)ceil_div(a.rows_b, 64);
   const int64_t total = (int64_t)a.tiles_a * a.tiles_b;
   const dim3 grid((unsigned)((total + 7) / 8 * 8), (unsigned)batches);
-  if (mm == kMmBf16)
-    launch((columns_gemm_kernel<kMmBf16, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
-  else if (mm == kMmSplit)
-    launch((columns_gemm_kernel<kMmSplit, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
-  else
-    launch((columns_gemm_kernel<kMmF32, 1, 1, TN>), grid, dim3(kClThreads), stream, a);
+  // Two groups of waves per tile where the tiles alone leave the SIMDs with a wave or two and the
+  // reduction is long enough to share (whole forward: 6 x 25 x 50, 96 -> 160, split 65 -> 55 us;
+  // 3 x 45 x 91, 200 -> 37, bf16 86 -> 67 us).  With fp32 MFMAs two waves of 512 tiles keep a SIMD
+  // busy as it is (1 x 128 x 256, 64 -> 64: 62 -> 67 us), and so do the splits of the weight
+  // gradient (57 -> 66 us).
+  const bool shared = !TN && total * batches <= (mm == kMmF32 ? 256 : 1024) && a.red >= 4 * kGk;
+#define CG(MMv)                                                                                   \
+  do {                                                                                            \
+    if constexpr (!TN) {                                                                          \
+      if (shared) {                                                                               \
+        launch((columns_gemm_kernel<MMv, false, 2>), grid, dim3(2 * kClThreads), stream, a);      \
+        break;                                                                                    \
+      }                                                                                           \
+    }                                                                                             \
+    launch((columns_gemm_kernel<MMv, TN, 1>), grid, dim3(kClThreads), stream, a);                 \
+  } while (0)
+  if (mm == kMmBf16) CG(kMmBf16); else if (mm == kMmSplit) CG(kMmSplit); else CG(kMmF32);
+#undef CG
   SDK_LAUNCH_CHECK("mapped_conv(columns product)");
   return SDK_OK;
 }
