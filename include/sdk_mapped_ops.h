@@ -565,7 +565,13 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
  *
  *   sdk_mapped_conv_by_columns(...)           1 when a call of these sizes does (transposed: of a
  *                                             transposed convolution), 0 otherwise
- *   sdk_mapped_conv_plan_build_columns(...)   fills, of a plan buffer of full size, the part
+ *   sdk_mapped_conv_plan_bytes_columns(...)   size of a plan that holds this too (0: this map's
+ *                                             calls never run so); sdk_mapped_conv_plan_build
+ *                                             fills all of a buffer of that size.  Build and
+ *                                             calls are given the same plan_bytes; with a
+ *                                             plan of sdk_mapped_conv_plan_bytes such calls
+ *                                             invert the map in their workspace.
+ *   sdk_mapped_conv_plan_build_columns(...)   fills, of a buffer of that size, only the part
  *                                             such calls read; for no other call
  *   sdk_mapped_conv_columns_enable(0 / 1)     turns the route off / on for the calling thread
  *                                             (to measure or test the tile kernels at small
@@ -576,12 +582,25 @@ int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_c
                                int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
                                int32_t interp, int32_t dtype, int32_t compute,
                                int32_t transposed);
+size_t sdk_mapped_conv_plan_bytes_columns(int64_t image_height, int64_t image_width,
+                                          int64_t map_height, int64_t map_width,
+                                          int64_t kernel_size, int32_t num_interp_pts,
+                                          int32_t interp, int32_t dtype);
 int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
                                        void* plan, size_t plan_bytes, int64_t image_height,
                                        int64_t image_width, int64_t map_height, int64_t map_width,
                                        int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
                                        int32_t dtype, sdk_stream_t stream);
 int sdk_mapped_conv_columns_enable(int32_t enabled);
+/* One part of the same plan: parts = 1 what the forward of a convolution, the backward-input of a
+ * transposed one and both weight gradients read; 2 what the backward-input of a convolution and
+ * the forward of a transposed one read (most of the time of a build); 3 both.  A call must find
+ * the parts it reads; a combined backward reads both. */
+int sdk_mapped_conv_plan_build_parts(const void* sample_map, const void* interp_weights, void* plan,
+                                     size_t plan_bytes, int64_t image_height, int64_t image_width,
+                                     int64_t map_height, int64_t map_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype,
+                                     int32_t parts, sdk_stream_t stream);
 int sdk_mapped_conv_forward_planned(const void* input, const void* sample_map, const void*
     interp_weights, const void* weight, const void* bias, void* output, void* workspace, size_t
     workspace_bytes, void* plan, size_t plan_bytes, int64_t batch, int64_t in_channels, int64_t

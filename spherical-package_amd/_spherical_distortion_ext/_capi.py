@@ -61,6 +61,7 @@ SIGNATURES = {
     "sdk_mapped_conv_backward_select": [_vp] * 9 + [_sz, _vp, _sz] + _CONV_DIMS,
     "sdk_mapped_transposed_conv_backward_select": [_vp] * 9 + [_sz, _vp, _sz] + _CONV_DIMS,
     "sdk_mapped_conv_plan_build": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
+    "sdk_mapped_conv_plan_build_parts": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 4 + [_vp],
     "sdk_mapped_conv_plan_build_columns": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
     "sdk_mapped_conv_by_columns": [_i64] * 8 + [_i32] * 5,
     "sdk_mapped_conv_columns_enable": [_i32],
@@ -114,6 +115,8 @@ def load():
     lib.sdk_voting_resample_workspace_bytes.argtypes = [_i64] * 4
     lib.sdk_voting_resample_workspace_bytes.restype = _sz
     lib.sdk_mapped_conv_plan_bytes.argtypes = [_i64] * 5 + [_i32] * 3
+    lib.sdk_mapped_conv_plan_bytes_columns.restype = _sz
+    lib.sdk_mapped_conv_plan_bytes_columns.argtypes = [_i64] * 5 + [_i32] * 3
     lib.sdk_mapped_avg_unpool_lists_bytes.restype = _sz
     lib.sdk_mapped_avg_unpool_lists_bytes.argtypes = [_i64] * 5 + [_i32] * 3
     lib.sdk_mapped_conv_plan_bytes.restype = _sz

@@ -80,7 +80,7 @@ int run(const char* what, Op op, const ConvGeom& g, int dtype, int compute, cons
     if (plan.buffer != nullptr) {
       rc = check_plan(what, g, dtype, compute, plan);
       if (rc) return rc;
-      load_cached_plan(g, plan.buffer, &cached);
+      load_cached_plan(g, plan.buffer, plan.bytes, &cached);
       cp = &cached;
     }
     const float* m = (const float*)map;
@@ -459,13 +459,14 @@ size_t sdk_mapped_conv_plan_bytes(int64_t image_height, int64_t image_width, int
   return cached_plan_bytes(g);
 }
 
-int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weights, void* plan,
-                               size_t plan_bytes, int64_t image_height, int64_t image_width,
-                               int64_t map_height, int64_t map_width, int64_t kernel_size,
-                               int32_t num_interp_pts, int32_t interp, int32_t dtype,
-                               sdk_stream_t stream) {
+int sdk_mapped_conv_plan_build_parts(const void* sample_map, const void* interp_weights, void* plan,
+                                     size_t plan_bytes, int64_t image_height, int64_t image_width,
+                                     int64_t map_height, int64_t map_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype,
+                                     int32_t parts, sdk_stream_t stream) {
   const char* what = "mapped_conv_plan_build";
   SDK_REQUIRE(sample_map && plan, "%s: NULL pointer", what);
+  SDK_REQUIRE(parts >= 1 && parts <= 3, "%s: parts = %d", what, parts);
   SDK_REQUIRE(num_interp_pts >= 0 && (num_interp_pts == 0 || interp_weights),
               "%s: weighted map needs interp_weights", what);
   const size_t need = sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width,
@@ -478,7 +479,17 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
   ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
              (int)kernel_size, num_interp_pts, interp, (int)map_width};
   return build_cached_plan(g, (const float*)sample_map, (const float*)interp_weights, plan,
-                           (hipStream_t)stream);
+                           plan_bytes, (hipStream_t)stream, parts);
+}
+
+int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weights, void* plan,
+                               size_t plan_bytes, int64_t image_height, int64_t image_width,
+                               int64_t map_height, int64_t map_width, int64_t kernel_size,
+                               int32_t num_interp_pts, int32_t interp, int32_t dtype,
+                               sdk_stream_t stream) {
+  return sdk_mapped_conv_plan_build_parts(sample_map, interp_weights, plan, plan_bytes,
+                                          image_height, image_width, map_height, map_width,
+                                          kernel_size, num_interp_pts, interp, dtype, 3, stream);
 }
 
 int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_channels,
@@ -497,6 +508,18 @@ int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_c
   return fused_supported(g) && plan_supported(g) && columns_first(g) ? 1 : 0;
 }
 
+size_t sdk_mapped_conv_plan_bytes_columns(int64_t image_height, int64_t image_width,
+                                          int64_t map_height, int64_t map_width,
+                                          int64_t kernel_size, int32_t num_interp_pts,
+                                          int32_t interp, int32_t dtype) {
+  if (sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width, kernel_size,
+                                 num_interp_pts, interp, dtype) == 0)
+    return 0;
+  ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
+             (int)kernel_size, num_interp_pts, interp, (int)map_width};
+  return cached_columns_plan_bytes(g);
+}
+
 int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
                                        void* plan, size_t plan_bytes, int64_t image_height,
                                        int64_t image_width, int64_t map_height, int64_t map_width,
@@ -506,10 +529,10 @@ int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* inter
   SDK_REQUIRE(sample_map && plan, "%s: NULL pointer", what);
   SDK_REQUIRE(num_interp_pts >= 0 && (num_interp_pts == 0 || interp_weights),
               "%s: weighted map needs interp_weights", what);
-  const size_t need = sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width,
-                                                 kernel_size, num_interp_pts, interp, dtype);
+  const size_t need = sdk_mapped_conv_plan_bytes_columns(
+      image_height, image_width, map_height, map_width, kernel_size, num_interp_pts, interp, dtype);
   if (need == 0)
-    return fail(SDK_ERR_UNSUPPORTED, "%s: no plan for this geometry (ask sdk_mapped_conv_plan_bytes)",
+    return fail(SDK_ERR_UNSUPPORTED, "%s: no plan for this geometry (ask sdk_mapped_conv_plan_bytes_columns)",
                 what);
   if (plan_bytes < need)
     return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, plan_bytes);

@@ -1173,7 +1173,7 @@ int fused_gemm_scatter(const ConvGeom& g, int compute, const float* pix, const f
       shared->pix_rows = true;
     }
     return columns_gemm_scatter(g, matrix_mode(compute), pix, map, wts, Wm, bias, img, workspace,
-                                stream, cached != nullptr ? cached->col2im_lists : nullptr);
+                                stream, cached != nullptr ? cached->columns_lists : nullptr);
   }
   const bool planned_fb = planned_scatter_supported(g);
   const int* generic_gate = nullptr;   // gate of the atomic scatter kernel at the end
@@ -1361,7 +1361,8 @@ int fused_gather_wgrad(const ConvGeom& g, int compute, const float* pix, const f
 namespace {
 struct CachedLayout {
   size_t plan, lists, lists4, inverse, inverse_lists, col2im, total;
-  bool has_inverse, has_col2im;
+  size_t columns, total_columns;   // ... with the inverted map of the columns route behind it
+  bool has_inverse, has_col2im, has_columns;
 };
 CachedLayout cached_layout(const ConvGeom& g) {
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -1376,9 +1377,17 @@ CachedLayout cached_layout(const ConvGeom& g) {
                   (int64_t)g.H * g.W * g.K < ((int64_t)1 << 31);
   l.inverse_lists = l.inverse + (l.has_inverse ? up(inverse_plan_bytes(g)) : 0);
   l.col2im = l.inverse_lists + (l.has_inverse ? up(tile_lists_bytes(inverse_geom(g))) : 0);
-  // the inverted map of the product and columns routes, where the map may take one of them
-  l.has_col2im = product_route_map(g) || columns_map(g);
+  // the inverted map of the product route (conv_product.hpp), where the map may take it
+  l.has_col2im = product_route_map(g);
   l.total = l.col2im + (l.has_col2im ? up(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp)) : 0);
+  // the columns route reads the same lists; a plan buffer of total_columns bytes holds them for the
+  // other maps too (apart, because they take as long to build as the rest, and a map seen once by
+  // a large forward needs neither)
+  l.has_columns = columns_map(g);
+  l.columns = l.has_col2im ? l.col2im : l.total;
+  l.total_columns =
+      l.total + (l.has_columns && !l.has_col2im
+                     ? up(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp)) : 0);
   return l;
 }
 }  // namespace
@@ -1388,7 +1397,11 @@ size_t cached_plan_bytes(const ConvGeom& g) {
   return cached_layout(g).total;
 }
 
-void load_cached_plan(const ConvGeom& g, void* buffer, CachedPlan* out) {
+size_t cached_columns_plan_bytes(const ConvGeom& g) {
+  return cached_plan_bytes(g) != 0 && columns_map(g) ? cached_layout(g).total_columns : 0;
+}
+
+void load_cached_plan(const ConvGeom& g, void* buffer, size_t bytes, CachedPlan* out) {
   const CachedLayout l = cached_layout(g);
   char* b = static_cast<char*>(buffer);
   load_plan(g, b + l.plan, &out->plan);
@@ -1400,19 +1413,24 @@ void load_cached_plan(const ConvGeom& g, void* buffer, CachedPlan* out) {
     load_tile_lists(out->inverse.plan, b + l.inverse_lists, &out->inverse_lists);
   }
   out->col2im_lists = l.has_col2im ? b + l.col2im : nullptr;
+  out->columns_lists = l.has_columns && bytes >= l.total_columns ? b + l.columns : nullptr;
 }
 
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
-                      hipStream_t stream) {
+                      size_t bytes, hipStream_t stream, int parts) {
   const CachedLayout l = cached_layout(g);
   char* b = static_cast<char*>(buffer);
   CachedPlan cp;
-  int rc = build_plan(g, map, wts, b + l.plan, stream, &cp.plan);
-  if (rc) return rc;
-  rc = build_tile_lists(cp.plan, b + l.lists, stream, &cp.lists, 0);
-  if (rc) return rc;
-  rc = build_tile_lists(cp.plan, b + l.lists4, stream, &cp.lists4, 4);
-  if (rc) return rc;
+  int rc = SDK_OK;
+  if (parts & kPlanGather) {
+    rc = build_plan(g, map, wts, b + l.plan, stream, &cp.plan);
+    if (rc) return rc;
+    rc = build_tile_lists(cp.plan, b + l.lists, stream, &cp.lists, 0);
+    if (rc) return rc;
+    rc = build_tile_lists(cp.plan, b + l.lists4, stream, &cp.lists4, 4);
+    if (rc) return rc;
+  }
+  if (!(parts & kPlanScatter)) return SDK_OK;
   if (l.has_inverse) {
     rc = build_inverse_plan(g, map, wts, b + l.inverse, stream, &cp.inverse);
     if (rc) return rc;
@@ -1424,14 +1442,16 @@ int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, voi
     rc = col2im_lists_build(map, wts, b + l.col2im, g.H, g.W, g.M, g.K, g.P, g.interp, stream);
     if (rc) return rc;
   }
+  if (l.has_columns && !l.has_col2im && bytes >= l.total_columns)
+    return build_cached_columns_plan(g, map, wts, buffer, stream);
   return SDK_OK;
 }
 
 int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                               hipStream_t stream) {
   const CachedLayout l = cached_layout(g);
-  if (!l.has_col2im) return SDK_OK;
-  return col2im_lists_build(map, wts, static_cast<char*>(buffer) + l.col2im, g.H, g.W, g.M, g.K,
+  if (!l.has_columns) return SDK_OK;
+  return col2im_lists_build(map, wts, static_cast<char*>(buffer) + l.columns, g.H, g.W, g.M, g.K,
                             g.P, g.interp, stream);
 }
 

@@ -31,17 +31,23 @@ struct CachedPlan {
   bool has_inverse = false;
   InversePlan inverse;
   TileLists inverse_lists;
-  const void* col2im_lists = nullptr;   // the inverted map of the product and columns routes, where kept
+  const void* col2im_lists = nullptr;   // the inverted map of the product route, where kept
+  const void* columns_lists = nullptr;  // ... of the columns route
 };
 // g: only H, W, M, OW, K, P and interp matter.  0 bytes: no plan for this geometry.
 size_t cached_plan_bytes(const ConvGeom& g);
+// ... with the inverted map that calls of the columns route read (0: this map's calls never do).
+size_t cached_columns_plan_bytes(const ConvGeom& g);
+// bytes: of the buffer; what a larger plan holds beside the rest is built where there is room.
+// parts: what gathers and weight gradients read, what scatters read, or both.
+constexpr int kPlanGather = 1, kPlanScatter = 2;
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
-                      hipStream_t stream);
-// The part of the same buffer that calls of the columns route (conv_columns.hpp) read.
+                      size_t bytes, hipStream_t stream, int parts = kPlanGather | kPlanScatter);
+// The part of a buffer of cached_columns_plan_bytes that those calls read, alone.
 int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                               hipStream_t stream);
 // Pointers into a buffer build_cached_plan filled for the same geometry.
-void load_cached_plan(const ConvGeom& g, void* buffer, CachedPlan* out);
+void load_cached_plan(const ConvGeom& g, void* buffer, size_t bytes, CachedPlan* out);
 
 // Calls every contraction of which runs as columns and products (conv_columns.hpp).
 bool columns_first(const ConvGeom& g);

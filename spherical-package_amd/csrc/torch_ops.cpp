@@ -86,7 +86,7 @@ struct Entry {
   c10::Storage keep_map, keep_wts;   // an address cannot be reused while its entry lives
   hipStream_t stream = nullptr;      // last user: a call on another stream is ordered behind it
   int complete = 0;
-  bool built = false;   // false: the buffer is there, nothing has needed its contents yet
+  int built = 0;   // parts of the buffer that are filled (each by the first call that reads it)
 };
 std::list<Entry> g_cache;   // most recently used last
 
@@ -172,11 +172,11 @@ Tensor bytes_on(const Tensor& ref, size_t n) {
 }
 
 // The kept plan of `key`, or one built by `build` (which returns the plan's size, 0 for none,
-// and fills the buffer it is handed on `stream`).  needed: false for a call that reads nothing of
-// the plan; its entry is made, and filled by the first call that does.
+// and fills the buffer it is handed on `stream`).  needed: the parts of the plan (bits) that this call
+// reads, 0 for none: its entry is made all the same.  build fills the parts it is asked for.
 template <typename Size, typename Build>
 PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor& wts,
-                 hipStream_t stream, Size size, Build build, bool needed = true) {
+                 hipStream_t stream, Size size, Build build, int needed = 1) {
   PlanRef out;
   if (!g_cache_enabled) return out;
   if (!tensor_key(map, &key.map) || !tensor_key(wts, &key.wts)) return out;
@@ -185,12 +185,13 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
     if (it->key == key) {
       g_cache.splice(g_cache.end(), g_cache, it);   // most recently used
       Entry& e = g_cache.back();
-      if (!e.built && (!needed || capturing(stream))) return out;
+      const int missing = needed & ~e.built;
+      if (needed == 0 || (missing != 0 && capturing(stream))) return out;
       order_behind(stream, e.stream);
       e.stream = stream;
-      if (!e.built) {
-        e.complete = build(e.plan.data_ptr(), e.nbytes);
-        e.built = true;
+      if (missing != 0) {
+        e.complete = build(e.plan.data_ptr(), e.nbytes, missing);
+        e.built |= missing;
       }
       out.plan = e.plan;
       out.nbytes = e.nbytes;
@@ -205,14 +206,14 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
   e.key = key;
   e.plan = bytes_on(ref, n);
   e.nbytes = n;
-  if (needed) e.complete = build(e.plan.data_ptr(), n);
+  if (needed != 0) e.complete = build(e.plan.data_ptr(), n, needed);
   e.built = needed;
   e.keep_map = map.storage();
   if (wts.has_value() && wts->defined()) e.keep_wts = wts->storage();
   e.stream = stream;
   while (g_cache.size() >= g_cache_max) g_cache.pop_front();
   g_cache.push_back(std::move(e));
-  if (!needed) return out;
+  if (needed == 0) return out;
   out.plan = g_cache.back().plan;
   out.nbytes = n;
   out.complete = g_cache.back().complete;
@@ -223,12 +224,14 @@ struct ConvDims {
   int64_t B, Cin, Cout, K;
 };
 
-// The plan of a (transposed) convolution call.  scatter: the call splats into the image (the
-// backward of a convolution, the forward of a transposed one); of the calls that run as columns
-// and products only those read a plan, and only the part with the inverted map.
+// The plan of a (transposed) convolution call.  gather: the call samples the image (the forward of
+// a convolution, the backward-input of a transposed one, both weight gradients); scatter: it
+// splats into it (the backward-input of a convolution, the forward of a transposed one).  Each
+// reads its part of the plan; of the calls that run as columns and products only scatters read
+// one, and only the inverted map.
 PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, const ConvDims& d,
                   int64_t img_h, int64_t img_w, int64_t P, int64_t interp, bool transposed,
-                  bool scatter, hipStream_t stream) {
+                  bool gather, bool scatter, hipStream_t stream) {
   if (ref.scalar_type() != at::kFloat) return PlanRef();
   const int64_t MH = map.size(0), MW = map.size(1), K = d.K;
   const bool columns =
@@ -244,17 +247,22 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, co
   key.interp = interp;
   return plan_for(
       key, ref, map, wts, stream,
-      [&] { return sdk_mapped_conv_plan_bytes(img_h, img_w, MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32); },
-      [&](void* buf, size_t n) {
+      [&] {
+        return columns ? sdk_mapped_conv_plan_bytes_columns(img_h, img_w, MH, MW, K, (int32_t)P,
+                                                            (int32_t)interp, SDK_F32)
+                       : sdk_mapped_conv_plan_bytes(img_h, img_w, MH, MW, K, (int32_t)P,
+                                                    (int32_t)interp, SDK_F32);
+      },
+      [&](void* buf, size_t n, int parts) {
         if (columns)
           SDK_CALL(sdk_mapped_conv_plan_build_columns, map.data_ptr(), cptr(wts), buf, n, img_h,
                    img_w, MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32, stream);
         else
-          SDK_CALL(sdk_mapped_conv_plan_build, map.data_ptr(), cptr(wts), buf, n, img_h, img_w, MH,
-                   MW, K, (int32_t)P, (int32_t)interp, SDK_F32, stream);
+          SDK_CALL(sdk_mapped_conv_plan_build_parts, map.data_ptr(), cptr(wts), buf, n, img_h, img_w,
+                   MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32, parts, stream);
         return 0;
       },
-      !columns || scatter);
+      columns ? (scatter ? 1 : 0) : (gather ? 1 : 0) | (scatter ? 2 : 0));
 }
 
 PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptTensor& wts,
@@ -280,7 +288,7 @@ PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptT
         return kind == kMaxUnpool ? sdk_mapped_max_unpool_workspace_bytes(out_h, out_w, dt)
                                   : sdk_resample_to_map_workspace_bytes(out_h, out_w, dt);
       },
-      [&](void* buf, size_t n) {
+      [&](void* buf, size_t n, int) {
         if (kind == kAvgUnpoolLists) {
           SDK_CALL(sdk_mapped_avg_unpool_lists_build, map.data_ptr(), cptr(wts), buf, n, out_h,
                    out_w, MH, MW, K, (int32_t)P, (int32_t)interp, dt, stream);
@@ -539,7 +547,7 @@ Tensor mapped_conv_forward(const Tensor& x, const Tensor& map, const OptTensor& 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, false, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -577,7 +585,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward(const Tensor& grad_outpu
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -611,7 +619,7 @@ Tensor mapped_transposed_conv_forward(const Tensor& x, const Tensor& map, const 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, out_h, out_w, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, true, s);
+  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, false, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -647,7 +655,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_transposed_conv_backward(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, OH, OW, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, OH, OW, P, interp, true, false, s);
+  PlanRef plan = conv_plan(x, map, wts, d, OH, OW, P, interp, true, true, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -689,7 +697,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward_select(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, img_h, img_w, map.size(0), map.size(1), P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, img_h, img_w, P, interp, transposed,
+  PlanRef plan = conv_plan(x, map, wts, d, img_h, img_w, P, interp, transposed, true,
                            !transposed && need_input, s);
   const auto ptr = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
   const auto call = transposed ? sdk_mapped_transposed_conv_backward_select

@@ -130,3 +130,26 @@ def test_the_inverted_map_is_built_by_the_first_backward(ops):
         eager = ops.ops.mapped_conv_backward(*args(tm))
         for o, e, r in zip(outs, eager, want):
             assert torch.equal(o.cpu(), r) and torch.equal(e.cpu(), r)
+
+
+def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):
+    """A convolution's forward builds what it gathers by, its backward the inverse; results are those
+    of a plan built at once, whichever call comes first, and of no plan."""
+    m, iw, x, w, b, g, bt = _arrays((2, 40, 72, 16, 24, 16, 24, 9, 0, 1))
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    tx, tw, tb, tg, tbt, K = t(x), t(w), t(b), t(g), t(bt), 9
+    calls = {
+        "forward": lambda tm: [ops.ops.mapped_conv_forward(tx, tm, None, tw, tb, K, 1)],
+        "weights": lambda tm: list(ops.ops.mapped_conv_backward_select(
+            tg, tm, None, tx, tw, K, 1, False, False, True))[1:],
+        "transposed": lambda tm: [ops.ops.mapped_transposed_conv_forward(tg, tm, None, tw, tbt, 16, 24, K, 1)],
+        "backward": lambda tm: list(ops.ops.mapped_conv_backward(tg, tm, None, tx, tw, tb, K, 1)),
+    }
+    ops.set_conv_plan_cache(False)
+    want = {n: f(t(m)) for n, f in calls.items()}
+    ops.set_conv_plan_cache(True)
+    for order in (list(calls), list(calls)[::-1], ["transposed", "forward", "backward", "weights"]):
+        tm = t(m)
+        for n in order:
+            for have, ref in zip(calls[n](tm), want[n]):
+                assert _rel(have.cpu().numpy(), ref.cpu().numpy()) <= 1e-6, (order, n)
