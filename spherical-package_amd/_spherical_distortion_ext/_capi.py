@@ -81,7 +81,8 @@ SIGNATURES = {
 OTHER_SYMBOLS = ("sdk_last_error", "sdk_version", "sdk_mapped_conv_workspace_bytes",
                  "sdk_resample_to_map_workspace_bytes", "sdk_mapped_max_unpool_workspace_bytes",
                  "sdk_resample_to_uv_maps_workspace_bytes", "sdk_voting_resample_workspace_bytes",
-                 "sdk_mapped_conv_plan_bytes")
+                 "sdk_mapped_conv_plan_bytes", "sdk_mapped_conv_plan_bytes_columns",
+                 "sdk_mapped_avg_unpool_lists_bytes")
 
 _lib = None
 
