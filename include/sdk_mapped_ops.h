@@ -592,10 +592,18 @@ int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* inter
                                        int64_t kernel_size, int32_t num_interp_pts, int32_t interp,
                                        int32_t dtype, sdk_stream_t stream);
 int sdk_mapped_conv_columns_enable(int32_t enabled);
-/* One part of the same plan: parts = 1 what the forward of a convolution, the backward-input of a
- * transposed one and both weight gradients read; 2 what the backward-input of a convolution and
- * the forward of a transposed one read (most of the time of a build); 3 both.  A call must find
- * the parts it reads; a combined backward reads both. */
+/* Parts of the same plan, a sum of bits: 1 the tap plan, 2 the inverse plan (most of the time of a
+ * build), 4 the inverted map; 7 is the whole.  A call must find the parts it reads:
+ * sdk_mapped_conv_plan_parts gives them for calls of these sizes that do not run by columns.
+ * gather: the call samples the image (the forward of a convolution, the backward-input of a
+ * transposed one); weights: it forms a weight gradient; scatter: it splats into the image (the
+ * other two).  0: it reads no plan. */
+int sdk_mapped_conv_plan_parts(int64_t batch, int64_t in_channels, int64_t out_channels,
+                               int64_t image_height, int64_t image_width, int64_t map_height,
+                               int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
+                               int32_t interp, int32_t dtype, int32_t compute,
+                               int32_t transposed, int32_t gather, int32_t weights,
+                               int32_t scatter);
 int sdk_mapped_conv_plan_build_parts(const void* sample_map, const void* interp_weights, void* plan,
                                      size_t plan_bytes, int64_t image_height, int64_t image_width,
                                      int64_t map_height, int64_t map_width, int64_t kernel_size,

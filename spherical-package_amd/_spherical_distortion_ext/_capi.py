@@ -64,6 +64,7 @@ SIGNATURES = {
     "sdk_mapped_conv_plan_build_parts": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 4 + [_vp],
     "sdk_mapped_conv_plan_build_columns": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],
     "sdk_mapped_conv_by_columns": [_i64] * 8 + [_i32] * 5,
+    "sdk_mapped_conv_plan_parts": [_i64] * 8 + [_i32] * 8,
     "sdk_mapped_conv_columns_enable": [_i32],
     # plans of the scatter direction
     "sdk_resample_to_map_plan_build": [_vp] * 3 + [_sz] + [_i64] * 5 + [_i32] * 3 + [_vp],

@@ -466,7 +466,7 @@ int sdk_mapped_conv_plan_build_parts(const void* sample_map, const void* interp_
                                      int32_t parts, sdk_stream_t stream) {
   const char* what = "mapped_conv_plan_build";
   SDK_REQUIRE(sample_map && plan, "%s: NULL pointer", what);
-  SDK_REQUIRE(parts >= 1 && parts <= 3, "%s: parts = %d", what, parts);
+  SDK_REQUIRE(parts >= 1 && parts <= kPlanAll, "%s: parts = %d", what, parts);
   SDK_REQUIRE(num_interp_pts >= 0 && (num_interp_pts == 0 || interp_weights),
               "%s: weighted map needs interp_weights", what);
   const size_t need = sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width,
@@ -489,7 +489,25 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
                                sdk_stream_t stream) {
   return sdk_mapped_conv_plan_build_parts(sample_map, interp_weights, plan, plan_bytes,
                                           image_height, image_width, map_height, map_width,
-                                          kernel_size, num_interp_pts, interp, dtype, 3, stream);
+                                          kernel_size, num_interp_pts, interp, dtype, kPlanAll,
+                                          stream);
+}
+
+// The geometry of a float32 call the fused kernels take; false for every other.
+static bool fused_geometry(int64_t batch, int64_t in_channels, int64_t out_channels,
+                           int64_t image_height, int64_t image_width, int64_t map_height,
+                           int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
+                           int32_t interp, int32_t dtype, int32_t compute, int32_t transposed,
+                           ConvGeom* g) {
+  if (dtype != SDK_F32 || compute == SDK_COMPUTE_UNFUSED || kernel_size < 1 || map_height < 1 ||
+      map_width < 1 || image_height < 1 || image_width < 1 || num_interp_pts < 0 ||
+      map_height * map_width >= ((int64_t)1 << 31) || image_height * image_width >= ((int64_t)1 << 31))
+    return false;
+  *g = ConvGeom{batch, (int)(transposed ? out_channels : in_channels), (int)image_height,
+                (int)image_width, (int)(transposed ? in_channels : out_channels),
+                (int)(map_height * map_width), (int)kernel_size, num_interp_pts, interp,
+                (int)map_width};
+  return fused_supported(*g) && plan_supported(*g);
 }
 
 int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_channels,
@@ -497,15 +515,24 @@ int sdk_mapped_conv_by_columns(int64_t batch, int64_t in_channels, int64_t out_c
                                int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
                                int32_t interp, int32_t dtype, int32_t compute,
                                int32_t transposed) {
-  if (dtype != SDK_F32 || compute == SDK_COMPUTE_UNFUSED || kernel_size < 1 || map_height < 1 ||
-      map_width < 1 || image_height < 1 || image_width < 1 || num_interp_pts < 0 ||
-      map_height * map_width >= ((int64_t)1 << 31) || image_height * image_width >= ((int64_t)1 << 31))
+  ConvGeom g;
+  return fused_geometry(batch, in_channels, out_channels, image_height, image_width, map_height,
+                        map_width, kernel_size, num_interp_pts, interp, dtype, compute,
+                        transposed, &g) && columns_first(g) ? 1 : 0;
+}
+
+int sdk_mapped_conv_plan_parts(int64_t batch, int64_t in_channels, int64_t out_channels,
+                               int64_t image_height, int64_t image_width, int64_t map_height,
+                               int64_t map_width, int64_t kernel_size, int32_t num_interp_pts,
+                               int32_t interp, int32_t dtype, int32_t compute,
+                               int32_t transposed, int32_t gather, int32_t weights,
+                               int32_t scatter) {
+  ConvGeom g;
+  if (!fused_geometry(batch, in_channels, out_channels, image_height, image_width, map_height,
+                      map_width, kernel_size, num_interp_pts, interp, dtype, compute, transposed,
+                      &g))
     return 0;
-  ConvGeom g{batch, (int)(transposed ? out_channels : in_channels), (int)image_height,
-             (int)image_width, (int)(transposed ? in_channels : out_channels),
-             (int)(map_height * map_width), (int)kernel_size, num_interp_pts, interp,
-             (int)map_width};
-  return fused_supported(g) && plan_supported(g) && columns_first(g) ? 1 : 0;
+  return plan_parts_read(g, gather != 0, weights != 0, scatter != 0);
 }
 
 size_t sdk_mapped_conv_plan_bytes_columns(int64_t image_height, int64_t image_width,

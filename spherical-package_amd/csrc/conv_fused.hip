@@ -1416,13 +1416,21 @@ void load_cached_plan(const ConvGeom& g, void* buffer, size_t bytes, CachedPlan*
   out->columns_lists = l.has_columns && bytes >= l.total_columns ? b + l.columns : nullptr;
 }
 
+int plan_parts_read(const ConvGeom& g, bool gather, bool wgrad, bool scatter) {
+  const bool small = small_conv_supported(g);
+  int parts = 0;
+  if ((gather && !small) || (wgrad && !small_wgrad_supported(g))) parts |= kPlanTaps;
+  if (scatter && !small) parts |= product_route(g) ? kPlanLists : kPlanInverse;
+  return parts;
+}
+
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                       size_t bytes, hipStream_t stream, int parts) {
   const CachedLayout l = cached_layout(g);
   char* b = static_cast<char*>(buffer);
   CachedPlan cp;
   int rc = SDK_OK;
-  if (parts & kPlanGather) {
+  if (parts & kPlanTaps) {
     rc = build_plan(g, map, wts, b + l.plan, stream, &cp.plan);
     if (rc) return rc;
     rc = build_tile_lists(cp.plan, b + l.lists, stream, &cp.lists, 0);
@@ -1430,14 +1438,14 @@ int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, voi
     rc = build_tile_lists(cp.plan, b + l.lists4, stream, &cp.lists4, 4);
     if (rc) return rc;
   }
-  if (!(parts & kPlanScatter)) return SDK_OK;
-  if (l.has_inverse) {
+  if ((parts & kPlanInverse) && l.has_inverse) {
     rc = build_inverse_plan(g, map, wts, b + l.inverse, stream, &cp.inverse);
     if (rc) return rc;
     rc = build_tile_lists(cp.inverse.plan, b + l.inverse_lists, stream, &cp.inverse_lists, 0,
                           kProductCap);
     if (rc) return rc;
   }
+  if (!(parts & kPlanLists)) return SDK_OK;
   if (l.has_col2im) {
     rc = col2im_lists_build(map, wts, b + l.col2im, g.H, g.W, g.M, g.K, g.P, g.interp, stream);
     if (rc) return rc;

@@ -39,10 +39,13 @@ size_t cached_plan_bytes(const ConvGeom& g);
 // ... with the inverted map that calls of the columns route read (0: this map's calls never do).
 size_t cached_columns_plan_bytes(const ConvGeom& g);
 // bytes: of the buffer; what a larger plan holds beside the rest is built where there is room.
-// parts: what gathers and weight gradients read, what scatters read, or both.
-constexpr int kPlanGather = 1, kPlanScatter = 2;
+// parts: the tap plan (gathers and weight gradients), the inverse plan (scatters), the inverted
+// map (scatters by the product route).
+constexpr int kPlanTaps = 1, kPlanInverse = 2, kPlanLists = 4, kPlanAll = 7;
+// Those that calls of g read, 0 for none: layers of a few image channels have kernels of their own.
+int plan_parts_read(const ConvGeom& g, bool gather, bool wgrad, bool scatter);
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
-                      size_t bytes, hipStream_t stream, int parts = kPlanGather | kPlanScatter);
+                      size_t bytes, hipStream_t stream, int parts = kPlanAll);
 // The part of a buffer of cached_columns_plan_bytes that those calls read, alone.
 int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                               hipStream_t stream);

@@ -173,7 +173,7 @@ Tensor bytes_on(const Tensor& ref, size_t n) {
 
 // The kept plan of `key`, or one built by `build` (which returns the plan's size, 0 for none,
 // and fills the buffer it is handed on `stream`).  needed: the parts of the plan (bits) that this call
-// reads, 0 for none: its entry is made all the same.  build fills the parts it is asked for.
+// reads, 0 for none: its entry is made all the same, without memory.  build fills the parts it is asked for.
 template <typename Size, typename Build>
 PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor& wts,
                  hipStream_t stream, Size size, Build build, int needed = 1) {
@@ -190,6 +190,7 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
       order_behind(stream, e.stream);
       e.stream = stream;
       if (missing != 0) {
+        if (!e.plan.defined()) e.plan = bytes_on(ref, e.nbytes);
         e.complete = build(e.plan.data_ptr(), e.nbytes, missing);
         e.built |= missing;
       }
@@ -204,9 +205,11 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
   if (n == 0) return out;
   Entry e;
   e.key = key;
-  e.plan = bytes_on(ref, n);
   e.nbytes = n;
-  if (needed != 0) e.complete = build(e.plan.data_ptr(), n, needed);
+  if (needed != 0) {
+    e.plan = bytes_on(ref, n);
+    e.complete = build(e.plan.data_ptr(), n, needed);
+  }
   e.built = needed;
   e.keep_map = map.storage();
   if (wts.has_value() && wts->defined()) e.keep_wts = wts->storage();
@@ -225,13 +228,15 @@ struct ConvDims {
 };
 
 // The plan of a (transposed) convolution call.  gather: the call samples the image (the forward of
-// a convolution, the backward-input of a transposed one, both weight gradients); scatter: it
-// splats into it (the backward-input of a convolution, the forward of a transposed one).  Each
-// reads its part of the plan; of the calls that run as columns and products only scatters read
-// one, and only the inverted map.
+// a convolution, the backward-input of a transposed one); weights: it forms a weight gradient;
+// scatter: it splats into the image (the other two).  Each reads its part of the plan, a layer
+// of a few image channels none; of the calls that run as columns and products only scatters
+// read one, the inverted map.  (Measured, first step on a new map, all parts of a plan built ->
+// those that are read: 4 x 512 x 1024, 3 -> 32 channels, no picture gradient 694 -> 342 us,
+// 64 x 128, 3 -> 16 547 -> 175 us; level-7 icosphere decoder block 3.24 -> 2.88 ms.)
 PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, const ConvDims& d,
                   int64_t img_h, int64_t img_w, int64_t P, int64_t interp, bool transposed,
-                  bool gather, bool scatter, hipStream_t stream) {
+                  bool gather, bool weights, bool scatter, hipStream_t stream) {
   if (ref.scalar_type() != at::kFloat) return PlanRef();
   const int64_t MH = map.size(0), MW = map.size(1), K = d.K;
   const bool columns =
@@ -262,7 +267,10 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, co
                    MH, MW, K, (int32_t)P, (int32_t)interp, SDK_F32, parts, stream);
         return 0;
       },
-      columns ? (scatter ? 1 : 0) : (gather ? 1 : 0) | (scatter ? 2 : 0));
+      columns ? (scatter ? 1 : 0)
+              : sdk_mapped_conv_plan_parts(d.B, d.Cin, d.Cout, img_h, img_w, MH, MW, K, (int32_t)P,
+                                           (int32_t)interp, SDK_F32, current_mode(),
+                                           transposed ? 1 : 0, gather, weights, scatter));
 }
 
 PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptTensor& wts,
@@ -547,7 +555,7 @@ Tensor mapped_conv_forward(const Tensor& x, const Tensor& map, const OptTensor& 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, false, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, false, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -585,7 +593,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward(const Tensor& grad_outpu
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, true, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, false, true, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -619,7 +627,7 @@ Tensor mapped_transposed_conv_forward(const Tensor& x, const Tensor& map, const 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, out_h, out_w, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, false, true, s);
+  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, false, false, true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -655,7 +663,7 @@ std::tuple<Tensor, Tensor, Tensor> mapped_transposed_conv_backward(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, OH, OW, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, OH, OW, P, interp, true, true, false, s);
+  PlanRef plan = conv_plan(x, map, wts, d, OH, OW, P, interp, true, true, true, false, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -697,8 +705,8 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward_select(
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, img_h, img_w, map.size(0), map.size(1), P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, img_h, img_w, P, interp, transposed, true,
-                           !transposed && need_input, s);
+  PlanRef plan = conv_plan(x, map, wts, d, img_h, img_w, P, interp, transposed,
+                           transposed && need_input, need_params, !transposed && need_input, s);
   const auto ptr = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
   const auto call = transposed ? sdk_mapped_transposed_conv_backward_select
                                : sdk_mapped_conv_backward_select;

@@ -153,3 +153,33 @@ def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):
         for n in order:
             for have, ref in zip(calls[n](tm), want[n]):
                 assert _rel(have.cpu().numpy(), ref.cpu().numpy()) <= 1e-6, (order, n)
+
+
+@pytest.mark.parametrize("shape", [
+    (2, 3, 24, 20, 36, 16, 24, 9, 0, 1),    # a first layer reads no plan
+    (1, 4, 128, 20, 36, 16, 24, 9, 0, 1),   # ... nor with two blocks of columns
+    (1, 4, 100, 13, 17, 24, 30, 25, 0, 1),  # its weight gradient does: too many accumulators
+    (2, 16, 24, 40, 72, 16, 24, 9, 0, 0),   # the scatter by the product route
+])
+def test_layers_on_a_shared_map_build_what_each_reads(ops, tile_kernels, shape):
+    """Layers of different widths on one map, in both orders: the parts one of them left out are
+    there for the next; results are those without plans."""
+    m, iw, x, w, b, g, bt = _arrays(shape)
+    K, interp = shape[7], shape[9]
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    wide = _arrays(shape[:1] + (40, 72) + shape[3:])
+
+    def step(tm, arrays):
+        _, _, x, w, b, g, bt = (None if a is None else t(a) for a in arrays)
+        return [ops.ops.mapped_conv_forward(x, tm, None, w, b, K, interp),
+                *ops.ops.mapped_conv_backward(g, tm, None, x, w, b, K, interp)]
+
+    layers = [(m, iw, x, w, b, g, bt), wide]
+    ops.set_conv_plan_cache(False)
+    want = [step(t(m), a) for a in layers]
+    ops.set_conv_plan_cache(True)
+    for order in ((0, 1, 0), (1, 0, 1)):
+        tm = t(m)
+        for i in order:
+            for have, ref in zip(step(tm, layers[i]), want[i]):
+                assert _rel(have.cpu().numpy(), ref.cpu().numpy()) <= 2e-6, (order, i)
