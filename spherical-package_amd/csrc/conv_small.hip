@@ -939,8 +939,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
 bool small_conv_supported(const ConvGeom& g) {
   return g.Cg >= 1 && g.Cg <= 4 && g.K >= 1 && g.K <= 25 && g.Cp >= 1 && g.Cp <= 128 &&
          g.B <= 65535 && (int64_t)g.Cg * g.H * g.W < ((int64_t)1 << 31) &&
-         (int64_t)g.M * g.K * (g.P > 0 ? g.P : 1) * 2 < ((int64_t)1 << 31) &&
-         g.M <= (1 << 22);   // 64 rows of the output within a 31-bit byte offset
+         (int64_t)g.M * g.K * (g.P > 0 ? g.P : 1) * 2 < ((int64_t)1 << 31);
 }
 
 static int padded_blocks(int64_t n) {
@@ -1020,7 +1019,10 @@ int small_forward(const ConvGeom& g, const float* img, const float* map, const f
   // the vector unit does Cg * K multiply-adds per output.  K = 9, bilinear, 4 x 256 x 512: 3 -> 16
   // channels 28 us per pixel against 30, 3 -> 32 43 against 32, 1 -> 32 21 against 23, 4 -> 48 62
   // against 57.
-  if (g.Cg == 1 || g.Cp <= 16)
+  // (A workgroup of the matrix kernel stores through one descriptor: 64 rows of the output have to
+  // lie within its 31-bit byte offsets.  Larger pictures take the kernel that addresses flatly.)
+  constexpr int kDescriptorPixels = 1 << 22;
+  if (g.Cg == 1 || g.Cp <= 16 || g.M > kDescriptorPixels)
     return small_pixel_forward(g, img, map, wts, Wm, bias, pix, stream);
   SmallTiling tl = small_tiling(g);
   const int64_t tiles = (int64_t)tl.nx * tl.ny;

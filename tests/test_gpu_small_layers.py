@@ -102,3 +102,24 @@ def test_zero_weight_taps_are_not_read(ops):
     assert torch.equal(y, torch.full_like(y, 3.0 * K))
     _, gw, _ = ops.mapped_conv_backward(_t(g), _t(m), None, _t(x), _t(w), _t(b), K, 1)
     assert torch.equal(gw, torch.full_like(gw, 4.0 * H * W))
+
+
+@pytest.mark.parametrize("OH,OW", [(2048, 2048), (2049, 2048)])
+def test_both_sides_of_the_stores_of_a_descriptor(ops, OH, OW):
+    """4194304 output pixels are the most the matrix kernel's stores reach; a picture of more takes
+    the flat forward, and its backward the same kernels as every first layer's."""
+    gen = torch.Generator(device=DEV).manual_seed(OH)
+    H, W, Cin, Cout = 32, 64, 3, 17
+    at = torch.randint(0, H * W, (OH, OW, 1), generator=gen, device=DEV)
+    m = torch.stack([at % W, at // W], -1).float()
+    x, w, b, g = (torch.randn(s, generator=gen, device=DEV) for s in (
+        (1, Cin, H, W), (Cout, Cin, 1), (Cout,), (1, Cout, OH, OW)))
+    y = ops.mapped_conv_forward(x, m, None, w, b, 1, 0)
+    gi, gw, gb = ops.mapped_conv_backward(g, m, None, x, w, b, 1, 0)
+    cols, wide = x.double().reshape(Cin, -1)[:, at.reshape(-1)], g.double().reshape(Cout, -1)
+    want = (w[..., 0].double() @ cols + b[:, None].double()).reshape(y.shape)
+    assert float((y - want).abs().max() / want.abs().max()) <= 1e-6    # sums of four terms
+    grad = torch.zeros(Cin, H * W, dtype=torch.float64, device=DEV)
+    grad.index_add_(1, at.reshape(-1), w[..., 0].double().T @ wide)
+    for got, ref in ((gi.reshape(Cin, -1), grad), (gw[..., 0], wide @ cols.T), (gb, wide.sum(1))):
+        assert float((got - ref).abs().max() / ref.abs().max()) <= 1e-4

@@ -315,3 +315,16 @@ def test_plan_cache_evicts_the_least_recently_used_entry():
         _ops._PLAN_CACHE.clear()
         _ops._PLAN_CACHE.update(saved)
         _ops._PLAN_CACHE_MAX = saved_max
+
+
+def test_first_layers_of_any_picture_size_read_no_plan():
+    """Layers of at most four image channels have kernels of their own, whatever the picture's
+    size (2048 x 4096 is 2^23 output pixels): no part of a plan is read for them."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    for h, w in ((64, 128), (2048, 2048), (2049, 2048), (1920, 3840), (2048, 4096)):
+        for cin, cout in ((3, 32), (1, 16), (4, 64)):
+            for transposed in (0, 1):
+                channels = (cout, cin) if transposed else (cin, cout)
+                assert lib.sdk_mapped_conv_plan_parts(1, *channels, h, w, h, w, 9, 0, 1,
+                                                      _capi.SDK_F32, 0, transposed, 1, 1, 1) == 0
