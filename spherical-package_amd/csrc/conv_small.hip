@@ -310,7 +310,9 @@ __device__ __forceinline__ int windows_at_once(const TileWindow& win, int batche
 // Copies the windows of `count` batch elements from img0 on into LDS, all channels of an element
 // together, a zero element behind each.  A wave takes 64 columns of a row at a time, of four
 // batch elements together; everything but a lane's column is uniform over the wave.
-template <int CG>
+// PAD: there may be fewer channels than CG (two at least), and the others have to read as zero: their
+// weights are zero, but zero times an infinity is not.
+template <int CG, bool PAD>
 __device__ __forceinline__ void stage_windows(const TileWindow& win, const float* __restrict__ img0,
                                               int count, size_t HW, int Cg, int W, int waves,
                                               float* __restrict__ lds) {
@@ -336,6 +338,10 @@ __device__ __forceinline__ void stage_windows(const TileWindow& win, const float
           const float* src = row + (size_t)min(j0 + i, count - 1) * Cg * HW;
 #pragma unroll
           for (int ch = 0; ch < CG; ++ch) v[i][ch] = (src + (size_t)(ch < Cg ? ch : 0) * HW)[col];
+          if constexpr (PAD) {
+#pragma unroll
+            for (int ch = 2; ch < CG; ++ch) v[i][ch] = ch < Cg ? v[i][ch] : 0.0f;
+          }
         }
         if (on) {
 #pragma unroll
@@ -343,7 +349,7 @@ __device__ __forceinline__ void stage_windows(const TileWindow& win, const float
             if (j0 + i < count) {
               Elem* dst = out + (j0 + i) * stride + at;
               if constexpr (CG == 1) *dst = v[i][0];
-              else *dst = f32x4{v[i][0], v[i][1], v[i][2], CG > 3 ? v[i][CG - 1] : 0.0f};
+              else *dst = f32x4{v[i][0], v[i][1], CG > 2 ? v[i][CG > 2 ? 2 : 0] : 0.0f, CG > 3 ? v[i][CG - 1] : 0.0f};
             }
           }
         }
@@ -363,7 +369,7 @@ __device__ __forceinline__ int opaque(int x) {
 
 // col[g][c] += the lane's column values of G samples.  The reads of a sample are requested before
 // the blend of the one before it.
-template <int INTERP, int CG, int G>
+template <int INTERP, int CG, int G, bool PAD>
 __device__ __forceinline__ void add_columns(const LaneTaps<INTERP, G>& t, bool fits,
                                             const float* __restrict__ window,
                                             const float* __restrict__ img_b, size_t HW, int Cg,
@@ -410,7 +416,8 @@ __device__ __forceinline__ void add_columns(const LaneTaps<INTERP, G>& t, bool f
       for (int i = 0; i < N; ++i)
 #pragma unroll
         for (int c = 0; c < CG; ++c)
-          col[g][c] = __builtin_fmaf(t.co[g][i], o[i] >= 0 ? d[i][c] : 0.0f, col[g][c]);
+          col[g][c] = __builtin_fmaf(t.co[g][i], o[i] >= 0 && (!PAD || c < 2 || c < Cg) ? d[i][c] : 0.0f,
+                                     col[g][c]);
       __builtin_amdgcn_sched_barrier(0);   // one sample's reads in flight: registers
     }
   }
@@ -549,6 +556,14 @@ __global__ __launch_bounds__(kSmThreads) void small_pixel_forward_kernel(
         for (int c = 0; c < CG; ++c) col[k0 + g][c] = 0.0f;
     }
   }
+  // what has no sample or channel of its own (the group's last repeated, channel 0) meets weights of
+  // zero, but zero times an infinity is not zero
+  if (K < KPAD || Cg < CG) {
+#pragma unroll
+    for (int k = 0; k < KPAD; ++k)
+#pragma unroll
+      for (int c = 0; c < CG; ++c) col[k][c] = k < K && c < Cg ? col[k][c] : 0.0f;
+  }
   float* out = pix + (size_t)blockIdx.y * Cp * M + m;
   for (int n = 0; n < Cp; ++n) {
     const float* wrow = wl + n * (CG * KMAX);
@@ -641,6 +656,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward
     const float* __restrict__ Wm, const float* __restrict__ bias, float* __restrict__ pix, int Cg,
     int H, int W, int Cp, int M, int OW, int K, int P, int B, SmallTiling tl) {
   constexpr int E = SmallElem<CG>::kFloats, HALF = NG * kSmGroup, STEPS = HALF * CG;
+  constexpr bool kPad = NG > 1;   // (CG is the image's own number of channels otherwise)
   extern __shared__ __align__(16) float lds[];
   float* window = lds;                                  // [kSmWindow + 1][E]
   float* wl = lds + (kSmWindow + 1) * E + (CG == 1 ? 3 : 0);   // [STEPS][64][NB]
@@ -680,7 +696,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward
     if (b == b_begin || j == at_once) {
       j = 0;
       __syncthreads();   // the windows' last readers are through (first round: red, wl, bl)
-      if (win.fits) stage_windows<CG>(win, img_b, min(at_once, b_end - b), HW, Cg, W, tl.waves, window);
+      if (win.fits) stage_windows<CG, kPad>(win, img_b, min(at_once, b_end - b), HW, Cg, W, tl.waves, window);
       __syncthreads();
     }
     const float* window_b = window + j * stride * E;
@@ -701,7 +717,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward
 #pragma unroll
         for (int c = 0; c < CG; ++c) col[g][c] = 0.0f;
       if constexpr (kHoist) {
-        add_columns<INTERP, CG, kSmGroup>(taps, win.fits, window_b, img_b, HW, Cg, col);
+        add_columns<INTERP, CG, kSmGroup, kPad>(taps, win.fits, window_b, img_b, HW, Cg, col);
       } else {
         const int q = WEIGHTED ? P : 1, k0 = gr * kSmGroup;
         for (int p = 0; p < q; ++p) {
@@ -710,7 +726,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward
           LaneSamples<INTERP, kSmGroup> s;
           decode<INTERP, WEIGHTED, kSmGroup>(pt, lp.samples - k0, win.anchor, H, W, s);
           place(s, win, W, E * 4, taps);
-          add_columns<INTERP, CG, kSmGroup>(taps, win.fits, window_b, img_b, HW, Cg, col);
+          add_columns<INTERP, CG, kSmGroup, kPad>(taps, win.fits, window_b, img_b, HW, Cg, col);
         }
       }
 #pragma unroll
@@ -843,7 +859,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
       if (b == b_begin || j == at_once) {
         j = 0;
         __syncthreads();   // the windows' last readers are through
-        if (win.fits) stage_windows<CG>(win, img_b, min(at_once, b_end - b), HW, Cg, W, tl.waves, window);
+        if (win.fits) stage_windows<CG, false>(win, img_b, min(at_once, b_end - b), HW, Cg, W, tl.waves, window);
         __syncthreads();
       }
       const float* window_b = window + j * stride * E;
@@ -855,7 +871,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
 #pragma unroll
           for (int c = 0; c < CG; ++c) col[g][c] = 0.0f;
         if constexpr (kHoist) {
-          add_columns<INTERP, CG, kSmGroup>(taps, win.fits, window_b, img_b, HW, Cg, col);
+          add_columns<INTERP, CG, kSmGroup, false>(taps, win.fits, window_b, img_b, HW, Cg, col);
         } else {
           const int q = WEIGHTED ? P : 1, k0 = gr * kSmGroup;
           for (int p = 0; p < q; ++p) {
@@ -864,7 +880,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
             LaneSamples<INTERP, kSmGroup> s;
             decode<INTERP, WEIGHTED, kSmGroup>(pt, lp.samples - k0, win.anchor, H, W, s);
             place(s, win, W, E * 4, taps);
-            add_columns<INTERP, CG, kSmGroup>(taps, win.fits, window_b, img_b, HW, Cg, col);
+            add_columns<INTERP, CG, kSmGroup, false>(taps, win.fits, window_b, img_b, HW, Cg, col);
           }
         }
 #pragma unroll
@@ -974,12 +990,14 @@ static SmallTiling small_tiling(const ConvGeom& g) {
       if (g.Cp <= 32) {                                                                      \
         constexpr int NBv = 1;                                                               \
         if (g.Cg <= 1) { constexpr int CGv = 1; CALL; }                                      \
-        else if (g.Cg <= 3) { constexpr int CGv = 3; CALL; }                                 \
+        else if (g.Cg == 2) { constexpr int CGv = 2; CALL; }                                 \
+        else if (g.Cg == 3) { constexpr int CGv = 3; CALL; }                                 \
         else { constexpr int CGv = 4; CALL; }                                                \
       } else {                                                                               \
         constexpr int NBv = 2;                                                               \
         if (g.Cg <= 1) { constexpr int CGv = 1; CALL; }                                      \
-        else if (g.Cg <= 3) { constexpr int CGv = 3; CALL; }                                 \
+        else if (g.Cg == 2) { constexpr int CGv = 2; CALL; }                                 \
+        else if (g.Cg == 3) { constexpr int CGv = 3; CALL; }                                 \
         else { constexpr int CGv = 4; CALL; }                                                \
       }                                                                                      \
     } else {                                                                                 \

@@ -123,3 +123,24 @@ def test_both_sides_of_the_stores_of_a_descriptor(ops, OH, OW):
     grad.index_add_(1, at.reshape(-1), w[..., 0].double().T @ wide)
     for got, ref in ((gi.reshape(Cin, -1), grad), (gw[..., 0], wide @ cols.T), (gb, wide.sum(1))):
         assert float((got - ref).abs().max() / ref.abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("wild", [0.0, 0.4])
+@pytest.mark.parametrize("Cin,Cout,K", [(3, 17, 9), (3, 17, 11), (2, 17, 9), (2, 17, 11), (2, 8, 9),
+                                        (2, 8, 11), (3, 8, 11)])
+def test_infinities_stay_in_their_channel(ops, oracle, Cin, Cout, K, wild):
+    """Window elements and weights are padded to three or four channels: an infinity of the image
+    gives infinities, no NaN from the padding's zero weights."""
+    rng = np.random.default_rng(Cin + K)
+    OH, OW = 37, 70
+    m = _near(rng, OH, OW, K, 1.6, wild)
+    x = rng.standard_normal((2, Cin, OH, OW)).astype(np.float32)
+    x[0, 0, 5, 7], x[1, Cin - 1, 20, 30] = np.inf, np.inf
+    w = rng.uniform(0.1, 1, (Cout, Cin, K)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    y = ops.mapped_conv_forward(_t(x), _t(m), None, _t(w), _t(b), K, 0).cpu().numpy()
+    want = oracle.mapped_conv_forward(x, m, w, b, K, 0, None)
+    assert np.isinf(want).any() and not np.isnan(want).any()
+    assert np.array_equal(np.isinf(y), np.isinf(want)) and not np.isnan(y).any()
+    on = np.isfinite(want)
+    assert relerr(y[on], want[on]) <= 1e-5
