@@ -51,6 +51,14 @@ inline void launch_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t s
 // behind the test of the tap it belongs to, one branch, one load and one wait per tap.
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 
+// Between the LDS writes of some lanes of a wave and the reads of others.  The hardware serves a
+// wave's LDS accesses in order; this keeps the compiler from moving them past each other.
+__device__ __forceinline__ void wave_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ----------------------------------------------------------------------------- column values
 // Pixel tiles: `waves` rows of 32 pixels where the grid has that many rows, else one row of
 // 32 * waves pixels (vertex lists).
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
 #pragma unroll
         for (int q = 0; q < 4; ++q) av[a][q] = next[a][q];
       if (b + 1 < b_end) request(b + 1);
-      // (a wave's LDS accesses are in order: its own writes are there when it reads them)
+      wave_exchange();
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         f32x4 bv[CB];
@@ -913,6 +921,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
                                                                 0, 0, 0);
           }
       }
+      wave_exchange();   // (the next batch element's columns go where these were)
     }
     lp = lp_next;
   }

@@ -53,9 +53,9 @@ def _near(rng, OH, OW, K, spread, wild, stride=1):
 
 @pytest.mark.parametrize("interp", [0, 1, 2])
 @pytest.mark.parametrize("B,Cin,Cout,OH,OW,K", [
-    (1, 1, 8, 3, 31, 9),      # fewer rows than waves, no full piece, one pixel row block
+    (1, 1, 8, 3, 31, 9),      # three rows, no full piece, one pixel row block
     (2, 3, 17, 5, 33, 10),    # one pixel in a second piece; the largest single sample group
-    (9, 3, 32, 40, 64, 9),    # four waves a workgroup; more batch elements than fit at once
+    (9, 3, 32, 40, 64, 9),    # full pieces; nine batch elements through the weight gradient
     (3, 4, 33, 37, 70, 11),   # a second 32-row block; the smallest of three sample groups
     (1, 2, 65, 1, 130, 1),    # one row, one sample, a second channel chunk
     (2, 4, 128, 9, 40, 25),
@@ -64,6 +64,38 @@ def test_edges_of_pieces_groups_and_blocks(ops, oracle, B, Cin, Cout, OH, OW, K,
     rng = np.random.default_rng(OH * OW + K)
     m = _near(rng, OH, OW, K, 1.6, 0.0)
     _check(ops, oracle, B, Cin, Cout, m, None, OH, OW, interp, 3)
+
+
+def _tiling(B, OH, OW):
+    """(waves of a workgroup, stacked?, tiles, batch elements of a forward's and of a weight gradient's
+    workgroup, workgroups of the latter that walk tiles), as small_tiling and its callers choose."""
+    pieces = -(-OW // 32)
+    waves = 4 if pieces * OH * B >= 1024 else 1
+    stacked = OH >= waves
+    tiles = pieces * -(-OH // waves) if stacked else -(-OW // (32 * waves)) * OH
+    want = min(768, max(64, int(8 * (tiles * B) ** 0.5)))
+    walkers = min(tiles, want)
+    return (waves, stacked, tiles, -(-B // min(B, -(-2048 // tiles))),
+            -(-B // min(B, max(1, want // walkers))), walkers)
+
+
+@pytest.mark.parametrize("Cin,Cout,K,B,OH,OW,stride", [
+    (3, 17, 7, 1, 1, 33001, 1),     # a vertex list: four waves side by side
+    (3, 17, 9, 1, 3, 12001, 1),     # fewer rows than a workgroup's waves
+    (3, 20, 9, 4, 101, 70, 1),      # four waves, the last tiles cut below and on the right
+    (3, 17, 9, 6, 245, 515, 1),     # several batch elements in the windows at once, more to come
+    (4, 33, 9, 4, 245, 515, 2),     # windows so large that each batch element has its own turn
+])
+def test_workgroups_of_four_waves(ops, oracle, Cin, Cout, K, B, OH, OW, stride):
+    waves, stacked, tiles, forward, weights, walkers = _tiling(B, OH, OW)
+    assert waves == 4 and stacked == (OH >= 4)
+    if OH == 245:    # the batch loops and the walk over several tiles
+        assert forward > 1 and weights == B and walkers < tiles
+    else:
+        assert OW % 32 and OH % 4
+    rng = np.random.default_rng(OW)
+    m = _near(rng, OH, OW, K, 1.6 if OH > 3 else 0.9, 0.0, stride)
+    _check(ops, oracle, B, Cin, Cout, m, None, OH * stride, OW * stride, 1, OH)
 
 
 @pytest.mark.parametrize("interp", [0, 1, 2])
