@@ -1835,27 +1835,62 @@ namespace {
 // FILL = false: counts the taps of every image element; true: writes them at the slots the
 // scanned counts reserve.  Taps outside the image and taps with a zero coefficient are left
 // out (by both passes alike).
+// A workgroup's taps of one element take one atomic together, through a table in LDS: an element
+// claims the table's place its number hashes to (where several do, one wins and the others' taps go
+// to memory singly).  Atomics on one address are served about every 10 ns: a tenth of 295 thousand
+// samples on one spot cost the two passes 2.5 ms one by one.
+constexpr int kInvertSlots = 1024;
+
 template <int INTERP, bool WEIGHTED, bool FILL>
 __global__ __launch_bounds__(kBlock) void col2im_invert_kernel(
     const float* __restrict__ map, const float* __restrict__ wts, int H, int W, int M, int K,
     int P, int* __restrict__ counter, int* __restrict__ src, float* __restrict__ co) {
-  const int pix = blockIdx.x * kBlock + threadIdx.x;   // sample m * K + k
-  if (pix >= M * K) return;
+  constexpr int N = PointTaps<float, INTERP>::N;
+  __shared__ int s_tag[kInvertSlots], s_count[kInvertSlots];
+  const int64_t pix = (int64_t)blockIdx.x * kBlock + threadIdx.x;   // sample m * K + k
+  const bool exists = pix < (int64_t)M * K;
   const int q = WEIGHTED ? P : 1;
   PointTaps<float, INTERP> t;
   for (int p = 0; p < q; ++p) {
-    const size_t s = (size_t)pix * q + p;
+    const size_t s = (size_t)(exists ? pix : 0) * q + p;
     t.set(map[s * 2], map[s * 2 + 1], H, W);
     const float wt = WEIGHTED ? wts[s] : 1.0f;
+    float c[N];
+    bool on[N];
+    int h[N], rank[N];
 #pragma unroll
-    for (int i = 0; i < PointTaps<float, INTERP>::N; ++i) {
-      const float c = INTERP == 0 ? wt : t.w[i] * wt;
-      if (t.off[i] >= 0 && c != 0.0f) {
-        const int slot = atomicAdd(&counter[t.off[i]], 1);
-        if constexpr (FILL) {
-          src[slot] = pix;
-          co[slot] = c;
-        }
+    for (int i = 0; i < N; ++i) {
+      c[i] = INTERP == 0 ? wt : t.w[i] * wt;
+      on[i] = exists && t.off[i] >= 0 && c[i] != 0.0f;
+      h[i] = (int)(((unsigned)t.off[i] * 2654435761u) >> 22);   // (top ten bits)
+    }
+    __syncthreads();   // (the table's last readers are through)
+    for (int e = threadIdx.x; e < kInvertSlots; e += kBlock) s_count[e] = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (on[i]) s_tag[h[i]] = t.off[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      rank[i] = on[i] && s_tag[h[i]] == t.off[i] ? atomicAdd(&s_count[h[i]], 1) : -1;
+    __syncthreads();
+    for (int e = threadIdx.x; e < kInvertSlots; e += kBlock) {
+      const int n = s_count[e];
+      if (n > 0) {
+        const int first = atomicAdd(&counter[s_tag[e]], n);
+        if constexpr (FILL) s_count[e] = first;
+      }
+    }
+    if constexpr (FILL) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      if (!on[i]) continue;
+      if constexpr (FILL) {
+        const int slot = rank[i] >= 0 ? s_count[h[i]] + rank[i] : atomicAdd(&counter[t.off[i]], 1);
+        src[slot] = (int)pix;
+        co[slot] = c[i];
+      } else if (rank[i] < 0) {
+        atomicAdd(&counter[t.off[i]], 1);
       }
     }
   }
@@ -1868,8 +1903,9 @@ constexpr int kScanPer = 16;
 constexpr int kScanTile = kBlock * kScanPer;
 
 // The block's exclusive scan of one value per thread; *total: the block's sum (every thread).
+template <int THREADS = kBlock>
 __device__ __forceinline__ int block_exclusive_scan(int mine, int* total) {
-  __shared__ int wave_sum[kBlock / 64];
+  __shared__ int wave_sum[THREADS / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = mine;
 #pragma unroll
@@ -1882,7 +1918,7 @@ __device__ __forceinline__ int block_exclusive_scan(int mine, int* total) {
   __syncthreads();
   int before = 0, all = 0;
 #pragma unroll
-  for (int w = 0; w < kBlock / 64; ++w) {
+  for (int w = 0; w < THREADS / 64; ++w) {
     before += w < wave ? wave_sum[w] : 0;
     all += wave_sum[w];
   }
@@ -1942,10 +1978,9 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(const int* __restric
 // Every element's entries sorted by source, then coefficient (the fill appends in the order
 // its atomics are served).  A wave takes one element after another, a list of at most kSortLds
 // entries in LDS, by a bitonic network whose exchanges all ascend, so that any length will do
-// (pairs past the end are left out: what is not there counts as larger than everything).  A
-// longer list, of a map that sends hundreds of samples to one image element, is sorted in
-// memory by the whole workgroup.  (One thread per list, by selection: a list of 100 entries, a 5 x 5
-// kernel's, costs it 5000 steps, one of ten thousand seconds.)
+// (pairs past the end are left out: what is not there counts as larger than everything).  Longer
+// lists are col2im_sort_long_kernel's.  (One thread per list, by selection: a list of 100 entries, a
+// 5 x 5 kernel's, costs it 5000 steps, one of ten thousand seconds.)
 constexpr int kSortLds = 512;
 constexpr int kSortTargets = 16;   // elements of a workgroup
 
@@ -1995,27 +2030,105 @@ __global__ __launch_bounds__(kBlock) void col2im_sort_kernel(const int* __restri
       co[beg + i] = lc[i];
     }
   }
-  for (int t = 0; t < kSortTargets && u0 + t < HW; ++t) {
-    const int beg = offset[u0 + t], n = offset[u0 + t + 1] - beg;
-    if (n <= kSortLds) continue;   // (uniform)
-    int* s = src + beg;
-    float* c = co + beg;
-    for (int64_t k = 2; k < 2 * (int64_t)n; k <<= 1) {
-      for (int64_t j = k >> 1; j > 0; j >>= 1) {
-        for (int i = threadIdx.x; i < n; i += kBlock) {
-          const int64_t o = j == (k >> 1) ? (i ^ (k - 1)) : (i ^ j);
-          if (o > i && o < n) {
-            const int si = s[i], so = s[o];
-            const float ci = c[i], cj = c[o];
-            if (entry_less(so, cj, si, ci)) {
-              s[i] = so;
-              c[i] = cj;
-              s[o] = si;
-              c[o] = ci;
+}
+
+// The lists of more than kSortLds entries, of a map that sends hundreds of samples to one image
+// element: a workgroup each.  Up to kSortLong entries are sorted in LDS by the same network.  A longer
+// list is made anew from the map, in the order of its points: a thread takes eight consecutive points,
+// and a scan over the workgroup gives its entries their places, so that the time is that of reading
+// the map once.  (First step of a 64 -> 64 layer, 1 x 128 x 256, a tenth of the 295 thousand samples on
+// one spot, lists of 29 thousand: 7474 us with the lists sorted in memory by one workgroup and an
+// atomic per tap in col2im_invert_kernel, 1721 now.)
+constexpr int kSortLong = 6144;
+constexpr int kSortLongThreads = 1024;
+
+template <int INTERP, bool WEIGHTED>
+__global__ __launch_bounds__(kSortLongThreads) void col2im_sort_long_kernel(
+    const float* __restrict__ map, const float* __restrict__ wts, int H, int W, int64_t points,
+    int P, const int* __restrict__ offset, int* __restrict__ src, float* __restrict__ co, int HW) {
+  constexpr int kPer = 8, kThreads = kSortLongThreads;
+  __shared__ int s_src[kSortLong];
+  __shared__ float s_co[kSortLong];
+  __shared__ int s_list[kThreads], s_lists;
+  const int q = WEIGHTED ? P : 1;
+  // neighbouring elements go to different workgroups: a crowded spot has four
+  for (int64_t u0 = blockIdx.x; u0 < HW; u0 += (int64_t)gridDim.x * kThreads) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_lists = 0;
+    __syncthreads();
+    const int64_t mine = u0 + (int64_t)gridDim.x * threadIdx.x;
+    if (mine < HW && offset[mine + 1] - offset[mine] > kSortLds)
+      s_list[atomicAdd(&s_lists, 1)] = (int)mine;
+    __syncthreads();
+    const int lists = s_lists;
+    for (int l = 0; l < lists; ++l) {
+      const int u = s_list[l], beg = offset[u], n = offset[u + 1] - beg;   // (uniform)
+      if (n <= kSortLong) {
+        for (int i = threadIdx.x; i < n; i += kThreads) {
+          s_src[i] = src[beg + i];
+          s_co[i] = co[beg + i];
+        }
+        for (int k = 2; k < 2 * n; k <<= 1)
+          for (int j = k >> 1; j > 0; j >>= 1) {
+            __syncthreads();
+            for (int i = threadIdx.x; i < n; i += kThreads) {
+              const int o = j == (k >> 1) ? (i ^ (k - 1)) : (i ^ j);
+              if (o > i && o < n) {
+                const int si = s_src[i], so = s_src[o];
+                const float ci = s_co[i], cj = s_co[o];
+                if (entry_less(so, cj, si, ci)) {
+                  s_src[i] = so;
+                  s_co[i] = cj;
+                  s_src[o] = si;
+                  s_co[o] = ci;
+                }
+              }
             }
           }
-        }
         __syncthreads();
+        for (int i = threadIdx.x; i < n; i += kThreads) {
+          src[beg + i] = s_src[i];
+          co[beg + i] = s_co[i];
+        }
+        __syncthreads();   // (the next list goes where this one was)
+        continue;
+      }
+      int placed = 0;
+      for (int64_t p0 = 0; p0 < points && placed < n; p0 += kThreads * kPer) {
+        const int64_t first = p0 + threadIdx.x * kPer;
+        // the thread's entries, counted (at < 0) or written from place `at` on
+        auto entries = [&](int at) {
+          int found = 0;
+          float x[kPer], y[kPer], wt[kPer];   // (all requested before the first is used)
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) {
+            const int64_t s = min(first + i, points - 1);
+            x[i] = map[s * 2];
+            y[i] = map[s * 2 + 1];
+            wt[i] = WEIGHTED ? wts[s] : 1.0f;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) {
+            PointTaps<float, INTERP> t;
+            t.set(x[i], y[i], H, W);
+#pragma unroll
+            for (int j = 0; j < PointTaps<float, INTERP>::N; ++j) {
+              const float c = INTERP == 0 ? wt[i] : t.w[j] * wt[i];
+              if (t.off[j] != u || c == 0.0f || first + i >= points) continue;
+              if (at >= 0 && at + found < n) {
+                src[beg + at + found] = (int)((first + i) / q);
+                co[beg + at + found] = c;
+              }
+              ++found;
+            }
+          }
+          return found;
+        };
+        int total;
+        const int before = block_exclusive_scan<kThreads>(entries(-1), &total);
+        if (total > 0) entries(placed + before);
+        placed += total;
       }
     }
   }
@@ -2230,6 +2343,11 @@ int col2im_lists_build(const float* map, const float* wts, void* lists, int H, i
                               stream, map, wts, H, W, M, K, P, l.cursor, l.src, l.co)));
   launch(col2im_sort_kernel, dim3((unsigned)ceil_div(HW, kSortTargets)), dim3(kBlock), stream,
          (const int*)l.offset, l.src, l.co, HW);
+  SDK_DISPATCH_INTERP(interp, P,
+                      (launch((col2im_sort_long_kernel<INTERP, WEIGHTED>),
+                              dim3((unsigned)std::min(HW, 256)), dim3(kSortLongThreads), stream,
+                              map, wts, H, W, (int64_t)M * K * (P > 0 ? P : 1), P,
+                              (const int*)l.offset, l.src, l.co, HW)));
   SDK_LAUNCH_CHECK("mapped_conv(inverted map)");
   return SDK_OK;
 }

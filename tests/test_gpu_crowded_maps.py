@@ -81,3 +81,17 @@ def test_a_crowded_map_does_not_stall_a_layer(ops):
         tm = _t(_crowded(np.random.default_rng(1), m, share))
         kept.append(_seconds(lambda: ops.mapped_conv_backward(g, tm, None, x, w, b, 9, 1))[1])
     assert kept[2] <= 4 * kept[1]
+
+
+def test_a_crowded_map_is_inverted_in_time(ops):
+    """The first step on a map as above, its lists included: 17 times the even map's when one
+    workgroup sorted lists of thirty thousand in memory."""
+    m = workloads.gnomonic_kernel_map(128, 256).astype(np.float32)
+    x, g = torch.randn(1, 64, 128, 256, device=DEV), torch.randn(1, 64, 128, 256, device=DEV)
+    w, b = torch.randn(64, 64, 9, device=DEV) / 24, torch.randn(64, device=DEV)
+    first = []
+    for share in (0.0, 0.0, 0.1):          # (the first warms up)
+        maps = [_t(_crowded(np.random.default_rng(i), m, share)) for i in range(3)]
+        first.append(min(_seconds(lambda tm=tm: ops.mapped_conv_backward(g, tm, None, x, w, b, 9, 1))[0]
+                         for tm in maps))
+    assert first[2] <= 6 * first[1]
