@@ -2211,30 +2211,87 @@ __global__ __launch_bounds__(kBlock) void col2im_gather_kernel(
 
 // Entries of one image element that come from the same pooled pixel (neighbours in a sorted
 // list) become one with the sum of their coefficients; src then names the pooled pixel and
-// count[u] the entries left.
+// count[u] the entries left.  A thread merges an element's list, the wave one of more than
+// kUnpoolLong entries (of a map that sends many samples to one element): 64 entries at a time, the sums
+// of equal neighbours by a segmented scan, the last of which goes on with the next 64.
+constexpr int kUnpoolLong = 256;
+
 __global__ __launch_bounds__(kBlock) void unpool_merge_kernel(const int* __restrict__ offset,
                                                               int* __restrict__ src,
                                                               float* __restrict__ co,
                                                               int* __restrict__ count, int HW,
                                                               int K) {
   const int u = blockIdx.x * kBlock + threadIdx.x;
-  if (u >= HW) return;
-  const int beg = offset[u], end = offset[u + 1];
-  int at = beg - 1, cur = -1;
-  float sum = 0.0f;
-  for (int e = beg; e < end; ++e) {
-    const int m = src[e] / K;
-    const float c = co[e];
-    if (m != cur) {
-      if (at >= beg) co[at] = sum;
-      src[++at] = m;
-      cur = m;
-      sum = 0.0f;
+  const int lane = threadIdx.x & 63;
+  const int beg = u < HW ? offset[u] : 0, end = u < HW ? offset[u + 1] : 0;
+  if (u < HW && end - beg <= kUnpoolLong) {
+    int at = beg - 1, cur = -1;
+    float sum = 0.0f;
+    for (int e = beg; e < end; ++e) {
+      const int m = src[e] / K;
+      const float c = co[e];
+      if (m != cur) {
+        if (at >= beg) co[at] = sum;
+        src[++at] = m;
+        cur = m;
+        sum = 0.0f;
+      }
+      sum += c;
     }
-    sum += c;
+    if (at >= beg) co[at] = sum;
+    count[u] = at - beg + 1;
   }
-  if (at >= beg) co[at] = sum;
-  count[u] = at - beg + 1;
+  unsigned long long crowds = __ballot(end - beg > kUnpoolLong);
+  while (crowds != 0) {
+    const int owner = __ffsll(crowds) - 1;
+    crowds &= crowds - 1;
+    const int b = __builtin_amdgcn_readlane(beg, owner), e = __builtin_amdgcn_readlane(end, owner);
+    int out = b;                  // entries written so far end here
+    int carry_m = -1;             // pooled pixel of the last one, its sum
+    float carry = 0.0f;
+    for (int e0 = b; e0 < e; e0 += 4 * 64) {
+      int ms[4];
+      float cs[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = min(e0 + 64 * i + lane, e - 1);
+        ms[i] = src[at] / K;
+        cs[i] = co[at];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int here = min(64, e - (e0 + 64 * i));   // entries of this piece (uniform)
+        if (here <= 0) break;
+        const int m = ms[i];
+        float c = cs[i];
+        int before = __shfl_up(m, 1);
+        if (lane == 0) before = carry_m;
+        const bool head = lane < here && m != before;
+        const unsigned long long heads = __ballot(head);
+        int started = head;       // a head lies between the lanes summed so far and this one
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const float cd = __shfl_up(c, d);
+          const int sd = __shfl_up(started, d);
+          if (lane >= d && !started) {
+            c += cd;
+            started = sd;
+          }
+        }
+        const int nth = __popcll(heads & (~0ull >> (63 - lane)));   // heads up to this lane
+        if (nth == 0) c += carry;
+        const bool last = lane < here && (lane + 1 == here || ((heads >> (lane + 1)) & 1) != 0);
+        if (last) {
+          src[out - 1 + nth] = m;
+          co[out - 1 + nth] = c;
+        }
+        out += __popcll(heads);
+        carry_m = __builtin_amdgcn_readlane(m, here - 1);
+        carry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), here - 1));
+      }
+    }
+    if (lane == owner) count[u] = out - b;
+  }
 }
 
 // Average unpooling of blended samples as a gather over the merged lists: a thread owns an image
@@ -2242,39 +2299,59 @@ __global__ __launch_bounds__(kBlock) void unpool_merge_kernel(const int* __restr
 // pixels, so the reads of a wave fall into few lines.  (The tile kernel adds K * 4 values per
 // pooled pixel and plane to LDS by compare-and-swap: 4 x 48 planes of 190 x 378 from 95 x 189,
 // 94 us; and a map whose windows it cannot hold, stride 1 at 256 x 512, went to atomics in
-// memory: 7.9 ms for 128 planes.)
+// memory: 7.9 ms for 128 planes.)  Lists of more than kUnpoolLong entries are the whole wave's, an
+// entry of four to each lane in turn, the lanes' sums added by a tree.  (2 x 16 planes of 256 x 512, stride
+// 1, a tenth of the samples on one spot, forward + backward: 18.3 ms with one thread a list, 0.81 now.)
 template <int PC>
 __global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
     const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
     const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
     int M, int planes, float K) {
   const int u = banded_pixel_block() * kBlock + threadIdx.x;
-  if (u >= HW) return;
   const int plane0 = blockIdx.y * PC;
   const int np = min(PC, planes - plane0);
-  const int beg = offset[u], n = count[u];
+  const int beg = u < HW ? offset[u] : 0, n = u < HW ? count[u] : 0;
   const float* g0 = gout + (size_t)plane0 * M;
-  float acc[PC];
+  // sum += entries first .. first + 3, first + step .. first + step + 3, ... of those before end
+  auto add = [&](int first, int end, int step, float (&sum)[PC]) {
 #pragma unroll
-  for (int j = 0; j < PC; ++j) acc[j] = 0.0f;
-  for (int e = 0; e < n; e += 4) {
-    int m[4];
-    float c[4], v[4][PC];
+    for (int j = 0; j < PC; ++j) sum[j] = 0.0f;
+    for (int e = first; e < end; e += step) {
+      int m[4];
+      float c[4], v[4][PC];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int at = beg + min(e + i, n - 1);
-      m[i] = src[at];
-      c[i] = co[at];
+      for (int i = 0; i < 4; ++i) {
+        const int at = min(e + i, end - 1);
+        m[i] = src[at];
+        c[i] = co[at];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) v[i][j] = g0[(size_t)(j < np ? j : 0) * M + m[i]];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) sum[j] += e + i < end ? c[i] * v[i][j] : 0.0f;
     }
+  };
+  float acc[PC];
+  add(beg, n <= kUnpoolLong ? beg + n : beg, 4, acc);
+  unsigned long long crowds = __ballot(n > kUnpoolLong);
+  while (crowds != 0) {
+    const int owner = __ffsll(crowds) - 1, lane = threadIdx.x & 63;
+    crowds &= crowds - 1;
+    const int b = __builtin_amdgcn_readlane(beg, owner), all = __builtin_amdgcn_readlane(n, owner);
+    float part[PC];
+    add(b + 4 * lane, b + all, 4 * 64, part);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < PC; ++j) {
 #pragma unroll
-      for (int j = 0; j < PC; ++j) v[i][j] = g0[(size_t)(j < np ? j : 0) * M + m[i]];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < PC; ++j) acc[j] += e + i < n ? c[i] * v[i][j] : 0.0f;
+      for (int d = 1; d < 64; d <<= 1) part[j] += __shfl_xor(part[j], d);
+      if (lane == owner) acc[j] = part[j];
+    }
   }
+  if (u >= HW) return;
 #pragma unroll
   for (int j = 0; j < PC; ++j)
     if (j < np) gin[(size_t)(plane0 + j) * HW + u] = acc[j] / K;

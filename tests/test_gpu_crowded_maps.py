@@ -95,3 +95,40 @@ def test_a_crowded_map_is_inverted_in_time(ops):
         first.append(min(_seconds(lambda tm=tm: ops.mapped_conv_backward(g, tm, None, x, w, b, 9, 1))[0]
                          for tm in maps))
     assert first[2] <= 6 * first[1]
+
+
+@pytest.mark.parametrize("share", [0.002, 0.02, 0.1, 0.3, 1.0])
+@pytest.mark.parametrize("C,P", [(3, 0), (11, 0), (2, 3)])
+def test_average_unpooling_of_crowded_maps(ops, oracle, C, P, share):
+    H, W, OH, OW, K = 24, 41, 48, 70, 9
+    rng = np.random.default_rng(int(1000 * share) + C)
+    shape = (OH, OW, K) + ((P,) if P else ())
+    m = np.stack([rng.uniform(-1, W, shape), rng.uniform(-1, H, shape)], -1)
+    m = _crowded(rng, m, share)
+    iw = rng.uniform(0.1, 1, shape).astype(np.float32) if P else None
+    g = rng.standard_normal((1, C, OH, OW)).astype(np.float32)
+    got = [ops.mapped_avg_unpool(_t(g), _t(m), _t(iw), H, W, K, 1) for _ in range(2)]
+    assert torch.equal(*got)             # two maps, two builds of their lists
+    f64 = lambda a: None if a is None else a.astype(np.float64)  # noqa: E731
+    want = oracle.mapped_avg_unpool(f64(g), f64(m), H, W, K, 1, f64(iw))
+    mag = oracle.mapped_avg_unpool(np.abs(f64(g)), f64(m), H, W, K, 1, f64(iw))
+    # n float32 additions of n terms each way (n: the samples on the spot at most, merged and then
+    # summed): 2 n * 2^-24 of the sum of magnitudes would bound any order; the longest chain is 256
+    # entries, or a wave's share of a list, and its tree
+    chain = max(256, OH * OW * K * max(P, 1) // 64 + 70)
+    assert np.all(np.abs(got[0].cpu().numpy() - want) <= chain * 2.0 ** -23 * mag + 4e-6 * np.abs(g).max())
+
+
+def test_a_crowded_map_does_not_stall_average_pooling(ops):
+    """2 x 16 planes of 256 x 512, stride 1, a tenth of the samples on one spot: 18 ms (the even
+    map's 0.1) with one entry after the other, the first step, lists included, 78 ms (0.5)."""
+    m = workloads.gnomonic_kernel_map(256, 512).astype(np.float32)
+    g = torch.randn(2, 16, 256, 512, device=DEV)
+    first, kept = [], []
+    for share in (0.0, 0.0, 0.1):          # (the first warms up)
+        maps = [_t(_crowded(np.random.default_rng(i), m, share)) for i in range(3)]
+        runs = [_seconds(lambda tm=tm: ops.mapped_avg_unpool(g, tm, None, 256, 512, 9, 1)) for tm in maps]
+        first.append(min(r[0] for r in runs))
+        kept.append(min(r[1] for r in runs))
+    print("first", first, "kept", kept)
+    assert kept[2] <= 25 * kept[1] and first[2] <= 40 * first[1]
