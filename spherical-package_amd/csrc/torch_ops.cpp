@@ -173,12 +173,13 @@ Tensor bytes_on(const Tensor& ref, size_t n) {
 
 // The kept plan of `key`, or one built by `build` (which returns the plan's size, 0 for none,
 // and fills the buffer it is handed on `stream`).  needed: the parts of the plan (bits) that this call
-// reads, 0 for none: its entry is made all the same, without memory.  build fills the parts it is asked for.
+// reads; build fills the parts it is asked for.  A call that reads none leaves the cache as it is: an
+// entry for it would hold nothing but its map, and push out a plan.
 template <typename Size, typename Build>
 PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor& wts,
                  hipStream_t stream, Size size, Build build, int needed = 1) {
   PlanRef out;
-  if (!g_cache_enabled) return out;
+  if (!g_cache_enabled || needed == 0) return out;
   if (!tensor_key(map, &key.map) || !tensor_key(wts, &key.wts)) return out;
   std::lock_guard<std::mutex> lock(g_mu);
   for (auto it = g_cache.begin(); it != g_cache.end(); ++it) {
@@ -186,11 +187,10 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
       g_cache.splice(g_cache.end(), g_cache, it);   // most recently used
       Entry& e = g_cache.back();
       const int missing = needed & ~e.built;
-      if (needed == 0 || (missing != 0 && capturing(stream))) return out;
+      if (missing != 0 && capturing(stream)) return out;
       order_behind(stream, e.stream);
       e.stream = stream;
       if (missing != 0) {
-        if (!e.plan.defined()) e.plan = bytes_on(ref, e.nbytes);
         e.complete = build(e.plan.data_ptr(), e.nbytes, missing);
         e.built |= missing;
       }
@@ -206,17 +206,14 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
   Entry e;
   e.key = key;
   e.nbytes = n;
-  if (needed != 0) {
-    e.plan = bytes_on(ref, n);
-    e.complete = build(e.plan.data_ptr(), n, needed);
-  }
+  e.plan = bytes_on(ref, n);
+  e.complete = build(e.plan.data_ptr(), n, needed);
   e.built = needed;
   e.keep_map = map.storage();
   if (wts.has_value() && wts->defined()) e.keep_wts = wts->storage();
   e.stream = stream;
   while (g_cache.size() >= g_cache_max) g_cache.pop_front();
   g_cache.push_back(std::move(e));
-  if (needed == 0) return out;
   out.plan = g_cache.back().plan;
   out.nbytes = n;
   out.complete = g_cache.back().complete;

@@ -47,6 +47,16 @@ def oracle():
     return _oracle
 
 
+@pytest.fixture
+def tile_kernels():
+    """Small float32 convolutions of this thread on the tile kernels instead of the columns route."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    before = lib.sdk_mapped_conv_columns_enable(0)
+    yield
+    lib.sdk_mapped_conv_columns_enable(before)
+
+
 # ---------------------------------------------------------------------------------------------
 # Builders shared by the oracle (CPU) and GPU replays of the reference's known-answer tests.
 # ---------------------------------------------------------------------------------------------

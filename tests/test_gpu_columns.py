@@ -1,8 +1,8 @@
 """Small convolution calls as columns and matrix products (csrc/conv_columns.hip) against the
 oracle in float64 accumulation, and the tile kernels at the same sizes.
 
-The tile kernels are reached at small sizes by turning the route off for the thread
-(sdk_mapped_conv_columns_enable); the plan tests then run on them.
+The tile kernels are reached at small sizes by turning the route off for the thread (the
+tile_kernels fixture); the plan tests then run on them.
 """
 import numpy as np
 import pytest
@@ -24,15 +24,6 @@ def ops():
 def oracle():
     from oracle import oracle as o
     return o
-
-
-@pytest.fixture
-def tile_kernels(ops):
-    from _spherical_distortion_ext import _capi
-    lib = _capi.load()
-    before = lib.sdk_mapped_conv_columns_enable(0)
-    yield
-    lib.sdk_mapped_conv_columns_enable(before)
 
 
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
@@ -103,8 +94,8 @@ def test_columns_route_matches_the_oracle(ops, oracle, tc, mode):
 
 
 def test_the_inverted_map_is_built_by_the_first_backward(ops):
-    """A forward makes the map's cache entry and builds nothing; results do not depend on which
-    call comes first, and a replayed capture whose entry is not built gives the eager result."""
+    """A forward builds nothing; results do not depend on which call comes first, and a replayed
+    capture whose entry is not built gives the eager result."""
     m, iw, x, w, b, g, _ = _arrays((2, 16, 24, 11, 13, 9, 10, 9, 0, 1))
     t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
     tx, tw, tb, tg, K = t(x), t(w), t(b), t(g), 9
@@ -113,8 +104,7 @@ def test_the_inverted_map_is_built_by_the_first_backward(ops):
     tm = t(m)
     before = ops.plan_cache_size()
     ops.ops.mapped_conv_forward(tx, tm, None, tw, tb, K, 1)
-    after = ops.plan_cache_size()
-    assert after - before in (0, 1)        # (0: the cache was full and dropped another)
+    assert ops.plan_cache_size() == before
     side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -130,6 +120,32 @@ def test_the_inverted_map_is_built_by_the_first_backward(ops):
         eager = ops.ops.mapped_conv_backward(*args(tm))
         for o, e, r in zip(outs, eager, want):
             assert torch.equal(o.cpu(), r) and torch.equal(e.cpu(), r)
+
+
+def test_calls_that_read_no_plan_leave_the_cache_alone(ops):
+    """Forwards on pictures of new sizes (columns, first layers) neither push out a plan nor keep
+    a map."""
+    t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
+    shapes = [(2, 16, 24, 11, 13, 9, 10, 9, 0, 1), (2, 3, 24, 20, 36, 16, 24, 9, 0, 1)]
+
+    def forward(tc):
+        m, _, x, w, b, _, _ = _arrays(tc)
+        ops.ops.mapped_conv_forward(t(x), t(m), None, t(w), t(b), tc[7], tc[9])
+
+    ops.set_conv_plan_cache(False)
+    ops.set_conv_plan_cache(True, max_entries=2)
+    try:
+        for h in (12, 13):      # two training maps with their inverted maps
+            m, _, x, w, b, g, _ = _arrays((2, 16, 24, 11, 13, h, 10, 9, 0, 1))
+            ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 9, 1)
+        assert ops.plan_cache_size() == 2
+        held = torch.cuda.memory_allocated()
+        for tc in shapes * 2:
+            forward(tc)
+        assert ops.plan_cache_size() == 2
+        assert torch.cuda.memory_allocated() == held     # (a plan let go, a map kept would show)
+    finally:
+        ops.set_conv_plan_cache(True, max_entries=16)
 
 
 def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):

@@ -102,7 +102,7 @@ def test_compiled_and_python_operators_agree(ops, weighted, dtype, interp, cache
         ops.set_conv_plan_cache(True)
 
 
-def test_compiled_layer_follows_the_compute_mode_and_the_cache_switches(ops):
+def test_compiled_layer_follows_the_compute_mode_and_the_cache_switches(ops, tile_kernels):
     if ops._native is None:
         pytest.skip("the compiled operator layer is not built")
     d = _inputs(False, np.float32)
