@@ -571,8 +571,13 @@ int sdk_mapped_conv_plan_build(const void* sample_map, const void* interp_weight
  *                                             calls are given the same plan_bytes; with a
  *                                             plan of sdk_mapped_conv_plan_bytes such calls
  *                                             invert the map in their workspace.
- *   sdk_mapped_conv_plan_build_columns(...)   fills, of a buffer of that size, only the part
- *                                             such calls read; for no other call
+ *   sdk_mapped_conv_columns_bytes(...)        size of a buffer with the inverted map alone (0 as
+ *                                             above), which only such calls take, told from a plan
+ *                                             by exactly this plan_bytes: 10 MB where the plan with
+ *                                             it has 100 (3 x 3 kernels, bilinear, 128 x 256)
+ *   sdk_mapped_conv_plan_build_columns(...)   fills such a buffer; or, of a buffer of
+ *                                             sdk_mapped_conv_plan_bytes_columns, only the part
+ *                                             such calls read, for no other call
  *   sdk_mapped_conv_columns_enable(0 / 1)     turns the route off / on for the calling thread
  *                                             (to measure or test the tile kernels at small
  *                                             sizes); returns the previous value.  Workspace
@@ -586,6 +591,9 @@ size_t sdk_mapped_conv_plan_bytes_columns(int64_t image_height, int64_t image_wi
                                           int64_t map_height, int64_t map_width,
                                           int64_t kernel_size, int32_t num_interp_pts,
                                           int32_t interp, int32_t dtype);
+size_t sdk_mapped_conv_columns_bytes(int64_t image_height, int64_t image_width, int64_t map_height,
+                                     int64_t map_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype);
 int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
                                        void* plan, size_t plan_bytes, int64_t image_height,
                                        int64_t image_width, int64_t map_height, int64_t map_width,

@@ -83,6 +83,7 @@ OTHER_SYMBOLS = ("sdk_last_error", "sdk_version", "sdk_mapped_conv_workspace_byt
                  "sdk_resample_to_map_workspace_bytes", "sdk_mapped_max_unpool_workspace_bytes",
                  "sdk_resample_to_uv_maps_workspace_bytes", "sdk_voting_resample_workspace_bytes",
                  "sdk_mapped_conv_plan_bytes", "sdk_mapped_conv_plan_bytes_columns",
+                 "sdk_mapped_conv_columns_bytes",
                  "sdk_mapped_avg_unpool_lists_bytes")
 
 _lib = None
@@ -117,6 +118,8 @@ def load():
     lib.sdk_voting_resample_workspace_bytes.argtypes = [_i64] * 4
     lib.sdk_voting_resample_workspace_bytes.restype = _sz
     lib.sdk_mapped_conv_plan_bytes.argtypes = [_i64] * 5 + [_i32] * 3
+    lib.sdk_mapped_conv_columns_bytes.restype = _sz
+    lib.sdk_mapped_conv_columns_bytes.argtypes = [_i64] * 5 + [_i32] * 3
     lib.sdk_mapped_conv_plan_bytes_columns.restype = _sz
     lib.sdk_mapped_conv_plan_bytes_columns.argtypes = [_i64] * 5 + [_i32] * 3
     lib.sdk_mapped_avg_unpool_lists_bytes.restype = _sz

@@ -61,7 +61,12 @@ int check_plan(const char* what, const ConvGeom& g, int dtype, int compute, Plan
   if (plan.buffer == nullptr || dtype != SDK_F32 || compute == SDK_COMPUTE_UNFUSED ||
       !fused_supported(g))
     return SDK_OK;
-  const size_t need = cached_plan_bytes(g);
+  const size_t need = cached_plan_bytes(g), alone = columns_alone_bytes(g);
+  if (alone != 0 && plan.bytes == alone)
+    return columns_first(g) ? SDK_OK
+                            : fail(SDK_ERR_WORKSPACE,
+                                   "%s: the plan buffer has %zu bytes, those of an inverted map alone, "
+                                   "which this call does not read", what, plan.bytes);
   if (need == 0 || plan.bytes < need)
     return fail(SDK_ERR_WORKSPACE, "%s: the plan buffer has %zu bytes, this geometry's plan %zu",
                 what, plan.bytes, need);
@@ -478,6 +483,9 @@ int sdk_mapped_conv_plan_build_parts(const void* sample_map, const void* interp_
     return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, plan_bytes);
   ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
              (int)kernel_size, num_interp_pts, interp, (int)map_width};
+  if (plan_bytes == columns_alone_bytes(g))
+    return fail(SDK_ERR_WORKSPACE, "%s: a buffer of %zu bytes is taken for an inverted map alone", what,
+                plan_bytes);
   return build_cached_plan(g, (const float*)sample_map, (const float*)interp_weights, plan,
                            plan_bytes, (hipStream_t)stream, parts);
 }
@@ -547,6 +555,17 @@ size_t sdk_mapped_conv_plan_bytes_columns(int64_t image_height, int64_t image_wi
   return cached_columns_plan_bytes(g);
 }
 
+size_t sdk_mapped_conv_columns_bytes(int64_t image_height, int64_t image_width, int64_t map_height,
+                                     int64_t map_width, int64_t kernel_size,
+                                     int32_t num_interp_pts, int32_t interp, int32_t dtype) {
+  if (sdk_mapped_conv_plan_bytes(image_height, image_width, map_height, map_width, kernel_size,
+                                 num_interp_pts, interp, dtype) == 0)
+    return 0;
+  ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
+             (int)kernel_size, num_interp_pts, interp, (int)map_width};
+  return columns_alone_bytes(g);
+}
+
 int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* interp_weights,
                                        void* plan, size_t plan_bytes, int64_t image_height,
                                        int64_t image_width, int64_t map_height, int64_t map_width,
@@ -561,12 +580,13 @@ int sdk_mapped_conv_plan_build_columns(const void* sample_map, const void* inter
   if (need == 0)
     return fail(SDK_ERR_UNSUPPORTED, "%s: no plan for this geometry (ask sdk_mapped_conv_plan_bytes_columns)",
                 what);
-  if (plan_bytes < need)
-    return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, got %zu", what, need, plan_bytes);
   ConvGeom g{1, 1, (int)image_height, (int)image_width, 1, (int)(map_height * map_width),
              (int)kernel_size, num_interp_pts, interp, (int)map_width};
+  if (plan_bytes < need && plan_bytes != columns_alone_bytes(g))
+    return fail(SDK_ERR_WORKSPACE, "%s: needs %zu bytes, or %zu for the inverted map alone, got %zu",
+                what, need, columns_alone_bytes(g), plan_bytes);
   return build_cached_columns_plan(g, (const float*)sample_map, (const float*)interp_weights, plan,
-                                   (hipStream_t)stream);
+                                   plan_bytes, (hipStream_t)stream);
 }
 
 int sdk_mapped_conv_forward(const void* input, const void* sample_map, const void* interp_weights,

@@ -1401,9 +1401,18 @@ size_t cached_columns_plan_bytes(const ConvGeom& g) {
   return cached_plan_bytes(g) != 0 && columns_map(g) ? cached_layout(g).total_columns : 0;
 }
 
+size_t columns_alone_bytes(const ConvGeom& g) {
+  if (cached_columns_plan_bytes(g) == 0) return 0;
+  return ((col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp) + 255) & ~(size_t)255) + 128;
+}
+
 void load_cached_plan(const ConvGeom& g, void* buffer, size_t bytes, CachedPlan* out) {
-  const CachedLayout l = cached_layout(g);
   char* b = static_cast<char*>(buffer);
+  if (bytes == columns_alone_bytes(g)) {
+    out->columns_lists = b;
+    return;
+  }
+  const CachedLayout l = cached_layout(g);
   load_plan(g, b + l.plan, &out->plan);
   load_tile_lists(out->plan, b + l.lists, &out->lists);
   load_tile_lists(out->plan, b + l.lists4, &out->lists4);
@@ -1451,16 +1460,17 @@ int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, voi
     if (rc) return rc;
   }
   if (l.has_columns && !l.has_col2im && bytes >= l.total_columns)
-    return build_cached_columns_plan(g, map, wts, buffer, stream);
+    return build_cached_columns_plan(g, map, wts, buffer, bytes, stream);
   return SDK_OK;
 }
 
 int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
-                              hipStream_t stream) {
+                              size_t bytes, hipStream_t stream) {
   const CachedLayout l = cached_layout(g);
   if (!l.has_columns) return SDK_OK;
-  return col2im_lists_build(map, wts, static_cast<char*>(buffer) + l.columns, g.H, g.W, g.M, g.K,
-                            g.P, g.interp, stream);
+  const size_t at = bytes == columns_alone_bytes(g) ? 0 : l.columns;
+  return col2im_lists_build(map, wts, static_cast<char*>(buffer) + at, g.H, g.W, g.M, g.K, g.P,
+                            g.interp, stream);
 }
 
 }  // namespace sdk

@@ -38,6 +38,9 @@ struct CachedPlan {
 size_t cached_plan_bytes(const ConvGeom& g);
 // ... with the inverted map that calls of the columns route read (0: this map's calls never do).
 size_t cached_columns_plan_bytes(const ConvGeom& g);
+// A buffer with that inverted map alone.  The size tells it from a plan: plans are multiples of 256
+// bytes, this is half of that more.
+size_t columns_alone_bytes(const ConvGeom& g);
 // bytes: of the buffer; what a larger plan holds beside the rest is built where there is room.
 // parts: the tap plan (gathers and weight gradients), the inverse plan (scatters), the inverted
 // map (scatters by the product route).
@@ -46,9 +49,10 @@ constexpr int kPlanTaps = 1, kPlanInverse = 2, kPlanLists = 4, kPlanAll = 7;
 int plan_parts_read(const ConvGeom& g, bool gather, bool wgrad, bool scatter);
 int build_cached_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
                       size_t bytes, hipStream_t stream, int parts = kPlanAll);
-// The part of a buffer of cached_columns_plan_bytes that those calls read, alone.
+// The part of a buffer of cached_columns_plan_bytes that those calls read, or a buffer of
+// columns_alone_bytes (bytes says which).
 int build_cached_columns_plan(const ConvGeom& g, const float* map, const float* wts, void* buffer,
-                              hipStream_t stream);
+                              size_t bytes, hipStream_t stream);
 // Pointers into a buffer build_cached_plan filled for the same geometry.
 void load_cached_plan(const ConvGeom& g, void* buffer, size_t bytes, CachedPlan* out);
 

@@ -66,8 +66,7 @@ bool tensor_key(const OptTensor& t, TensorKey* k) {
   return true;
 }
 
-enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kConvColumns = 4,
-            kAvgUnpoolLists = 5 };
+enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kAvgUnpoolLists = 4 };
 
 struct Key {
   int kind = 0, device = 0, dtype = 0;
@@ -79,14 +78,21 @@ struct Key {
   }
 };
 
-struct Entry {
-  Key key;
+struct Buffer {
   Tensor plan;
   size_t nbytes = 0;
+  int built = 0;   // parts of the buffer that are filled (each by the first call that reads it)
+};
+// kSide: the inverted map that convolutions by columns read (much smaller than the plan of the others
+// on the same map).
+enum Slot { kMain = 0, kSide = 1 };
+
+struct Entry {
+  Key key;
+  Buffer buffers[2];   // by Slot, each made by the first call that reads it
   c10::Storage keep_map, keep_wts;   // an address cannot be reused while its entry lives
   hipStream_t stream = nullptr;      // last user: a call on another stream is ordered behind it
   int complete = 0;
-  int built = 0;   // parts of the buffer that are filled (each by the first call that reads it)
 };
 std::list<Entry> g_cache;   // most recently used last
 
@@ -177,46 +183,54 @@ Tensor bytes_on(const Tensor& ref, size_t n) {
 // entry for it would hold nothing but its map, and push out a plan.
 template <typename Size, typename Build>
 PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor& wts,
-                 hipStream_t stream, Size size, Build build, int needed = 1) {
+                 hipStream_t stream, Size size, Build build, int needed = 1, Slot slot = kMain) {
   PlanRef out;
   if (!g_cache_enabled || needed == 0) return out;
   if (!tensor_key(map, &key.map) || !tensor_key(wts, &key.wts)) return out;
   std::lock_guard<std::mutex> lock(g_mu);
   for (auto it = g_cache.begin(); it != g_cache.end(); ++it) {
-    if (it->key == key) {
-      g_cache.splice(g_cache.end(), g_cache, it);   // most recently used
-      Entry& e = g_cache.back();
-      const int missing = needed & ~e.built;
-      if (missing != 0 && capturing(stream)) return out;
-      order_behind(stream, e.stream);
-      e.stream = stream;
-      if (missing != 0) {
-        e.complete = build(e.plan.data_ptr(), e.nbytes, missing);
-        e.built |= missing;
+    if (!(it->key == key)) continue;
+    g_cache.splice(g_cache.end(), g_cache, it);   // most recently used
+    Entry& e = g_cache.back();
+    Buffer& buf = e.buffers[slot];
+    const int missing = needed & ~buf.built;
+    if (missing != 0) {
+      if (capturing(stream)) return out;
+      if (!buf.plan.defined()) {
+        buf.nbytes = size();
+        if (buf.nbytes == 0) return out;
+        buf.plan = bytes_on(ref, buf.nbytes);
       }
-      out.plan = e.plan;
-      out.nbytes = e.nbytes;
-      out.complete = e.complete;
-      return out;
     }
+    order_behind(stream, e.stream);
+    e.stream = stream;
+    if (missing != 0) {
+      e.complete = build(buf.plan.data_ptr(), buf.nbytes, missing);
+      buf.built |= missing;
+    }
+    out.plan = buf.plan;
+    out.nbytes = buf.nbytes;
+    out.complete = e.complete;
+    return out;
   }
   if (capturing(stream)) return out;
   const size_t n = size();
   if (n == 0) return out;
   Entry e;
   e.key = key;
-  e.nbytes = n;
-  e.plan = bytes_on(ref, n);
-  e.complete = build(e.plan.data_ptr(), n, needed);
-  e.built = needed;
+  Buffer& buf = e.buffers[slot];
+  buf.nbytes = n;
+  buf.plan = bytes_on(ref, n);
+  e.complete = build(buf.plan.data_ptr(), n, needed);
+  buf.built = needed;
   e.keep_map = map.storage();
   if (wts.has_value() && wts->defined()) e.keep_wts = wts->storage();
   e.stream = stream;
+  out.plan = buf.plan;
+  out.nbytes = n;
+  out.complete = e.complete;
   while (g_cache.size() >= g_cache_max) g_cache.pop_front();
   g_cache.push_back(std::move(e));
-  out.plan = g_cache.back().plan;
-  out.nbytes = n;
-  out.complete = g_cache.back().complete;
   return out;
 }
 
@@ -240,7 +254,7 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, co
       sdk_mapped_conv_by_columns(d.B, d.Cin, d.Cout, img_h, img_w, MH, MW, K, (int32_t)P,
                                  (int32_t)interp, SDK_F32, current_mode(), transposed ? 1 : 0) == 1;
   Key key;
-  key.kind = columns ? kConvColumns : kConv;
+  key.kind = kConv;
   key.device = ref.device().index();
   key.a = img_h;
   key.b = img_w;
@@ -250,8 +264,8 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, co
   return plan_for(
       key, ref, map, wts, stream,
       [&] {
-        return columns ? sdk_mapped_conv_plan_bytes_columns(img_h, img_w, MH, MW, K, (int32_t)P,
-                                                            (int32_t)interp, SDK_F32)
+        return columns ? sdk_mapped_conv_columns_bytes(img_h, img_w, MH, MW, K, (int32_t)P,
+                                                       (int32_t)interp, SDK_F32)
                        : sdk_mapped_conv_plan_bytes(img_h, img_w, MH, MW, K, (int32_t)P,
                                                     (int32_t)interp, SDK_F32);
       },
@@ -267,7 +281,8 @@ PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, co
       columns ? (scatter ? 1 : 0)
               : sdk_mapped_conv_plan_parts(d.B, d.Cin, d.Cout, img_h, img_w, MH, MW, K, (int32_t)P,
                                            (int32_t)interp, SDK_F32, current_mode(),
-                                           transposed ? 1 : 0, gather, weights, scatter));
+                                           transposed ? 1 : 0, gather, weights, scatter),
+      columns ? kSide : kMain);
 }
 
 PlanRef scatter_plan(Kind kind, const Tensor& ref, const Tensor& map, const OptTensor& wts,

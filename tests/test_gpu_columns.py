@@ -148,6 +148,79 @@ def test_calls_that_read_no_plan_leave_the_cache_alone(ops):
         ops.set_conv_plan_cache(True, max_entries=16)
 
 
+def test_columns_layers_keep_their_lists_alone(ops):
+    """64 -> 64 channels at 1 x 128 x 256 keep 10 MB of lists, not room for a plan of 100; a layer on
+    the same map that runs on a plan shares the map's entry."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    size = (128, 256, 128, 256, 9, 0, 1, _capi.SDK_F32)
+    m, _, x, w, b, g, _ = _arrays((1, 64, 64, 128, 256, 128, 256, 9, 0, 1))
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    args = (t(g), t(m), None, t(x), t(w), t(b), 9, 1)
+    ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 9, 1)     # (side streams' memory)
+    ops.set_conv_plan_cache(False)
+    ops.set_conv_plan_cache(True)
+    try:
+        before = torch.cuda.memory_allocated()
+        ops.ops.mapped_conv_backward(*args)
+        held = torch.cuda.memory_allocated() - before
+        assert 0 < held <= lib.sdk_mapped_conv_columns_bytes(*size) + 1024 < 11e6
+        assert ops.plan_cache_size() == 1
+        lib.sdk_mapped_conv_columns_enable(0)
+        ops.ops.mapped_conv_backward(*args)
+        lib.sdk_mapped_conv_columns_enable(1)
+        assert ops.plan_cache_size() == 1
+        assert torch.cuda.memory_allocated() - before >= lib.sdk_mapped_conv_plan_bytes(*size)
+        ops.ops.mapped_conv_backward(*args)
+    finally:
+        lib.sdk_mapped_conv_columns_enable(1)
+
+
+def test_every_buffer_a_columns_call_may_be_given(ops):
+    """No plan, the inverted map alone, a plan with it (built whole, or that part of it) and one
+    without: the same gradient; the inverted map alone is refused by calls of the tile kernels."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    B, Cin, Cout, H, W, K = 1, 40, 48, 40, 64, 9
+    m, _, x, w, _, g, _ = _arrays((B, Cin, Cout, H, W, H, W, K, 0, 1))
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    tm, tg, tw = t(m), t(g), t(w)
+    size = (H, W, H, W, K, 0, 1, _capi.SDK_F32)
+    plain, both, alone = (int(f(*size)) for f in (
+        lib.sdk_mapped_conv_plan_bytes, lib.sdk_mapped_conv_plan_bytes_columns,
+        lib.sdk_mapped_conv_columns_bytes))
+    assert plain % 256 == both % 256 == 0 and alone % 256 == 128 and alone < both - plain + 256
+    nws = lib.sdk_mapped_conv_workspace_bytes(B, Cin, Cout, H, W, H, W, K, 0, 1, _capi.SDK_F32, 0)
+    ws = torch.empty(nws, dtype=torch.uint8, device=DEV)
+    p, stream = (lambda a: a.data_ptr()), torch.cuda.current_stream().cuda_stream  # noqa: E731
+
+    def call(plan):
+        out = torch.empty(B, Cin, H, W, device=DEV)
+        rc = lib.sdk_mapped_conv_backward_input_planned(
+            p(tg), p(tm), None, p(tw), p(out), p(ws), nws, None if plan is None else p(plan),
+            0 if plan is None else plan.numel(), B, Cin, H, W, Cout, H, W, K, 0, 1, _capi.SDK_F32, 0,
+            stream)
+        return rc, out
+
+    want = call(None)[1]
+    for build, n in (("sdk_mapped_conv_plan_build_columns", alone), ("sdk_mapped_conv_plan_build", plain),
+                     ("sdk_mapped_conv_plan_build_columns", both), ("sdk_mapped_conv_plan_build", both)):
+        plan = torch.empty(n, dtype=torch.uint8, device=DEV)
+        assert getattr(lib, build)(p(tm), None, p(plan), n, *size, stream) == 0
+        rc, out = call(plan)
+        assert rc == 0 and torch.equal(out, want), (build, n)
+    plan = torch.empty(alone, dtype=torch.uint8, device=DEV)
+    assert lib.sdk_mapped_conv_plan_build_columns(p(tm), None, p(plan), alone - 128, *size, stream) == -3
+    assert lib.sdk_mapped_conv_plan_build(p(tm), None, p(plan), alone, *size, stream) == -3
+    lib.sdk_mapped_conv_columns_enable(0)
+    try:
+        nws = lib.sdk_mapped_conv_workspace_bytes(B, Cin, Cout, H, W, H, W, K, 0, 1, _capi.SDK_F32, 0)
+        ws = torch.empty(nws, dtype=torch.uint8, device=DEV)
+        assert call(plan)[0] == -3 and b"inverted map alone" in lib.sdk_last_error()
+    finally:
+        lib.sdk_mapped_conv_columns_enable(1)
+
+
 def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):
     """A convolution's forward builds what it gathers by, its backward the inverse; results are those
     of a plan built at once, whichever call comes first, and of no plan."""
