@@ -234,7 +234,8 @@ def _conv_plan(ref, sample_map, interp_weights, dims, img_h, img_w, P, interp, t
     """(plan tensor, bytes) for a call on this map, built on first use; (None, 0) when the library
     has no plan for it, the call reads none or the cache is off.  dims: (B, Cin, Cout, K); scatter:
     the call splats into the image (the backward of a convolution, the forward of a transposed one).
-    Calls that run by columns read at most the inverted map, and that only to scatter."""
+    Calls that run by columns read at most the inverted map, and that only to scatter (a forward
+    whose input requires a gradient has it built for its backward)."""
     if not _plan_cache_enabled or ref.dtype != torch.float32:
         return None, 0
     MH, MW = int(sample_map.shape[0]), int(sample_map.shape[1])
@@ -595,7 +596,7 @@ def mapped_conv_forward(x, sample_map, interp_weights, weight, bias, kernel_size
     with torch.cuda.device(x.device):
         ws, nws = _workspace(x, B, Cin, Cout, H, W, OH, OW, K, P, int(interp))
         plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), H, W, P,
-                                 int(interp), False, False)
+                                 int(interp), False, x.requires_grad)
         dims = (B, Cin, H, W, Cout, OH, OW, K, P, int(interp), _DTYPES[x.dtype], _current_mode(),
                 _stream(x))
         if plan is None:

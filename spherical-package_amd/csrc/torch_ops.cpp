@@ -242,7 +242,9 @@ struct ConvDims {
 // a convolution, the backward-input of a transposed one); weights: it forms a weight gradient;
 // scatter: it splats into the image (the other two).  Each reads its part of the plan, a layer
 // of a few image channels none; of the calls that run as columns and products only scatters
-// read one, the inverted map.  (Measured, first step on a new map, all parts of a plan built ->
+// read one, the inverted map.  A forward whose input requires a gradient asks for what the input's
+// gradient reads too: a backward captured into a graph after it finds its plan whole, where
+// nothing could be built.  (Measured, first step on a new map, all parts of a plan built ->
 // those that are read: 4 x 512 x 1024, 3 -> 32 channels, no picture gradient 694 -> 342 us,
 // 64 x 128, 3 -> 16 547 -> 175 us; level-7 icosphere decoder block 3.24 -> 2.88 ms.)
 PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, const ConvDims& d,
@@ -567,7 +569,7 @@ Tensor mapped_conv_forward(const Tensor& x, const Tensor& map, const OptTensor& 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, H, W, OH, OW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, false, false, s);
+  PlanRef plan = conv_plan(x, map, wts, d, H, W, P, interp, false, true, false, x.requires_grad(), s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())
@@ -639,7 +641,8 @@ Tensor mapped_transposed_conv_forward(const Tensor& x, const Tensor& map, const 
   hipStream_t s = stream_of(x);
   size_t nws = 0;
   Tensor ws = workspace(x, d, out_h, out_w, IH, IW, P, interp, &nws);
-  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, false, false, true, s);
+  PlanRef plan = conv_plan(x, map, wts, d, out_h, out_w, P, interp, true, x.requires_grad(), false,
+                           true, s);
   const int dt = dtype_code(x), mode = current_mode();
   void* wsp = nws ? ws.data_ptr() : nullptr;
   if (!plan.plan.defined())

@@ -221,6 +221,59 @@ def test_every_buffer_a_columns_call_may_be_given(ops):
         lib.sdk_mapped_conv_columns_enable(1)
 
 
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("columns", [0, 1])
+def test_a_backward_captured_after_a_forward_finds_its_plan(ops, columns, transposed):
+    """Nothing is built under capture: a forward whose input requires a gradient builds what the
+    input's gradient reads, and the replays rebuild nothing."""
+    from _spherical_distortion_ext import _capi
+    import spherical_distortion.nn as snn
+    H, W, C = (40, 64, 40) if columns else (256, 256, 16)
+    m, _, x, _, _, _, _ = _arrays((1, C, C, H, W, H, W, 9, 0, 1))
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    cls = snn.MappedTransposedConvolution if transposed else snn.MappedConvolution
+    layer, tx = cls(C, C, 9).to(DEV), t(x).requires_grad_()
+    args = lambda tm: (H, W, tm) if transposed else (tm,)  # noqa: E731
+    name = "mapped_transposed_conv_backward" if transposed else "mapped_conv_backward"
+    w, b, g = layer.weight.detach(), layer.bias.detach(), t(x)
+    lib = _capi.load()
+    lib.sdk_mapped_conv_columns_enable(columns)
+    times = {}
+    try:
+        want = getattr(ops.ops, name)(g, t(m), None, tx.detach(), w, b, 9, 1)
+        for warm in ("nothing", "forward", "step"):
+            tm = t(m)
+            if warm != "nothing":
+                y = layer(tx, *args(tm))
+                if warm == "step":
+                    torch.autograd.grad(y, [tx], g)
+            outs = [torch.empty_like(o) for o in want]
+            graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                with torch.cuda.graph(graph, stream=side):
+                    for o, r in zip(outs, getattr(ops.ops, name)(g, tm, None, tx.detach(), w, b, 9, 1)):
+                        o.copy_(r)
+            times[warm] = 1e9
+            for _ in range(8):
+                for o in outs:
+                    o.zero_()
+                start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                start.record()
+                graph.replay()
+                end.record()
+                torch.cuda.synchronize()
+                times[warm] = min(times[warm], start.elapsed_time(end))
+                for o, r in zip(outs, want):
+                    assert _rel(o.cpu().numpy(), r.cpu().numpy()) <= 2e-6
+    finally:
+        lib.sdk_mapped_conv_columns_enable(1)
+    print(times)
+    # (the columns' gathers read no plan: nothing to rebuild in the backward of a transposed layer)
+    assert times["forward"] <= 1.1 * times["step"]
+    assert (columns and transposed) or times["forward"] <= 0.95 * times["nothing"]
+
+
 def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):
     """A convolution's forward builds what it gathers by, its backward the inverse; results are those
     of a plan built at once, whichever call comes first, and of no plan."""
