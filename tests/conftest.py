@@ -57,6 +57,23 @@ def tile_kernels():
     lib.sdk_mapped_conv_columns_enable(before)
 
 
+@pytest.fixture(params=["tiles", "columns"])
+def conv_route(request):
+    """Both routes of small float32 convolutions in turn: the kernels of large calls at the test's
+    sizes, and the columns such calls take by themselves."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    before = lib.sdk_mapped_conv_columns_enable(int(request.param == "columns"))
+    yield request.param
+    lib.sdk_mapped_conv_columns_enable(before)
+
+
+def runs_by_columns(B, Cin, Cout, H, W, OH, OW, K, P, interp, transposed=0):
+    from _spherical_distortion_ext import _capi
+    return _capi.load().sdk_mapped_conv_by_columns(B, Cin, Cout, H, W, OH, OW, K, P, interp,
+                                                   _capi.SDK_F32, 0, transposed) == 1
+
+
 # ---------------------------------------------------------------------------------------------
 # Builders shared by the oracle (CPU) and GPU replays of the reference's known-answer tests.
 # ---------------------------------------------------------------------------------------------

@@ -145,7 +145,7 @@ def test_planned_calls_match_plain_calls_and_the_oracle(ops, oracle, tc, mode):
     assert relerr(tgi1, ti) <= tol_b and relerr(tgw1, tw) <= tol_b and relerr(tgb1, tb) <= tol_b
 
 
-def test_cache_misses_after_an_in_place_change_of_the_map(ops, oracle):
+def test_cache_misses_after_an_in_place_change_of_the_map(ops, oracle, conv_route):
     Cin, Cout, H, W, OH, OW, K, P, interp, kind = CASES[0]
     m, iw, x, w, b, g, _ = _case(3, *CASES[0])
     tm = _t(m)
@@ -206,7 +206,7 @@ def test_every_planned_entry_point_refuses_a_plan_that_is_too_small(ops):
     assert float(gb.abs().max()) == 0.0       # no bias gradient was launched by a refused call
 
 
-def test_maps_made_under_inference_mode_go_past_the_cache(ops, oracle):
+def test_maps_made_under_inference_mode_go_past_the_cache(ops, oracle, conv_route):
     """A tensor created under torch.inference_mode() has no version counter; the cached
     operators take the uncached entry points for it instead of failing."""
     Cin, Cout, H, W, OH, OW, K, P, interp, kind = CASES[0]
@@ -227,7 +227,7 @@ def test_maps_made_under_inference_mode_go_past_the_cache(ops, oracle):
     assert relerr(up, oracle.resample_to_map(x, m[:, :, 0], H, W, interp)) <= 1e-4
 
 
-def test_a_plan_is_not_built_under_graph_capture(ops):
+def test_a_plan_is_not_built_under_graph_capture(ops, conv_route):
     """A key that misses while the stream is being captured takes the uncached entry points:
     nothing is inserted into the cache, and the replayed graph gives the eager result."""
     Cin, Cout, H, W, OH, OW, K, P, interp, kind = CASES[0]

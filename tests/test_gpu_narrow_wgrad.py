@@ -3,13 +3,14 @@ interpolation weights), which has a kernel of its own: every kernel size it is b
 widths of the output-channel block, a grid whose right edge cuts a tile, channel counts that
 leave the last chunk and the last rows partly empty, taps outside the image, and a launch in
 which every workgroup walks several tiles (the requests for a tile are made while the one
-before it is multiplied).
+before it is multiplied).  Calls as small as most of these run by columns: every one is made on both
+routes.
 """
 import numpy as np
 import pytest
 import torch
 
-from conftest import relerr
+from conftest import relerr, runs_by_columns
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -45,7 +46,8 @@ def _nearest_case(seed, B, Cin, Cout, H, W, K):
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
 @pytest.mark.parametrize("Cout", [24, 48])
 @pytest.mark.parametrize("K", range(1, 11))
-def test_every_kernel_size_and_block_width(ops, oracle, K, Cout, mode):
+def test_every_kernel_size_and_block_width(ops, oracle, conv_route, K, Cout, mode):
+    assert runs_by_columns(2, 40, Cout, 20, 37, 20, 37, K, 0, 0) == (conv_route == "columns")
     m, x, w, b, g = _nearest_case(100 * K + Cout, 2, 40, Cout, 20, 37, K)
     ops.set_conv_compute(mode)
     try:
@@ -61,7 +63,7 @@ def test_every_kernel_size_and_block_width(ops, oracle, K, Cout, mode):
 
 @pytest.mark.parametrize("mode", ["native", "split"])
 @pytest.mark.parametrize("Cout,K", [(40, 7), (8, 9), (64, 4)])
-def test_workgroups_that_walk_several_tiles(ops, oracle, Cout, K, mode):
+def test_workgroups_that_walk_several_tiles(ops, oracle, conv_route, Cout, K, mode):
     # 8 batch elements x 8 chunks of image channels: eight workgroups per kind share the 24
     # tiles of the 48 x 64 grid, three each
     m, x, w, b, g = _nearest_case(7 + Cout + K, 8, 256, Cout, 48, 64, K)

@@ -3,6 +3,7 @@ with shapes, channel counts, kernel sizes, interpolation, point counts and map c
 (locally coherent or scattered) drawn per seed.  The fixed cases of test_gpu_parity.py pin known
 corners; this sweep looks for the ones nobody thought of (tile remainders, channel paddings,
 plan / inverse-map / tiled-unpool paths and their fallbacks meeting odd sizes).
+Convolutions run on both routes: sizes this small take columns by themselves.
 Tolerances as everywhere: nearest gather and pooling bit-exact, float32 forward 1e-5, float32
 backward 1e-4, norm-relative.
 """
@@ -92,7 +93,7 @@ def _conv_case(seed):
 
 
 @pytest.mark.parametrize("seed", range(100, 116))
-def test_convolution_bf16_operands(ops, oracle, seed):
+def test_convolution_bf16_operands(ops, oracle, conv_route, seed):
     """The bf16 compute mode (operands rounded to bf16, fp32 accumulation) on the same sweep:
     1e-2 norm-relative against the float32 oracle."""
     rng, interp, K, H, W, OH, OW, B, Cin, Cout, m, iw, x, w, b, g = _conv_case(seed)
@@ -109,7 +110,7 @@ def test_convolution_bf16_operands(ops, oracle, seed):
 
 
 @pytest.mark.parametrize("seed", range(300, 324))
-def test_convolution_split_operands(ops, oracle, seed):
+def test_convolution_split_operands(ops, oracle, conv_route, seed):
     """The split compute mode (float32 operands as three bf16 pieces, fp32 accumulation) on the
     same sweep, at the float32 tolerances."""
     rng, interp, K, H, W, OH, OW, B, Cin, Cout, m, iw, x, w, b, g = _conv_case(seed)
@@ -126,7 +127,7 @@ def test_convolution_split_operands(ops, oracle, seed):
 
 
 @pytest.mark.parametrize("seed", range(40))
-def test_convolution_and_transposed(ops, oracle, seed):
+def test_convolution_and_transposed(ops, oracle, conv_route, seed):
     rng, interp, K, H, W, OH, OW, B, Cin, Cout, m, iw, x, w, b, g = _conv_case(seed)
     y = _n(ops.mapped_conv_forward(_t(x), _t(m), _t(iw), _t(w), _t(b), K, interp))
     assert relerr(y, oracle.mapped_conv_forward(x, m, w, b, K, interp, iw)) <= FWD
@@ -226,7 +227,7 @@ def test_uv_resampling_voting_and_generated_maps(ops, oracle, seed):
 
 
 @pytest.mark.parametrize("seed", [11, 12, 13])
-def test_fused_kernels_against_the_unfused_path_on_random_layers(ops, seed):
+def test_fused_kernels_against_the_unfused_path_on_random_layers(ops, conv_route, seed):
     """Twenty random layers per seed (nearest, bilinear and bispherical taps, 1 to 12 samples,
     3 to 136 output channels, unit stride and stride 2, one-row grids of thousands of pixels,
     batches that make workgroups walk several tiles): the plan-driven and window kernels against
