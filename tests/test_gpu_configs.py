@@ -94,11 +94,13 @@ def test_configuration3_reduced(ops, oracle):
         assert relerr(got, want) <= BWD
 
 
+@pytest.mark.usefixtures("conv_route")
 def test_configuration4_reduced(ops, oracle):
     """Weighted (P = 4) bispherical convolution on a 32 x 64 grid, 40 -> 24 channels."""
     _conv_both_ways(ops, oracle, workloads.config4(batch=2, cin=40, cout=24, H=32, W=64))
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("order", ["hierarchical", "append"])
 def test_configuration5_reduced(ops, oracle, order):
     """Level-3 icosphere (642 vertices): vertex convolution and transposed up-sampling from

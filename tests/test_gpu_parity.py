@@ -304,6 +304,7 @@ CONV_CASES = [(i, wgt, dt) for i in (0, 1, 2) for wgt in (False, True)
               for dt in (np.float32, np.float64)]
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("case", CONV_CASES, ids=_ids)
 def test_mapped_convolution(ops, oracle, case):
     interp, weighted, dt = case
@@ -324,6 +325,7 @@ def test_mapped_convolution(ops, oracle, case):
     assert relerr(_n(gb), wb) <= BWD_TOL[dt]
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("case", CONV_CASES, ids=_ids)
 def test_mapped_transposed_convolution(ops, oracle, case):
     interp, weighted, dt = case
@@ -377,6 +379,7 @@ TILE_CASES = [
 ]
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("tc", TILE_CASES, ids=lambda t: "x".join(map(str, t)))
 def test_fused_conv_tile_edges(ops, oracle, tc):
     Cin, Cout, H, W, OH, OW, K, P, interp = tc
@@ -413,6 +416,7 @@ def test_fused_conv_tile_edges(ops, oracle, tc):
     assert relerr(_n(gb), wb) <= 1e-4
 
 
+@pytest.mark.usefixtures("conv_route")
 def test_weight_gradient_without_partial_sums(ops, oracle):
     """The weight gradient normally leaves per-workgroup sums in the workspace and a second
     kernel adds them up; a call whose sums would need more than 160 MB adds to grad_weight
@@ -466,6 +470,7 @@ PLAN_CASES = [
 ]
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("tc", PLAN_CASES, ids=lambda t: "x".join(map(str, t)))
 def test_fused_conv_coherent_maps(ops, oracle, tc):
     """Maps with the locality the LDS-window kernels are built for, at shapes that hit their
@@ -501,6 +506,7 @@ def test_fused_conv_coherent_maps(ops, oracle, tc):
     assert relerr(_n(gw), ww) <= 1e-4
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("crowded", [False, True], ids=["injective", "crowded"])
 def test_nearest_scatter_inverse_map_and_its_fallback(ops, oracle, crowded):
     """Nearest unweighted maps run the scatter contractions as a gather over the inverse map
@@ -536,6 +542,7 @@ def bf16_compute(ops):
     ops.set_conv_compute("native")
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("tc", TILE_CASES[:4], ids=lambda t: "x".join(map(str, t)))
 def test_bf16_compute_within_1e_2(ops, oracle, bf16_compute, tc):
     """bf16 operands with fp32 accumulation in the MFMA contraction: every output within
@@ -574,6 +581,7 @@ def split_compute(ops):
     ops.set_conv_compute("native")
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("tc", TILE_CASES + PLAN_CASES, ids=lambda t: "x".join(map(str, t)))
 def test_split_compute_keeps_float32_accuracy(ops, oracle, split_compute, tc):
     """float32 operands split into three bf16 pieces each (six piece products, fp32
@@ -608,6 +616,7 @@ def test_split_compute_keeps_float32_accuracy(ops, oracle, split_compute, tc):
     assert relerr(got, want) <= 1e-4
 
 
+@pytest.mark.usefixtures("conv_route")
 def test_split_compute_on_values_that_stress_the_pieces(ops, oracle, split_compute):
     """Operands whose low mantissa bits matter: large offsets plus small signals, powers of two,
     denormal-range and huge magnitudes; and float64 tensors, which run as in the native mode."""
@@ -749,6 +758,7 @@ def test_gather_at_index_and_unpool_layer(ops, oracle, case):
             eps=1e-6, atol=1e-7, nondet_tol=1e-9)
 
 
+@pytest.mark.usefixtures("conv_route")
 @pytest.mark.parametrize("mode", ["native", "bf16", "split"])
 @pytest.mark.parametrize("shape", [(9, 12), (16, 20), (8, 28), (20, 36)],
                          ids=lambda s: "%dx%d" % s)
