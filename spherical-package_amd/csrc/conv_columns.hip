@@ -165,6 +165,10 @@ __global__ __launch_bounds__(kClThreads) void columns_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kGk = 32;
 constexpr int kGld = 36;
+// A split of the weight gradient's reduction is hundreds of pixels; added up one after the other they
+// lose twice the bits of the tile kernels' sums (6 x 25 x 50 pixels, 96 -> 160: 4.5e-7 of the float64
+// norm against 2.1e-7), so two steps at a time are summed apart and then added: 1.7e-7, for 2 us of the
+// layer's 174.
 
 struct GemmArgs {
   const float *A, *B;
@@ -254,9 +258,8 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   if (threadIdx.x < BM)
     s_bias[threadIdx.x] = !TN && g.bias != nullptr ? g.bias[min(i0 + (int)threadIdx.x, g.rows_a - 1)] : 0.0f;
 
-  floatx16 acc;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  const floatx16 none = {};
+  floatx16 acc = none, all = none;   // (TN: all = the sums of two steps each, acc those under way)
 
   auto load8 = [&](const float* p, float (&f)[8]) {
     const vec4 lo = *reinterpret_cast<const vec4*>(p), hi = *reinterpret_cast<const vec4*>(p + 4);
@@ -268,6 +271,7 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   };
 
   auto multiply = [&](int buf) {
+    if (TN && buf == 0) acc = none;
 #pragma unroll
     for (int s = 0; s < kGk / 16; ++s) {
       float fa[8], fb[8];
@@ -310,8 +314,10 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
     multiply(1);   // (a step past the end multiplies zeros)
     __builtin_amdgcn_sched_barrier(0);
     stash(0, r0 + 2 * kStep, ra[0], rbv[0]);
+    if constexpr (TN) all += acc;
     __syncthreads();
   }
+  if constexpr (TN) acc = all;
   if constexpr (KS == 2) {
     // the second group's sums join the first's through LDS, [register][thread]
     float* sums = &lds[1][0][0];
@@ -346,7 +352,8 @@ __global__ __launch_bounds__(kClThreads) void columns_wgrad_sum_kernel(
 #pragma unroll
     for (int x = 0; x < 8; ++x) v[x] = partial[(size_t)min(s + x, splits - 1) * split_stride + e];
 #pragma unroll
-    for (int x = 0; x < 8; ++x) sum += s + x < splits ? v[x] : 0.0f;
+    for (int x = 0; x < 8; ++x) v[x] = s + x < splits ? v[x] : 0.0f;
+    sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
   gW[((size_t)i * Cg + c) * K + k] = sum;
 }
