@@ -904,6 +904,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
         for (int q = 0; q < 4; ++q) av[a][q] = next[a][q];
       if (b + 1 < b_end) request(b + 1);
       wave_exchange();
+      float sum_b[NB] = {};   // (this batch element's sixteen pixels apart: half the error of one chain)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         f32x4 bv[CB];
@@ -914,13 +915,15 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
         for (int i = 0; i < 4; ++i)
 #pragma unroll
           for (int a = 0; a < NB; ++a) {
-            row_sum[a] += av[a][q][i];
+            sum_b[a] += av[a][q][i];
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
               acc[a][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a][q][i], bv[cb][i], acc[a][cb],
                                                                 0, 0, 0);
           }
       }
+#pragma unroll
+      for (int a = 0; a < NB; ++a) row_sum[a] += sum_b[a];
       wave_exchange();   // (the next batch element's columns go where these were)
     }
     lp = lp_next;
@@ -951,10 +954,18 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, 1 + NB * small_columns(
     if (n < Cp && k < K && c < Cg) atomic_add_noret(gW + ((size_t)n * Cg + c) * K + k, sum[e]);
   }
   if (gbias != nullptr) {
+    // (the waves' sums together: an atomic each, one after the other on the channel, lost twice the bits)
+    __syncthreads();   // the readers of sum are through
 #pragma unroll
     for (int a = 0; a < NB; ++a) {
       const float s = row_sum[a] + __shfl_xor(row_sum[a], 32);
-      if (h == 0 && n0 + 32 * a + nl < Cp) atomic_add_noret(gbias + n0 + 32 * a + nl, s);
+      if (h == 0) sum[(wave * NB + a) * 32 + nl] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < 32 * NB && n0 + (int)threadIdx.x < Cp) {
+      float s = sum[threadIdx.x];
+      for (int w = 1; w < tl.waves; ++w) s += sum[w * NB * 32 + threadIdx.x];
+      atomic_add_noret(gbias + n0 + threadIdx.x, s);
     }
   }
 }
