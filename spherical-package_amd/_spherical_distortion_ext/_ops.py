@@ -217,6 +217,8 @@ def _cache_lookup(key, cur):
     if ent.stream != cur:
         cur.wait_stream(ent.stream)
         ent.stream = cur
+        if isinstance(ent.plan, torch.Tensor):   # once let go, its memory waits for this stream's calls
+            ent.plan.record_stream(cur)
     return ent
 
 

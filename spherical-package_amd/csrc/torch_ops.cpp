@@ -15,6 +15,7 @@
 //
 // Built with the host compiler against the torch headers; no device code here.
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -104,7 +105,6 @@ struct PlanRef {
 };
 
 void order_behind(hipStream_t cur, hipStream_t last) {
-  if (cur == last) return;
   hipEvent_t ev = nullptr;
   if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return;
   if (hipEventRecord(ev, last) == hipSuccess) (void)hipStreamWaitEvent(cur, ev, 0);
@@ -202,8 +202,14 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
         buf.plan = bytes_on(ref, buf.nbytes);
       }
     }
-    order_behind(stream, e.stream);
-    e.stream = stream;
+    if (stream != e.stream) {
+      order_behind(stream, e.stream);
+      e.stream = stream;
+      // once let go, the buffers' memory waits for the calls of this stream too
+      const auto here = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(ref.device().index());
+      for (Buffer& b : e.buffers)
+        if (b.plan.defined()) b.plan.record_stream(here.unwrap());
+    }
     if (missing != 0) {
       e.complete = build(buf.plan.data_ptr(), buf.nbytes, missing);
       buf.built |= missing;

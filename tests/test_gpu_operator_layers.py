@@ -152,3 +152,29 @@ def test_both_layers_refuse_the_same_arguments(ops):
         for fn in (getattr(ops.ops, name), ops.PYTHON_IMPL[name]):
             with pytest.raises(RuntimeError, match=what):
                 fn(*args)
+
+
+@pytest.mark.parametrize("layer", ["compiled", "python"])
+def test_a_plan_let_go_is_not_reused_under_a_call_of_another_stream(ops, tile_kernels, layer):
+    """A plan made on one stream and read on another returns to the first one's memory when the
+    cache drops it: not before the call on the other stream is through."""
+    d = _inputs(False, np.float32)
+    run = ops.ops.mapped_conv_forward if layer == "compiled" else ops.PYTHON_IMPL["mapped_conv_forward"]
+    m, side, kept = d["m"].clone(), torch.cuda.Stream(), 0
+    pending = lambda s: s["active_bytes.all.current"] - s["allocated_bytes.all.current"]  # noqa: E731
+    ops.set_conv_plan_cache(False)
+    ops.set_conv_plan_cache(True)
+    try:
+        before = torch.cuda.memory_allocated()
+        run(d["x"], m, None, d["w"], d["b"], d["K"], 1)
+        kept = torch.cuda.memory_allocated() - before
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(100_000_000)       # (some tens of milliseconds)
+            run(d["x"], m, None, d["w"], d["b"], d["K"], 1)
+        ops.set_conv_plan_cache(False)           # lets go of the plan while that call waits
+        stats, busy = torch.cuda.memory_stats(), not side.query()
+        torch.cuda.synchronize()
+    finally:
+        ops.set_conv_plan_cache(True)
+    assert busy and kept > 0 and pending(stats) >= kept
