@@ -164,12 +164,25 @@ class _PlanEntry:
     """A kept plan: the buffer, its size, the storages of the map it was built from, the
     stream that used it last (every call reads the plan, and the max-unpool call rewrites the
     plan's gate word, so a call on another stream is ordered behind the last user) and the
-    `complete` verdict of a scatter plan."""
-    __slots__ = ("plan", "nbytes", "keep", "stream", "complete")
+    `complete` verdict of a scatter plan.  captured: a graph reads the plan by its address; it stays
+    as long as anyone beside the cache holds the map (the graph's owner has to)."""
+    __slots__ = ("plan", "nbytes", "keep", "stream", "complete", "captured")
 
     def __init__(self, plan, nbytes, keep, stream, complete=0):
         self.plan, self.nbytes, self.keep, self.stream, self.complete = \
             plan, nbytes, keep, stream, complete
+        self.captured = False
+
+    def needed(self):
+        return self.captured and torch._C._storage_Use_Count(self.keep[0]._cdata) > 1
+
+
+def _shrink_cache(most):
+    for key in list(_PLAN_CACHE):
+        if len(_PLAN_CACHE) <= most:
+            break
+        if not _PLAN_CACHE[key].needed():
+            del _PLAN_CACHE[key]
 
 
 def set_conv_plan_cache(enabled, max_entries=None):
@@ -185,8 +198,7 @@ def set_conv_plan_cache(enabled, max_entries=None):
         _PLAN_CACHE_MAX = int(max_entries)
     if not enabled:
         _PLAN_CACHE.clear()
-    while len(_PLAN_CACHE) > _PLAN_CACHE_MAX:
-        _PLAN_CACHE.pop(next(iter(_PLAN_CACHE)))
+    _shrink_cache(_PLAN_CACHE_MAX)
     if _native is not None:
         _native.sdk_torch_set_plan_cache(1 if enabled else 0, _PLAN_CACHE_MAX)
 
@@ -214,6 +226,8 @@ def _cache_lookup(key, cur):
     if ent is None:
         return None
     _PLAN_CACHE[key] = ent
+    ent.captured = ent.captured or (isinstance(ent.plan, torch.Tensor)
+                                    and torch.cuda.is_current_stream_capturing())
     if ent.stream != cur:
         cur.wait_stream(ent.stream)
         ent.stream = cur
@@ -223,8 +237,7 @@ def _cache_lookup(key, cur):
 
 
 def _cache_insert(key, ent):
-    while len(_PLAN_CACHE) >= _PLAN_CACHE_MAX:
-        _PLAN_CACHE.pop(next(iter(_PLAN_CACHE)))
+    _shrink_cache(_PLAN_CACHE_MAX - 1)
     _PLAN_CACHE[key] = ent
 
 

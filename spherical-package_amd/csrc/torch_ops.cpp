@@ -22,6 +22,7 @@
 #include <torch/library.h>
 
 #include <cstdint>
+#include <iterator>
 #include <list>
 #include <mutex>
 #include <string>
@@ -94,8 +95,16 @@ struct Entry {
   c10::Storage keep_map, keep_wts;   // an address cannot be reused while its entry lives
   hipStream_t stream = nullptr;      // last user: a call on another stream is ordered behind it
   int complete = 0;
+  bool captured = false;             // a graph reads the plan
 };
 std::list<Entry> g_cache;   // most recently used last
+
+// Lets go of the least recently used entries until `most` are left.  A plan that a captured graph reads
+// by its address stays as long as anyone beside the cache holds its map (the graph's owner has to).
+void shrink_cache(size_t most) {
+  for (auto it = g_cache.begin(); g_cache.size() > most && it != g_cache.end();)
+    it = it->captured && it->keep_map.use_count() > 1 ? std::next(it) : g_cache.erase(it);
+}
 
 struct PlanRef {
   Tensor plan;   // undefined: none
@@ -194,8 +203,9 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
     Entry& e = g_cache.back();
     Buffer& buf = e.buffers[slot];
     const int missing = needed & ~buf.built;
+    const bool captured = capturing(stream);
     if (missing != 0) {
-      if (capturing(stream)) return out;
+      if (captured) return out;
       if (!buf.plan.defined()) {
         buf.nbytes = size();
         if (buf.nbytes == 0) return out;
@@ -214,6 +224,7 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
       e.complete = build(buf.plan.data_ptr(), buf.nbytes, missing);
       buf.built |= missing;
     }
+    e.captured |= captured;
     out.plan = buf.plan;
     out.nbytes = buf.nbytes;
     out.complete = e.complete;
@@ -235,7 +246,7 @@ PlanRef plan_for(Key key, const Tensor& ref, const Tensor& map, const OptTensor&
   out.plan = buf.plan;
   out.nbytes = n;
   out.complete = e.complete;
-  while (g_cache.size() >= g_cache_max) g_cache.pop_front();
+  shrink_cache(g_cache_max - 1);
   g_cache.push_back(std::move(e));
   return out;
 }
@@ -778,7 +789,7 @@ void sdk_torch_set_plan_cache(int enabled, int max_entries) {
   g_cache_enabled = enabled != 0;
   if (max_entries > 0) g_cache_max = (size_t)max_entries;
   if (!g_cache_enabled) g_cache.clear();
-  while (g_cache.size() > g_cache_max) g_cache.pop_front();
+  shrink_cache(g_cache_max);
 }
 int sdk_torch_plan_cache_size(void) {
   std::lock_guard<std::mutex> lock(g_mu);

@@ -178,3 +178,49 @@ def test_a_plan_let_go_is_not_reused_under_a_call_of_another_stream(ops, tile_ke
     finally:
         ops.set_conv_plan_cache(True)
     assert busy and kept > 0 and pending(stats) >= kept
+
+
+@pytest.mark.parametrize("layer", ["compiled", "python"])
+def test_a_plan_that_a_graph_reads_is_not_let_go(ops, tile_kernels, layer):
+    """A captured call reads its plan by address: the cache keeps it beyond its sixteen entries as
+    long as the map is held outside, and no longer."""
+    d = _inputs(False, np.float32)
+    run = ops.ops.mapped_conv_forward if layer == "compiled" else ops.PYTHON_IMPL["mapped_conv_forward"]
+    step = lambda m: run(d["x"], m, None, d["w"], d["b"], d["K"], 1)  # noqa: E731
+    want = step(d["m"])
+    small = d["x"][:, :, :2, :2].contiguous()                # (smaller plans)
+    others = [d["m"][:2].clone() for _ in range(4)]
+    other_calls = lambda: [run(small, o, None, d["w"], d["b"], d["K"], 1) for o in others]  # noqa: E731
+    sizes = []
+    for call in (lambda: step(d["m"]), lambda: run(small, others[0], None, d["w"], d["b"], d["K"], 1)):
+        ops.set_conv_plan_cache(False)
+        ops.set_conv_plan_cache(True, max_entries=2)
+        sizes.append(-torch.cuda.memory_allocated())
+        call()
+        sizes[-1] += torch.cuda.memory_allocated()
+    ops.set_conv_plan_cache(False)
+    ops.set_conv_plan_cache(True)
+    assert sizes[0] > sizes[1] > 0
+    try:
+        m, side, graph = d["m"].clone(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        out = torch.empty_like(want)
+        before = torch.cuda.memory_allocated()
+        step(m)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            with torch.cuda.graph(graph, stream=side):
+                out.copy_(step(m))
+        other_calls()
+        assert ops.plan_cache_size() == 2
+        assert torch.cuda.memory_allocated() - before >= sizes[0] + sizes[1]
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+        del graph, m
+        other_calls()
+        assert ops.plan_cache_size() == 2
+        assert torch.cuda.memory_allocated() - before < sizes[0] + sizes[1]
+    finally:
+        ops.set_conv_plan_cache(True, max_entries=16)
