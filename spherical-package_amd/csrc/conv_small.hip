@@ -655,8 +655,9 @@ __global__ __launch_bounds__(kSmThreads) void small_scatter_kernel(
 //
 // 3 -> 32 channels at 512 x 1024, B = 4, bilinear, K = 9 (268 MB written): 148 us with a thread
 // per pixel that gathered from global memory and multiplied on the vector unit, 101 us now, of
-// which 34 us are vector and 30 us matrix instructions; those add up, and four waves per SIMD
-// do not cover all of a tile's serial start (map, box, window).  A window per wave instead of
+// which 32 us are vector (1015 instructions a wave) and 31 us matrix instructions; those add up, and
+// four waves per SIMD do not cover all of a tile's serial start (map, box, window): waves wait 0.42
+// of their cycles.  A window per wave instead of
 // per workgroup saves the two barriers and doubles the window reads: 119 us.
 template <int INTERP, bool WEIGHTED, int CG, int NG, int NB>
 __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward_kernel(
@@ -780,7 +781,7 @@ __global__ __launch_bounds__(kSmThreads, small_waves(NG, NB)) void small_forward
 // the workgroup as one float atomic per element of gW.  gbias (optional): the sums of the
 // pixel-side rows, from the same registers, one atomic per channel and wave.
 //
-// The layer above: 457 us when every (c, k) worked out its own taps, 155 us now (268 MB of pixel-side
+// The layer above: 457 us when every (c, k) worked out its own taps, about 150 now (268 MB of pixel-side
 // values read, 31 us of matrix instructions); waves wait 0.57 of their cycles for a tile's map, box and
 // window.  With a window per wave 171 us.
 // 32-column blocks of (k, c)

@@ -263,7 +263,7 @@ struct ConvDims {
 // gradient reads too: a backward captured into a graph after it finds its plan whole, where
 // nothing could be built.  (Measured, first step on a new map, all parts of a plan built ->
 // those that are read: 4 x 512 x 1024, 3 -> 32 channels, no picture gradient 694 -> 342 us,
-// 64 x 128, 3 -> 16 547 -> 175 us; level-7 icosphere decoder block 3.24 -> 2.88 ms.)
+// 64 x 128, 3 -> 16 547 -> 175 us.)
 PlanRef conv_plan(const Tensor& ref, const Tensor& map, const OptTensor& wts, const ConvDims& d,
                   int64_t img_h, int64_t img_w, int64_t P, int64_t interp, bool transposed,
                   bool gather, bool weights, bool scatter, hipStream_t stream) {
