@@ -245,32 +245,25 @@ def _uncacheable(*keys):
     return any(k is _NO_KEY for k in keys)
 
 
-def _conv_plan(ref, sample_map, interp_weights, dims, img_h, img_w, P, interp, transposed, scatter):
-    """(plan tensor, bytes) for a call on this map, built on first use; (None, 0) when the library
-    has no plan for it, the call reads none or the cache is off.  dims: (B, Cin, Cout, K); scatter:
-    the call splats into the image (the backward of a convolution, the forward of a transposed one).
-    Calls that run by columns read at most the inverted map, and that only to scatter (a forward
-    whose input requires a gradient has it built for its backward)."""
+def _conv_plan(ref, sample_map, interp_weights, img_h, img_w, K, P, interp, columns=False):
+    """(plan tensor, bytes) for this map and geometry, built on first use; (None, 0) when the
+    library has no plan for it or the cache is off.  columns: the inverted map alone, for calls that
+    run by columns."""
     if not _plan_cache_enabled or ref.dtype != torch.float32:
         return None, 0
     MH, MW = int(sample_map.shape[0]), int(sample_map.shape[1])
     km, kw = _tensor_key(sample_map), _tensor_key(interp_weights)
     if _uncacheable(km, kw):
         return None, 0
-    B, Cin, Cout, K = (int(d) for d in dims)
-    size = (int(img_h), int(img_w), MH, MW, K, int(P), int(interp), _capi.SDK_F32)
-    lib = _capi.load()
-    columns = lib.sdk_mapped_conv_by_columns(B, Cin, Cout, *size, _current_mode(),
-                                             int(transposed)) == 1
-    if columns and not scatter:
-        return None, 0
-    key = (columns, ref.device, km, kw, int(img_h), int(img_w), K, int(P), int(interp))
+    key = (bool(columns), ref.device, km, kw, int(img_h), int(img_w), int(K), int(P), int(interp))
     cur = torch.cuda.current_stream(ref.device)
     ent = _cache_lookup(key, cur)
     if ent is not None:
         return ent.plan, ent.nbytes
     if torch.cuda.is_current_stream_capturing():
         return None, 0
+    lib = _capi.load()
+    size = (int(img_h), int(img_w), MH, MW, int(K), int(P), int(interp), _capi.SDK_F32)
     n = (lib.sdk_mapped_conv_columns_bytes if columns else lib.sdk_mapped_conv_plan_bytes)(*size)
     if n == 0:
         return None, 0
@@ -281,6 +274,23 @@ def _conv_plan(ref, sample_map, interp_weights, dims, img_h, img_w, P, interp, t
             None if interp_weights is None else interp_weights.untyped_storage())
     _cache_insert(key, _PlanEntry(plan, n, keep, cur))
     return plan, n
+
+
+def _plan_of_call(ref, sample_map, interp_weights, dims, img_h, img_w, P, interp, transposed,
+                  scatter):
+    """_conv_plan as a call of these sizes reads it.  dims: (B, Cin, Cout, K); scatter: the call splats
+    into the image (the backward of a convolution, the forward of a transposed one).  Calls that run
+    by columns read at most the inverted map, and that only to scatter (a forward whose input
+    requires a gradient has it built for its backward)."""
+    if ref.dtype != torch.float32:
+        return None, 0
+    B, Cin, Cout, K = (int(d) for d in dims)
+    columns = _capi.load().sdk_mapped_conv_by_columns(
+        B, Cin, Cout, int(img_h), int(img_w), int(sample_map.shape[0]), int(sample_map.shape[1]), K,
+        int(P), int(interp), _capi.SDK_F32, _current_mode(), int(transposed)) == 1
+    if columns and not scatter:
+        return None, 0
+    return _conv_plan(ref, sample_map, interp_weights, img_h, img_w, K, P, interp, columns)
 
 
 def _scatter_plan(kind, ref, sample_map, interp_weights, out_h, out_w, K, P, interp):
@@ -610,8 +620,8 @@ def mapped_conv_forward(x, sample_map, interp_weights, weight, bias, kernel_size
     out = torch.empty((B, Cout, OH, OW), dtype=x.dtype, device=x.device)
     with torch.cuda.device(x.device):
         ws, nws = _workspace(x, B, Cin, Cout, H, W, OH, OW, K, P, int(interp))
-        plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), H, W, P,
-                                 int(interp), False, x.requires_grad)
+        plan, nplan = _plan_of_call(x, sample_map, interp_weights, (B, Cin, Cout, K), H, W, P,
+                                    int(interp), False, x.requires_grad)
         dims = (B, Cin, H, W, Cout, OH, OW, K, P, int(interp), _DTYPES[x.dtype], _current_mode(),
                 _stream(x))
         if plan is None:
@@ -643,8 +653,8 @@ def mapped_conv_backward(grad_output, sample_map, interp_weights, x, weight, bia
         ws, nws = _workspace(x, B, Cin, Cout, H, W, OH, OW, K, P, int(interp))
         s = _stream(x)
         dims = (B, Cin, H, W, Cout, OH, OW, K, P, int(interp), dt, _current_mode(), s)
-        plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), H, W, P,
-                                 int(interp), False, True)
+        plan, nplan = _plan_of_call(x, sample_map, interp_weights, (B, Cin, Cout, K), H, W, P,
+                                    int(interp), False, True)
         if plan is None:
             _capi.call("sdk_mapped_conv_backward", _ptr(grad_output), _ptr(sample_map),
                        _ptr(interp_weights), _ptr(x), _ptr(weight), _ptr(gi), _ptr(gw), _ptr(gb),
@@ -670,8 +680,8 @@ def mapped_transposed_conv_forward(x, sample_map, interp_weights, weight, bias, 
     out = torch.empty((B, Cout, OH, OW), dtype=x.dtype, device=x.device)
     with torch.cuda.device(x.device):
         ws, nws = _workspace(x, B, Cin, Cout, OH, OW, IH, IW, K, P, int(interp))
-        plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), OH, OW, P,
-                                 int(interp), True, True)
+        plan, nplan = _plan_of_call(x, sample_map, interp_weights, (B, Cin, Cout, K), OH, OW, P,
+                                    int(interp), True, True)
         dims = (B, Cin, IH, IW, Cout, OH, OW, K, P, int(interp), _DTYPES[x.dtype], _current_mode(),
                 _stream(x))
         if plan is None:
@@ -702,8 +712,8 @@ def mapped_transposed_conv_backward(grad_output, sample_map, interp_weights, x, 
         ws, nws = _workspace(x, B, Cin, Cout, OH, OW, IH, IW, K, P, int(interp))
         s = _stream(x)
         dims = (B, Cin, IH, IW, Cout, OH, OW, K, P, int(interp), dt, _current_mode(), s)
-        plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), OH, OW, P,
-                                 int(interp), True, False)
+        plan, nplan = _plan_of_call(x, sample_map, interp_weights, (B, Cin, Cout, K), OH, OW, P,
+                                    int(interp), True, False)
         if plan is None:
             _capi.call("sdk_mapped_transposed_conv_backward", _ptr(grad_output), _ptr(sample_map),
                        _ptr(interp_weights), _ptr(x), _ptr(weight), _ptr(gi), _ptr(gw), _ptr(gb),
@@ -734,8 +744,8 @@ def mapped_conv_backward_select(grad_output, sample_map, interp_weights, x, weig
             else "sdk_mapped_conv_backward_select")
     with torch.cuda.device(x.device):
         ws, nws = _workspace(x, B, Cin, Cout, *img, *grid, K, P, int(interp))
-        plan, nplan = _conv_plan(x, sample_map, interp_weights, (B, Cin, Cout, K), *img, P,
-                                 int(interp), transposed, need_input and not transposed)
+        plan, nplan = _plan_of_call(x, sample_map, interp_weights, (B, Cin, Cout, K), *img, P,
+                                    int(interp), transposed, need_input and not transposed)
         _capi.call(name, _ptr(grad_output), _ptr(sample_map), _ptr(interp_weights), _ptr(x),
                    _ptr(weight), _ptr(gi), _ptr(gw), _ptr(gb), _ptr(ws), nws, _ptr(plan), nplan,
                    B, Cin, IH, IW, Cout, OH, OW, K, P, int(interp), _DTYPES[x.dtype],
