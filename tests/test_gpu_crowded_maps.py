@@ -98,8 +98,8 @@ def test_a_crowded_map_is_inverted_in_time(ops):
 
 
 @pytest.mark.parametrize("share", [0.002, 0.02, 0.1, 0.3, 1.0])
-@pytest.mark.parametrize("C,P", [(3, 0), (11, 0), (2, 3)])
-def test_average_unpooling_of_crowded_maps(ops, oracle, C, P, share):
+@pytest.mark.parametrize("C,P,interp", [(3, 0, 1), (11, 0, 2), (2, 3, 1), (2, 2, 0), (1, 2, 2)])
+def test_average_unpooling_of_crowded_maps(ops, oracle, C, P, interp, share):
     H, W, OH, OW, K = 24, 41, 48, 70, 9
     rng = np.random.default_rng(int(1000 * share) + C)
     shape = (OH, OW, K) + ((P,) if P else ())
@@ -107,11 +107,11 @@ def test_average_unpooling_of_crowded_maps(ops, oracle, C, P, share):
     m = _crowded(rng, m, share)
     iw = rng.uniform(0.1, 1, shape).astype(np.float32) if P else None
     g = rng.standard_normal((1, C, OH, OW)).astype(np.float32)
-    got = [ops.mapped_avg_unpool(_t(g), _t(m), _t(iw), H, W, K, 1) for _ in range(2)]
+    got = [ops.mapped_avg_unpool(_t(g), _t(m), _t(iw), H, W, K, interp) for _ in range(2)]
     assert torch.equal(*got)             # two maps, two builds of their lists
     f64 = lambda a: None if a is None else a.astype(np.float64)  # noqa: E731
-    want = oracle.mapped_avg_unpool(f64(g), f64(m), H, W, K, 1, f64(iw))
-    mag = oracle.mapped_avg_unpool(np.abs(f64(g)), f64(m), H, W, K, 1, f64(iw))
+    want = oracle.mapped_avg_unpool(f64(g), f64(m), H, W, K, interp, f64(iw))
+    mag = oracle.mapped_avg_unpool(np.abs(f64(g)), f64(m), H, W, K, interp, f64(iw))
     # n float32 additions of n terms each way (n: the samples on the spot at most, merged and then
     # summed): 2 n * 2^-24 of the sum of magnitudes would bound any order; the longest chain is 256
     # entries, or a wave's share of a list, and its tree
@@ -132,3 +132,19 @@ def test_a_crowded_map_does_not_stall_average_pooling(ops):
         kept.append(min(r[1] for r in runs))
     print("first", first, "kept", kept)
     assert kept[2] <= 25 * kept[1] and first[2] <= 40 * first[1]
+
+
+@pytest.mark.parametrize("share", [0.03, 0.1, 0.6])
+def test_products_gathered_on_crowded_maps(ops, oracle, share):
+    """Up-sampling layers of nearest taps gather their products through the same lists."""
+    H, W, OH, OW, K, Cin, Cout = 96, 129, 48, 64, 9, 12, 24
+    rng = np.random.default_rng(int(100 * share))
+    m = np.stack([rng.uniform(-1, W, (OH, OW, K)), rng.uniform(-1, H, (OH, OW, K))], -1)
+    m = _crowded(rng, m, share)
+    x = rng.standard_normal((2, Cout, OH, OW)).astype(np.float32)
+    w = (rng.standard_normal((Cout, Cin, K)) / np.sqrt(Cin * K)).astype(np.float32)
+    b = rng.standard_normal(Cin).astype(np.float32)
+    y = [ops.mapped_transposed_conv_forward(_t(x), _t(m), None, _t(w), _t(b), H, W, K, 0) for _ in range(2)]
+    assert torch.equal(*y)
+    want = oracle.mapped_transposed_conv_forward(x, m, w, b, H, W, K, 0, None)
+    assert relerr(y[0].cpu().numpy(), want) <= 1e-4
