@@ -271,8 +271,8 @@ def test_a_backward_captured_after_a_forward_finds_its_plan(ops, columns, transp
         lib.sdk_mapped_conv_columns_enable(1)
     print(times)
     # (the columns' gathers read no plan: nothing to rebuild in the backward of a transposed layer)
-    assert times["forward"] <= 1.1 * times["step"]
-    assert (columns and transposed) or times["forward"] <= 0.95 * times["nothing"]
+    assert times["forward"] <= 1.15 * times["step"]
+    assert (columns and transposed) or times["forward"] <= 0.97 * times["nothing"]
 
 
 def test_plan_parts_are_built_by_the_calls_that_read_them(ops, tile_kernels):
