@@ -253,4 +253,13 @@ __device__ __forceinline__ int set_rank(const WindowSet& ws, int n, int off) {
   return lo;
 }
 
+// Pixel (0..31) of a wave's 32 that lane position j = l % 32 works on.  A 16-byte LDS read serves
+// 16 lanes at a time, {0-3, 12-15, 20-23, 24-27} and {4-11, 16-19, 28-31} of each half wave: giving
+// each of those sets one row of 16 tile pixels makes their window elements consecutive, whatever
+// the window's width, and the 36-float stride spreads 16 consecutive elements over every bank.
+// (Two rows of a window 18 elements wide, pixels in lane order: 8.3 cycles a read instead of 4.4.)
+__device__ __forceinline__ int lane_pixel(int j) {
+  return 4 * (int)((0x73261540u >> (4 * (j >> 2))) & 7u) + (j & 3);   // nibble j / 4: pixel / 4
+}
+
 }  // namespace sdk

@@ -9,21 +9,35 @@
 // side, and the column values are produced straight into MFMA B fragments:
 //
 //   workgroup  = one 2-D tile of 128 pixels x TN = 32 * NB pixel-side channels x one batch element
-//   wave w     = pixels 32w .. 32w+31 of the tile x all TN channels (NB accumulators of 32 x 32)
-//   lane l     = pixel j = l % 32, reduction half h = l / 32
+//   wave w     = pixels 32 (w % 4) .. + 31 of the tile x all TN channels (NB accumulators of 32 x 32)
+//   lane l     = one pixel (lane_pixel), reduction half h = l / 32: channels 16 h .. 16 h + 15
 //
-// v_mfma_f32_32x32x2_f32 step s contracts channels 2s + h, so a lane needs the 16 channels
-// {h, h+2, ...} of its pixel; v_mfma_f32_32x32x16_bf16 instruction t contracts channels
-// 16t + 8h + 0..7.  The window and the weight tile keep the 32 channels of a chunk in that
-// order (position 16h + s, or 16h + 8t + j), so a lane reads its 16 values of one tap, and its
-// 16 weights of one row n, as four 16-byte LDS reads.  Per kernel sample and chunk a wave issues
-// 16 NB MFMAs, 64 fused multiply-adds, about 16 + 4 NB LDS reads and no global gather; plan rows
-// (window index, coefficient) are read from global memory one sample ahead, weights are staged
-// through a double-buffered LDS tile, and there is one barrier per sample.
+// v_mfma_f32_32x32x2_f32 step s contracts channels s and 16 + s of the chunk,
+// v_mfma_f32_32x32x16_bf16 instruction t channels 8 t .. 8 t + 7 and 16 + 8 t .. (which two a step
+// takes is free as long as both operands agree), so a lane reads its 16 values of one tap as four
+// 16-byte LDS reads.  The weights are laid out beforehand as the A operands they become, rounded or
+// split already (window_weight_kernel): a sample's tile is copied to LDS as it lies and read back
+// lane by lane, without conflicts and without conversions in the loop.  There is one buffer of it:
+// it is filled while the column values are gathered, behind one barrier, read by the MFMAs, and
+// free again behind the next.  That is what lets three workgroups share a CU, and three workgroups
+// at different points of a sample are what hides its waits.  Requests that cost no registers or
+// vector instructions are made through buffer descriptors (uniform base and offset).
+//
+// 8 x 128 x 256 x 512 -> 128, four-tap samples, the tiles inside their window (seven eighths):
+// float32 2411 -> 2208 us (two workgroups with a skewed window and two weight tiles before), bf16
+// 919 -> 615, split 1926 -> 1542; the polar eighth (big windows, one workgroup of two groups) 464 ->
+// 416, 253 -> 179 and 456 -> 327.  The inverse direction likewise (2537 -> 2397, 1097 -> 756,
+// 2082 -> 1685).  float32 is bound by its matrix products (1.73 ms of the 2.21 at the sustained
+// clock, to which vector instructions add); bf16 by its vector instructions (95 a sample and chunk, 64 of them
+// the blend), its sixteen window reads and what three workgroups leave of a window's latency:
+// without any global read it takes 400 of the 615 us, without its MFMAs 560.
 //
 // Rows padded by the plan (coefficient 0) are pointed at a zero element behind the window, so
 // a non-finite image value never meets a zero coefficient.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "conv_fused.hpp"
 #include "conv_plan.hpp"
@@ -36,40 +50,65 @@ namespace sdk {
 namespace {
 
 constexpr int kWgThreads = 256;
-constexpr int kWE = 36;   // floats per window element / weight row: 32 channels + 4 of skew
+constexpr int kWE = 36;   // floats per window element: 32 channels + 4 of skew
 
-// Position of channel c (0..31 inside its chunk) in a window element or weight row.
-__host__ __device__ constexpr int chunk_pos(int c, bool bf16) {
-  return bf16 ? 16 * ((c >> 3) & 1) + 8 * (c >> 4) + (c & 7) : 16 * (c & 1) + (c >> 1);
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Reads at uniform base + lane offset + uniform offset, both in bytes: no vector address arithmetic.
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc rsrc_of(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }
 
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
+// 16-byte pieces a lane reads of a 32 x 32 weight block, each 64 lanes wide: four of float32 (four
+// channels each), two of bf16 (eight), six of split operands (hi, mid, lo of two times eight).
+template <int MM>
+constexpr int kPieces = MM == kMmF32 ? 4 : (MM == kMmBf16 ? 2 : 6);
 
-// Wp[k][chunk][n][pos] (n padded to CpP, channels to whole chunks, zeros in the padding):
-// one (k, chunk, 128-row block) is 16 KB of consecutive memory.
+// The weights as A operands: piece p of row 32 blk + l % 32, sample k, chunk, for lane l (channels
+// 16 (l / 32) + .. of the chunk) is out[(((k chunks + chunk) blks + blk) kPieces + p) 64 + l].
+// Split: pieces hi of both eights, then mid, then lo.  Zeros past Cp and Cg.
 // swapped: the roles of the two channel indices of Wm are exchanged (Wm is [Cg, Cp * K]): the
 // contraction over the inverse plan gathers the pixel side and produces the image side.
+template <int MM>
 __global__ __launch_bounds__(kWgThreads) void window_weight_kernel(
-    const float* __restrict__ Wm, float* __restrict__ out, int Cp, int Cg, int K, int CpP,
-    int chunks, int bf16, int swapped) {
-  const size_t total = (size_t)K * chunks * CpP * kCC;
+    const float* __restrict__ Wm, u32x4* __restrict__ out, int Cp, int Cg, int K, int blks,
+    int chunks, int swapped) {
+  const size_t total = (size_t)K * chunks * blks * 128;
   for (size_t e = (size_t)blockIdx.x * kWgThreads + threadIdx.x; e < total;
        e += (size_t)gridDim.x * kWgThreads) {
-    const int pos = (int)(e % kCC);
-    const int n = (int)((e / kCC) % CpP);
-    const size_t rest = e / ((size_t)kCC * CpP);
+    const int lane = (int)(e & 63), t = (int)(e >> 6) & 1;
+    const size_t unit = e >> 7;
+    const int blk = (int)(unit % blks);
+    const size_t rest = unit / blks;
     const int chunk = (int)(rest % chunks), k = (int)(rest / chunks);
-    // inverse of chunk_pos
-    const int hh = pos >> 4, lo = pos & 15;
-    const int cl = bf16 ? 16 * (lo >> 3) + 8 * hh + (lo & 7) : 2 * lo + hh;
-    const int c = chunk * kCC + cl;
-    float v = 0.0f;
-    if (n < Cp && c < Cg)
-      v = swapped ? Wm[(size_t)c * Cp * K + (size_t)n * K + k]
-                  : Wm[(size_t)n * Cg * K + (size_t)c * K + k];
-    out[e] = v;
+    const int n = 32 * blk + (lane & 31), c0 = chunk * kCC + 16 * (lane >> 5) + 8 * t;
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int c = c0 + i;
+      f[i] = 0.0f;
+      if (n < Cp && c < Cg)
+        f[i] = swapped ? Wm[(size_t)c * Cp * K + (size_t)n * K + k]
+                       : Wm[(size_t)n * Cg * K + (size_t)c * K + k];
+    }
+    u32x4* dst = out + unit * kPieces<MM> * 64 + lane;
+    if constexpr (MM == kMmF32) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const u32x4 w = {__float_as_uint(f[4 * q]), __float_as_uint(f[4 * q + 1]),
+                         __float_as_uint(f[4 * q + 2]), __float_as_uint(f[4 * q + 3])};
+        dst[(2 * t + q) * 64] = w;
+      }
+    } else if constexpr (MM == kMmBf16) {
+      dst[t * 64] = __builtin_bit_cast(u32x4, pack_bf16x8(f));
+    } else {
+      const Bf16Split w = split_bf16x8(f);
+      dst[t * 64] = __builtin_bit_cast(u32x4, w.hi);
+      dst[(2 + t) * 64] = __builtin_bit_cast(u32x4, w.mid);
+      dst[(4 + t) * 64] = __builtin_bit_cast(u32x4, w.lo);
+    }
   }
 }
 
@@ -351,69 +390,75 @@ __global__ __launch_bounds__(1024) void tile_lists_kernel(const int* __restrict_
 }
 
 
-// CAP: elements of the LDS window.  kRegionCap: the tiles of `list` lie inside their window,
-// two workgroups share a CU.  kBigCap: `list` holds big tiles, whose window is their list in
-// big_lut; it takes most of a CU's LDS and one workgroup runs per CU.
+// MM: the matrix arithmetic.
+// CAP: elements of the LDS window.  kRegionCap: the tiles of `list` lie inside their window.
+// kBigCap: `list` holds big tiles, whose window is their list in big_lut; it takes most of a CU's
+// LDS and one workgroup runs per CU, of G = 2 groups of four waves: group g takes samples
+// g, g + 2, ... and the sums meet in LDS.
 // XR: plan rows beyond the first four that are requested ahead as well (0 or 2).  The lists of
 // an inverse plan are as long as targets have sources: at unit scale a third of the samples
 // of a weighted bispherical map have six rows somewhere in a tile.
 // RBT: plan rows requested and applied together: 4, or 1 for plans whose samples have a single
 // row (nearest taps without interpolation weights; three rows of padding would cost three
 // quarters of the gather's LDS reads and multiply-adds).
-template <int MM, int NB, int CAP, int XR, int RBT = 4>
-__global__ __launch_bounds__(kWgThreads, CAP > kRegionCap ? 1 : 2) void window_gemm_kernel(
-    const float* __restrict__ img, const int* __restrict__ hdr, const int* __restrict__ ns,
-    const int2* __restrict__ taps, const int* __restrict__ list, const int* __restrict__ count,
-    const float* __restrict__ Wp, const float* __restrict__ bias, float* __restrict__ pix, int Cg,
-    int H, int W, int Cp, int K, int S, int CpP, int chunks, PixelTiling pt, int tiles,
-    int n_tiles, const int* __restrict__ gate, const int* __restrict__ big_lut) {
+// SWZ: window elements of 32 floats whose 16-byte pieces change places (piece p of element e at
+// p ^ (e / 2) % 8) instead of 36 with a skew: 4 KB less, which is what a third workgroup needs
+// beside the float32 weight tile of 128 rows, for three more vector instructions a tap.
+template <int MM, int NB, int CAP, int XR, int RBT, int G, bool SWZ>
+__global__ __launch_bounds__(kWgThreads * G, CAP > kRegionCap || MM == kMmSplit ? 2 : 3) void
+window_gemm_kernel(const float* __restrict__ img, const int* __restrict__ hdr,
+                   const int* __restrict__ ns, const int2* __restrict__ taps,
+                   const int* __restrict__ list, const int* __restrict__ count,
+                   const u32x4* __restrict__ Wp, const float* __restrict__ bias,
+                   float* __restrict__ pix, int Cg, int H, int W, int Cp, int K, int S, int blks,
+                   int chunks, PixelTiling pt, int n_tiles, const int* __restrict__ gate,
+                   const int* __restrict__ big_lut) {
   if (gate != nullptr && *gate != 0) return;   // the plan is not valid: another kernel does the work
-  constexpr bool BF16 = MM != kMmF32;
   constexpr bool BIG = CAP > kRegionCap;
   constexpr int TN = 32 * NB;
-  __shared__ __align__(16) float region[(CAP + 1) * kWE];
-  __shared__ __align__(16) float As[2][TN * kWE];
-  __shared__ int src[CAP];
-  __shared__ int ns_l[kPlanKMax];   // rows per sample (a scalar load here would sit in the LDS waits)
+  constexpr int NW = 4 * G;          // waves
+  constexpr int CW = kCC / NW;       // channels of a chunk that a wave stages
+  constexpr int WT = NB * kPieces<MM> * 64;   // 16-byte pieces of a weight tile
+  constexpr int E = SWZ ? 32 : kWE;  // floats per window element
+  constexpr int WPT = (WT + kWgThreads - 1) / kWgThreads;
+  static_assert(G == 1 || TN * 128 <= (CAP + 1) * E, "the groups' sums meet in the window");
+  __shared__ __align__(128) float region[(CAP + 1) * E];
+  __shared__ __align__(16) u32x4 As[G * WT];
+  __shared__ unsigned char ns_l[kPlanKMax];   // (at most 32 rows, plan_supported)
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, h = lane >> 5;
-  // Workgroup ids go round-robin over the 8 XCDs (each with its own L2): XCD x takes the
-  // list entries [x * per, (x + 1) * per), so neighbouring tiles meet in one L2 and every XCD
-  // gets the same share of the list however long it is.
+  const int pw = wave & 3, group = wave >> 2;
   const int cnt = *count;
   const int per = (cnt + 7) >> 3;
   const int wg = blockIdx.x / n_tiles;
   const int slot = (wg & 7) * per + (wg >> 3);
   if ((wg >> 3) >= per || slot >= cnt) return;
   const int tile = list[slot];
-  const int n0 = (blockIdx.x % n_tiles) * TN;
+  const int nt = blockIdx.x % n_tiles, n0 = nt * TN;
   const int ty0 = (tile / pt.tiles_x) * pt.TY(), tx0 = (tile % pt.tiles_x) << pt.tx_shift;
   const int M = pt.OH * pt.OW;
   const size_t HW = (size_t)H * W;
   const float* img_b = img + (size_t)blockIdx.y * Cg * HW;
 
-  // this lane's pixel and its plan rows: row r of sample k at rows_p[(k * S + r) * 128]
-  const int p_local = 32 * wave + j;
-  int RS;
-  const int2* rows_p = taps + (size_t)tile * K * S * 128 + p_local;
-  if constexpr (BIG) {
-    const int* bl = big_lut + (size_t)tile * kBigStride;
-    RS = min(bl[0], CAP);
-    for (int e = tid; e < RS; e += kWgThreads) src[e] = bl[kBigLut + e];
-  } else {
-    RS = hdr[tile * kHdrStride + 2] * hdr[tile * kHdrStride + 3];
-    load_region_lut(hdr + (size_t)tile * kHdrStride, RS, src);
+  const int p_local = 32 * pw + lane_pixel(j);
+  // the window elements this lane stages (the same for every chunk): lane, lane + 64, ...
+  constexpr int ITER = (CAP + 63) / 64;
+  const int* lut = BIG ? big_lut + (size_t)tile * kBigStride : hdr + (size_t)tile * kHdrStride;
+  const int RS = BIG ? min(lut[0], CAP) : lut[2] * lut[3];
+  int wo[ITER];
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) {
+    const int e = lane + 64 * it;
+    const int o = e < RS ? lut[(BIG ? kBigLut : kHdrLut) + e] : -1;
+    wo[it] = o >= 0 ? o * 4 : 0x7ffffffc;
   }
-  if (tid < kWE) region[RS * kWE + tid] = 0.0f;   // the zero element padded rows point at
-  for (int k = tid; k < K; k += kWgThreads) ns_l[k] = ns[(size_t)tile * K + k];
+  if (tid < E) region[RS * E + tid] = 0.0f;   // the zero element padded rows point at
+  for (int k = tid; k < K; k += kWgThreads * G) ns_l[k] = (unsigned char)ns[(size_t)tile * K + k];
 
-  // The accumulators start at the bias of their rows (register v of lane l: row
-  // 8 (v / 4) + 4 (l / 32) + v % 4): the reads are issued here, with the window's, and the
-  // epilogue is stores alone.  (Read behind each store they serialise: on this part a wait
-  // for the load also waits for the store before it, 64 round trips per tile and wave.)
   floatx16 acc[NB];
-  if (bias != nullptr) {
+  if (bias != nullptr && group == 0) {
 #pragma unroll
     for (int a = 0; a < NB; ++a)
 #pragma unroll
@@ -429,189 +474,212 @@ __global__ __launch_bounds__(kWgThreads, CAP > kRegionCap ? 1 : 2) void window_g
       for (int v = 0; v < 16; ++v) acc[a][v] = 0.0f;
   }
 
-  // weight tile of (k, chunk): TN rows of 32 values, 16-byte pieces e = tid + 256 i
-  constexpr int WPT = TN * kCC / 4 / kWgThreads;   // float4 per thread: 4 (TN = 128), 2 or 1
-  static_assert(WPT == 4 || WPT == 2 || WPT == 1, "weight tile of 128, 64 or 32 rows");
-  float4 w0, w1, w2, w3;   // (named registers: an array here ends up in scratch memory)
-  w0 = w1 = w2 = w3 = make_float4(0.f, 0.f, 0.f, 0.f);
-#define SDK_LOAD_WEIGHTS(kv, chunkv)                                              \
-  do {                                                                            \
-    const float4* srcw = reinterpret_cast<const float4*>(                         \
-        Wp + (((size_t)(kv) * chunks + (chunkv)) * CpP + n0) * kCC) + tid;        \
-    w0 = srcw[0];                                                                 \
-    if constexpr (WPT >= 2) w1 = srcw[kWgThreads];                                \
-    if constexpr (WPT == 4) {                                                     \
-      w2 = srcw[2 * kWgThreads];                                                  \
-      w3 = srcw[3 * kWgThreads];                                                  \
-    }                                                                             \
+  // weight tile of (k, chunk): WT pieces in operand order, copied as they lie
+  const int gt = tid & (kWgThreads - 1);
+  u32x4 wq[WPT];
+  const Rsrc w_rs = rsrc_of(Wp + (size_t)nt * WT);
+#define SDK_LOAD_WEIGHTS(kv, chunkv)                                                           \
+  do {                                                                                         \
+    const int wso = ((kv) * chunks + (chunkv)) * blks * (kPieces<MM> * 1024);                  \
+    _Pragma("unroll") for (int i = 0; i < WPT; ++i) wq[i] = __builtin_amdgcn_raw_buffer_load_b128( \
+        w_rs, min(gt + i * kWgThreads, WT - 1) * 16, wso, 0);                                  \
   } while (0)
-#define SDK_STORE_WEIGHTS(bufv)                                                   \
-  do {                                                                            \
-    float* dstw = &As[bufv][(tid >> 3) * kWE + 4 * (tid & 7)];                    \
-    *reinterpret_cast<float4*>(dstw) = w0;                                        \
-    if constexpr (WPT >= 2) *reinterpret_cast<float4*>(dstw + 32 * kWE) = w1;     \
-    if constexpr (WPT == 4) {                                                     \
-      *reinterpret_cast<float4*>(dstw + 64 * kWE) = w2;                           \
-      *reinterpret_cast<float4*>(dstw + 96 * kWE) = w3;                           \
-    }                                                                             \
+#define SDK_STORE_WEIGHTS()                                                                    \
+  do {                                                                                         \
+    _Pragma("unroll") for (int i = 0; i < WPT; ++i)                                            \
+      if ((i + 1) * kWgThreads <= WT || gt + i * kWgThreads < WT)                              \
+        As[group * WT + gt + i * kWgThreads] = wq[i];                                          \
   } while (0)
 
-  // Plan rows of one sample: the first four are requested a whole sample ahead, without
-  // conditions (rows past the sample's count re-read its last slot and are masked when they
-  // are used), so that no branch and no wait sits between a request and the MFMAs that cover
-  // its latency.  Samples with more than four rows fetch the others when they need them.
+  // Plan rows of one sample, requested a whole sample ahead (rows past the sample's count re-read
+  // its last slot and are masked when they are used); the others when they are needed.
   constexpr int RB = RBT;
-  int2 rows[RB], rows_next[RB];
-  int2 xrows[XR > 0 ? XR : 1], xrows_next[XR > 0 ? XR : 1];
-#define SDK_LOAD_ROWS_N(dst, kv, r0v, NR)                                         \
-  do {                                                                            \
-    _Pragma("unroll") for (int u = 0; u < (NR); ++u)                              \
-      dst[u] = rows_p[((size_t)(kv) * S + min((r0v) + u, S - 1)) * 128];          \
-  } while (0)
-#define SDK_LOAD_ROWS(dst, kv, r0v) SDK_LOAD_ROWS_N(dst, kv, r0v, RB)
-  // col[] += the taps of up to four rows (FIRST: col[] = ..., the product of the first row
-  // instead of a register clear and a multiply-add)
-#define SDK_GATHER_ROWS(src, r0v, FIRST) SDK_GATHER_ROWS_N(src, r0v, FIRST, RB)
-#define SDK_GATHER_ROWS_N(src, r0v, FIRST, NR)                                    \
-  do {                                                                            \
-    int e[RB];                                                                    \
-    float co[RB];                                                                 \
-    _Pragma("unroll") for (int u = 0; u < (NR); ++u) {                            \
-      co[u] = (r0v) + u < n_rows ? __int_as_float(src[u].y) : 0.0f;               \
-      e[u] = co[u] != 0.0f ? src[u].x : RS;                                       \
-    }                                                                             \
-    _Pragma("unroll") for (int u = 0; u < (NR); ++u) {                            \
-      const float4* rp = reinterpret_cast<const float4*>(region + e[u] * kWE + 16 * h); \
-      const float4 d0 = rp[0], d1 = rp[1], d2 = rp[2], d3 = rp[3];                \
-      const float d[16] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w,        \
-                           d2.x, d2.y, d2.z, d2.w, d3.x, d3.y, d3.z, d3.w};       \
-      _Pragma("unroll") for (int i = 0; i < 16; ++i)                              \
-        colv[i] = (FIRST) && u == 0 ? co[u] * d[i] : __builtin_fmaf(co[u], d[i], colv[i]); \
-    }                                                                             \
-  } while (0)
-
-  int buf = 0;
-  SDK_LOAD_WEIGHTS(0, 0);
-  int n_rows = ns[(size_t)tile * K];
-  SDK_LOAD_ROWS(rows, 0, 0);
-  if constexpr (XR > 0) SDK_LOAD_ROWS_N(xrows, 0, RB, XR);
-  for (int chunk = 0; chunk < chunks; ++chunk) {
-    const int c0 = chunk * kCC;
-    __syncthreads();   // every wave is done with the previous chunk's window (and src is built)
-    {
-      // wave w stages channels 8w .. 8w+7 of every window element; a lane owns elements
-      // lane, lane + 64, ... and has all its loads in flight before the first LDS write
-      constexpr int ITER = (CAP + 63) / 64;
-      const int cw = c0 + 8 * wave;
-      const char* cbase = reinterpret_cast<const char*>(img_b + (size_t)min(cw, Cg - 1) * HW);
-      const unsigned plane = (unsigned)HW * 4u;
-      float v[ITER][8];
+  const Rsrc rows_rs = rsrc_of(taps + (size_t)tile * K * S * 128);
+  int2 rows[RB], xrows[XR > 0 ? XR : 1];
+  auto row_at = [&](int kv, int r) {
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rows_rs, p_local * 8,
+                                                         (kv * S + min(r, S - 1)) * 1024, 0);
+    return make_int2((int)v.x, (int)v.y);
+  };
+  const char* regb = reinterpret_cast<const char*>(region) + (SWZ ? 0 : 64 * h);
+  float colv[16];
+  // coefficient and window position of up to N rows, the zero element where there is none
+  auto decode = [&](const int2* rw, int r0, int n_rows, float* co, unsigned* at, auto count_c) {
+    constexpr int N = decltype(count_c)::value;
 #pragma unroll
-      for (int it = 0; it < ITER; ++it) {
-        const int e = lane + 64 * it;
-        const int o = e < RS ? src[e] : -1;
+    for (int u = 0; u < N; ++u) {
+      co[u] = r0 + u < n_rows ? __int_as_float(rw[u].y) : 0.0f;
+      const unsigned e = co[u] != 0.0f ? rw[u].x : RS;
+      at[u] = SWZ ? (e << 7) | (((4u * h) ^ ((e >> 1) & 7u)) << 4) : __umul24(e, E * 4u);
+    }
+  };
+  auto piece = [&](unsigned at, unsigned q) {
+    return *reinterpret_cast<const float4*>(regb + (SWZ ? at ^ (q << 4) : at + (q << 4)));
+  };
+  // colv += their taps (first: colv = ...), the next row's reads in flight behind a row's sums
+  auto gather = [&](const float* co, const unsigned* at, bool first, auto count_c) {
+    constexpr int N = decltype(count_c)::value;
+    float4 d[2][4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const bool ok = o >= 0 && cw + i < Cg;
-          const float d = *reinterpret_cast<const float*>(
-              cbase + (ok ? (unsigned)i * plane + (unsigned)o * 4u : 0u));
-          v[it][i] = ok ? d : 0.0f;
-        }
+    for (int q = 0; q < 4; ++q) d[0][q] = piece(at[0], q);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (u + 1 < N) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[(u + 1) & 1][q] = piece(at[u + 1], q);
+        asm volatile("" ::: "memory");
       }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 v = d[u & 1][q];
+        const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          colv[4 * q + i] = first && u == 0 ? co[u] * f[i]
+                                            : __builtin_fmaf(co[u], f[i], colv[4 * q + i]);
+      }
+    }
+  };
+
+  const int k_first = min(group, K - 1);
+  const int steps = (K + G - 1) / G;
+  SDK_LOAD_WEIGHTS(k_first, 0);
+#pragma unroll
+  for (int u = 0; u < RB; ++u) rows[u] = row_at(k_first, u);
+  if constexpr (XR > 0) {
+#pragma unroll
+    for (int u = 0; u < XR; ++u) xrows[u] = row_at(k_first, RB + u);
+  }
+  for (int chunk = 0; chunk < chunks; ++chunk) {
+    // wave w stages channels CW w .. of every window element
+    {
+      // Channels past the last come from an empty descriptor and elements outside the image from
+      // an offset past any: such reads return zero.
+      const int cw = chunk * kCC + CW * wave;
+      const float* cbase = img_b + (size_t)min(cw, Cg - 1) * HW;
+      const int plane = (int)(HW * 4u), valid = min(CW, Cg - cw);
+      float v[ITER][CW];
+#pragma unroll
+      for (int i = 0; i < CW; ++i) {
+        const Rsrc ch = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(cbase), 0, i < valid ? valid * plane : 0, 0x00020000);
+#pragma unroll
+        for (int it = 0; it < ITER; ++it)
+          v[it][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              ch, wo[it], i < valid ? i * plane : 0, 0));
+      }
+      __syncthreads();   // every wave is done with the previous chunk's window
 #pragma unroll
       for (int it = 0; it < ITER; ++it) {
         const int e = lane + 64 * it;
         if (e < RS) {
-          float* dst = region + e * kWE;
-          if constexpr (BF16) {
-            float4* d4 = reinterpret_cast<float4*>(dst + 16 * (wave & 1) + 8 * (wave >> 1));
-            d4[0] = make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
-            d4[1] = make_float4(v[it][4], v[it][5], v[it][6], v[it][7]);
-          } else {
-            *reinterpret_cast<float4*>(dst + 4 * wave) =
-                make_float4(v[it][0], v[it][2], v[it][4], v[it][6]);
-            *reinterpret_cast<float4*>(dst + 16 + 4 * wave) =
-                make_float4(v[it][1], v[it][3], v[it][5], v[it][7]);
+#pragma unroll
+          for (int i = 0; i < CW / 4; ++i) {
+            const int p = CW / 4 * wave + i;
+            *reinterpret_cast<float4*>(region + e * E + 4 * (SWZ ? p ^ ((e >> 1) & 7) : p)) =
+                make_float4(v[it][4 * i], v[it][4 * i + 1], v[it][4 * i + 2], v[it][4 * i + 3]);
           }
         }
       }
     }
-    if (chunk == 0) SDK_STORE_WEIGHTS(buf);   // (later chunks: stored behind the previous chunk's last sample)
     __syncthreads();
 
-    for (int k = 0; k < K; ++k) {
+    for (int step = 0; step < steps; ++step) {
+      const int k = group + step * G;
+      const bool live = G == 1 || k < K;
+      // As is free (a barrier lies behind its last reads): this sample's weights go in while its
+      // column values are gathered
+      SDK_STORE_WEIGHTS();
+      const int n_rows = live ? __builtin_amdgcn_readfirstlane(ns_l[k]) : 0;
+      float co[RB], xco[XR > 0 ? XR : 1];
+      unsigned at[RB], xat[XR > 0 ? XR : 1];
+      decode(rows, 0, n_rows, co, at, std::integral_constant<int, RB>{});
+      if constexpr (XR > 0) decode(xrows, RB, n_rows, xco, xat, std::integral_constant<int, XR>{});
       // ---- request the next sample's weights and first rows (after the last sample of the
       // last chunk: the first ones again, unused)
-      const bool last_k = k + 1 == K;
-      const int kn = last_k ? 0 : k + 1;
-      const int chunk_n = last_k ? (chunk + 1 < chunks ? chunk + 1 : 0) : chunk;
+      const bool wrap = k + G >= K;
+      const int kn = wrap ? k_first : k + G;
+      const int chunk_n = wrap ? (chunk + 1 < chunks ? chunk + 1 : 0) : chunk;
       SDK_LOAD_WEIGHTS(kn, chunk_n);
-      SDK_LOAD_ROWS(rows_next, kn, 0);
-      if constexpr (XR > 0) SDK_LOAD_ROWS_N(xrows_next, kn, RB, XR);
-      const int n_rows_next = __builtin_amdgcn_readfirstlane(ns_l[kn]);
-      asm volatile("" ::: "memory");   // the requests stay here, ahead of the gather and the MFMAs
-
-      // ---- gather: col[c][pixel j] for this lane's 16 channels of the chunk
-      float colv[16];
-      SDK_GATHER_ROWS(rows, 0, true);
-      if (n_rows > RB) {
-        if constexpr (XR > 0) SDK_GATHER_ROWS_N(xrows, RB, false, XR);
-        for (int r0 = RB + XR; r0 < n_rows; r0 += RB) {
-          int2 more[RB];
-          SDK_LOAD_ROWS(more, k, r0);
-          SDK_GATHER_ROWS(more, r0, false);
-        }
-      }
-      // ---- contraction
-      const float* at = &As[buf][j * kWE + 16 * h];
-      if constexpr (MM == kMmF32) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float4 aq[NB];
-#pragma unroll
-          for (int a = 0; a < NB; ++a)
-            aq[a] = *reinterpret_cast<const float4*>(at + a * 32 * kWE + 4 * q);
-#pragma unroll
-          for (int a = 0; a < NB; ++a) {
-            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[a].x, colv[4 * q + 0], acc[a], 0, 0, 0);
-            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[a].y, colv[4 * q + 1], acc[a], 0, 0, 0);
-            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[a].z, colv[4 * q + 2], acc[a], 0, 0, 0);
-            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[a].w, colv[4 * q + 3], acc[a], 0, 0, 0);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const float fb[8] = {colv[8 * t + 0], colv[8 * t + 1], colv[8 * t + 2], colv[8 * t + 3],
-                               colv[8 * t + 4], colv[8 * t + 5], colv[8 * t + 6], colv[8 * t + 7]};
-          Bf16Frag b16;
-          Bf16Split b3;
-          if constexpr (MM == kMmSplit) b3 = split_bf16x8(fb);
-          else b16 = pack_bf16x8(fb);
-#pragma unroll
-          for (int a = 0; a < NB; ++a) {
-            const float4 lo = *reinterpret_cast<const float4*>(at + a * 32 * kWE + 8 * t);
-            const float4 hi = *reinterpret_cast<const float4*>(at + a * 32 * kWE + 8 * t + 4);
-            const float fa[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            if constexpr (MM == kMmSplit) acc[a] = mfma_split(split_bf16x8(fa), b3, acc[a]);
-            else acc[a] = mfma_bf16(pack_bf16x8(fa), b16, acc[a]);
-          }
-        }
-      }
-      SDK_STORE_WEIGHTS(buf ^ 1);
-      lds_barrier();
-      buf ^= 1;
-      n_rows = n_rows_next;
-#pragma unroll
-      for (int u = 0; u < RB; ++u) rows[u] = rows_next[u];
+      for (int u = 0; u < RB; ++u) rows[u] = row_at(kn, u);
       if constexpr (XR > 0) {
 #pragma unroll
-        for (int u = 0; u < XR; ++u) xrows[u] = xrows_next[u];
+        for (int u = 0; u < XR; ++u) xrows[u] = row_at(kn, RB + u);
       }
+      asm volatile("" ::: "memory");   // the requests stay here, ahead of the gather and the MFMAs
+      if (live) {
+        gather(co, at, true, std::integral_constant<int, RB>{});
+        if (n_rows > RB) {
+          if constexpr (XR > 0) gather(xco, xat, false, std::integral_constant<int, XR>{});
+          for (int r0 = RB + XR; r0 < n_rows; r0 += RB) {
+            int2 more[RB];
+#pragma unroll
+            for (int u = 0; u < RB; ++u) more[u] = row_at(k, r0 + u);
+            decode(more, r0, n_rows, co, at, std::integral_constant<int, RB>{});
+            gather(co, at, false, std::integral_constant<int, RB>{});
+          }
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (live) {
+        const u32x4* at = As + group * WT + lane;
+        if constexpr (MM == kMmF32) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            f32x4 aq[NB];
+#pragma unroll
+            for (int a = 0; a < NB; ++a) aq[a] = __builtin_bit_cast(f32x4, at[(a * 4 + q) * 64]);
+#pragma unroll
+            for (int a = 0; a < NB; ++a)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(aq[a][i], colv[4 * q + i], acc[a], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const float fb[8] = {colv[8 * t + 0], colv[8 * t + 1], colv[8 * t + 2], colv[8 * t + 3],
+                                 colv[8 * t + 4], colv[8 * t + 5], colv[8 * t + 6], colv[8 * t + 7]};
+            if constexpr (MM == kMmBf16) {
+              const Bf16Frag b16 = pack_bf16x8(fb);
+#pragma unroll
+              for (int a = 0; a < NB; ++a)
+                acc[a] = mfma_bf16(__builtin_bit_cast(Bf16Frag, at[(a * 2 + t) * 64]), b16, acc[a]);
+            } else {
+              const Bf16Split b3 = split_bf16x8(fb);
+#pragma unroll
+              for (int a = 0; a < NB; ++a) {
+                Bf16Split a3;
+                a3.hi = __builtin_bit_cast(Bf16Frag, at[(a * 6 + t) * 64]);
+                a3.mid = __builtin_bit_cast(Bf16Frag, at[(a * 6 + 2 + t) * 64]);
+                a3.lo = __builtin_bit_cast(Bf16Frag, at[(a * 6 + 4 + t) * 64]);
+                acc[a] = mfma_split(a3, b3, acc[a]);
+              }
+            }
+          }
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
   }
-  // ---- epilogue: store.  Accumulator register v of lane l: row 8*(v/4) + 4*h + v%4
-  // (pixel-side channel), column j (pixel).
+  if constexpr (G > 1) {
+    // the second group's sums, added by the first: register-major, lane fastest
+    __syncthreads();
+    float* s = region + pw * (NB * 16 * 64) + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s[(a * 16 + v) * 64] = acc[a][v];
+    }
+    __syncthreads();
+    if (group == 1) return;
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][v] += s[(a * 16 + v) * 64];
+  }
   const int oy = ty0 + (p_local >> pt.tx_shift), ox = tx0 + (p_local & (pt.TX() - 1));
   if (oy < pt.OH && ox < pt.OW) {
     float* out = pix + (size_t)blockIdx.y * Cp * M + (size_t)oy * pt.OW + ox;
@@ -625,10 +693,6 @@ __global__ __launch_bounds__(kWgThreads, CAP > kRegionCap ? 1 : 2) void window_g
   }
 #undef SDK_LOAD_WEIGHTS
 #undef SDK_STORE_WEIGHTS
-#undef SDK_LOAD_ROWS
-#undef SDK_LOAD_ROWS_N
-#undef SDK_GATHER_ROWS
-#undef SDK_GATHER_ROWS_N
 }
 
 
@@ -657,8 +721,8 @@ template <int CH, int NBP>
 __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_kernel(
     const float* __restrict__ img, const int* __restrict__ hdr, const int* __restrict__ ns,
     const int2* __restrict__ taps, const int* __restrict__ list, const int* __restrict__ count,
-    const float* __restrict__ Wp, const float* __restrict__ bias, float* __restrict__ pix, int Cg,
-    int H, int W, int Cp, int K, int S, int CpP, int chunks, PixelTiling pt, int n_tiles,
+    const float4* __restrict__ Wp, const float* __restrict__ bias, float* __restrict__ pix, int Cg,
+    int H, int W, int Cp, int K, int S, int blks, int chunks, PixelTiling pt, int n_tiles,
     const int* __restrict__ gate) {
   if (gate != nullptr && *gate != 0) return;
   constexpr int XS = 32 * CH + 4;   // floats per source pixel in the window
@@ -694,8 +758,7 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
     Tl[(i / kPrT) * TSZ + kProductCap * kPrT + i % kPrT] = 0.0f;
   __syncthreads();
   {
-    // window: lane = source pixel, wave w = channels 8w .. 8w+7 of every chunk; the channels of
-    // a chunk lie in the order the MFMA steps take them (as in window_gemm_kernel)
+    // window: lane = source pixel, wave w = channels 8w .. 8w+7 of every chunk
     const int o = lane < RS ? src[lane] : -1;
     for (int chunk = 0; chunk < chunks; ++chunk) {
       const int cw = chunk * kCC + 8 * wave;
@@ -710,8 +773,8 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
         v[i] = ok ? d : 0.0f;
       }
       float* dst = X + lane * XS + chunk * kCC;
-      *reinterpret_cast<float4*>(dst + 4 * wave) = make_float4(v[0], v[2], v[4], v[6]);
-      *reinterpret_cast<float4*>(dst + 16 + 4 * wave) = make_float4(v[1], v[3], v[5], v[7]);
+      *reinterpret_cast<float4*>(dst + 8 * wave) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(dst + 8 * wave + 4) = make_float4(v[4], v[5], v[6], v[7]);
     }
   }
 
@@ -727,10 +790,9 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
   // MFMA role
   const int pb = wave & 1, cb = wave >> 1;
   const float* xrow = X + (32 * pb + j) * XS + 16 * h;
-  // weights of (k, chunk), rows n0 + HN cb + 32 a + j, this lane's 16 values: 4 x 16 bytes
-  auto weight_ptr = [&](int k, int chunk, int a) {
-    return reinterpret_cast<const float4*>(
-        Wp + (((size_t)k * chunks + chunk) * CpP + n0 + HN * cb + 32 * a + j) * kCC + 16 * h);
+  // weights of (k, chunk), rows n0 + HN cb + 32 a + j, this lane's 16 values: piece q of four
+  auto weight_at = [&](int k, int chunk, int a, int q) {
+    return Wp[((((size_t)k * chunks + chunk) * blks + (n0 + HN * cb) / 32 + a) * 4 + q) * 64 + lane];
   };
   // Weights come from global memory (the L2) straight into A operands.  Where the registers
   // allow it (WS) all of a sample's weights are requested a whole sample ahead; otherwise one
@@ -743,7 +805,7 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
 #pragma unroll
     for (int a = 0; a < NBP; ++a)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) wa[c][a][q] = weight_ptr(0, min(c, chunks - 1), a)[q];
+      for (int q = 0; q < 4; ++q) wa[c][a][q] = weight_at(0, min(c, chunks - 1), a, q);
   __syncthreads();   // the window is complete
 
   for (int k = 0; k < K; ++k) {
@@ -776,7 +838,7 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
 #pragma unroll
         for (int a = 0; a < NBP; ++a)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) wn[c][a][q] = weight_ptr(kn, min(c, chunks - 1), a)[q];
+          for (int q = 0; q < 4; ++q) wn[c][a][q] = weight_at(kn, min(c, chunks - 1), a, q);
 #pragma unroll
       for (int c = 0; c < WC; ++c)
         if (c < chunks) SDK_PRODUCT_CHUNK(c, wa[c]);
@@ -794,7 +856,7 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
 #pragma unroll
         for (int a = 0; a < NBP; ++a)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) wn[0][a][q] = weight_ptr(kn, cn, a)[q];
+          for (int q = 0; q < 4; ++q) wn[0][a][q] = weight_at(kn, cn, a, q);
         SDK_PRODUCT_CHUNK(chunk, wa[0]);
 #pragma unroll
         for (int a = 0; a < NBP; ++a)
@@ -857,9 +919,9 @@ bool window_gemm_supported(const ConvGeom& g) {
 }
 
 size_t window_gemm_weight_bytes(const ConvGeom& g) {
-  const size_t CpP = (size_t)(g.Cp + 127) / 128 * 128;
+  const size_t blks = (size_t)(g.Cp + 127) / 128 * 4;
   const size_t chunks = (size_t)(g.Cg + kCC - 1) / kCC;
-  return (size_t)g.K * chunks * CpP * kCC * sizeof(float);
+  return (size_t)g.K * chunks * blks * kPieces<kMmSplit> * 1024;   // (the largest arithmetic)
 }
 
 size_t tile_lists_bytes(const ConvGeom& g) {
@@ -891,17 +953,20 @@ int build_tile_lists(const Plan& plan, void* workspace, hipStream_t stream, Tile
 int window_gemm(const ConvGeom& g, int mm, const Plan& plan, const TileLists& tl,
                 const float* img, const float* Wm, bool swapped, const float* bias, float* pix,
                 float* weights, const int* gate, hipStream_t stream, int which) {
-  const int CpP = (g.Cp + 127) / 128 * 128;
+  const int blks = (g.Cp + 127) / 128 * 4;
   const int chunks = (g.Cg + kCC - 1) / kCC;
   const bool big = which == kListBig;
+  u32x4* wp = reinterpret_cast<u32x4*>(weights);
+  if (big && plan.big_lut == nullptr) return SDK_OK;
   if (!big) {
-    const size_t total = (size_t)g.K * chunks * CpP * kCC;
-    const int blocks = (int)std::min<size_t>((total + kWgThreads - 1) / kWgThreads, 2048);
-    launch(window_weight_kernel, dim3(blocks), dim3(kWgThreads), stream, Wm, weights, g.Cp, g.Cg,
-           g.K, CpP, chunks, mm != kMmF32 ? 1 : 0, swapped ? 1 : 0);
+    const size_t total = (size_t)g.K * chunks * blks * 128;
+    const dim3 wgrid((unsigned)std::min<size_t>((total + kWgThreads - 1) / kWgThreads, 2048));
+#define WW(MMv)                                                                              \
+  launch(window_weight_kernel<MMv>, wgrid, dim3(kWgThreads), stream, Wm, wp, g.Cp, g.Cg, g.K, \
+         blks, chunks, swapped ? 1 : 0)
+    if (mm == kMmBf16) WW(kMmBf16); else if (mm == kMmSplit) WW(kMmSplit); else WW(kMmF32);
+#undef WW
     SDK_LAUNCH_CHECK("window_weight");
-  } else if (big && plan.big_lut == nullptr) {
-    return SDK_OK;
   }
   const bool wide = g.Cp > 64, thin = g.Cp <= 32;
   const int TN = wide ? 128 : (thin ? 32 : 64);
@@ -914,25 +979,20 @@ int window_gemm(const ConvGeom& g, int mm, const Plan& plan, const TileLists& tl
   // (wide layers only: with fewer MFMAs per sample the two extra requests cost more than the
   // exposed reads they save; configuration 5's up-sampling layer 0.35 -> 0.38 ms)
   const bool more_rows = swapped && plan.S > 4 && wide;
-#define WG4(MMv, NBv, CAPv, XRv)                                                               \
-  launch(window_gemm_kernel<MMv, NBv, CAPv, XRv>, grid, dim3(kWgThreads), stream, img,         \
-         plan.hdr, plan.ns, plan.taps, list, count, (const float*)weights, bias, pix, g.Cg,    \
-         g.H, g.W, g.Cp, g.K, plan.S, CpP, chunks, plan.pt, plan.tiles, n_tiles, gate,         \
-         plan.big_lut)
-#define WG3(MMv, NBv, CAPv)                                                    \
-  do {                                                                         \
-    if (more_rows) WG4(MMv, NBv, CAPv, 2); else WG4(MMv, NBv, CAPv, 0);        \
+#define WG5(MMv, NBv, CAPv, XRv, RBv, Gv)                                                       \
+  launch(window_gemm_kernel<MMv, NBv, CAPv, XRv, RBv, Gv, (MMv == kMmF32 && NBv == 4 && Gv == 1)>, \
+         grid, dim3(kWgThreads * Gv), stream, img, plan.hdr, plan.ns, plan.taps, list, count,   \
+         (const u32x4*)wp, bias, pix, g.Cg, g.H, g.W, g.Cp, g.K, plan.S, blks, chunks, plan.pt, \
+         n_tiles, gate, plan.big_lut)
+#define WG3(MMv, NBv, CAPv, Gv)                                                          \
+  do {                                                                                   \
+    if (more_rows) WG5(MMv, NBv, CAPv, 2, 4, Gv); else WG5(MMv, NBv, CAPv, 0, 4, Gv);    \
   } while (0)
-#define WG1R(MMv, NBv)                                                                         \
-  launch(window_gemm_kernel<MMv, NBv, kRegionCap, 0, 1>, grid, dim3(kWgThreads), stream, img,  \
-         plan.hdr, plan.ns, plan.taps, list, count, (const float*)weights, bias, pix, g.Cg,    \
-         g.H, g.W, g.Cp, g.K, plan.S, CpP, chunks, plan.pt, plan.tiles, n_tiles, gate,         \
-         plan.big_lut)
 #define WG2(MMv, NBv)                                                 \
   do {                                                                \
-    if (big) WG3(MMv, NBv, kBigCap);                                  \
-    else if (plan.S == 1) WG1R(MMv, NBv);                             \
-    else WG3(MMv, NBv, kRegionCap);                                   \
+    if (big) WG3(MMv, NBv, kBigCap, 2);                               \
+    else if (plan.S == 1) WG5(MMv, NBv, kRegionCap, 0, 1, 1);         \
+    else WG3(MMv, NBv, kRegionCap, 1);                                \
   } while (0)
 #define WG1(MMv)                                                            \
   do {                                                                      \
@@ -942,10 +1002,9 @@ int window_gemm(const ConvGeom& g, int mm, const Plan& plan, const TileLists& tl
   else if (mm == kMmSplit) WG1(kMmSplit);
   else WG1(kMmF32);
 #undef WG1
-#undef WG1R
 #undef WG2
 #undef WG3
-#undef WG4
+#undef WG5
   SDK_LAUNCH_CHECK(big ? "window_gemm(big)" : "window_gemm");
   return SDK_OK;
 }
@@ -957,15 +1016,16 @@ bool window_product_supported(const ConvGeom& g, int mm) {
 int window_product(const ConvGeom& g, const Plan& plan, const TileLists& tl, const float* img,
                    const float* bias, float* pix, const float* weights, const int* gate,
                    hipStream_t stream) {
-  const int CpP = (g.Cp + 127) / 128 * 128;
+  const int blks = (g.Cp + 127) / 128 * 4;
   const int chunks = (g.Cg + kCC - 1) / kCC;
   const bool wide = g.Cp > 64;
   const int n_tiles = (int)ceil_div(g.Cp, wide ? 128 : 64);
   const dim3 grid((unsigned)((plan.tiles + 7) / 8 * 8 * n_tiles), (unsigned)g.B);
 #define WP2(CHv, NBPv)                                                                        \
   launch(window_product_kernel<CHv, NBPv>, grid, dim3(kWgThreads), stream, img, plan.hdr,     \
-         plan.ns, plan.taps, tl.product, tl.count + 4, weights, bias, pix, g.Cg, g.H, g.W,    \
-         g.Cp, g.K, plan.S, CpP, chunks, plan.pt, n_tiles, gate)
+         plan.ns, plan.taps, tl.product, tl.count + 4,                                        \
+         reinterpret_cast<const float4*>(weights), bias, pix, g.Cg, g.H, g.W,                 \
+         g.Cp, g.K, plan.S, blks, chunks, plan.pt, n_tiles, gate)
 #define WP(CHv)                                     \
   do {                                              \
     if (wide) WP2(CHv, 2); else WP2(CHv, 1);        \

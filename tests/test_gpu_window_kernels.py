@@ -1,0 +1,86 @@
+"""The LDS-window convolution kernels (csrc/conv_window_*.hip) on values
+whose every product and sum is a float32 number, rounded to bf16 or not: integers of at most four
+bits and sample positions at halves, so blended values are multiples of 1/4 below 2^6 and sums stay
+below 2^24 quarters.  Every arithmetic then has one right answer, the oracle's, to the bit."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+# (batch, Cin, Cout, H, W, OH, OW, K, interp, points): channels around a chunk of 32, rows around the
+# 32, 64 and 128 a workgroup multiplies, widths no multiple of 4 or of a tile's 16 pixels, every way
+# the samples are shared among the waves (K % 4, K = 10 in eight waves), single-row plans, more than
+# four rows a sample, tiles inside their window and (strided, scattered samples) big ones
+SIZES = [
+    (1, 5, 65, 9, 20, 9, 20, 9, 1, 0),
+    (2, 32, 128, 17, 33, 17, 33, 9, 1, 0),
+    (1, 33, 130, 16, 32, 16, 32, 10, 2, 0),
+    (1, 70, 96, 10, 19, 10, 19, 7, 0, 0),
+    (2, 40, 72, 48, 96, 24, 48, 9, 1, 0),
+    (1, 64, 100, 40, 80, 20, 40, 4, 2, 0),
+    (1, 37, 66, 12, 24, 12, 24, 1, 1, 0),
+    (1, 34, 68, 8, 11, 8, 11, 2, 1, 0),
+    (1, 8, 80, 9, 16, 9, 16, 3, 0, 2),
+    (2, 31, 33, 14, 18, 14, 18, 5, 1, 0),
+    (1, 36, 127, 16, 40, 16, 40, 6, 2, 0),
+    (1, 64, 66, 24, 40, 12, 20, 8, 0, 2),
+    (3, 20, 129, 32, 64, 32, 64, 9, 0, 2),
+]
+
+
+def _arrays(tc):
+    B, Cin, Cout, H, W, OH, OW, K, interp, P = tc
+    rng = np.random.default_rng(sum(tc))
+    side = int(np.ceil(np.sqrt(K)))
+    k = np.arange(K)
+    ys = np.arange(OH)[:, None, None] * (H / OH) + (k // side - 1) * 1.5
+    xs = np.arange(OW)[None, :, None] * (W / OW) + (k % side - 1) * 1.5
+    ys, xs = (np.broadcast_to(a, (OH, OW, K)) + rng.integers(-1, 2, (OH, OW, K)) * 0.5
+              for a in (ys, xs))
+    ys = np.round(ys * 2) / 2
+    xs = np.round(xs * 2) / 2 % W
+    iw = None
+    if P:
+        ys, xs = (np.stack([a + p for p in range(P)], -1) for a in (np.floor(ys), np.floor(xs)))
+        iw = np.broadcast_to(np.array([0.5, 0.25, 0.25, 0.5][:P]), ys.shape).astype(np.float32).copy()
+    m = np.stack([xs, ys], -1).astype(np.float32)
+    f = lambda *s: rng.integers(-4, 5, s).astype(np.float32)  # noqa: E731
+    return m, iw, f(B, Cin, H, W), f(Cout, Cin, K), f(Cout), f(B, Cout, OH, OW)
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
+def test_exact_values(oracle, tile_kernels, tc, mode):
+    import _spherical_distortion_ext._ops as ops
+    K, interp = tc[7], tc[8]
+    m, iw, x, w, b, g = _arrays(tc)
+    t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
+    tx, tm, tiw, tw, tb, tg = map(t, (x, m, iw, w, b, g))
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(tx, tm, tiw, tw, tb, K, interp)
+        gi, gw, gb = ops.ops.mapped_conv_backward(tg, tm, tiw, tx, tw, tb, K, interp)
+    assert np.array_equal(y.cpu().numpy(), oracle.mapped_conv_forward(x, m, w, b, K, interp, iw))
+    wi, ww, wb = oracle.mapped_conv_backward(g, m, x, w, b, K, interp, iw)
+    for have, want in ((gi, wi), (gw, ww), (gb, wb)):
+        assert np.array_equal(have.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+def test_values_that_are_not_finite_stay_where_they_are(tile_kernels, mode):
+    """An infinite pixel reaches the outputs and weights that read it and no others (padding of
+    plans, channels and rows multiplies zeros by zeros)."""
+    import _spherical_distortion_ext._ops as ops
+    tc = (1, 33, 70, 16, 36, 16, 36, 9, 1, 0)
+    m, _, x, w, b, g = _arrays(tc)
+    w[w == 0], g[g == 0] = 1, 1
+    x[0, 32, 5, 7] = np.inf
+    m[..., 0] = np.minimum(np.abs(m[..., 0]), 34)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(t(x), t(m), None, t(w), t(b), 9, 1).cpu().numpy()
+        gw = ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 9, 1)[1].cpu().numpy()
+    reads = ((np.abs(m[..., 0] - 7) < 1) & (np.abs(m[..., 1] - 5) < 1)).any(-1)
+    assert np.array_equal(~np.isfinite(y[0]).all(0), reads)
+    assert np.isfinite(gw[:, :32]).all() and not np.isfinite(gw[:, 32]).all()
