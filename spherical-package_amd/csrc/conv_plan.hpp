@@ -163,6 +163,12 @@ int window_wgrad_narrow(const ConvGeom& g, int mm, const Plan& plan, const TileL
                         const float* pix, const float* img, float* gW, float* partial,
                         hipStream_t stream);
 
+// Its bf16 arithmetic (conv_window_wgrad16.hip): leaves accumulator register 16 k + v of row block
+// (thread / 64), K * 16 * 256 floats a workgroup, in `partial`.
+int window_wgrad16(const ConvGeom& g, const Plan& plan, const int* list, const int* count, bool big,
+                   const float* pix, const float* img, float* partial, int groups, int c_chunks,
+                   int n_tiles, int64_t slots, hipStream_t stream);
+
 size_t window_wgrad_partial_bytes(const ConvGeom& g);
 // big: the sums over the tiles of tl.big, from their big windows.
 int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& tl,

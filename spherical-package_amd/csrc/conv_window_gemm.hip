@@ -23,11 +23,11 @@
 // at different points of a sample are what hides its waits.  Requests that cost no registers or
 // vector instructions are made through buffer descriptors (uniform base and offset).
 //
-// 8 x 128 x 256 x 512 -> 128, four-tap samples, the tiles inside their window (seven eighths):
+// 8 x 128 x 256 x 512 -> 128, four-tap samples, the tiles inside their window (seven eighths; kernel times):
 // float32 2411 -> 2208 us (two workgroups with a skewed window and two weight tiles before), bf16
 // 919 -> 615, split 1926 -> 1542; the polar eighth (big windows, one workgroup of two groups) 464 ->
 // 416, 253 -> 179 and 456 -> 327.  The inverse direction likewise (2537 -> 2397, 1097 -> 756,
-// 2082 -> 1685).  float32 is bound by its matrix products (1.73 ms of the 2.21 at the sustained
+// 2082 -> 1685).  float32 is bound by its matrix products (1.72 ms at the published rate, 1.97 at the sustained
 // clock, to which vector instructions add); bf16 by its vector instructions (95 a sample and chunk, 64 of them
 // the blend), its sixteen window reads and what three workgroups leave of a window's latency:
 // without any global read it takes 400 of the 615 us, without its MFMAs 560.

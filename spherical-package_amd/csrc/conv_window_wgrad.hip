@@ -1,5 +1,5 @@
 // Weight gradient of mapped convolution from an LDS window, driven by a tap plan (gfx950,
-// float32 tensors, fp32 MFMA):
+// float32 tensors, fp32 MFMA or operands split into bf16 pieces):
 //
 //   gW[n][c][k] += sum_{b, m} pix[b][n][m] * col[b][(c, k)][m]
 //   col[b][(c, k)][m] = sum_r coefficient(m, k, r) * img[b][c][tap(m, k, r)]
@@ -386,7 +386,8 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
 #undef SDK_VALS_ISSUE
 #undef SDK_BLEND
       } else {
-        // ---- bf16 matrix unit (operands rounded to bf16, or split into three bf16 pieces):
+        // ---- bf16 matrix unit, operands split into three bf16 pieces (rounded operands have a
+        // kernel of their own, conv_window_wgrad16.hip):
         // one instruction contracts 16 pixels, lane (j, h) supplying its row / channel for the
         // eight pixels 8 h .. 8 h + 7 of the group.  A lane therefore builds eight column values
         // per sample and instruction from the window (the same reads and multiply-adds per
@@ -397,8 +398,7 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
 #pragma unroll 1
         for (int grp = 0; grp < 2; ++grp) {
           const int m0 = 16 * grp + 8 * h;   // first of this lane's eight pixels of the quarter
-          Bf16Frag b16[KW];
-          Bf16Split b3[MM == kMmSplit ? KW : 1];
+          Bf16Split b3[KW];
 #pragma unroll
           for (int c = 0; c < KW; ++c) {
             const int k = c < KP ? wave * KP + c : 4 * KP + (c - KP);
@@ -416,8 +416,7 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
               t = __builtin_fmaf(__int_as_float(r23.y), v2, t);
               bv[i] = __builtin_fmaf(__int_as_float(r23.w), v3, t);
             }
-            if constexpr (MM == kMmSplit) b3[c] = split_bf16x8(bv);
-            else b16[c] = pack_bf16x8(bv);
+            b3[c] = split_bf16x8(bv);
           }
           // A fragments: rows 32 a + j (and 32 wave + j for the remaining samples)
           auto a_values = [&](int row, float (&f)[8]) {
@@ -431,29 +430,17 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
             if constexpr (KP > 0) {
               float f[8];
               a_values(32 * a + j, f);
-              if constexpr (MM == kMmSplit) {
-                const Bf16Split a3 = split_bf16x8(f);
+              const Bf16Split a3 = split_bf16x8(f);
 #pragma unroll
-                for (int kk = 0; kk < KP; ++kk) accF[kk][a] = mfma_split(a3, b3[kk], accF[kk][a]);
-              } else {
-                const Bf16Frag a16 = pack_bf16x8(f);
-#pragma unroll
-                for (int kk = 0; kk < KP; ++kk) accF[kk][a] = mfma_bf16(a16, b16[kk], accF[kk][a]);
-              }
+              for (int kk = 0; kk < KP; ++kk) accF[kk][a] = mfma_split(a3, b3[kk], accF[kk][a]);
             }
           }
           if constexpr (R > 0) {
             float f[8];
             a_values(32 * wave + j, f);
-            if constexpr (MM == kMmSplit) {
-              const Bf16Split a3 = split_bf16x8(f);
+            const Bf16Split a3 = split_bf16x8(f);
 #pragma unroll
-              for (int r = 0; r < R; ++r) accR[r] = mfma_split(a3, b3[KP + r], accR[r]);
-            } else {
-              const Bf16Frag a16 = pack_bf16x8(f);
-#pragma unroll
-              for (int r = 0; r < R; ++r) accR[r] = mfma_bf16(a16, b16[KP + r], accR[r]);
-            }
+            for (int r = 0; r < R; ++r) accR[r] = mfma_split(a3, b3[KP + r], accR[r]);
           }
         }
       }
@@ -581,7 +568,14 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
   const int TX = plan.pt.TX();
   const int vec4 = (g.OW % 4 == 0 && TX >= 16 && reinterpret_cast<uintptr_t>(pix) % 16 == 0) ? 1 : 0;
   const dim3 grid((unsigned)w.slots);
-  const int KP = g.K / 4, R = g.K % 4;
+  int KP = g.K / 4, R = g.K % 4;
+  if (mm == kMmBf16) {
+    const int rc = window_wgrad16(g, plan, list, count, big, pix, img, partial, w.groups,
+                                  w.c_chunks, w.n_tiles, w.slots, stream);
+    if (rc) return rc;
+    KP = 0;   // (its accumulators: one row block a wave for every sample)
+    R = g.K;
+  } else {
 #define WW3(KPv, Rv, CAPv, MMv)                                                                  \
   launch(window_wgrad_kernel<KPv, Rv, CAPv, MMv>, grid, dim3(kWwThreads), stream, pix, img,      \
          plan.hdr, plan.ns, plan.taps, list, count, partial, g.Cg, g.H, g.W, g.Cp, plan.S,       \
@@ -592,8 +586,7 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
          plan.pt, w.groups, (int)g.B, w.c_chunks, w.n_tiles, vec4, plan.big_lut)
 #define WW2(KPv, Rv, CAPv)                                                       \
   do {                                                                           \
-    if (mm == kMmBf16) WW3(KPv, Rv, CAPv, kMmBf16);                              \
-    else if (mm == kMmSplit) WW3(KPv, Rv, CAPv, kMmSplit);                       \
+    if (mm == kMmSplit) WW3(KPv, Rv, CAPv, kMmSplit);                            \
     else if (plan.S == 1) WW3ONE(KPv, Rv, CAPv);                                 \
     else WW3(KPv, Rv, CAPv, kMmF32);                                             \
   } while (0)
@@ -618,6 +611,7 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
 #undef WW3
 #undef WW3ONE
   SDK_LAUNCH_CHECK(big ? "window_wgrad(big)" : "window_wgrad");
+  }
   const int kinds0 = w.c_chunks * w.n_tiles, total = (int)g.B * w.groups;
   const int parts = (int)std::min<int64_t>(std::min(total, 16),
                                            ceil_div(2048, (int64_t)w.nreg * kinds0));
