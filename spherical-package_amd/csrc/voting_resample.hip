@@ -4,7 +4,8 @@
 // (ext_modules/include/core/interpolation.h:249-265, core/resample.h:163-172,
 // common/resample.h:109-130, src/cpp/voting_resample_layer.cpp:8-37).  Here the histogram is a
 // caller-provided workspace of 32-bit counters (a pixel cannot collect 2^31 votes), reused
-// pass after pass for as many batch elements as it holds; the first label with the most votes wins, label 0 where nobody voted.
+// pass after pass for as many batch elements as it holds; the first label with the most votes wins,
+// label 0 where nobody voted.  Where the map is coherent the histogram never leaves LDS (below).
 // With more than one channel the reference's histograms overlap (its channel offset lacks the
 // factor `candidates`); label images have one channel, and the overlap is reproduced as it is.
 #include <hip/hip_runtime.h>
@@ -18,13 +19,147 @@ namespace sdk {
 
 constexpr int kVoteBlock = 256;
 
-__global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restrict__ p, size_t n16) {
+// ---------------------------------------------------------------------------------------------
+// Coherent maps: neighbouring pixels vote for neighbouring cells.  vote_boxes_kernel leaves, per
+// tile of 16 x 16 input pixels, the box of the cells its pixels vote for; a workgroup of
+// vote_tile_kernel owns a tile of output cells, finds the input tiles whose box meets it, counts
+// their votes in LDS and writes the winners.  Every label is read about once, every histogram
+// counter stays in LDS: 4 x 512 x 1024 labels, 13 classes, halved: clear 12 + votes 35 + argmax 10
+// us (27 MB of counters cleared, added to by atomics and scanned) -> boxes 6 + cells 10.  A cell tile
+// that more than kVoteMeet input tiles vote into says so in a flag, and the histogram kernels, launched
+// behind it on that flag, do the whole pass again; they cost 2 us each where they have nothing
+// to do (57 -> 27 us a call; a scrambled map, which pays for both, 103 -> 114).
+// ---------------------------------------------------------------------------------------------
+constexpr int kVoteTile = 16;        // input tile side
+constexpr int kVoteMeet = 64;        // input tiles (16384 pixels) a workgroup takes on
+constexpr int kVoteTiles = 8192;     // input tiles: every workgroup looks through all boxes (64 KB)
+constexpr int kVoteCounters = 4096;  // LDS counters of a workgroup
+constexpr int kVoteGridX = 256;      // blocks per plane of a launch that may find nothing to do
+
+__global__ __launch_bounds__(kVoteTile * kVoteTile) void vote_boxes_kernel(
+    const int64_t* __restrict__ map, ushort4* __restrict__ boxes, int* __restrict__ flag, int IH,
+    int IW, int tiles_x, int OH, int OW) {
+  __shared__ int box[4];
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0 && tid == 0) *flag = 0;
+  if (tid < 4) box[tid] = tid < 2 ? 0xffff : 0;
+  __syncthreads();
+  const int iy = (blockIdx.x / tiles_x) * kVoteTile + tid / kVoteTile;
+  const int ix = (blockIdx.x % tiles_x) * kVoteTile + tid % kVoteTile;
+  int x0 = 0xffff, y0 = 0xffff, x1 = 0, y1 = 0;   // (x1, y1: one past the last)
+  if (iy < IH && ix < IW) {
+    const longlong2 t = reinterpret_cast<const longlong2*>(map)[(size_t)iy * IW + ix];
+    if (t.x >= 0 && t.x < OW && t.y >= 0 && t.y < OH) {
+      x0 = (int)t.x;
+      y0 = (int)t.y;
+      x1 = x0 + 1;
+      y1 = y0 + 1;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    x0 = min(x0, __shfl_xor(x0, o));
+    y0 = min(y0, __shfl_xor(y0, o));
+    x1 = max(x1, __shfl_xor(x1, o));
+    y1 = max(y1, __shfl_xor(y1, o));
+  }
+  if ((tid & 63) == 0) {
+    atomicMin(&box[0], x0);
+    atomicMin(&box[1], y0);
+    atomicMax(&box[2], x1);
+    atomicMax(&box[3], y1);
+  }
+  __syncthreads();
+  if (tid == 0)
+    boxes[blockIdx.x] = make_ushort4((unsigned short)box[0], (unsigned short)box[1],
+                                     (unsigned short)box[2], (unsigned short)box[3]);
+}
+
+// Workgroup: 2^cell_shift x 2^cell_shift output cells (at most one a thread) of batch element
+// blockIdx.y.
+__global__ __launch_bounds__(kVoteBlock) void vote_tile_kernel(
+    const int64_t* __restrict__ labels, const int64_t* __restrict__ map,
+    const ushort4* __restrict__ boxes, int* __restrict__ flag, int64_t* __restrict__ out, int IH,
+    int IW, int tiles, int tiles_x, int OH, int OW, int cells_x, int cell_shift, int candidates) {
+  __shared__ unsigned votes[kVoteCounters];
+  __shared__ int meet[kVoteMeet];
+  __shared__ int n_meet;
+  const int tid = threadIdx.x, side = 1 << cell_shift, cells = side << cell_shift;
+  const int ox0 = (blockIdx.x % cells_x) << cell_shift, oy0 = (blockIdx.x / cells_x) << cell_shift;
+  const int ox1 = min(ox0 + side, OW), oy1 = min(oy0 + side, OH);
+  if (tid == 0) n_meet = 0;
+  for (int i = tid; i < cells * candidates; i += kVoteBlock) votes[i] = 0;
+  __syncthreads();
+  for (int t0 = tid; t0 < tiles; t0 += 8 * kVoteBlock) {   // (eight reads in flight)
+    ushort4 b[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = boxes[min(t0 + u * kVoteBlock, tiles - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int t = t0 + u * kVoteBlock;
+      if (t < tiles && b[u].x < ox0 + side && b[u].z > ox0 && b[u].y < oy0 + side && b[u].w > oy0) {
+        const int at = atomicAdd(&n_meet, 1);
+        if (at < kVoteMeet) meet[at] = t;
+      }
+    }
+  }
+  __syncthreads();
+  if (n_meet > kVoteMeet) {
+    if (tid == 0) *flag = 1;   // (every writer writes the same)
+    return;
+  }
+  const int64_t* plane = labels + (size_t)blockIdx.y * IH * IW;
+  const int py = tid / kVoteTile, px = tid % kVoteTile;
+  constexpr int U = 4;   // input tiles whose pixels are requested together
+  for (int i0 = 0; i0 < n_meet; i0 += U) {
+    longlong2 t[U];
+    long long label[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int m = meet[min(i0 + u, n_meet - 1)];
+      const int iy = (m / tiles_x) * kVoteTile + py, ix = (m % tiles_x) * kVoteTile + px;
+      const size_t at = iy < IH && ix < IW ? (size_t)iy * IW + ix : 0;
+      t[u] = reinterpret_cast<const longlong2*>(map)[at];
+      label[u] = plane[at];
+      if (i0 + u >= n_meet || iy >= IH || ix >= IW) label[u] = -1;   // no pixel: no vote
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // (cells past the image's edge belong to no workgroup: such votes are not cast)
+      if (t[u].x >= ox0 && t[u].x < ox1 && t[u].y >= oy0 && t[u].y < oy1 && label[u] >= 0 &&
+          label[u] < candidates) {
+        const int cell = (((int)t[u].y - oy0) << cell_shift) + ((int)t[u].x - ox0);
+        atomicAdd(&votes[cell * candidates + (int)label[u]], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  const int ox = ox0 + (tid & (side - 1)), oy = oy0 + (tid >> cell_shift);
+  if (tid < cells && ox < OW && oy < OH) {
+    const unsigned* v = votes + tid * candidates;
+    unsigned best = 0;
+    int arg = 0;
+    for (int k = 0; k < candidates; ++k) {
+      const unsigned n = v[k];
+      if (n > best) {   // strict: the first of equal counts stays
+        best = n;
+        arg = k;
+      }
+    }
+    out[((size_t)blockIdx.y * OH + oy) * OW + ox] = arg;
+  }
+}
+
+// flag (optional): the kernel runs only if *flag != 0.
+__global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restrict__ p, size_t n16,
+                                                                const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
   const size_t stride = (size_t)gridDim.x * kVoteBlock;
   for (size_t i = (size_t)blockIdx.x * kVoteBlock + threadIdx.x; i < n16; i += stride)
     p[i] = make_uint4(0, 0, 0, 0);
 }
 
-// One thread per input pixel, grid.y over (batch element of this pass, channel): the plane
+// One thread per input pixel (and grid width), grid.y over (batch element of this pass, channel): the plane
 // arithmetic is per workgroup, and the pixel's target (16 bytes of the map) and its label are
 // requested together.  A label outside [0, candidates) casts no vote (the reference would
 // write outside its histogram).  Neighbouring lanes often vote for the same cell (pixels of a
@@ -33,24 +168,28 @@ __global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restric
 __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
     const int64_t* __restrict__ labels, const int64_t* __restrict__ map,
     unsigned* __restrict__ votes, int in_pixels, int channels, int OH, int OW, int candidates,
-    size_t element_stride) {
-  const int pix = blockIdx.x * kVoteBlock + threadIdx.x;
+    size_t element_stride, const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
-  const int at = min(pix, in_pixels - 1);
-  const long long x = map[(size_t)at * 2], y = map[(size_t)at * 2 + 1];
-  const long long label = labels[(size_t)plane * in_pixels + at];
-  const bool ok = pix < in_pixels && x >= 0 && x <= OW - 1 && y >= 0 && y <= OH - 1 &&
-                  label >= 0 && label < candidates;
-  // channel offset in histogram elements as the reference has it (common/resample.h:127-129):
-  // c * OH * OW, not c whole histograms, so the histograms of several channels overlap
-  const long long cell = ok ? (long long)(e * element_stride + (size_t)c * OH * OW +
-                                          ((size_t)y * OW + (size_t)x) * candidates +
-                                          (size_t)label)
-                            : -1;
-  const long long below = __shfl_up(cell, 1);
-  const LaneRuns runs(below == cell);
-  if (ok && runs.tail) atomicAdd(&votes[cell], (unsigned)(runs.dist + 1));
+  for (long long first = (long long)blockIdx.x * kVoteBlock; first < in_pixels;
+       first += (long long)gridDim.x * kVoteBlock) {
+    const long long pix = first + threadIdx.x;
+    const int at = (int)min(pix, (long long)in_pixels - 1);
+    const long long x = map[(size_t)at * 2], y = map[(size_t)at * 2 + 1];
+    const long long label = labels[(size_t)plane * in_pixels + at];
+    const bool ok = pix < in_pixels && x >= 0 && x <= OW - 1 && y >= 0 && y <= OH - 1 &&
+                    label >= 0 && label < candidates;
+    // channel offset in histogram elements as the reference has it (common/resample.h:127-129):
+    // c * OH * OW, not c whole histograms, so the histograms of several channels overlap
+    const long long cell = ok ? (long long)(e * element_stride + (size_t)c * OH * OW +
+                                            ((size_t)y * OW + (size_t)x) * candidates +
+                                            (size_t)label)
+                              : -1;
+    const long long below = __shfl_up(cell, 1);
+    const LaneRuns runs(below == cell);
+    if (ok && runs.tail) atomicAdd(&votes[cell], (unsigned)(runs.dist + 1));
+  }
 }
 
 // One thread per output pixel, grid.y over (batch element of this pass, channel): index of
@@ -58,33 +197,36 @@ __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
 // the first is compared.
 __global__ __launch_bounds__(kVoteBlock) void vote_argmax_kernel(
     const unsigned* __restrict__ votes, int64_t* __restrict__ out, int out_pixels, int channels,
-    int candidates, size_t element_stride) {
-  const int pix = blockIdx.x * kVoteBlock + threadIdx.x;
-  if (pix >= out_pixels) return;
+    int candidates, size_t element_stride, const int* __restrict__ flag) {
+  if (flag != nullptr && *flag == 0) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
-  const unsigned* v =
-      votes + e * element_stride + ((size_t)c * out_pixels + pix) * (size_t)candidates;
-  unsigned best = 0;
-  int arg = 0;
-  for (int k0 = 0; k0 < candidates; k0 += 8) {
-    unsigned n[8];
+  for (long long pix = (long long)blockIdx.x * kVoteBlock + threadIdx.x; pix < out_pixels;
+       pix += (long long)gridDim.x * kVoteBlock) {
+    const unsigned* v =
+        votes + e * element_stride + ((size_t)c * out_pixels + pix) * (size_t)candidates;
+    unsigned best = 0;
+    int arg = 0;
+    for (int k0 = 0; k0 < candidates; k0 += 8) {
+      unsigned n[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) n[i] = v[min(k0 + i, candidates - 1)];
+      for (int i = 0; i < 8; ++i) n[i] = v[min(k0 + i, candidates - 1)];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (k0 + i < candidates && n[i] > best) {   // strict: the first of equal counts stays
-        best = n[i];
-        arg = k0 + i;
-      }
+      for (int i = 0; i < 8; ++i)
+        if (k0 + i < candidates && n[i] > best) {   // strict: the first of equal counts stays
+          best = n[i];
+          arg = k0 + i;
+        }
+    }
+    out[(size_t)plane * out_pixels + pix] = arg;
   }
-  out[(size_t)plane * out_pixels + pix] = arg;
 }
 
 static size_t vote_bytes(int64_t channels, int64_t oh, int64_t ow, int64_t candidates) {
   const size_t n = (size_t)channels * oh * ow * candidates * sizeof(unsigned);
   return (n + 255) & ~(size_t)255;
 }
+constexpr size_t kVoteFlagBytes = 256;
 
 }  // namespace sdk
 
@@ -95,7 +237,7 @@ extern "C" {
 size_t sdk_voting_resample_workspace_bytes(int64_t channels, int64_t out_height,
                                            int64_t out_width, int64_t num_candidates) {
   if (channels < 1 || out_height < 1 || out_width < 1 || num_candidates < 1) return 0;
-  return vote_bytes(channels, out_height, out_width, num_candidates);
+  return vote_bytes(channels, out_height, out_width, num_candidates) + kVoteFlagBytes;
 }
 
 int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, int64_t* out,
@@ -127,18 +269,48 @@ int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, 
   // as many batch elements per pass as the workspace holds histograms (and grid.y planes)
   const int64_t per_pass = std::min<int64_t>(
       std::min<int64_t>(batch, (int64_t)(workspace_bytes / need)), 65535 / channels);
+  // The LDS kernels: one channel (several share cells), boxes of 16-bit coordinates, few enough
+  // input tiles and counters; the boxes lie where the histogram would, the flag behind it (a
+  // workspace without room for it: the histogram).  A workgroup's cells are as many as its counters allow.
+  const int tiles_x = (int)ceil_div(in_width, kVoteTile);
+  const int64_t tiles = (int64_t)tiles_x * ceil_div(in_height, kVoteTile);
+  int shift = 4;
+  while (shift > 2 && (num_candidates << (2 * shift)) > kVoteCounters) --shift;
+  const int* flag = nullptr;
+  if (channels == 1 && out_height < 0xffff && out_width < 0xffff && tiles <= kVoteTiles &&
+      batch <= 65535 && (num_candidates << (2 * shift)) <= kVoteCounters &&
+      tiles * sizeof(ushort4) <= need * (size_t)per_pass && (uintptr_t)sample_map % 16 == 0 &&
+      workspace_bytes >= need * (size_t)per_pass + kVoteFlagBytes) {
+    ushort4* boxes = static_cast<ushort4*>(workspace);
+    int* raised = reinterpret_cast<int*>(static_cast<char*>(workspace) + need * (size_t)per_pass);
+    launch(vote_boxes_kernel, dim3((unsigned)tiles), dim3(kVoteTile * kVoteTile), s, sample_map,
+           boxes, raised, (int)in_height, (int)in_width, tiles_x, (int)out_height, (int)out_width);
+    const int64_t cells_x = ceil_div(out_width, 1 << shift);
+    launch(vote_tile_kernel,
+           dim3((unsigned)(cells_x * ceil_div(out_height, 1 << shift)), (unsigned)batch),
+           dim3(kVoteBlock), s, input, sample_map, (const ushort4*)boxes, raised, out,
+           (int)in_height, (int)in_width, (int)tiles, tiles_x, (int)out_height, (int)out_width,
+           (int)cells_x, shift, (int)num_candidates);
+    flag = raised;
+  }
   for (int64_t b = 0; b < batch; b += per_pass) {
     const int64_t nb = std::min<int64_t>(per_pass, batch - b);
     const size_t n16 = need / 16 * (size_t)nb;
-    const int clear_blocks = (int)std::min<int64_t>(ceil_div((int64_t)n16, kVoteBlock), 4096);
-    launch(vote_clear_kernel, dim3(clear_blocks), dim3(kVoteBlock), s, (uint4*)workspace, n16);
+    // (behind a flag: narrow grids, whose blocks are quick to find nothing to do)
+    const int64_t most = flag != nullptr ? kVoteGridX : ((int64_t)1 << 31) - 1;
+    const int64_t clear_blocks =
+        std::min<int64_t>(ceil_div((int64_t)n16, kVoteBlock), flag != nullptr ? kVoteGridX : 4096);
+    launch(vote_clear_kernel, dim3((unsigned)clear_blocks), dim3(kVoteBlock), s, (uint4*)workspace,
+           n16, flag);
     const unsigned planes = (unsigned)(nb * channels);
-    launch(vote_kernel, dim3((unsigned)ceil_div(in_pixels, kVoteBlock), planes), dim3(kVoteBlock),
-           s, input + (size_t)b * n_in, sample_map, votes, in_pixels, (int)channels,
-           (int)out_height, (int)out_width, (int)num_candidates, need / sizeof(unsigned));
-    launch(vote_argmax_kernel, dim3((unsigned)ceil_div(out_pixels, kVoteBlock), planes),
+    launch(vote_kernel, dim3((unsigned)std::min(ceil_div(in_pixels, kVoteBlock), most), planes),
+           dim3(kVoteBlock), s, input + (size_t)b * n_in, sample_map, votes, in_pixels,
+           (int)channels, (int)out_height, (int)out_width, (int)num_candidates,
+           need / sizeof(unsigned), flag);
+    launch(vote_argmax_kernel,
+           dim3((unsigned)std::min(ceil_div(out_pixels, kVoteBlock), most), planes),
            dim3(kVoteBlock), s, (const unsigned*)votes, out + (size_t)b * n_out, out_pixels,
-           (int)channels, (int)num_candidates, need / sizeof(unsigned));
+           (int)channels, (int)num_candidates, need / sizeof(unsigned), flag);
   }
   SDK_LAUNCH_CHECK("voting_resample_to_map");
   return SDK_OK;
