@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include <cfloat>
 #include <climits>
@@ -462,10 +463,16 @@ __global__ __launch_bounds__(kBlock) void uv_scatter_kernel(
 // workgroup per (texture, plane chunk) sums its bucket into an LDS copy of the texture and
 // writes that out with plain stores, zeros included, so no fill of the output is needed.
 //
-// Lanes own consecutive bucket entries, which are consecutive image pixels of one row wherever
-// the map is coherent; these hit the same texel in runs.  Each run is summed across lanes first
-// (segmented scan over shuffles) and only its last lane adds to LDS, which keeps the
-// compare-and-swap adds nearly free of collisions.
+// The sums are held in double in LDS: ds_add_f64 takes 8 cycles a wave, without an answer to wait
+// for, where a float sum is a compare-and-swap loop of a read and 12 cycles a turn (ds_add_f32
+// takes 224).  Lanes own consecutive bucket entries, which are consecutive image pixels of one row
+// wherever the map is coherent; these hit the same texel in runs, which the LDS would serve one
+// lane after the other: each is summed across its lanes first, within rows of 16 lanes, where a
+// step of the scan is a vector instruction and no shuffle, and its last lane adds to LDS.  26
+// planes, 80 textures of 64 x 64, 512 x 1024 pixels: 131 -> 55 us (compare-and-swap adds and
+// shuffles across the wave before; 80 with the textures in their own order, the largest buckets
+// last; 290 without the scan; without the adds 43).
+// Textures whose doubles do not fit kUvLdsBytes keep compare-and-swap adds (ACC = T).
 // ---------------------------------------------------------------------------
 constexpr int kUvMaxTextures = 1 << 20;
 constexpr int kUvLdsBytes = 64 * 1024;
@@ -539,23 +546,44 @@ __global__ __launch_bounds__(kBlock) void uv_fill_kernel(const int64_t* __restri
 
 constexpr int kUvBlock = 1024;   // 16 waves: a long bucket (a polar face) takes few rounds
 
-template <typename T, int INTERP, int PL>
+
+template <typename T, int INTERP, int PL, typename ACC>
 __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
     const T* __restrict__ in, const T* __restrict__ uv, const int* __restrict__ offset,
     const int* __restrict__ list, T* __restrict__ textures, int planes, int NT, int TH, int TW,
     int MP) {
   extern __shared__ __align__(16) unsigned char uv_lds[];
-  T* acc = reinterpret_cast<T*>(uv_lds);             // [PL][TH * TW]
+  constexpr bool DIRECT = std::is_same<ACC, double>::value;   // native adds
+  ACC* acc = reinterpret_cast<ACC*>(uv_lds);         // [PL][TH * TW]
   const int THW = TH * TW;
-  const int t = blockIdx.x;
-  const int plane0 = blockIdx.y * PL;
+  // Longest buckets first, all their plane chunks: a polar texture's takes three times as long as
+  // the others', and started last it runs alone at the end.
+  int t = blockIdx.x, chunk = blockIdx.y;
+  if (NT <= kUvBlock) {
+    __shared__ int size[kUvBlock];
+    __shared__ int chosen;
+    const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / (int)gridDim.y;
+    chunk = id % (int)gridDim.y;
+    const int i = threadIdx.x;
+    if (i < NT) size[i] = offset[i + 1] - offset[i];
+    __syncthreads();
+    if (i < NT) {
+      const int mine = size[i];
+      int above = 0;
+      for (int k = 0; k < NT; ++k) above += (size[k] > mine || (size[k] == mine && k < i)) ? 1 : 0;
+      if (above == rank) chosen = i;
+    }
+    __syncthreads();
+    t = chosen;
+  }
+  const int plane0 = chunk * PL;
   const int np = min(PL, planes - plane0);
   // segment of the texture's bucket this workgroup sums (gridDim.z > 1: several workgroups
   // share a texture and add their sums to the zero-filled output)
   const int lo0 = offset[t], hi0 = offset[t + 1];
   const int per = (hi0 - lo0 + (int)gridDim.z - 1) / (int)gridDim.z;
   const int lo = lo0 + (int)blockIdx.z * per, hi = min(hi0, lo + per);
-  for (int i = threadIdx.x; i < PL * THW; i += kUvBlock) acc[i] = T(0);
+  for (int i = threadIdx.x; i < PL * THW; i += kUvBlock) acc[i] = ACC(0);
   __syncthreads();
   constexpr int N = PointTaps<T, INTERP>::N;
   // this round's pixel, point and values are loaded during the round before
@@ -583,8 +611,8 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
     pix_next = e + kUvBlock < hi ? list[e + kUvBlock] : 0;
     // lanes whose first tap is the same texel form a run: all their taps coincide
     const int ky = live ? taps.ty[0] : INT_MIN, kx = live ? taps.tx[0] : (int)threadIdx.x;
-    const int by = __shfl_up(ky, 1), bx = __shfl_up(kx, 1);
-    const LaneRuns runs(by == ky && bx == kx);
+    const int by = row_below<1>(ky), bx = row_below<1>(kx);
+    const RowRuns runs(by == ky && bx == kx);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const T w = taps.off[i] >= 0 ? (INTERP == 0 ? T(1) : taps.w[i]) : T(0);
@@ -593,7 +621,13 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
 #pragma unroll
       for (int j = 0; j < PL; ++j) {
         const T total = runs.sum(w * cur[j]);
-        if (live && runs.tail && inside && total != T(0)) lds_add(acc + j * THW + o, total);
+        if (live && runs.tail && inside && total != T(0)) {
+          if constexpr (DIRECT)
+            __hip_atomic_fetch_add(acc + j * THW + o, (double)total, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+          else
+            lds_add(acc + j * THW + o, total);
+        }
       }
     }
   }
@@ -604,7 +638,7 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
     for (int j = 0; j < PL; ++j) {
       if (j < np) {
         T* dst = textures + (size_t)(plane0 + j) * stride + (size_t)t * THW + i;
-        const T v = acc[j * THW + i];
+        const T v = (T)acc[j * THW + i];
         if (gridDim.z == 1) *dst = v;
         else if (v != T(0)) atomicAdd(dst, v);
       }
@@ -1613,8 +1647,10 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
     if (rc != SDK_OK) return rc;
     // planes per workgroup: as many as LDS holds while the grid still fills the GPU; few
     // textures: several workgroups share one and add their parts to a zero-filled output
+    const bool direct = THW * sizeof(double) <= (size_t)kUvLdsBytes;
+    const size_t sum = direct ? sizeof(double) : sizeof(T);
     int pl = 1;
-    while (pl < 4 && (size_t)(2 * pl) * THW * sizeof(T) <= (size_t)kUvLdsBytes &&
+    while (pl < 4 && (size_t)(2 * pl) * THW * sum <= (size_t)kUvLdsBytes &&
            (int64_t)NT * ceil_div(planes, 2 * pl) >= 1024)
       pl *= 2;
     const int64_t groups = (int64_t)NT * ceil_div(planes, pl);
@@ -1627,12 +1663,16 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
       if (rc != SDK_OK) return rc;
     }
     const dim3 grid((unsigned)NT, (unsigned)ceil_div(planes, pl), (unsigned)split);
-#define UVS(PLv)                                                                              \
-  SDK_DISPATCH_INTERP_ONLY(interp, (uv_texture_scatter_kernel<T, INTERP, PLv>                 \
-                                    <<<grid, dim3(kUvBlock), (size_t)PLv * THW * sizeof(T), stream>>>( \
+#define UVS(PLv, ACCv)                                                                        \
+  SDK_DISPATCH_INTERP_ONLY(interp, (uv_texture_scatter_kernel<T, INTERP, PLv, ACCv>           \
+                                    <<<grid, dim3(kUvBlock), (size_t)PLv * THW * sum, stream>>>( \
                                         in, uv, (const int*)offset, (const int*)list, textures, \
                                         (int)planes, NT, TH, TW, MP)))
-    if (pl == 4) UVS(4); else if (pl == 2) UVS(2); else UVS(1);
+    if (direct) {
+      if (pl == 4) UVS(4, double); else if (pl == 2) UVS(2, double); else UVS(1, double);
+    } else {   // (such a texture takes half of kUvLdsBytes or more)
+      UVS(1, T);
+    }
 #undef UVS
     SDK_LAUNCH_CHECK("resample_to_uv_maps(by texture)");
     return SDK_OK;

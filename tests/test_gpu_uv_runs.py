@@ -1,0 +1,43 @@
+"""The texture gradient of UV resampling by texture (csrc/mapped_gather_scatter.hip,
+uv_texture_scatter_kernel) on values with one right answer: integers, texture points at halves, so
+every product is a multiple of 1/4 and every sum a float32 number.  Compared to the bit."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import _spherical_distortion_ext._ops as o
+    return o
+
+
+# (batch, channels, textures, TH, TW, H, W): odd plane counts, one texture (its bucket shared among
+# workgroups), more textures than threads of a workgroup, textures whose double sums are just in and
+# just out of the LDS (8192 texels), buckets of less and more than one round of 1024 pixels
+SIZES = [(1, 1, 1, 1, 1, 1, 1), (2, 3, 5, 8, 9, 33, 47), (1, 13, 80, 16, 16, 60, 128),
+         (1, 5, 1030, 4, 3, 40, 77), (1, 2, 3, 64, 128, 50, 90), (1, 3, 2, 91, 91, 64, 64),
+         (3, 2, 1, 16, 16, 100, 120)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("interp", [0, 1, 2])
+@pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
+def test_texture_gradient(ops, oracle, tc, interp, dtype):
+    B, C, NT, TH, TW, H, W = tc
+    rng = np.random.default_rng(sum(tc) + interp)
+    # runs of 1 to 70 neighbouring pixels on one point, over the rows of 16 lanes and the waves'
+    # ends; some points and textures outside
+    n = H * W
+    length = rng.integers(1, 71, n)
+    run = np.repeat(np.arange(n), length)[:n]
+    quad = rng.integers(-1, NT + 1, n)[run].reshape(H, W)
+    uv = (rng.integers(-4, 2 * np.array([TW, TH]) + 4, (n, 2)) / 2)[run].reshape(H, W, 2)
+    uv = uv.astype(dtype)
+    g = rng.integers(-3, 4, (B, C, H, W)).astype(dtype)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)  # noqa: E731
+    have = ops.ops.resample_to_uv_maps(t(g), t(quad), t(uv), NT, TH, TW, interp).cpu().numpy()
+    assert np.array_equal(have, oracle.resample_to_uv_maps(g, quad, uv, NT, TH, TW, interp))
