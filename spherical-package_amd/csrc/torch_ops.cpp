@@ -97,7 +97,10 @@ struct Entry {
   int complete = 0;
   bool captured = false;             // a graph reads the plan
 };
-std::list<Entry> g_cache;   // most recently used last
+// Most recently used last.  Never destroyed: at the process's end the GPU runtime may be gone before this
+// library's statics, and freeing a plan that several streams used (an event is recorded for each)
+// then throws, which aborts the process.
+std::list<Entry>& g_cache = *new std::list<Entry>;
 
 // Lets go of the least recently used entries until `most` are left.  A plan that a captured graph reads
 // by its address stays as long as anyone beside the cache holds its map (the graph's owner has to).
