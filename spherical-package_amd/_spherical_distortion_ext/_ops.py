@@ -989,7 +989,7 @@ def _load_native():
     for name in ("sdk_torch_set_default_mode", "sdk_torch_set_plan_cache",
                  "sdk_torch_set_unpool_workspace"):
         getattr(lib, name).restype = None
-    lib.sdk_torch_native_select.restype = ctypes.c_char_p
+    lib.sdk_torch_native_more.restype = ctypes.c_char_p
     return lib, frozenset(lib.sdk_torch_native_ops().decode().split(","))
 
 
@@ -997,11 +997,11 @@ _library = torch.library.Library(_NS, "DEF")
 for _name, _schema, _fn in _SCHEMAS:
     _library.define(_name + _schema)
 _native, _NATIVE_OPS = _load_native()
-# the operator the compiled layer implements beside those of the reference's extension modules
-_NATIVE_SELECT = frozenset() if _native is None else \
-    frozenset([_native.sdk_torch_native_select().decode()])
+# operators the compiled layer implements beside the ones sdk_torch_native_ops names
+_NATIVE_MORE = frozenset() if _native is None else \
+    frozenset(_native.sdk_torch_native_more().decode().split(","))
 for _name, _schema, _fn in _SCHEMAS:
-    if _name not in _NATIVE_OPS | _NATIVE_SELECT:
+    if _name not in _NATIVE_OPS | _NATIVE_MORE:
         _library.impl(_name, _fn, "CUDA")
 
 
@@ -1010,5 +1010,5 @@ for _name, _schema, _fn in _SCHEMAS:
 # that callers of this module and callers of torch.ops.sdk_mapped_ops run the same code.
 ops = getattr(torch.ops, _NS)
 PYTHON_IMPL = {_name: _fn for _name, _schema, _fn in _SCHEMAS}
-for _name in _NATIVE_OPS | _NATIVE_SELECT:
+for _name in _NATIVE_OPS | _NATIVE_MORE:
     globals()[_name] = getattr(ops, _name)

@@ -21,11 +21,13 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <iterator>
 #include <list>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "sdk_mapped_ops.h"
@@ -68,7 +70,8 @@ bool tensor_key(const OptTensor& t, TensorKey* k) {
   return true;
 }
 
-enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kAvgUnpoolLists = 4 };
+enum Kind { kConv = 0, kResample = 1, kAvgUnpool = 2, kMaxUnpool = 3, kAvgUnpoolLists = 4,
+            kUvScatter = 5 };
 
 struct Key {
   int kind = 0, device = 0, dtype = 0;
@@ -753,12 +756,112 @@ std::tuple<Tensor, Tensor, Tensor> mapped_conv_backward_select(
   return {gi, gw, gb};
 }
 
+// ----------------------------------------------------------------------------- textures, labels
+void check_uv(const Tensor& ref, const Tensor& quad, const Tensor& uv) {
+  check_one(ref, "quad_idx", quad, true);
+  check_one(ref, "tex_uv", uv);
+  TORCH_CHECK(quad.scalar_type() == at::kLong && quad.dim() == 2,
+              "quad_idx must be a 2-D int64 tensor, got ", quad.scalar_type(), " ", quad.sizes());
+  TORCH_CHECK(uv.dim() == 3 && uv.size(0) == quad.size(0) && uv.size(1) == quad.size(1) &&
+                  uv.size(2) == 2,
+              "tex_uv ", uv.sizes(), " must be quad_idx ", quad.sizes(), " + (2,)");
+}
+
+Tensor resample_from_uv_maps(const Tensor& textures, const Tensor& quad, const Tensor& uv,
+                             int64_t interp) {
+  check_first(textures);
+  check_one(textures, "textures", textures);
+  check_uv(textures, quad, uv);
+  TORCH_CHECK(textures.dim() == 5, "textures must be [B, C, T, TH, TW], got ", textures.sizes());
+  const int64_t B = textures.size(0), C = textures.size(1), H = quad.size(0), W = quad.size(1);
+  Tensor out = at::empty({B, C, H, W}, textures.options());
+  c10::DeviceGuard guard(textures.device());
+  SDK_CALL(sdk_resample_from_uv_maps, textures.data_ptr(), quad.data_ptr<int64_t>(), uv.data_ptr(),
+           out.data_ptr(), B, C, textures.size(2), textures.size(3), textures.size(4), H, W,
+           (int32_t)interp, dtype_code(textures), stream_of(textures));
+  return out;
+}
+
+Tensor resample_to_uv_maps(const Tensor& x, const Tensor& quad, const Tensor& uv, int64_t NT,
+                           int64_t TH, int64_t TW, int64_t interp) {
+  check_first(x);
+  check_one(x, "x", x);
+  check_uv(x, quad, uv);
+  const int64_t H = quad.size(0), W = quad.size(1);
+  TORCH_CHECK(x.dim() == 4 && x.size(2) == H && x.size(3) == W, "input ", x.sizes(),
+              " must be [B, C, ", H, ", ", W, "]");
+  const int64_t B = x.size(0), C = x.size(1);
+  const int dt = dtype_code(x);
+  Tensor out = at::empty({B, C, NT, TH, TW}, x.options());
+  c10::DeviceGuard guard(x.device());
+  hipStream_t s = stream_of(x);
+  const size_t nws = sdk_resample_to_uv_maps_workspace_bytes(NT, TH, TW, H, W, dt);
+  // the pixels bucketed by texture, a function of quad_idx alone
+  Key key;
+  key.kind = kUvScatter;
+  key.device = x.device().index();
+  key.dtype = dt;
+  key.a = NT;
+  key.b = TH;
+  key.K = TW;
+  PlanRef plan = plan_for(
+      key, x, quad, OptTensor(), s, [&] { return nws; },
+      [&](void* buf, size_t n, int) {
+        SDK_CALL(sdk_resample_to_uv_maps_plan_build, quad.data_ptr<int64_t>(), buf, n, NT, TH, TW,
+                 H, W, dt, s);
+        return 1;
+      });
+  if (plan.plan.defined()) {
+    SDK_CALL(sdk_resample_to_uv_maps_planned, x.data_ptr(), quad.data_ptr<int64_t>(), uv.data_ptr(),
+             out.data_ptr(), plan.ptr(), plan.nbytes, B, C, NT, TH, TW, H, W, (int32_t)interp, dt,
+             s);
+    return out;
+  }
+  Tensor ws;
+  if (nws) ws = bytes_on(x, nws);
+  SDK_CALL(sdk_resample_to_uv_maps, x.data_ptr(), quad.data_ptr<int64_t>(), uv.data_ptr(),
+           out.data_ptr(), nws ? ws.data_ptr() : nullptr, nws, B, C, NT, TH, TW, H, W,
+           (int32_t)interp, dt, s);
+  return out;
+}
+
+Tensor voting_resample_to_map(const Tensor& labels, const Tensor& map, int64_t out_h, int64_t out_w,
+                              int64_t candidates) {
+  const std::pair<const char*, const Tensor*> named[2] = {{"input", &labels}, {"sample_map", &map}};
+  for (const auto& t : named) {
+    TORCH_CHECK(t.second->is_cuda(), "this backend runs on the GPU only: ", t.first,
+                " must be a CUDA/HIP tensor");
+    TORCH_CHECK(t.second->scalar_type() == at::kLong, t.first, " must be int64 (got ",
+                t.second->scalar_type(), ")");
+    TORCH_CHECK(t.second->is_contiguous(), t.first, " must be contiguous");
+  }
+  TORCH_CHECK(labels.dim() == 4 && map.dim() == 3 && map.size(0) == labels.size(2) &&
+                  map.size(1) == labels.size(3) && map.size(2) == 2,
+              "input ", labels.sizes(), " must be [B, C, IH, IW] and sample_map ", map.sizes(),
+              " [IH, IW, 2]");
+  const int64_t B = labels.size(0), C = labels.size(1);
+  Tensor out = at::empty({B, C, out_h, out_w}, labels.options());
+  c10::DeviceGuard guard(labels.device());
+  // room for several batch elements per pass, within 256 MiB
+  size_t nws = sdk_voting_resample_workspace_bytes(C, out_h, out_w, candidates);
+  const int64_t fit = (int64_t)(((size_t)256 << 20) / std::max<size_t>(nws, 1));
+  nws *= (size_t)std::max<int64_t>(1, std::min<int64_t>(B, fit));
+  Tensor ws = bytes_on(labels, std::max<size_t>(nws, 16));
+  SDK_CALL(sdk_voting_resample_to_map, labels.data_ptr<int64_t>(), map.data_ptr<int64_t>(),
+           out.data_ptr<int64_t>(), ws.data_ptr(), nws, B, C, labels.size(2), labels.size(3), out_h,
+           out_w, candidates, stream_of(labels));
+  return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(sdk_mapped_ops, CUDA, m) {
   m.impl("resample_from_map", &resample_from_map);
   m.impl("resample_to_map", &resample_to_map);
   m.impl("resample_to_map_normalized", &resample_to_map_normalized);
+  m.impl("resample_from_uv_maps", &resample_from_uv_maps);
+  m.impl("resample_to_uv_maps", &resample_to_uv_maps);
+  m.impl("voting_resample_to_map", &voting_resample_to_map);
   m.impl("mapped_max_pool", &mapped_max_pool);
   m.impl("mapped_max_unpool", &mapped_max_unpool);
   m.impl("mapped_avg_pool", &mapped_avg_pool);
@@ -778,7 +881,11 @@ const char* sdk_torch_native_ops(void) {
          "mapped_max_unpool,mapped_avg_pool,mapped_avg_unpool,mapped_conv_forward,"
          "mapped_conv_backward,mapped_transposed_conv_forward,mapped_transposed_conv_backward";
 }
-const char* sdk_torch_native_select(void) { return "mapped_conv_backward_select"; }
+// ... and those for textures and labels, and the backward that forms only the gradients asked for
+const char* sdk_torch_native_more(void) {
+  return "mapped_conv_backward_select,resample_from_uv_maps,resample_to_uv_maps,"
+         "voting_resample_to_map";
+}
 void sdk_torch_set_default_mode(int mode) { g_default_mode = mode; }
 // mode < 0 removes the override; returns the previous override (-1: none)
 int sdk_torch_set_thread_mode(int mode) {

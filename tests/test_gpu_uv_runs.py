@@ -41,3 +41,35 @@ def test_texture_gradient(ops, oracle, tc, interp, dtype):
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)  # noqa: E731
     have = ops.ops.resample_to_uv_maps(t(g), t(quad), t(uv), NT, TH, TW, interp).cpu().numpy()
     assert np.array_equal(have, oracle.resample_to_uv_maps(g, quad, uv, NT, TH, TW, interp))
+
+
+def test_compiled_and_python_operators_agree(ops):
+    if ops._native is None:
+        pytest.skip("the compiled operator layer is not built")
+    rng = np.random.default_rng(3)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    quad, uv = t(rng.integers(-1, 6, (20, 31))), t(rng.uniform(-1, 9, (20, 31, 2)))
+    tex, g = t(rng.integers(-4, 5, (2, 3, 5, 8, 9)) * 1.0), t(rng.integers(-4, 5, (2, 3, 20, 31)) * 1.0)
+    labels, vmap = t(rng.integers(0, 7, (2, 1, 20, 31))), t(rng.integers(0, 5, (20, 31, 2)))
+    calls = {"resample_from_uv_maps": (tex, quad, uv, 1),
+             "resample_to_uv_maps": (g, quad, uv, 5, 8, 9, 0),
+             "voting_resample_to_map": (labels, vmap, 5, 5, 7)}
+    for name, args in calls.items():
+        assert getattr(ops, name) is getattr(ops.ops, name)
+        assert torch.equal(getattr(ops.ops, name)(*args), ops.PYTHON_IMPL[name](*args))
+        for i, a in enumerate(args):   # a tensor of another type, layout or shape: refused by both
+            if not isinstance(a, torch.Tensor):
+                continue
+            for bad in (a.int(), a.transpose(-1, -2), a[:, :-1].contiguous(), a.cpu()):
+                for fn in (getattr(ops.ops, name), ops.PYTHON_IMPL[name]):
+                    if name == "resample_from_uv_maps" and i == 0 and bad.dim() == 5 and \
+                            bad.is_cuda and bad.dtype == a.dtype and bad.is_contiguous():
+                        continue   # (fewer channels are an ordinary call)
+                    if name != "voting_resample_to_map" and i == 0 and bad.shape[2:] == a.shape[2:] \
+                            and bad.is_cuda and bad.dtype == a.dtype:
+                        continue
+                    if name == "voting_resample_to_map" and i == 0 and bad.shape[1] == 0 and \
+                            bad.is_cuda and bad.dtype == a.dtype:
+                        continue
+                    with pytest.raises(RuntimeError):
+                        fn(*args[:i], bad, *args[i + 1:])
