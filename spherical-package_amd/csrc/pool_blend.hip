@@ -12,9 +12,10 @@
 // 16-byte LDS read serves a tap of four planes.  A band too tall for four planes takes two or
 // one per pass, past that its taps come from global memory; the choice is made per workgroup.
 // Results are the per-pixel kernels' bit for bit: the same products, summed in the same order.
-// (Measured, average / maximum: 4 x 48 planes of 190 x 378, stride 2, 80 -> 58 / 82 -> 61 us;
+// (Measured, average / maximum: 4 x 48 planes of 190 x 378, stride 2, 80 -> 52 / 82 -> 55 us (58 / 61
+// with the band read an element at a time);
 // 8 x 64 planes of 256 x 512, stride 2, 335 -> 126 / 360 -> 141 us.  Two workgroups per CU of 256
-// registers: at three the nine samples' positions and weights spill, 68 us.)
+// registers: at three the nine samples' positions and weights spill, 69 us.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -65,23 +66,41 @@ __device__ __forceinline__ void run_blend(const float* __restrict__ in, float* _
   if (t == 0) band[band_elems] = vecp(0.0f);
   for (int p = p_begin; p < p_end; p += PG) {
     const float* src = in + (size_t)p * HW + row_start;
-    // four elements of PG planes in flight per thread; planes past the range repeat the last
-    for (int e0 = t; e0 < band_elems; e0 += 4 * nt) {
-      float v[4][PG];
+    // The band is one run of memory: four neighbours of PG planes a read (16 bytes from any element
+    // boundary), AHEAD such groups in flight per thread; planes past the range repeat the last, the
+    // last groups overlap (and store the same values).
+    typedef float vec4 __attribute__((ext_vector_type(4)));
+    constexpr int AHEAD = 2;
+    if (band_elems >= 4) {
+      for (int e0 = 4 * t; e0 < band_elems; e0 += AHEAD * 4 * nt) {
+        vec4 v[AHEAD][PG];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int e = min(e0 + i * nt, band_elems - 1);
+        for (int i = 0; i < AHEAD; ++i) {
+          const int e = min(e0 + i * 4 * nt, band_elems - 4);
 #pragma unroll
-        for (int g = 0; g < PG; ++g) v[i][g] = src[(size_t)min(g, p_end - 1 - p) * HW + e];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (e0 + i * nt < band_elems) {
-          vecp x;
-#pragma unroll
-          for (int g = 0; g < PG; ++g) x[g] = v[i][g];
-          band[e0 + i * nt] = x;
+          for (int g = 0; g < PG; ++g)
+            __builtin_memcpy(&v[i][g], src + (size_t)min(g, p_end - 1 - p) * HW + e, sizeof(vec4));
         }
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+          if (i > 0 && e0 + i * 4 * nt >= band_elems) break;
+          const int e = min(e0 + i * 4 * nt, band_elems - 4);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            vecp y;
+#pragma unroll
+            for (int g = 0; g < PG; ++g) y[g] = v[i][g][x];
+            band[e + x] = y;
+          }
+        }
+      }
+    } else {
+      for (int e = t; e < band_elems; e += nt) {
+        vecp y;
+#pragma unroll
+        for (int g = 0; g < PG; ++g) y[g] = src[(size_t)min(g, p_end - 1 - p) * HW + e];
+        band[e] = y;
+      }
     }
     __syncthreads();
     if (on) {
