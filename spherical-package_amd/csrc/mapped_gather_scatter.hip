@@ -2335,22 +2335,19 @@ __global__ __launch_bounds__(kBlock) void unpool_merge_kernel(const int* __restr
 }
 
 // Average unpooling of blended samples as a gather over the merged lists: a thread owns an image
-// element in PC planes, four entries in flight.  Neighbouring elements draw on the same few pooled
-// pixels, so the reads of a wave fall into few lines.  (The tile kernel adds K * 4 values per
-// pooled pixel and plane to LDS by compare-and-swap: 4 x 48 planes of 190 x 378 from 95 x 189,
-// 94 us; and a map whose windows it cannot hold, stride 1 at 256 x 512, went to atomics in
-// memory: 7.9 ms for 128 planes.)  Lists of more than kUnpoolLong entries are the whole wave's, an
-// entry of four to each lane in turn, the lanes' sums added by a tree.  (2 x 16 planes of 256 x 512, stride
-// 1, a tenth of the samples on one spot, forward + backward: 18.3 ms with one thread a list, 0.81 now.)
+// element.  (The tile kernel adds K * 4 values per pooled pixel and plane to LDS by
+// compare-and-swap: 4 x 48 planes of 190 x 378 from 95 x 189, 94 us; and a map whose windows it cannot
+// hold, stride 1 at 256 x 512, went to atomics in memory: 7.9 ms for 128 planes.)  Lists of more
+// than kUnpoolLong entries are the whole wave's, an entry of four to each lane in turn, the lanes' sums
+// added by a tree.  (2 x 16 planes of 256 x 512, stride 1, a tenth of the samples on one spot, forward +
+// backward: 18.3 ms with one thread a list, 0.81 now.)
+
+// gin of element u (of all the wave's, u >= HW: none) in planes plane0 .. plane0 + np - 1, read from
+// memory: four entries and PC planes in flight.
 template <int PC>
-__global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
-    const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
-    const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
-    int M, int planes, float K) {
-  const int u = banded_pixel_block() * kBlock + threadIdx.x;
-  const int plane0 = blockIdx.y * PC;
-  const int np = min(PC, planes - plane0);
-  const int beg = u < HW ? offset[u] : 0, n = u < HW ? count[u] : 0;
+__device__ __forceinline__ void unpool_from_memory(
+    const float* __restrict__ gout, const int* __restrict__ src, const float* __restrict__ co,
+    float* __restrict__ gin, int u, int beg, int n, int HW, int M, int plane0, int np, float K) {
   const float* g0 = gout + (size_t)plane0 * M;
   // sum += entries first .. first + 3, first + step .. first + step + 3, ... of those before end
   auto add = [&](int first, int end, int step, float (&sum)[PC]) {
@@ -2395,6 +2392,131 @@ __global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
 #pragma unroll
   for (int j = 0; j < PC; ++j)
     if (j < np) gin[(size_t)(plane0 + j) * HW + u] = acc[j] / K;
+}
+
+template <int PC>
+__global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
+    const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
+    const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
+    int M, int planes, float K) {
+  const int u = banded_pixel_block() * kBlock + threadIdx.x;
+  const int plane0 = blockIdx.y * PC;
+  const int beg = u < HW ? offset[u] : 0, n = u < HW ? count[u] : 0;
+  unpool_from_memory<PC>(gout, src, co, gin, u, beg, n, HW, M, plane0, min(PC, planes - plane0), K);
+}
+
+// The same sums with the sources in LDS: a workgroup owns kUnpoolSpan neighbouring image elements and
+// a range of planes.  Where the map is coherent the lists of neighbours draw on a few rows of pooled
+// pixels; per pass those of eight planes (or four, or two, as many as fit) go to LDS side by side,
+// [pooled pixel][plane], so that one or two 16-byte reads serve an entry of all of them, and a thread
+// keeps the first kUnpoolKept entries of its list in registers over the passes.  A workgroup whose
+// sources span too much, or one of whose lists is long, reads them from memory as above.  Same
+// products in the same order as there: the same bits.  4 x 48 planes of 190 x 378 from 95 x 189:
+// 60 -> 34 us, 8 x 64 of 256 x 512 285 -> 119 (bound by the requests of 4-byte reads, one per entry and
+// plane, before).  Not for maps as dense as their image, whose spans touch five times their own
+// length in pooled pixels and whose lists are longer than what is kept (192 planes of 256 x 512, stride 1: 541 us
+// from memory, 1058 so), nor below 64 planes (32 of 190 x 378: 14 against 21).
+constexpr int kUnpoolSpan = 512;
+constexpr int kUnpoolKept = 8;
+constexpr int kUnpoolLdsBytes = 40 * 1024;   // four workgroups per CU
+
+template <int PG>
+__device__ __forceinline__ void unpool_from_lds(
+    const float* __restrict__ gout, const int* __restrict__ src, const float* __restrict__ co,
+    float* __restrict__ gin, float* lds, int u, int beg, int n, int most, int m0, int span, int HW,
+    int M, int p_begin, int p_end, float K) {
+  typedef float vecp __attribute__((ext_vector_type(PG)));
+  vecp* g = reinterpret_cast<vecp*>(lds);
+  int at[kUnpoolKept];
+  float c[kUnpoolKept];
+#pragma unroll
+  for (int i = 0; i < kUnpoolKept; ++i) {
+    at[i] = i < n ? src[beg + i] - m0 : 0;
+    c[i] = i < n ? co[beg + i] : 0.0f;
+  }
+  for (int p = p_begin; p < p_end; p += PG) {
+    for (int e = threadIdx.x; e < span; e += kUnpoolSpan) {
+      vecp v;
+#pragma unroll
+      for (int j = 0; j < PG; ++j)
+        v[j] = gout[(size_t)min(p + j, p_end - 1) * M + m0 + e];   // (past the range: the last again)
+      g[e] = v;
+    }
+    __syncthreads();
+    vecp acc(0.0f);
+#pragma unroll
+    for (int i = 0; i < kUnpoolKept; ++i) {
+      if (i >= most) break;   // (uniform over the workgroup)
+      const vecp v = g[at[i]];
+#pragma unroll
+      for (int j = 0; j < PG; ++j) acc[j] += i < n ? c[i] * v[j] : 0.0f;
+    }
+    for (int i = kUnpoolKept; i < n; ++i) {
+      const vecp v = g[src[beg + i] - m0];
+      const float ci = co[beg + i];
+#pragma unroll
+      for (int j = 0; j < PG; ++j) acc[j] += ci * v[j];
+    }
+    if (u < HW) {
+#pragma unroll
+      for (int j = 0; j < PG; ++j)
+        if (p + j < p_end) gin[(size_t)(p + j) * HW + u] = acc[j] / K;
+    }
+    __syncthreads();
+  }
+}
+
+// grid.x = 8 * blocks * ceil(chunks / 8): an XCD takes whole plane chunks, whose pooled rows its L2
+// then keeps for the neighbouring spans.
+__global__ __launch_bounds__(kUnpoolSpan) void unpool_spans_kernel(
+    const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
+    const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
+    int M, int planes, int blocks, int chunks, float K) {
+  __shared__ __align__(16) float lds[kUnpoolLdsBytes / 4];
+  __shared__ int s_first, s_last, s_most;
+  const int within = blockIdx.x >> 3;
+  const int chunk = (within / blocks) * 8 + (blockIdx.x & 7);
+  if (chunk >= chunks) return;
+  const int p_begin = (int)((int64_t)chunk * planes / chunks);
+  const int p_end = (int)((int64_t)(chunk + 1) * planes / chunks);
+  const int u = (within % blocks) * kUnpoolSpan + threadIdx.x;
+  const int beg = u < HW ? offset[u] : 0, n = u < HW ? count[u] : 0;
+  if (threadIdx.x == 0) {
+    s_first = INT_MAX;
+    s_last = -1;
+    s_most = 0;
+  }
+  __syncthreads();
+  // (merged lists ascend: the first and the last entry bound a list's sources)
+  int first = n > 0 ? src[beg] : INT_MAX, last = n > 0 ? src[beg + n - 1] : -1, most = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    first = min(first, __shfl_xor(first, d));
+    last = max(last, __shfl_xor(last, d));
+    most = max(most, __shfl_xor(most, d));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMin(&s_first, first);
+    atomicMax(&s_last, last);
+    atomicMax(&s_most, most);
+  }
+  __syncthreads();
+  const int m0 = s_last < 0 ? 0 : s_first, span = s_last < 0 ? 1 : s_last - s_first + 1;
+  const int longest = s_most;
+  if (longest <= kUnpoolLong && span <= kUnpoolLdsBytes / 8) {
+    if (span <= kUnpoolLdsBytes / 32)
+      unpool_from_lds<8>(gout, src, co, gin, lds, u, beg, n, longest, m0, span, HW, M, p_begin,
+                         p_end, K);
+    else if (span <= kUnpoolLdsBytes / 16)
+      unpool_from_lds<4>(gout, src, co, gin, lds, u, beg, n, longest, m0, span, HW, M, p_begin,
+                         p_end, K);
+    else
+      unpool_from_lds<2>(gout, src, co, gin, lds, u, beg, n, longest, m0, span, HW, M, p_begin,
+                         p_end, K);
+  } else {
+    for (int p = p_begin; p < p_end; p += 4)
+      unpool_from_memory<4>(gout, src, co, gin, u, beg, n, HW, M, p, min(4, p_end - p), K);
+  }
 }
 
 struct Col2imLists {
@@ -2487,6 +2609,22 @@ static int launch_unpool_lists(const float* gout, float* gin, const void* lists,
                                int H, int W, int M, int K, int P, int interp, hipStream_t stream) {
   const Col2imLists l = col2im_lists_at(const_cast<void*>(lists), H, W, M, K, P, interp);
   const int HW = H * W;
+  // From LDS where the map has half the image's pixels or fewer and there are planes to take the staging
+  // and the lists for (both sides at unpool_spans_kernel); chunks of planes in eighths, about four
+  // workgroups per CU.
+  const int64_t spans = ceil_div(HW, kUnpoolSpan);
+  if (planes >= 64 && 2 * (int64_t)M <= HW) {
+    int64_t chunks = std::max<int64_t>(8, std::min<int64_t>(planes / 16, 1024 / spans) / 8 * 8);
+    chunks = std::min<int64_t>(chunks, planes);
+    const int64_t grid = 8 * spans * ceil_div(chunks, 8);
+    if (grid < ((int64_t)1 << 31)) {
+      launch(unpool_spans_kernel, dim3((unsigned)grid), dim3(kUnpoolSpan), stream, gout,
+             (const int*)l.offset, (const int*)l.count, (const int*)l.src, (const float*)l.co, gin,
+             HW, M, (int)planes, (int)spans, (int)chunks, (float)K);
+      SDK_LAUNCH_CHECK("mapped_avg_unpool(lists, spans)");
+      return SDK_OK;
+    }
+  }
 #define UL(PCv)                                                                                \
   launch(unpool_lists_kernel<PCv>, dim3(banded_grid_x(HW), (unsigned)ceil_div(planes, PCv)),   \
          dim3(kBlock), stream, gout, (const int*)l.offset, (const int*)l.count,                \
