@@ -341,7 +341,7 @@ __global__ __launch_bounds__(1024) void tile_lists_kernel(const int* __restrict_
                                                           int* __restrict__ lists,
                                                           int* __restrict__ count, int max_rows,
                                                           int small_cap) {
-  constexpr int NC = 7;
+  constexpr int NC = 6;
   __shared__ int wave_n[NC][16];
   __shared__ int base[NC];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -361,7 +361,6 @@ __global__ __launch_bounds__(1024) void tile_lists_kernel(const int* __restrict_
     cls[3] = cls[1] && !cls[2];
     cls[4] = small;
     cls[5] = fit && !small;
-    cls[6] = live && !cls[2];
     unsigned long long mask[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -926,6 +925,7 @@ size_t window_gemm_weight_bytes(const ConvGeom& g) {
 
 size_t tile_lists_bytes(const ConvGeom& g) {
   const PixelTiling pt = plan_tiling(g.M / g.OW, g.OW);
+  // (the seventh list's place is not in use; a plan buffer that a caller holds has it)
   return ((size_t)7 * pt.tiles_x * pt.tiles_y + 8) * sizeof(int);
 }
 
@@ -937,7 +937,6 @@ void load_tile_lists(const Plan& plan, void* workspace, TileLists* out) {
   out->rest_small = lists + (size_t)3 * plan.tiles;
   out->product = lists + (size_t)4 * plan.tiles;
   out->inside_large = lists + (size_t)5 * plan.tiles;
-  out->not_big = lists + (size_t)6 * plan.tiles;
   out->count = lists + (size_t)7 * plan.tiles;
 }
 

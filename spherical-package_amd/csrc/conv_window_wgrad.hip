@@ -12,7 +12,7 @@
 //
 //   workgroup = 32 image channels (one chunk) x 128 pixel-side channels x all K samples x one
 //               batch element x every groups-th tile of the list
-//   wave w    = samples w KP .. w KP + KP - 1 for all four 32-row blocks of n ("full" samples,
+//   wave w    = samples w KP .. w KP + KP - 1 for all four (A) 32-row blocks of n ("full" samples,
 //               K = 4 KP + R), and row block w for each of the R remaining samples
 //
 // so a wave builds the column values of its own samples itself, straight into B operands:
@@ -23,6 +23,10 @@
 // quarter's plan rows are staged in LDS once per quarter, the window once per tile.  The
 // accumulators ((4 KP + R) x 16 registers) stay in registers over all tiles and leave the
 // workgroup once, into a partial-sum buffer that window_wgrad_reduce_kernel adds up.
+//
+// What bounds it: fp32 MFMAs and vector instructions do not overlap on a SIMD (9 MFMAs 576 cycles,
+// 18, 36 and 72 multiply-adds of either wave beside them 654, 723, 862, two waves a SIMD), so the blends
+// add to the MFMAs, which are busy for 63 % of the time at 8 x 128 -> 128 channels, 256 x 512.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -50,8 +54,15 @@ constexpr int kWwRows = 4; // plan rows per sample this kernel applies
 // offsets of the next tile's window, before a quarter's MFMAs.
 // ONE: every sample of the plan has a single row (nearest taps without interpolation weights);
 // the step loop then reads and applies that row alone instead of four, three of them padding.
-template <int KP, int R, int CAP, int MM, bool ONE = false>
-__global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_wgrad_kernel(
+// A: row blocks of the pixel-side tile, 4, or 2 where there are at most 64 pixel-side channels.  With
+// two, a remaining sample's pixels go half to waves 0 and 1 and half to waves 2 and 3 (row block
+// w % 2), so that no wave multiplies rows that do not exist.
+// G: groups of four waves that share a window, each with quarter tiles of its own (q % G); the sums
+// of the second are added to those of the first at the end.  Two where the LDS holds one window
+// only and the registers allow it: 1-rings of 163842 icosphere vertices, batch 4, 64 -> 64, the big
+// tiles: four row blocks (half of them padding) 279 us, two 213, two groups as well 162.
+template <int KP, int R, int CAP, int MM, bool ONE = false, int A = 4, int G = 1>
+__global__ __launch_bounds__(kWwThreads * G, CAP > kRegionCap && G == 1 ? 1 : 2) void window_wgrad_kernel(
     const float* __restrict__ pix, const float* __restrict__ img, const int* __restrict__ hdr,
     const int* __restrict__ ns, const int2* __restrict__ taps, const int* __restrict__ list,
     const int* __restrict__ count, float* __restrict__ partial, int Cg, int H, int W, int Cp,
@@ -61,14 +72,19 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
   constexpr bool BIG = CAP > kRegionCap;
   // (with two workgroups per CU the registers are not there: the requests spill and the kernel
   // takes half as long again)
-  constexpr bool PIPE = BIG;
+  constexpr bool PIPE = BIG && G == 1;
+  constexpr int ROWS = ONE ? 1 : kWwRows;   // plan rows held per sample and pixel
   __shared__ __align__(16) float region[(CAP + 1) * kWwE];
-  __shared__ __align__(16) float gt[128 * kWwG];
-  __shared__ __align__(16) int2 rowsL[K * kWwQ * kWwRows];
+  __shared__ __align__(16) float gt_[G][32 * A * kWwG];
+  __shared__ __align__(16) int2 rows_[G][K * kWwQ * ROWS];
   __shared__ int src[BIG ? 1 : CAP];
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (a scalar for the compiler)
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // (scalars)
+  const int wave = wave_all & 3, part = wave_all >> 2;
+  const int tid = threadIdx.x & (kWwThreads - 1);   // within the group
+  float* gt = gt_[part];
+  int2* rowsL = rows_[part];
   const int j = lane & 31, h = lane >> 5;
   // Workgroup ids go round-robin over the 8 XCDs.  All workgroups of one tile run (every
   // batch element and channel chunk) read the same plan rows, those of one batch element the
@@ -85,12 +101,12 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
   const float* img_b = img + ((size_t)batch * Cg) * HW;
   const float* pix_b = pix + ((size_t)batch * Cp) * M;
 
-  floatx16 accF[KP > 0 ? KP : 1][4];
+  floatx16 accF[KP > 0 ? KP : 1][A];
   floatx16 accR[R > 0 ? R : 1];
 #pragma unroll
   for (int i = 0; i < (KP > 0 ? KP : 1); ++i)
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < A; ++a)
 #pragma unroll
       for (int v = 0; v < 16; ++v) accF[i][a][v] = 0.0f;
 #pragma unroll
@@ -102,21 +118,22 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
   const char* regb = reinterpret_cast<const char*>(region) + 4 * j;
   // pixel-side tile staging role: row n_s, pixels 16 hr_s .. 16 hr_s + 15 of the quarter
   const int n_s = tid >> 1, hr_s = tid & 1;
-  const bool n_ok = n0 + n_s < Cp;
+  const bool n_ok = n_s < 32 * A && n0 + n_s < Cp;
   const float* pix_row = pix_b + (size_t)(n_ok ? n0 + n_s : 0) * M;
 
-  // ---- staging pieces.  Window: wave w stages channels 8w .. 8w+7 of every element; a lane
+  // ---- staging pieces.  Window: wave w stages CW channels from CW w on of every element; a lane
   // owns elements lane, lane + 64, ... and has all its loads in flight before the first LDS write.
   constexpr int ITER = (CAP + 63) / 64;
-  const int cw = c0 + 8 * wave;
+  constexpr int CW = 8 / G;
+  const int cw = c0 + CW * wave_all;
   const char* cbase = reinterpret_cast<const char*>(img_b + (size_t)min(cw, Cg - 1) * HW);
   const unsigned plane = (unsigned)HW * 4u;
   // wv[it][i] = channel cw + i of the element at flat offset wo[it] (-1: none)
-  auto fetch_window = [&](const int (&wo)[ITER], float (&wv)[ITER][8]) {
+  auto fetch_window = [&](const int (&wo)[ITER], float (&wv)[ITER][CW]) {
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < CW; ++i) {
         // Plain loads from a valid address, nothing that could become a branch around a load
         // (with a condition on the load the generated code took one of the eight of every
         // round behind a branch and waited for it there: five round trips per window instead
@@ -129,32 +146,30 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
       }
     }
   };
-  auto store_window = [&](int RS, const int (&wo)[ITER], const float (&wv)[ITER][8]) {
+  auto store_window = [&](int RS, const int (&wo)[ITER], const float (&wv)[ITER][CW]) {
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
       const int e = lane + 64 * it;
       if (e < RS) {
-        float4* d4 = reinterpret_cast<float4*>(region + e * kWwE + 8 * wave);
-        if (wo[it] >= 0) {
-          d4[0] = make_float4(wv[it][0], wv[it][1], wv[it][2], wv[it][3]);
-          d4[1] = make_float4(wv[it][4], wv[it][5], wv[it][6], wv[it][7]);
-        } else {
-          d4[0] = make_float4(0.f, 0.f, 0.f, 0.f);
-          d4[1] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+        float4* d4 = reinterpret_cast<float4*>(region + e * kWwE + CW * wave_all);
+#pragma unroll
+        for (int i = 0; i < CW / 4; ++i)
+          d4[i] = wo[it] >= 0 ? make_float4(wv[it][4 * i], wv[it][4 * i + 1], wv[it][4 * i + 2],
+                                            wv[it][4 * i + 3])
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
       }
     }
   };
   // Quarter q of a tile: this thread's 16 values of the pixel-side tile (row n_s, pixels
   // 16 hr_s .. + 15) and its share of the plan rows, entry idx = tid + 256 u = (k, r, m), with
   // the rows its sample has (the row itself is read whether it exists or not, clamped to S).
-  constexpr int TOTAL = K * kWwRows * kWwQ;
+  constexpr int TOTAL = K * ROWS * kWwQ;
   constexpr int NR = (TOTAL + kWwThreads - 1) / kWwThreads;
   unsigned row_off[NR], row_k[NR];
 #pragma unroll
   for (int u = 0; u < NR; ++u) {
     const int idx = min(kWwThreads * u + tid, TOTAL - 1);
-    const int k = idx >> 7, r = (idx >> 5) & 3, m = idx & 31;
+    const int k = idx / (ROWS * kWwQ), r = (idx / kWwQ) % ROWS, m = idx % kWwQ;
     row_k[u] = k;
     row_off[u] = (k * S + min(r, S - 1)) * 128 + m;
   }
@@ -195,15 +210,17 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
   auto store_quarter = [&](int RS, const float4 (&gq)[4], const int2 (&pr)[NR],
                            const int (&pn)[NR]) {
     float4* dst = reinterpret_cast<float4*>(gt + n_s * kWwG + 16 * hr_s);
+    if (A == 4 || wave < A) {   // (a wave stages 32 rows)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = gq[i];
+      for (int i = 0; i < 4; ++i) dst[i] = gq[i];
+    }
 #pragma unroll
     for (int u = 0; u < NR; ++u) {
       const int idx = kWwThreads * u + tid;
       if (idx < TOTAL) {
-        const int k = idx >> 7, r = (idx >> 5) & 3, m = idx & 31;
-        const bool on = r < min(pn[u], min(S, kWwRows)) && __int_as_float(pr[u].y) != 0.0f;
-        rowsL[(k * kWwQ + m) * kWwRows + r] =
+        const int k = idx / (ROWS * kWwQ), r = (idx / kWwQ) % ROWS, m = idx % kWwQ;
+        const bool on = r < min(pn[u], min(S, ROWS)) && __int_as_float(pr[u].y) != 0.0f;
+        rowsL[(k * kWwQ + m) * ROWS + r] =
             make_int2((on ? pr[u].x : RS) * (kWwE * 4), on ? pr[u].y : 0);
       }
     }
@@ -229,11 +246,11 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
   // The workgroups of one XCD take neighbouring tiles of the list at the same time: their
   // windows share cache lines, which then meet in that XCD's L2.
   const int first_ti = (group & 7) * (groups >> 3) + (group >> 3);
-  if constexpr (PIPE) {
+  if constexpr (BIG) {
     if (first_ti < cnt) {
       const int first = list[first_ti];
-      if constexpr (BIG) fetch_offsets(first);
-      fetch_quarter(first, 0, pg, pr, pn);
+      fetch_offsets(first);
+      if constexpr (PIPE) fetch_quarter(first, part, pg, pr, pn);
     }
   }
   for (int ti = first_ti; ti < cnt; ti += groups) {
@@ -251,16 +268,16 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
     const int tile_next = has_next ? list[ti + groups] : tile;
 
     __syncthreads();   // every wave is done with the previous tile
-    if (tid < kWwE) region[RS * kWwE + tid] = 0.0f;   // the zero element inactive rows point at
+    if (threadIdx.x < kWwE) region[RS * kWwE + threadIdx.x] = 0.0f;   // the zero element inactive rows point at
     if constexpr (BIG) {
-      float sv[ITER][8];
+      float sv[ITER][CW];
       fetch_window(wo, sv);
       store_window(RS, wo, sv);
     } else {
-      for (int e = tid; e < RS; e += kWwThreads) src[e] = lut[kHdrLut + e];
+      for (int e = threadIdx.x; e < RS; e += kWwThreads * G) src[e] = lut[kHdrLut + e];
       __syncthreads();
       int so[ITER];
-      float sv[ITER][8];
+      float sv[ITER][CW];
 #pragma unroll
       for (int it = 0; it < ITER; ++it) {
         const int e = lane + 64 * it;
@@ -271,8 +288,8 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
     }
 
 #pragma unroll 1
-    for (int q = 0; q < 4; ++q) {
-      if (q > 0) __syncthreads();   // the previous quarter's reads of gt / rowsL are done
+    for (int q = part; q < 4; q += G) {
+      if (q >= G) __syncthreads();   // the previous quarter's reads of gt / rowsL are done
       if constexpr (PIPE) {
         store_quarter(RS, pg, pr, pn);
       } else {
@@ -281,14 +298,13 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
         fetch_quarter(tile, q, pg, pr, pn);
         store_quarter(RS, pg, pr, pn);
       }
-      __syncthreads();   // (for q == 0 this also publishes the window)
-      if constexpr (PIPE) {
-        // requests for what comes next, answered while this quarter's MFMAs run
-        if (q < 3) fetch_quarter(tile, q + 1, pg, pr, pn);
-        else if (has_next) {
-          fetch_quarter(tile_next, 0, pg, pr, pn);
-          if constexpr (BIG) fetch_offsets(tile_next);
-        }
+      __syncthreads();   // (for the first one this also publishes the window)
+      // requests for what comes next, answered while this quarter's MFMAs run
+      if (q + G < 4) {
+        if constexpr (PIPE) fetch_quarter(tile, q + G, pg, pr, pn);
+      } else if (has_next) {
+        if constexpr (PIPE) fetch_quarter(tile_next, part, pg, pr, pn);
+        if constexpr (BIG) fetch_offsets(tile_next);
       }
 
       if constexpr (MM == kMmF32) {
@@ -299,26 +315,32 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
       int4 R01[KW], R23[KW];       // plan rows, two steps ahead
       float co[KW][4], val[KW][4]; // coefficients and window values, one step ahead
       float bcur[KW];
-      const int2* rows_h = rowsL + (16 * h) * kWwRows;
+      const int2* rows_h = rowsL + (16 * h) * ROWS;
+      // A == 2: the remaining samples take part in every second step, with this wave's half of
+      // the pixels
+      const int half8 = A == 2 ? 8 * (wave >> 1) : 0;
+#define SDK_IN_STEP(c, stepv) (A == 4 || (c) < KP || ((stepv) & 1) == 0)
 #define SDK_ROWS_ISSUE(stepv)                                                        \
   do {                                                                               \
-    const int st = (stepv) < 16 ? (stepv) : 15;                                      \
     _Pragma("unroll") for (int c = 0; c < KW; ++c) {                                 \
+      if (!SDK_IN_STEP(c, stepv)) continue;                                          \
+      const int st = A == 4 || c < KP ? (stepv) : (stepv) / 2 + half8;               \
       const int k = c < KP ? wave * KP + c : 4 * KP + (c - KP);                      \
-      const int4* rp = reinterpret_cast<const int4*>(rows_h + (k * kWwQ + st) * kWwRows); \
+      const int2* rp2 = rows_h + (k * kWwQ + st) * ROWS;                             \
       if constexpr (ONE) {                                                           \
-        const int2 r0 = *reinterpret_cast<const int2*>(rp);                          \
-        R01[c].x = r0.x;                                                             \
-        R01[c].y = r0.y;                                                             \
+        R01[c].x = rp2->x;                                                           \
+        R01[c].y = rp2->y;                                                           \
       } else {                                                                       \
+        const int4* rp = reinterpret_cast<const int4*>(rp2);                         \
         R01[c] = rp[0];                                                              \
         R23[c] = rp[1];                                                              \
       }                                                                              \
     }                                                                                \
   } while (0)
-#define SDK_VALS_ISSUE()                                                             \
+#define SDK_VALS_ISSUE(stepv)                                                        \
   do {                                                                               \
     _Pragma("unroll") for (int c = 0; c < KW; ++c) {                                 \
+      if (!SDK_IN_STEP(c, stepv)) continue;                                          \
       val[c][0] = *reinterpret_cast<const float*>(regb + R01[c].x);                  \
       co[c][0] = __int_as_float(R01[c].y);                                           \
       if constexpr (!ONE) {                                                          \
@@ -331,9 +353,10 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
       }                                                                              \
     }                                                                                \
   } while (0)
-#define SDK_BLEND(dst)                                                               \
+#define SDK_BLEND(dst, stepv)                                                        \
   do {                                                                               \
     _Pragma("unroll") for (int c = 0; c < KW; ++c) {                                 \
+      if (!SDK_IN_STEP(c, stepv)) continue;                                          \
       float bv = co[c][0] * val[c][0];                                               \
       if constexpr (!ONE) {                                                          \
         bv = __builtin_fmaf(co[c][1], val[c][1], bv);                                \
@@ -344,44 +367,47 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
     }                                                                                \
   } while (0)
       SDK_ROWS_ISSUE(0);
-      SDK_VALS_ISSUE();    // step 0
+      SDK_VALS_ISSUE(0);
       SDK_ROWS_ISSUE(1);
-      SDK_BLEND(bcur);     // step 0
-      SDK_VALS_ISSUE();    // step 1
+      SDK_BLEND(bcur, 0);
+      SDK_VALS_ISSUE(1);
       SDK_ROWS_ISSUE(2);
-      float4 A[4], Aw;
+      float4 Af[A], Aw;
 #pragma unroll
       for (int step = 0; step < 16; ++step) {
         if ((step & 3) == 0) {
 #pragma unroll
-          for (int a = 0; a < 4; ++a)
-            A[a] = *reinterpret_cast<const float4*>(gt + (32 * a + j) * kWwG + 16 * h + step);
-          Aw = *reinterpret_cast<const float4*>(gt + (32 * wave + j) * kWwG + 16 * h + step);
+          for (int a = 0; a < A; ++a)
+            Af[a] = *reinterpret_cast<const float4*>(gt + (32 * a + j) * kWwG + 16 * h + step);
         }
-        const int ss = step & 3;
-        const float a0 = ss == 0 ? A[0].x : (ss == 1 ? A[0].y : (ss == 2 ? A[0].z : A[0].w));
-        const float a1 = ss == 0 ? A[1].x : (ss == 1 ? A[1].y : (ss == 2 ? A[1].z : A[1].w));
-        const float a2 = ss == 0 ? A[2].x : (ss == 1 ? A[2].y : (ss == 2 ? A[2].z : A[2].w));
-        const float a3 = ss == 0 ? A[3].x : (ss == 1 ? A[3].y : (ss == 2 ? A[3].z : A[3].w));
-        const float aw = ss == 0 ? Aw.x : (ss == 1 ? Aw.y : (ss == 2 ? Aw.z : Aw.w));
+        const int rstep = A == 4 ? step : step / 2;
+        if (SDK_IN_STEP(KP, step) && (rstep & 3) == 0)
+          Aw = *reinterpret_cast<const float4*>(gt + (32 * (wave & (A - 1)) + j) * kWwG + 16 * h +
+                                                half8 + rstep);
+        auto of = [](const float4& f, int s) {
+          return s == 0 ? f.x : (s == 1 ? f.y : (s == 2 ? f.z : f.w));
+        };
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kk = 0; kk < KP; ++kk) {
-          accF[kk][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, bcur[kk], accF[kk][0], 0, 0, 0);
-          accF[kk][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, bcur[kk], accF[kk][1], 0, 0, 0);
-          accF[kk][2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a2, bcur[kk], accF[kk][2], 0, 0, 0);
-          accF[kk][3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a3, bcur[kk], accF[kk][3], 0, 0, 0);
-        }
+        for (int kk = 0; kk < KP; ++kk)
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-          accR[r] = __builtin_amdgcn_mfma_f32_32x32x2f32(aw, bcur[KP + r], accR[r], 0, 0, 0);
+          for (int a = 0; a < A; ++a)
+            accF[kk][a] = __builtin_amdgcn_mfma_f32_32x32x2f32(of(Af[a], step & 3), bcur[kk],
+                                                               accF[kk][a], 0, 0, 0);
+        if (SDK_IN_STEP(KP, step)) {
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+            accR[r] = __builtin_amdgcn_mfma_f32_32x32x2f32(of(Aw, rstep & 3), bcur[KP + r],
+                                                           accR[r], 0, 0, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
         if (step < 15) {
-          SDK_BLEND(bcur);                      // step + 1
-          if (step < 14) SDK_VALS_ISSUE();      // step + 2
+          SDK_BLEND(bcur, step + 1);
+          if (step < 14) SDK_VALS_ISSUE(step + 2);
           if (step < 13) SDK_ROWS_ISSUE(step + 3);
         }
       }
+#undef SDK_IN_STEP
 #undef SDK_ROWS_ISSUE
 #undef SDK_VALS_ISSUE
 #undef SDK_BLEND
@@ -401,6 +427,7 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
           Bf16Split b3[KW];
 #pragma unroll
           for (int c = 0; c < KW; ++c) {
+            if (A == 2 && c >= KP && grp != (wave >> 1)) continue;   // (the other waves' pixels)
             const int k = c < KP ? wave * KP + c : 4 * KP + (c - KP);
             const int4* rp = reinterpret_cast<const int4*>(rowsL + (k * kWwQ + m0) * kWwRows);
             float bv[8];
@@ -418,7 +445,7 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
             }
             b3[c] = split_bf16x8(bv);
           }
-          // A fragments: rows 32 a + j (and 32 wave + j for the remaining samples)
+          // A fragments: rows 32 a + j (and of the wave's row block for the remaining samples)
           auto a_values = [&](int row, float (&f)[8]) {
             const float4* ap = reinterpret_cast<const float4*>(gt + row * kWwG + m0);
             const float4 lo = ap[0], hi = ap[1];
@@ -426,7 +453,7 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
             f[4] = hi.x; f[5] = hi.y; f[6] = hi.z; f[7] = hi.w;
           };
 #pragma unroll
-          for (int a = 0; a < 4; ++a) {
+          for (int a = 0; a < A; ++a) {
             if constexpr (KP > 0) {
               float f[8];
               a_values(32 * a + j, f);
@@ -435,9 +462,9 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
               for (int kk = 0; kk < KP; ++kk) accF[kk][a] = mfma_split(a3, b3[kk], accF[kk][a]);
             }
           }
-          if constexpr (R > 0) {
+          if (R > 0 && (A == 4 || grp == (wave >> 1))) {
             float f[8];
-            a_values(32 * wave + j, f);
+            a_values(32 * (wave & (A - 1)) + j, f);
             const Bf16Split a3 = split_bf16x8(f);
 #pragma unroll
             for (int r = 0; r < R; ++r) accR[r] = mfma_split(a3, b3[KP + r], accR[r]);
@@ -447,33 +474,66 @@ __global__ __launch_bounds__(kWwThreads, CAP > kRegionCap ? 1 : 2) void window_w
     }
   }
 
+  // ---- the second group's sums, through the window's LDS
+  if constexpr (G == 2) {
+    static_assert((A * KP + R) * 16 * kWwThreads <= (CAP + 1) * kWwE, "sums fit the window");
+    __syncthreads();
+    float* sums = region + tid;
+    if (part == 1) {
+#pragma unroll
+      for (int kk = 0; kk < KP; ++kk)
+#pragma unroll
+        for (int a = 0; a < A; ++a)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) sums[((kk * A + a) * 16 + v) * kWwThreads] = accF[kk][a][v];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sums[((KP * A + r) * 16 + v) * kWwThreads] = accR[r][v];
+    }
+    __syncthreads();
+    if (part == 1) return;
+#pragma unroll
+    for (int kk = 0; kk < KP; ++kk)
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) accF[kk][a][v] += sums[((kk * A + a) * 16 + v) * kWwThreads];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) accR[r][v] += sums[((KP * A + r) * 16 + v) * kWwThreads];
+  }
+
   // ---- every accumulator register is stored as it lies (register-major, thread fastest)
-  constexpr int NREG = (4 * KP + R) * 16;
+  constexpr int NREG = (A * KP + R) * 16;
   float* dst = partial + (size_t)blockIdx.x * (NREG * kWwThreads) + tid;
 #pragma unroll
   for (int kk = 0; kk < KP; ++kk)
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < A; ++a)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) dst[((kk * 4 + a) * 16 + v) * kWwThreads] = accF[kk][a][v];
+      for (int v = 0; v < 16; ++v) dst[((kk * A + a) * 16 + v) * kWwThreads] = accF[kk][a][v];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) dst[((KP * 4 + r) * 16 + v) * kWwThreads] = accR[r][v];
+    for (int v = 0; v < 16; ++v) dst[((KP * A + r) * 16 + v) * kWwThreads] = accR[r][v];
 }
 
 // Sums the accumulator copies of window_wgrad_kernel and adds them to gW.  Block (x, y, z):
 // accumulator register x of thread threadIdx.x, for the workgroup kind y = (channel chunk,
-// row tile), over every z-th of the batches * groups workgroups of that kind.
+// row tile), over every z-th of the batches * groups workgroups of that kind.  A: the row blocks
+// of the summing kernel.
 __global__ __launch_bounds__(kWwThreads) void window_wgrad_reduce_kernel(
     const float* __restrict__ partial, float* __restrict__ gW, int Cg, int Cp, int K, int KP,
-    int R, int groups, int batches, int c_chunks, int n_tiles, const int* __restrict__ count) {
+    int R, int A, int groups, int batches, int c_chunks, int n_tiles,
+    const int* __restrict__ count) {
   if (*count == 0) return;   // nothing was summed
   const int tid = threadIdx.x, reg = blockIdx.x;
   const int nt = blockIdx.y % n_tiles, cc = blockIdx.y / n_tiles;
   const int kinds = c_chunks * n_tiles * batches;
   const int total = batches * groups;
-  const size_t per_wg = (size_t)(4 * KP + R) * 16 * kWwThreads;
+  const size_t per_wg = (size_t)(A * KP + R) * 16 * kWwThreads;
   // four reads in flight per thread (a plain loop waits for each in turn)
   auto at = [&](int i) {
     const int ic = min(i, total - 1);
@@ -496,16 +556,21 @@ __global__ __launch_bounds__(kWwThreads) void window_wgrad_reduce_kernel(
   const int wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
   const int v = reg & 15, blk = reg >> 4;
   int k, a;
-  if (blk < 4 * KP) {
-    k = wave * KP + blk / 4;
-    a = blk & 3;
+  if (blk < A * KP) {
+    k = wave * KP + blk / A;
+    a = blk & (A - 1);
   } else {
-    k = 4 * KP + (blk - 4 * KP);
-    a = wave;
+    k = 4 * KP + (blk - A * KP);
+    a = wave & (A - 1);
   }
   const int n = nt * 128 + 32 * a + 8 * (v >> 2) + 4 * h + (v & 3);
   const int c = cc * kCC + j;
   if (c < Cg && n < Cp && k < K) atomic_add_noret(gW + (size_t)n * Cg * K + (size_t)c * K + k, s);
+}
+
+// G of window_wgrad_kernel
+constexpr int ww_parts(int cap, int mm, int a) {
+  return cap > kRegionCap && mm == kMmF32 && a == 2 ? 2 : 1;
 }
 
 struct WwGrid {
@@ -535,13 +600,13 @@ bool window_wgrad_big_supported(const ConvGeom& g, int mm) {
 }
 
 bool window_wgrad_supported(const ConvGeom& g, int mm) {
-  // (every wave multiplies four 32-row blocks: with 64 rows or fewer half of that is padding.
-  // On tiles inside an ordinary window the plan-driven kernel, which splits the pixels
-  // instead, is then the faster one; on big tiles, which it reads from global memory, the
-  // padded window kernel still is, down to a few rows: 3 x 3 bilinear at stride 2 on a
-  // 64 x 128 grid, 4 x 128 -> 64 channels: 346 against 162 us; 128 -> 13 channels: the whole
-  // backward call 0.49 against 0.29 ms.)
-  return window_wgrad_big_supported(g, mm) && g.Cp > 64;
+  // (single-row plans and at most 64 rows: window_wgrad_narrow, whose operands are copies.  With
+  // 64 rows or fewer, two row blocks a wave; the kernel that works from global memory, which took
+  // these layers before, is the slower one down to 8 rows and 8 channels.  9 samples, 256 x 512,
+  // batch 8, weight gradient in us, there and here: 64 -> 64 float32 1627 / 1075, split 1550 / 1156,
+  // bf16 1248 / 508; 128 -> 32 float32 2773 / 2012; 8 -> 16 float32 658 / 495; 180 x 360, 64 -> 8
+  // 761 / 543; 220 x 440, batch 1, 48 -> 40 252 / 143)
+  return window_wgrad_big_supported(g, mm) && (g.Cp > 64 || !window_wgrad_narrow_supported(g, mm));
 }
 
 size_t window_wgrad_partial_bytes(const ConvGeom& g) {
@@ -568,7 +633,7 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
   const int TX = plan.pt.TX();
   const int vec4 = (g.OW % 4 == 0 && TX >= 16 && reinterpret_cast<uintptr_t>(pix) % 16 == 0) ? 1 : 0;
   const dim3 grid((unsigned)w.slots);
-  int KP = g.K / 4, R = g.K % 4;
+  int KP = g.K / 4, R = g.K % 4, A = 4;
   if (mm == kMmBf16) {
     const int rc = window_wgrad16(g, plan, list, count, big, pix, img, partial, w.groups,
                                   w.c_chunks, w.n_tiles, w.slots, stream);
@@ -576,23 +641,24 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
     KP = 0;   // (its accumulators: one row block a wave for every sample)
     R = g.K;
   } else {
-#define WW3(KPv, Rv, CAPv, MMv)                                                                  \
-  launch(window_wgrad_kernel<KPv, Rv, CAPv, MMv>, grid, dim3(kWwThreads), stream, pix, img,      \
-         plan.hdr, plan.ns, plan.taps, list, count, partial, g.Cg, g.H, g.W, g.Cp, plan.S,       \
+    if (g.Cp <= 64) A = 2;
+#define WW3(KPv, Rv, CAPv, MMv, ONEv, Av)                                                         \
+  launch(window_wgrad_kernel<KPv, Rv, CAPv, MMv, ONEv, Av, ww_parts(CAPv, MMv, Av)>, grid,         \
+         dim3(kWwThreads * ww_parts(CAPv, MMv, Av)), stream, pix, img, plan.hdr, plan.ns, plan.taps, list, count, partial, g.Cg, g.H, g.W, g.Cp, plan.S,   \
          plan.pt, w.groups, (int)g.B, w.c_chunks, w.n_tiles, vec4, plan.big_lut)
-#define WW3ONE(KPv, Rv, CAPv)                                                                    \
-  launch(window_wgrad_kernel<KPv, Rv, CAPv, kMmF32, true>, grid, dim3(kWwThreads), stream, pix,   \
-         img, plan.hdr, plan.ns, plan.taps, list, count, partial, g.Cg, g.H, g.W, g.Cp, plan.S,   \
-         plan.pt, w.groups, (int)g.B, w.c_chunks, w.n_tiles, vec4, plan.big_lut)
-#define WW2(KPv, Rv, CAPv)                                                       \
+#define WW2(KPv, Rv, CAPv, Av)                                                   \
   do {                                                                           \
-    if (mm == kMmSplit) WW3(KPv, Rv, CAPv, kMmSplit);                            \
-    else if (plan.S == 1) WW3ONE(KPv, Rv, CAPv);                                 \
-    else WW3(KPv, Rv, CAPv, kMmF32);                                             \
+    if (mm == kMmSplit) WW3(KPv, Rv, CAPv, kMmSplit, false, Av);                 \
+    else if (plan.S == 1) WW3(KPv, Rv, CAPv, kMmF32, true, Av);                  \
+    else WW3(KPv, Rv, CAPv, kMmF32, false, Av);                                  \
+  } while (0)
+#define WW1(KPv, Rv, CAPv)                                                       \
+  do {                                                                           \
+    if (A == 2) WW2(KPv, Rv, CAPv, 2); else WW2(KPv, Rv, CAPv, 4);               \
   } while (0)
 #define WW(KPv, Rv)                                                   \
   do {                                                                \
-    if (big) WW2(KPv, Rv, kBigCap); else WW2(KPv, Rv, kRegionCap);    \
+    if (big) WW1(KPv, Rv, kBigCap); else WW1(KPv, Rv, kRegionCap);    \
   } while (0)
   switch (g.K) {
     case 1: WW(0, 1); break;
@@ -607,16 +673,17 @@ int window_wgrad(const ConvGeom& g, int mm, const Plan& plan, const TileLists& t
     default: WW(2, 2); break;
   }
 #undef WW
+#undef WW1
 #undef WW2
 #undef WW3
-#undef WW3ONE
   SDK_LAUNCH_CHECK(big ? "window_wgrad(big)" : "window_wgrad");
   }
   const int kinds0 = w.c_chunks * w.n_tiles, total = (int)g.B * w.groups;
+  const int nreg = (A * KP + R) * 16;
   const int parts = (int)std::min<int64_t>(std::min(total, 16),
-                                           ceil_div(2048, (int64_t)w.nreg * kinds0));
-  launch(window_wgrad_reduce_kernel, dim3((unsigned)w.nreg, (unsigned)kinds0, (unsigned)std::max(parts, 1)),
-         dim3(kWwThreads), stream, (const float*)partial, gW, g.Cg, g.Cp, g.K, KP, R, w.groups,
+                                           ceil_div(2048, (int64_t)nreg * kinds0));
+  launch(window_wgrad_reduce_kernel, dim3((unsigned)nreg, (unsigned)kinds0, (unsigned)std::max(parts, 1)),
+         dim3(kWwThreads), stream, (const float*)partial, gW, g.Cg, g.Cp, g.K, KP, R, A, w.groups,
          (int)g.B, w.c_chunks, w.n_tiles, count);
   SDK_LAUNCH_CHECK("window_wgrad_reduce");
   return SDK_OK;

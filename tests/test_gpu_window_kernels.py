@@ -27,6 +27,15 @@ SIZES = [
     (1, 36, 127, 16, 40, 16, 40, 6, 2, 0),
     (1, 64, 66, 24, 40, 12, 20, 8, 0, 2),
     (3, 20, 129, 32, 64, 32, 64, 9, 0, 2),
+    # at most 64 rows: two row blocks a wave, the remaining samples' pixels shared by two waves,
+    # big tiles by two groups of waves
+    (1, 33, 1, 9, 20, 9, 20, 3, 1, 0),
+    (2, 5, 32, 17, 33, 17, 33, 4, 2, 0),
+    (1, 40, 33, 48, 96, 24, 48, 9, 1, 0),
+    (2, 70, 64, 48, 96, 24, 48, 10, 2, 0),
+    (1, 32, 64, 40, 80, 20, 40, 7, 0, 0),
+    (1, 64, 63, 24, 40, 12, 20, 6, 0, 2),
+    (1, 20, 40, 12, 9, 12, 9, 2, 0, 0),
 ]
 
 
