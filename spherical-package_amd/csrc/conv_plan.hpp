@@ -145,9 +145,9 @@ int planned_wgrad(const ConvGeom& g, int mm, const Plan& plan, const float* pix,
                   const float* img, float* gW, float* partial, hipStream_t stream,
                   const int* tile_list = nullptr, const int* tile_count = nullptr);
 
-// The same sums over the tiles of tl.inside, from an LDS window with the column values built
-// straight into MFMA operands (conv_window_wgrad.hip; K <= 10, at most four plan rows per
-// sample: build the lists with max_rows = 4; mm: the matrix arithmetic).  partial: window_wgrad_partial_bytes(g).
+// The same sums over the tiles of tl.inside, from an LDS window (conv_window_wgrad.hip; K <= 10, at
+// most four plan rows per sample: build the lists with max_rows = 4; mm: the matrix arithmetic).
+// partial: window_wgrad_partial_bytes(g).
 bool window_wgrad_supported(const ConvGeom& g, int mm);
 // ... for the big tiles alone (window_wgrad(..., big = true)): also the layers whose other tiles
 // window_wgrad_narrow takes.
@@ -161,9 +161,16 @@ int window_wgrad_narrow(const ConvGeom& g, int mm, const Plan& plan, const TileL
                         const float* pix, const float* img, float* gW, float* partial,
                         hipStream_t stream);
 
-// Its bf16 arithmetic (conv_window_wgrad16.hip): leaves accumulator register 16 k + v of row block
-// (thread / 64), K * 16 * 256 floats a workgroup, in `partial`.
+// Its kernels (conv_window_wgrad_quarter.hpp), by matrix arithmetic: leave accumulator register 16 k + v of
+// row block (thread / 64) % window_wgrad_blocks(g), K * 16 * 256 floats a workgroup, in `partial`.
+inline int window_wgrad_blocks(const ConvGeom& g) { return g.Cp <= 64 ? 2 : 4; }
 int window_wgrad16(const ConvGeom& g, const Plan& plan, const int* list, const int* count, bool big,
+                   const float* pix, const float* img, float* partial, int groups, int c_chunks,
+                   int n_tiles, int64_t slots, hipStream_t stream);
+int window_wgrad32(const ConvGeom& g, const Plan& plan, const int* list, const int* count, bool big,
+                   const float* pix, const float* img, float* partial, int groups, int c_chunks,
+                   int n_tiles, int64_t slots, hipStream_t stream);
+int window_wgrad_split(const ConvGeom& g, const Plan& plan, const int* list, const int* count, bool big,
                    const float* pix, const float* img, float* partial, int groups, int c_chunks,
                    int n_tiles, int64_t slots, hipStream_t stream);
 

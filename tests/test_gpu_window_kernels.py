@@ -27,8 +27,11 @@ SIZES = [
     (1, 36, 127, 16, 40, 16, 40, 6, 2, 0),
     (1, 64, 66, 24, 40, 12, 20, 8, 0, 2),
     (3, 20, 129, 32, 64, 32, 64, 9, 0, 2),
-    # at most 64 rows: two row blocks a wave, the remaining samples' pixels shared by two waves,
-    # big tiles by two groups of waves
+    # big tiles whose samples do not halve among the two groups of waves
+    (1, 34, 100, 48, 96, 12, 24, 1, 1, 0),
+    (1, 34, 70, 48, 96, 12, 24, 3, 2, 0),
+    (2, 40, 40, 48, 96, 12, 24, 5, 0, 0),
+    # at most 64 rows: two row blocks, each with half of the pixels in two waves
     (1, 33, 1, 9, 20, 9, 20, 3, 1, 0),
     (2, 5, 32, 17, 33, 17, 33, 4, 2, 0),
     (1, 40, 33, 48, 96, 24, 48, 9, 1, 0),
