@@ -473,15 +473,16 @@ window_gemm_kernel(const float* __restrict__ img, const int* __restrict__ hdr,
       for (int v = 0; v < 16; ++v) acc[a][v] = 0.0f;
   }
 
-  // weight tile of (k, chunk): WT pieces in operand order, copied as they lie
+  // weight tile of (k, chunk): WT pieces in operand order, copied as they lie (a descriptor of its
+  // own: all the weights may be more than the 2 GB that one reaches)
   const int gt = tid & (kWgThreads - 1);
   u32x4 wq[WPT];
-  const Rsrc w_rs = rsrc_of(Wp + (size_t)nt * WT);
 #define SDK_LOAD_WEIGHTS(kv, chunkv)                                                           \
   do {                                                                                         \
-    const int wso = ((kv) * chunks + (chunkv)) * blks * (kPieces<MM> * 1024);                  \
-    _Pragma("unroll") for (int i = 0; i < WPT; ++i) wq[i] = __builtin_amdgcn_raw_buffer_load_b128( \
-        w_rs, min(gt + i * kWgThreads, WT - 1) * 16, wso, 0);                                  \
+    const Rsrc w_rs = rsrc_of(Wp + (size_t)nt * WT + ((size_t)(kv) * chunks + (chunkv)) *      \
+                              (size_t)(blks * (kPieces<MM> * 64)));                            \
+    _Pragma("unroll") for (int i = 0; i < WPT; ++i) wq[i] = __builtin_amdgcn_raw_buffer_load_b128(\
+        w_rs, min(gt + i * kWgThreads, WT - 1) * 16, 0, 0);                                    \
   } while (0)
 #define SDK_STORE_WEIGHTS()                                                                    \
   do {                                                                                         \

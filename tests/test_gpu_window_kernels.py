@@ -96,3 +96,23 @@ def test_values_that_are_not_finite_stay_where_they_are(tile_kernels, mode):
     reads = ((np.abs(m[..., 0] - 7) < 1) & (np.abs(m[..., 1] - 5) < 1)).any(-1)
     assert np.array_equal(~np.isfinite(y[0]).all(0), reads)
     assert np.isfinite(gw[:, :32]).all() and not np.isfinite(gw[:, 32]).all()
+
+
+@pytest.mark.parametrize("mode", ["native", "split"])
+def test_more_than_two_gigabytes_of_weights(tile_kernels, mode):
+    """The last output channel's row of a weight tensor past 2^31 bytes, integers as above."""
+    import _spherical_distortion_ext._ops as ops
+    C, K, H, W = 7744, 9, 8, 16
+    rng = np.random.default_rng(7)
+    x = torch.from_numpy(rng.integers(-4, 5, (1, C, H, W)).astype(np.float32)).to(DEV)
+    row = torch.from_numpy(rng.integers(-4, 5, (C, K)).astype(np.float32)).to(DEV)
+    at = torch.from_numpy(rng.integers(0, H * W, (H, W, K))).to(DEV)
+    w = torch.zeros(C, C, K, device=DEV)
+    assert w.numel() * 4 > 2 ** 31
+    w[-1] = row
+    m = torch.stack([at % W, at // W], -1).float().contiguous()
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(x, m, None, w, torch.zeros(C, device=DEV), K, 0)
+    want = (x.flatten(2)[0][:, at].double() * row.double()[:, None, None, :]).sum((0, 3))
+    assert torch.equal(y[0, -1].double(), want)
+    assert not y[0, :-1].any()
