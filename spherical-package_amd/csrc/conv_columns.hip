@@ -165,10 +165,37 @@ __global__ __launch_bounds__(kClThreads) void columns_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kGk = 32;
 constexpr int kGld = 36;
+// bf16 operands (CONV) are formed on the way to LDS, once per workgroup: a wave that forms its own from
+// float32 rows repeats what the neighbour of the same rows does, and six vector instructions an element
+// weigh as much as the products.  A row then holds 64 bytes a piece (one, or the three of the split)
+// and 16 of skew.  6 x 25 x 50 pixels, 96 -> 160, split, weight gradient 41.7 -> 39.0 us; 325 x 648, batch 2,
+// 16 -> 29, bf16, map and forward 251 -> 232.  Two groups on split operands keep float32 rows: two
+// workgroups would no longer share a CU.
+constexpr bool columns_conv(int mm, int ks) { return mm == kMmBf16 || (mm == kMmSplit && ks == 1); }
+constexpr int columns_row_bytes(int mm, int ks) {
+  return !columns_conv(mm, ks) ? kGld * 4 : (mm == kMmBf16 ? 64 : 192) + 16;
+}
 // A split of the weight gradient's reduction is hundreds of pixels; added up one after the other they
 // lose twice the bits of the tile kernels' sums (6 x 25 x 50 pixels, 96 -> 160: 4.5e-7 of the float64
 // norm against 2.1e-7), so two steps at a time are summed apart and then added: 1.7e-7, for 2 us of the
 // layer's 174.
+
+// (as split_bf16x8)
+__device__ __forceinline__ void split_bf16x4(const vec4& f, uint2 (&piece)[3]) {
+  unsigned u[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float r = f[i];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      u[p][i] = __float_as_uint(r) & 0xffff0000u;
+      r -= __uint_as_float(u[p][i]);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    piece[p] = make_uint2((u[p][0] >> 16) | u[p][1], (u[p][2] >> 16) | u[p][3]);
+}
 
 struct GemmArgs {
   const float *A, *B;
@@ -187,7 +214,9 @@ template <int MM, bool TN, int KS>
 __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs g) {
   constexpr int BM = 64, BN = 64;
   constexpr int LA = BM / 32, LB = BN / 32;   // 16-byte pieces per thread and step
-  __shared__ __attribute__((aligned(16))) float lds[KS][2][(BM + BN) * kGld];
+  constexpr bool CONV = columns_conv(MM, KS);
+  constexpr int RB = columns_row_bytes(MM, KS);
+  __shared__ __attribute__((aligned(16))) char lds[KS][2][(BM + BN) * RB];
   __shared__ float s_bias[BM];
   // consecutive slots of one XCD share the tile of the larger operand (workgroup ids go
   // round-robin over the 8 XCDs)
@@ -200,8 +229,8 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   const int tid = threadIdx.x % kClThreads, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  float* As[2] = {lds[group][0], lds[group][1]};
-  float* Bs[2] = {lds[group][0] + BM * kGld, lds[group][1] + BM * kGld};
+  char* As[2] = {lds[group][0], lds[group][1]};
+  char* Bs[2] = {lds[group][0] + BM * RB, lds[group][1] + BM * RB};
   const float* B = TN ? g.B : g.B + (size_t)blockIdx.y * g.batch_b;
   float* C = g.C + (size_t)blockIdx.y * g.batch_c;
   const int r_begin = TN ? (int)blockIdx.y * g.split : 0;
@@ -234,23 +263,36 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
       }
     }
   };
+  // four reduction elements, quad kb of a row
+  auto put = [&](char* row, const vec4& v) {
+    if constexpr (!CONV) {
+      *reinterpret_cast<vec4*>(row + 16 * kb) = v;
+    } else if constexpr (MM == kMmBf16) {
+      *reinterpret_cast<uint2*>(row + 8 * kb) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    } else {
+      uint2 piece[3];
+      split_bf16x4(v, piece);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(row + 64 * p + 8 * kb) = piece[p];
+    }
+  };
   auto stash = [&](int buf, int r0, const vec4 (&ga)[LA], const vec4 (&gb)[LB]) {
     if constexpr (!TN) {
       const bool on = r0 + 4 * kb < r_end;
 #pragma unroll
       for (int i = 0; i < LA; ++i)
-        *reinterpret_cast<vec4*>(&As[buf][(rb + 32 * i) * kGld + 4 * kb]) = on ? ga[i] : zero;
+        put(As[buf] + (rb + 32 * i) * RB, on ? ga[i] : zero);
 #pragma unroll
       for (int i = 0; i < LB; ++i)
-        *reinterpret_cast<vec4*>(&Bs[buf][(rb + 32 * i) * kGld + 4 * kb]) = on ? gb[i] : zero;
+        put(Bs[buf] + (rb + 32 * i) * RB, on ? gb[i] : zero);
     } else {
-      float* dst = (tid < 128 ? As[buf] : Bs[buf]) + 4 * (rb & 15) * kGld + 4 * kb;
+      char* dst = (tid < 128 ? As[buf] : Bs[buf]) + 4 * (rb & 15) * RB;
       const int r = r0 + 4 * kb;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const vec4 v = {r < r_end ? ga[0][e] : 0.0f, r + 1 < r_end ? ga[1][e] : 0.0f,
                         r + 2 < r_end ? gb[0][e] : 0.0f, r + 3 < r_end ? gb[1][e] : 0.0f};
-        *reinterpret_cast<vec4*>(dst + e * kGld) = v;
+        put(dst + e * RB, v);
       }
     }
   };
@@ -261,8 +303,8 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   const floatx16 none = {};
   floatx16 acc = none, all = none;   // (TN: all = the sums of two steps each, acc those under way)
 
-  auto load8 = [&](const float* p, float (&f)[8]) {
-    const vec4 lo = *reinterpret_cast<const vec4*>(p), hi = *reinterpret_cast<const vec4*>(p + 4);
+  auto load8 = [&](const char* p, float (&f)[8]) {
+    const vec4 lo = *reinterpret_cast<const vec4*>(p), hi = *reinterpret_cast<const vec4*>(p + 16);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       f[e] = lo[e];
@@ -274,17 +316,30 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
     if (TN && buf == 0) acc = none;
 #pragma unroll
     for (int s = 0; s < kGk / 16; ++s) {
-      float fa[8], fb[8];
-      load8(&As[buf][(wr + j) * kGld + 16 * s + 8 * h], fa);
-      load8(&Bs[buf][(wc + j) * kGld + 16 * s + 8 * h], fb);
-      if constexpr (MM == kMmF32) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
-      } else if constexpr (MM == kMmBf16) {
-        acc = mfma_bf16(pack_bf16x8(fa), pack_bf16x8(fb), acc);
+      if constexpr (CONV) {
+        auto piece = [&](const char* row, int p) {
+          return __builtin_bit_cast(Bf16Frag, *reinterpret_cast<const uint4*>(row + 64 * p));
+        };
+        const char* pa = As[buf] + (wr + j) * RB + 32 * s + 16 * h;
+        const char* pb = Bs[buf] + (wc + j) * RB + 32 * s + 16 * h;
+        if constexpr (MM == kMmBf16) {
+          acc = mfma_bf16(piece(pa, 0), piece(pb, 0), acc);
+        } else {
+          const Bf16Split a = {piece(pa, 0), piece(pa, 1), piece(pa, 2)};
+          const Bf16Split b = {piece(pb, 0), piece(pb, 1), piece(pb, 2)};
+          acc = mfma_split(a, b, acc);
+        }
       } else {
-        acc = mfma_split(split_bf16x8(fa), split_bf16x8(fb), acc);
+        float fa[8], fb[8];
+        load8(As[buf] + (wr + j) * RB + 64 * s + 32 * h, fa);
+        load8(Bs[buf] + (wc + j) * RB + 64 * s + 32 * h, fb);
+        if constexpr (MM == kMmF32) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
+        } else {
+          acc = mfma_split(split_bf16x8(fa), split_bf16x8(fb), acc);
+        }
       }
     }
   };
@@ -320,7 +375,8 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   if constexpr (TN) acc = all;
   if constexpr (KS == 2) {
     // the second group's sums join the first's through LDS, [register][thread]
-    float* sums = &lds[1][0][0];
+    static_assert(2 * (BM + BN) * RB >= 16 * kClThreads * (int)sizeof(float), "sums fit a group's rows");
+    float* sums = reinterpret_cast<float*>(lds[1][0]);
     if (group == 1) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) sums[v * kClThreads + tid] = acc[v];
