@@ -551,28 +551,38 @@ template <typename T, int INTERP, int PL, typename ACC>
 __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
     const T* __restrict__ in, const T* __restrict__ uv, const int* __restrict__ offset,
     const int* __restrict__ list, T* __restrict__ textures, int planes, int NT, int TH, int TW,
-    int MP) {
+    int MP, int ordered) {
   extern __shared__ __align__(16) unsigned char uv_lds[];
   constexpr bool DIRECT = std::is_same<ACC, double>::value;   // native adds
   ACC* acc = reinterpret_cast<ACC*>(uv_lds);         // [PL][TH * TW]
   const int THW = TH * TW;
-  // Longest buckets first, all their plane chunks: a polar texture's takes three times as long as
-  // the others', and started last it runs alone at the end.
+  // ordered (NT <= kUvBlock): longest buckets first, all their plane chunks: a polar texture's takes
+  // three times as long as the others', and started last it runs alone at the end.  The textures of
+  // longer buckets are counted by kUvBlock / NT threads for each texture (by one, 320 textures cost a
+  // workgroup 15 us).
   int t = blockIdx.x, chunk = blockIdx.y;
-  if (NT <= kUvBlock) {
-    __shared__ int size[kUvBlock];
+  if (ordered) {
+    __shared__ int size[kUvBlock], above[kUvBlock];
     __shared__ int chosen;
     const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / (int)gridDim.y;
     chunk = id % (int)gridDim.y;
-    const int i = threadIdx.x;
-    if (i < NT) size[i] = offset[i + 1] - offset[i];
-    __syncthreads();
-    if (i < NT) {
-      const int mine = size[i];
-      int above = 0;
-      for (int k = 0; k < NT; ++k) above += (size[k] > mine || (size[k] == mine && k < i)) ? 1 : 0;
-      if (above == rank) chosen = i;
+    const int i = threadIdx.x % NT, part = threadIdx.x / NT, parts = kUvBlock / NT;
+    if (part == 0) {
+      size[i] = offset[i + 1] - offset[i];
+      above[i] = 0;
     }
+    __syncthreads();
+    if (part < parts) {
+      const int per = (NT + parts - 1) / parts, end = min((part + 1) * per, NT);
+      const int mine = size[i];
+      int n = 0;
+#pragma unroll 4
+      for (int k = part * per; k < end; ++k)
+        n += (size[k] > mine || (size[k] == mine && k < i)) ? 1 : 0;
+      atomicAdd(&above[i], n);
+    }
+    __syncthreads();
+    if (part == 0 && above[i] == rank) chosen = i;
     __syncthreads();
     t = chosen;
   }
@@ -1663,11 +1673,15 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
       if (rc != SDK_OK) return rc;
     }
     const dim3 grid((unsigned)NT, (unsigned)ceil_div(planes, pl), (unsigned)split);
+    // buckets of less than a round of the workgroup are as good in any order, and choosing costs as
+    // much as they do (12 planes, 320 textures of 43 x 43, 65 x 130 pixels: 24 us a pass, 69 where
+    // every workgroup chose)
+    const int ordered = NT <= kUvBlock && MP >= (int64_t)NT * kUvBlock ? 1 : 0;
 #define UVS(PLv, ACCv)                                                                        \
   SDK_DISPATCH_INTERP_ONLY(interp, (uv_texture_scatter_kernel<T, INTERP, PLv, ACCv>           \
                                     <<<grid, dim3(kUvBlock), (size_t)PLv * THW * sum, stream>>>( \
                                         in, uv, (const int*)offset, (const int*)list, textures, \
-                                        (int)planes, NT, TH, TW, MP)))
+                                        (int)planes, NT, TH, TW, MP, ordered)))
     if (direct) {
       if (pl == 4) UVS(4, double); else if (pl == 2) UVS(2, double); else UVS(1, double);
     } else {   // (such a texture takes half of kUvLdsBytes or more)

@@ -17,10 +17,11 @@ def ops():
 
 # (batch, channels, textures, TH, TW, H, W): odd plane counts, one texture (its bucket shared among
 # workgroups), more textures than threads of a workgroup, textures whose double sums are just in and
-# just out of the LDS (8192 texels), buckets of less and more than one round of 1024 pixels
+# just out of the LDS (8192 texels), buckets of less and more than one round of 1024 pixels (then
+# taken by falling size)
 SIZES = [(1, 1, 1, 1, 1, 1, 1), (2, 3, 5, 8, 9, 33, 47), (1, 13, 80, 16, 16, 60, 128),
          (1, 5, 1030, 4, 3, 40, 77), (1, 2, 3, 64, 128, 50, 90), (1, 3, 2, 91, 91, 64, 64),
-         (3, 2, 1, 16, 16, 100, 120)]
+         (3, 2, 1, 16, 16, 100, 120), (1, 3, 33, 5, 6, 180, 200)]
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
