@@ -34,6 +34,10 @@ constexpr int kVoteTile = 16;        // input tile side
 constexpr int kVoteMeet = 64;        // input tiles (16384 pixels) a workgroup takes on
 constexpr int kVoteTiles = 8192;     // input tiles: every workgroup looks through all boxes (64 KB)
 constexpr int kVoteCounters = 4096;  // LDS counters of a workgroup
+// Histograms of fewer bytes than this in all stay in memory: the caches hold them, and five launches
+// cost more than three.  (4 x 101 x 314 labels halved, 25 classes, 3.1 MB: 11.2 us there, 12.6 here;
+// 5 x 128 x 529, 26 classes, 8.8 MB: 20.2 and 14.3; below 0.5 MB 7 and 14.)
+constexpr size_t kVoteBytes = (size_t)4 << 20;
 constexpr int kVoteGridX = 256;      // blocks per plane of a launch that may find nothing to do
 
 __global__ __launch_bounds__(kVoteTile * kVoteTile) void vote_boxes_kernel(
@@ -278,7 +282,8 @@ int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, 
   while (shift > 2 && (num_candidates << (2 * shift)) > kVoteCounters) --shift;
   const int* flag = nullptr;
   if (channels == 1 && out_height < 0xffff && out_width < 0xffff && tiles <= kVoteTiles &&
-      batch <= 65535 && (num_candidates << (2 * shift)) <= kVoteCounters &&
+      need * (size_t)batch >= kVoteBytes && batch <= 65535 &&
+      (num_candidates << (2 * shift)) <= kVoteCounters &&
       tiles * sizeof(ushort4) <= need * (size_t)per_pass && (uintptr_t)sample_map % 16 == 0 &&
       workspace_bytes >= need * (size_t)per_pass + kVoteFlagBytes) {
     ushort4* boxes = static_cast<ushort4*>(workspace);

@@ -35,19 +35,30 @@ def _coherent(ih, iw, oh, ow):
 # and without remainders, one pixel, one cell, each square's last number of classes and the next
 SIZES = [(1, 1, 1, 1, 1, 1), (3, 33, 47, 16, 23, 13), (2, 64, 96, 32, 48, 16), (1, 50, 70, 25, 35, 17),
          (2, 48, 80, 17, 33, 64), (1, 40, 64, 20, 31, 65), (1, 32, 32, 9, 7, 256),
-         (1, 32, 32, 9, 7, 257), (1, 20, 30, 60, 90, 5), (2, 128, 100, 1, 1, 3)]
+         (1, 32, 32, 9, 7, 257), (1, 20, 30, 60, 90, 5), (2, 48, 40, 1, 1, 256)]
 
 
+def _hist(oh, ow, nc):
+    return (4 * oh * ow * nc + 255) // 256 * 256
+
+
+def _enough(oh, ow, nc):
+    """Batch elements from which a call's histograms (4 MB) are kept in LDS."""
+    return -(-(4 << 20) // _hist(oh, ow, nc))
+
+
+@pytest.mark.parametrize("few", [False, True], ids=["lds", "histogram"])
 @pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
-def test_coherent_maps(oracle, tc):
+def test_coherent_maps(oracle, tc, few):
     B, ih, iw, oh, ow, nc = tc
+    B = B if few else _enough(oh, ow, nc)
     rng = np.random.default_rng(sum(tc))
     labels = rng.integers(-1, nc + 1, (B, 1, ih, iw))   # some outside [0, classes)
     vmap = _coherent(ih, iw, oh, ow)
     want = oracle.voting_resample_to_map(labels, vmap, oh, ow, nc)
     assert np.array_equal(_call(labels, vmap, oh, ow, nc), want)
     # the least workspace (histogram, no flag), and one with room for the flag but not all elements
-    hist = (4 * oh * ow * nc + 255) // 256 * 256
+    hist = _hist(oh, ow, nc)
     for ws in (hist, hist + 256):
         assert np.array_equal(_call(labels, vmap, oh, ow, nc, ws), want)
 
@@ -55,7 +66,8 @@ def test_coherent_maps(oracle, tc):
 @pytest.mark.parametrize("nc", [4, 40])
 @pytest.mark.parametrize("kind", ["scrambled", "one cell", "two halves"])
 def test_maps_that_raise_the_flag(oracle, kind, nc):
-    B, ih, iw, oh, ow = 2, 160, 208, 40, 52
+    ih, iw, oh, ow = 160, 208, 40, 52
+    B = _enough(oh, ow, nc)
     rng = np.random.default_rng(nc)
     labels = rng.integers(0, nc, (B, 1, ih, iw))
     vmap = _coherent(ih, iw, oh, ow)
