@@ -76,9 +76,9 @@ WwGrid ww_grid(const ConvGeom& g, int tiles, bool big) {
 
 bool window_wgrad_big_supported(const ConvGeom& g, int mm) {
   (void)mm;   // every matrix arithmetic
-  // (32-bit byte offsets over 32 planes, of the image and of the pixel-side tensor)
+  // (32-bit byte offsets over 32 planes of the image)
   return planned_wgrad_supported(g) && g.K >= 1 && g.K <= 10 && g.Cp >= 1 &&
-         (int64_t)g.H * g.W <= ((int64_t)1 << 24) && g.M <= (1 << 24);
+         (int64_t)g.H * g.W <= ((int64_t)1 << 24);
 }
 
 bool window_wgrad_supported(const ConvGeom& g, int mm) {

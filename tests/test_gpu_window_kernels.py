@@ -116,3 +116,40 @@ def test_more_than_two_gigabytes_of_weights(tile_kernels, mode):
     want = (x.flatten(2)[0][:, at].double() * row.double()[:, None, None, :]).sum((0, 3))
     assert torch.equal(y[0, -1].double(), want)
     assert not y[0, :-1].any()
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", [(66, 4096, 4104, 2, 1), (66, 4097, 4099, 1, 0), (40, 4096, 4104, 3, 0)],
+                         ids=lambda t: "x".join(map(str, t)))
+def test_weight_gradient_of_more_than_2_24_pixels(oracle, tile_kernels, tc, mode):
+    """Planes of which 32 are more than 2^31 bytes; 16-byte reads and, on an odd width, single ones;
+    the window kernels take such a layer (they leave their sums in a workspace with room for them)."""
+    import _spherical_distortion_ext._ops as ops
+    from _spherical_distortion_ext import _capi
+    Cout, OH, OW, K, interp = tc
+    Cin, H, W = 8, 64, 96
+    assert OH * OW > 2 ** 24
+    rng = np.random.default_rng(sum(tc))
+    k = np.arange(K)
+    y, x = torch.arange(OH, device=DEV) * H // OH, torch.arange(OW, device=DEV) * W // OW
+    m = torch.stack([x.expand(OH, OW)[..., None] + torch.from_numpy(k % 2 * 0.5).to(DEV),
+                     y[:, None].expand(OH, OW)[..., None] - torch.from_numpy(k // 2 * 0.5).to(DEV)], -1)
+    m = m.float().contiguous()
+    # gradients at some pixels, the corners among them: few enough for the oracle, and the sums exact
+    at = np.unique(np.concatenate([rng.integers(0, OH * OW, 4000),
+                                   [0, OW - 1, (OH - 1) * OW, OH * OW - 1, 2 ** 24 - 1, 2 ** 24]]))
+    values = rng.integers(-4, 5, (1, Cout, at.size)).astype(np.float32)
+    g = torch.zeros(1, Cout, OH, OW, device=DEV)
+    tat = torch.from_numpy(at).to(DEV)
+    g.view(1, Cout, -1)[..., tat] = torch.from_numpy(values).to(DEV)
+    img = rng.integers(-4, 5, (1, Cin, H, W)).astype(np.float32)
+    w = np.zeros((Cout, Cin, K), np.float32)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    with ops.conv_compute(mode):
+        _, gw, gb = ops.ops.mapped_conv_backward_select(g, m, None, t(img), t(w), K, interp, False,
+                                                        False, True)
+    few = m.view(1, -1, K, 2)[:, tat].cpu().numpy()
+    _, want, wb = oracle.mapped_conv_backward(values[:, :, None], few, img, w,
+                                              np.zeros(Cout, np.float32), K, interp, None)
+    assert np.array_equal(gw.cpu().numpy(), want)
+    assert np.array_equal(gb.cpu().numpy(), wb)

@@ -328,3 +328,12 @@ def test_first_layers_of_any_picture_size_read_no_plan():
                 channels = (cout, cin) if transposed else (cin, cout)
                 assert lib.sdk_mapped_conv_plan_parts(1, *channels, h, w, h, w, 9, 0, 1,
                                                       _capi.SDK_F32, 0, transposed, 1, 1, 1) == 0
+
+
+def test_window_weight_gradient_has_no_limit_of_output_pixels():
+    """Past 2^24 output pixels too a call reserves what the window kernels leave their sums in."""
+    from _spherical_distortion_ext import _capi
+    for cout, compute in ((96, 0), (96, 1), (96, 3), (40, 0)):
+        at_limit, past = (_capi.load().sdk_mapped_conv_workspace_bytes(
+            1, 32, cout, 512, 512, 4096, w, 9, 0, 1, _capi.SDK_F32, compute) for w in (4096, 4097))
+        assert past >= at_limit > 0
