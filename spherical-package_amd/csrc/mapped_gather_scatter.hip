@@ -471,7 +471,10 @@ __global__ __launch_bounds__(kBlock) void uv_scatter_kernel(
 // step of the scan is a vector instruction and no shuffle, and its last lane adds to LDS.  26
 // planes, 80 textures of 64 x 64, 512 x 1024 pixels: 131 -> 55 us (compare-and-swap adds and
 // shuffles across the wave before; 80 with the textures in their own order, the largest buckets
-// last; 290 without the scan; without the adds 43).
+// last; 290 without the scan; without the adds 43).  Where the buckets are longer than a round the
+// workgroups take them by falling size, an order that is made once with them: chosen by every
+// workgroup anew it cost as much as the sums of short buckets (128 planes, 320 textures of 32 x 32,
+// 512 x 1024: 588 -> 331 us, 64 planes, 320 of 80 x 80, 768 x 1536: 697 -> 395; 26 planes as above 47 -> 45).
 // Textures whose doubles do not fit kUvLdsBytes keep compare-and-swap adds (ACC = T).
 // ---------------------------------------------------------------------------
 constexpr int kUvMaxTextures = 1 << 20;
@@ -495,11 +498,20 @@ __global__ __launch_bounds__(kBlock) void uv_count_kernel(const int64_t* __restr
 // Exclusive scan in bucket order (texture-major, copy-minor): cursor[r][t] = first slot of part
 // r of texture t; offset[t] = first slot of texture t, offset[NT] = number of pixels listed.
 // One workgroup; every thread owns a contiguous strip of the NT * R counters, so the counters
-// are read in one sweep of independent loads.
-__global__ __launch_bounds__(kBlock) void uv_scan_kernel(const int* __restrict__ count, int NT,
-                                                         int R, int* __restrict__ offset,
-                                                         int* __restrict__ cursor) {
+// are read in one sweep of independent loads.  ordered: the first NT counters then make room for
+// the textures by falling bucket size, in classes of a quarter of a power of two (the order within
+// a class is that of the atomics).
+constexpr int kUvClasses = 128;
+__device__ __forceinline__ int uv_size_class(int size) {   // 0: the largest
+  const int top = 31 - __clz(max(size, 1));
+  return kUvClasses - 1 - (4 * top + (top >= 2 ? (size >> (top - 2)) & 3 : 0));
+}
+
+__global__ __launch_bounds__(kBlock) void uv_scan_kernel(int* __restrict__ count, int NT, int R,
+                                                         int* __restrict__ offset,
+                                                         int* __restrict__ cursor, int ordered) {
   __shared__ int wave_total[kBlock / 64];
+  __shared__ int place[kUvClasses], first_of[kUvClasses];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = NT * R;
   const int strip = (n + kBlock - 1) / kBlock;
@@ -522,6 +534,20 @@ __global__ __launch_bounds__(kBlock) void uv_scan_kernel(const int* __restrict__
     run += count[(size_t)r * NT + t];
   }
   if (threadIdx.x == kBlock - 1) offset[NT] = run;
+  if (!ordered) return;
+  if (threadIdx.x < kUvClasses) place[threadIdx.x] = 0;
+  __syncthreads();
+  for (int t = threadIdx.x; t < NT; t += kBlock)
+    atomicAdd(&place[uv_size_class(offset[t + 1] - offset[t])], 1);
+  __syncthreads();
+  if (threadIdx.x < kUvClasses) {
+    int before = 0;
+    for (int c = 0; c < (int)threadIdx.x; ++c) before += place[c];
+    first_of[threadIdx.x] = before;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < NT; t += kBlock)
+    count[atomicAdd(&first_of[uv_size_class(offset[t + 1] - offset[t])], 1)] = t;
 }
 
 __global__ __launch_bounds__(kBlock) void uv_fill_kernel(const int64_t* __restrict__ quad, int NT,
@@ -546,45 +572,22 @@ __global__ __launch_bounds__(kBlock) void uv_fill_kernel(const int64_t* __restri
 
 constexpr int kUvBlock = 1024;   // 16 waves: a long bucket (a polar face) takes few rounds
 
-
 template <typename T, int INTERP, int PL, typename ACC>
 __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
     const T* __restrict__ in, const T* __restrict__ uv, const int* __restrict__ offset,
-    const int* __restrict__ list, T* __restrict__ textures, int planes, int NT, int TH, int TW,
-    int MP, int ordered) {
+    const int* __restrict__ list, const int* __restrict__ order, T* __restrict__ textures, int planes,
+    int NT, int TH, int TW, int MP) {
   extern __shared__ __align__(16) unsigned char uv_lds[];
   constexpr bool DIRECT = std::is_same<ACC, double>::value;   // native adds
   ACC* acc = reinterpret_cast<ACC*>(uv_lds);         // [PL][TH * TW]
-  const int THW = TH * TW;
-  // ordered (NT <= kUvBlock): longest buckets first, all their plane chunks: a polar texture's takes
-  // three times as long as the others', and started last it runs alone at the end.  The textures of
-  // longer buckets are counted by kUvBlock / NT threads for each texture (by one, 320 textures cost a
-  // workgroup 15 us).
+  const int THW = TH * TW, threads = blockDim.x;
+  // order (optional): longest buckets first, all their plane chunks: a polar texture's takes three
+  // times as long as the others', and started last it runs alone at the end.
   int t = blockIdx.x, chunk = blockIdx.y;
-  if (ordered) {
-    __shared__ int size[kUvBlock], above[kUvBlock];
-    __shared__ int chosen;
-    const int id = blockIdx.y * gridDim.x + blockIdx.x, rank = id / (int)gridDim.y;
+  if (order != nullptr) {
+    const int id = blockIdx.y * gridDim.x + blockIdx.x;
+    t = order[id / (int)gridDim.y];
     chunk = id % (int)gridDim.y;
-    const int i = threadIdx.x % NT, part = threadIdx.x / NT, parts = kUvBlock / NT;
-    if (part == 0) {
-      size[i] = offset[i + 1] - offset[i];
-      above[i] = 0;
-    }
-    __syncthreads();
-    if (part < parts) {
-      const int per = (NT + parts - 1) / parts, end = min((part + 1) * per, NT);
-      const int mine = size[i];
-      int n = 0;
-#pragma unroll 4
-      for (int k = part * per; k < end; ++k)
-        n += (size[k] > mine || (size[k] == mine && k < i)) ? 1 : 0;
-      atomicAdd(&above[i], n);
-    }
-    __syncthreads();
-    if (part == 0 && above[i] == rank) chosen = i;
-    __syncthreads();
-    t = chosen;
   }
   const int plane0 = chunk * PL;
   const int np = min(PL, planes - plane0);
@@ -593,7 +596,7 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
   const int lo0 = offset[t], hi0 = offset[t + 1];
   const int per = (hi0 - lo0 + (int)gridDim.z - 1) / (int)gridDim.z;
   const int lo = lo0 + (int)blockIdx.z * per, hi = min(hi0, lo + per);
-  for (int i = threadIdx.x; i < PL * THW; i += kUvBlock) acc[i] = ACC(0);
+  for (int i = threadIdx.x; i < PL * THW; i += threads) acc[i] = ACC(0);
   __syncthreads();
   constexpr int N = PointTaps<T, INTERP>::N;
   // this round's pixel, point and values are loaded during the round before
@@ -603,8 +606,8 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
   T val[PL];
 #pragma unroll
   for (int j = 0; j < PL; ++j) val[j] = in[(size_t)(plane0 + (j < np ? j : 0)) * MP + pix];
-  int pix_next = e + kUvBlock < hi ? list[e + kUvBlock] : 0;
-  for (int base = lo; base < hi; base += kUvBlock) {   // uniform trip count over the workgroup
+  int pix_next = e + threads < hi ? list[e + threads] : 0;
+  for (int base = lo; base < hi; base += threads) {   // uniform trip count over the workgroup
     const bool live = e < hi;
     PointTaps<T, INTERP> taps;
     taps.set(pu, pv, TH, TW);
@@ -612,13 +615,13 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
 #pragma unroll
     for (int j = 0; j < PL; ++j) cur[j] = (live && j < np) ? val[j] : T(0);
     // next round's loads
-    e += kUvBlock;
+    e += threads;
     pix = pix_next;
     pu = uv[(size_t)pix * 2];
     pv = uv[(size_t)pix * 2 + 1];
 #pragma unroll
     for (int j = 0; j < PL; ++j) val[j] = in[(size_t)(plane0 + (j < np ? j : 0)) * MP + pix];
-    pix_next = e + kUvBlock < hi ? list[e + kUvBlock] : 0;
+    pix_next = e + threads < hi ? list[e + threads] : 0;
     // lanes whose first tap is the same texel form a run: all their taps coincide
     const int ky = live ? taps.ty[0] : INT_MIN, kx = live ? taps.tx[0] : (int)threadIdx.x;
     const int by = row_below<1>(ky), bx = row_below<1>(kx);
@@ -643,7 +646,7 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
   }
   __syncthreads();
   const size_t stride = (size_t)NT * THW;
-  for (int i = threadIdx.x; i < THW; i += kUvBlock) {
+  for (int i = threadIdx.x; i < THW; i += threads) {
 #pragma unroll
     for (int j = 0; j < PL; ++j) {
       if (j < np) {
@@ -1599,7 +1602,7 @@ static int uv_counter_copies(int64_t NT) {
   return r;
 }
 
-// Workspace of the adjoint by texture: count [R][NT] | offset (NT + 1) | cursor [R][NT] |
+// Workspace of the adjoint by texture: count [R][NT], then order [NT] | offset (NT + 1) | cursor [R][NT] |
 // bucket (MP pixels).
 static size_t uv_layout(int64_t NT, int64_t MP, size_t (&off)[4]) {
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -1614,6 +1617,9 @@ static size_t uv_layout(int64_t NT, int64_t MP, size_t (&off)[4]) {
 static bool uv_by_texture_fits(int64_t NT, int64_t THW, size_t esz) {
   return NT <= kUvMaxTextures && THW * (int64_t)esz <= kUvLdsBytes;
 }
+
+// Buckets of less than a round of the workgroup are as good in any order.
+static bool uv_ordered(int64_t NT, int64_t MP) { return MP >= NT * kUvBlock; }
 
 // The image pixels bucketed by texture (a function of quad_idx alone) into `workspace`
 // (uv_layout bytes): offset[t] .. offset[t + 1] - 1 of `list` are texture t's pixels.
@@ -1631,8 +1637,8 @@ static int build_uv_buckets(const int64_t* quad, void* workspace, int NT, int MP
   const dim3 pixel_grid((unsigned)ceil_div(MP, kBlock));
   const int copies = uv_counter_copies(NT);
   launch(uv_count_kernel, pixel_grid, dim3(kBlock), stream, quad, NT, MP, copies, count);
-  launch(uv_scan_kernel, dim3(1), dim3(kBlock), stream, (const int*)count, NT, copies, offset,
-         cursor);
+  launch(uv_scan_kernel, dim3(1), dim3(kBlock), stream, count, NT, copies, offset, cursor,
+         uv_ordered(NT, MP) ? 1 : 0);
   launch(uv_fill_kernel, pixel_grid, dim3(kBlock), stream, quad, NT, MP, copies, cursor, list);
   SDK_LAUNCH_CHECK("resample_to_uv_maps(bucket)");
   return SDK_OK;
@@ -1673,15 +1679,17 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
       if (rc != SDK_OK) return rc;
     }
     const dim3 grid((unsigned)NT, (unsigned)ceil_div(planes, pl), (unsigned)split);
-    // buckets of less than a round of the workgroup are as good in any order, and choosing costs as
-    // much as they do (12 planes, 320 textures of 43 x 43, 65 x 130 pixels: 24 us a pass, 69 where
-    // every workgroup chose)
-    const int ordered = NT <= kUvBlock && MP >= (int64_t)NT * kUvBlock ? 1 : 0;
+    // (short buckets of one large texture: three workgroups of 512 share a CU where two of 1024 would.
+    // 64 planes, 320 textures of 80 x 80, 256 x 512 pixels: 207 -> 178 us)
+    const bool halves = !uv_ordered(NT, MP) && pl == 1 && groups >= 1536 &&
+                        3 * THW * sum <= (size_t)150 * 1024;
+    const int threads = halves ? kUvBlock / 2 : kUvBlock;
+    const int* order = uv_ordered(NT, MP) ? reinterpret_cast<const int*>(ws + off[0]) : nullptr;
 #define UVS(PLv, ACCv)                                                                        \
   SDK_DISPATCH_INTERP_ONLY(interp, (uv_texture_scatter_kernel<T, INTERP, PLv, ACCv>           \
-                                    <<<grid, dim3(kUvBlock), (size_t)PLv * THW * sum, stream>>>( \
-                                        in, uv, (const int*)offset, (const int*)list, textures, \
-                                        (int)planes, NT, TH, TW, MP, ordered)))
+                                    <<<grid, dim3(threads), (size_t)PLv * THW * sum, stream>>>( \
+                                        in, uv, (const int*)offset, (const int*)list, order,  \
+                                        textures, (int)planes, NT, TH, TW, MP)))
     if (direct) {
       if (pl == 4) UVS(4, double); else if (pl == 2) UVS(2, double); else UVS(1, double);
     } else {   // (such a texture takes half of kUvLdsBytes or more)

@@ -22,6 +22,10 @@ def ops():
 SIZES = [(1, 1, 1, 1, 1, 1, 1), (2, 3, 5, 8, 9, 33, 47), (1, 13, 80, 16, 16, 60, 128),
          (1, 5, 1030, 4, 3, 40, 77), (1, 2, 3, 64, 128, 50, 90), (1, 3, 2, 91, 91, 64, 64),
          (3, 2, 1, 16, 16, 100, 120), (1, 3, 33, 5, 6, 180, 200)]
+# by falling bucket size in chunks of two and of four planes, the last one ragged, and with more textures
+# than threads of a workgroup; short buckets of large textures (workgroups of 512)
+SIZES += [(1, 103, 20, 8, 8, 150, 160), (5, 41, 20, 8, 8, 150, 160), (1, 3, 1030, 4, 3, 1024, 1040),
+          (1, 5, 320, 65, 70, 100, 110)]
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
