@@ -2434,10 +2434,11 @@ __global__ __launch_bounds__(kBlock) void unpool_lists_kernel(
 // keeps the first kUnpoolKept entries of its list in registers over the passes.  A workgroup whose
 // sources span too much, or one of whose lists is long, reads them from memory as above.  Same
 // products in the same order as there: the same bits.  4 x 48 planes of 190 x 378 from 95 x 189:
-// 60 -> 34 us, 8 x 64 of 256 x 512 285 -> 119 (bound by the requests of 4-byte reads, one per entry and
+// 60 -> 34 us, 8 x 64 of 256 x 512 285 -> 118 (bound by the requests of 4-byte reads, one per entry and
 // plane, before).  Not for maps as dense as their image, whose spans touch five times their own
 // length in pooled pixels and whose lists are longer than what is kept (192 planes of 256 x 512, stride 1: 541 us
-// from memory, 1058 so), nor below 64 planes (32 of 190 x 378: 14 against 21).
+// from memory, 1058 so), nor below 64 planes (us from memory and so, stride 2: 190 x 378, 32 planes 13 and 19, 48
+// 18 and 19.5, 64 22 and 19; 512 x 1024, 32 69 and 98, 48 102 and 102, 64 134 and 69).
 constexpr int kUnpoolSpan = 512;
 constexpr int kUnpoolKept = 8;
 constexpr int kUnpoolLdsBytes = 40 * 1024;   // four workgroups per CU
@@ -2488,20 +2489,78 @@ __device__ __forceinline__ void unpool_from_lds(
   }
 }
 
-// grid.x = 8 * blocks * ceil(chunks / 8): an XCD takes whole plane chunks, whose pooled rows its L2
-// then keeps for the neighbouring spans.
+// From memory, four planes at a time, the kept entries in registers over the passes: for spans whose
+// sources lie far apart.  (2 x 256 planes of 256 x 512, stride 2, the pooled grid transposed: 1046 us
+// with the lists read again for each four planes, 784 now, 933 by eight planes in unpool_lists_kernel;
+// in random order 1081, 967, 864, of 192 planes 320, 261, 330.)
+__device__ __forceinline__ void unpool_scattered(
+    const float* __restrict__ gout, const int* __restrict__ src, const float* __restrict__ co,
+    float* __restrict__ gin, int u, int beg, int n, int most, int HW, int M, int p_begin, int p_end,
+    float K) {
+  constexpr int PC = 4;
+  int at[kUnpoolKept];
+  float c[kUnpoolKept];
+#pragma unroll
+  for (int i = 0; i < kUnpoolKept; ++i) {
+    at[i] = i < n ? src[beg + i] : 0;
+    c[i] = i < n ? co[beg + i] : 0.0f;
+  }
+  for (int p = p_begin; p < p_end; p += PC) {
+    const float* g0 = gout + (size_t)p * M;
+    const int np = min(PC, p_end - p);
+    float acc[PC] = {};
+    float v[4][PC];
+#pragma unroll
+    for (int q = 0; q < kUnpoolKept; q += 4) {
+      if (q >= most) break;   // (uniform over the workgroup)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) v[i][j] = g0[(size_t)(j < np ? j : 0) * M + at[q + i]];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) acc[j] += q + i < n ? c[q + i] * v[i][j] : 0.0f;
+    }
+    for (int e = kUnpoolKept; e < n; e += 4) {
+      int m[4];
+      float w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int x = beg + min(e + i, n - 1);
+        m[i] = src[x];
+        w[i] = co[x];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) v[i][j] = g0[(size_t)(j < np ? j : 0) * M + m[i]];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < PC; ++j) acc[j] += e + i < n ? w[i] * v[i][j] : 0.0f;
+    }
+    if (u < HW) {
+#pragma unroll
+      for (int j = 0; j < PC; ++j)
+        if (j < np) gin[(size_t)(p + j) * HW + u] = acc[j] / K;
+    }
+  }
+}
+
+// Workgroup: a span of elements in `per` planes.  An XCD takes an eighth of the spans of all plane
+// chunks in turn, so whole chunks or parts of one, whose pooled rows its L2 then keeps for the
+// neighbouring spans.
 __global__ __launch_bounds__(kUnpoolSpan) void unpool_spans_kernel(
     const float* __restrict__ gout, const int* __restrict__ offset, const int* __restrict__ count,
     const int* __restrict__ src, const float* __restrict__ co, float* __restrict__ gin, int HW,
-    int M, int planes, int blocks, int chunks, float K) {
+    int M, int planes, int blocks, int per, float K) {
   __shared__ __align__(16) float lds[kUnpoolLdsBytes / 4];
   __shared__ int s_first, s_last, s_most;
-  const int within = blockIdx.x >> 3;
-  const int chunk = (within / blocks) * 8 + (blockIdx.x & 7);
-  if (chunk >= chunks) return;
-  const int p_begin = (int)((int64_t)chunk * planes / chunks);
-  const int p_end = (int)((int64_t)(chunk + 1) * planes / chunks);
-  const int u = (within % blocks) * kUnpoolSpan + threadIdx.x;
+  const int unit = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int p_begin = unit / blocks * per, p_end = min(p_begin + per, planes);
+  if (p_begin >= planes) return;
+  const int u = (unit % blocks) * kUnpoolSpan + threadIdx.x;
   const int beg = u < HW ? offset[u] : 0, n = u < HW ? count[u] : 0;
   if (threadIdx.x == 0) {
     s_first = INT_MAX;
@@ -2525,7 +2584,7 @@ __global__ __launch_bounds__(kUnpoolSpan) void unpool_spans_kernel(
   __syncthreads();
   const int m0 = s_last < 0 ? 0 : s_first, span = s_last < 0 ? 1 : s_last - s_first + 1;
   const int longest = s_most;
-  if (longest <= kUnpoolLong && span <= kUnpoolLdsBytes / 8) {
+  if (__builtin_expect(longest <= kUnpoolLong && span <= kUnpoolLdsBytes / 8, 1)) {
     if (span <= kUnpoolLdsBytes / 32)
       unpool_from_lds<8>(gout, src, co, gin, lds, u, beg, n, longest, m0, span, HW, M, p_begin,
                          p_end, K);
@@ -2535,6 +2594,8 @@ __global__ __launch_bounds__(kUnpoolSpan) void unpool_spans_kernel(
     else
       unpool_from_lds<2>(gout, src, co, gin, lds, u, beg, n, longest, m0, span, HW, M, p_begin,
                          p_end, K);
+  } else if (longest <= kUnpoolLong) {
+    unpool_scattered(gout, src, co, gin, u, beg, n, longest, HW, M, p_begin, p_end, K);
   } else {
     for (int p = p_begin; p < p_end; p += 4)
       unpool_from_memory<4>(gout, src, co, gin, u, beg, n, HW, M, p, min(4, p_end - p), K);
@@ -2632,17 +2693,25 @@ static int launch_unpool_lists(const float* gout, float* gin, const void* lists,
   const Col2imLists l = col2im_lists_at(const_cast<void*>(lists), H, W, M, K, P, interp);
   const int HW = H * W;
   // From LDS where the map has half the image's pixels or fewer and there are planes to take the staging
-  // and the lists for (both sides at unpool_spans_kernel); chunks of planes in eighths, about four
-  // workgroups per CU.
+  // and the lists for (both sides at unpool_spans_kernel).
   const int64_t spans = ceil_div(HW, kUnpoolSpan);
   if (planes >= 64 && 2 * (int64_t)M <= HW) {
-    int64_t chunks = std::max<int64_t>(8, std::min<int64_t>(planes / 16, 1024 / spans) / 8 * 8);
-    chunks = std::min<int64_t>(chunks, planes);
-    const int64_t grid = 8 * spans * ceil_div(chunks, 8);
+    // Planes of a workgroup.  Where all workgroups are at work at once (three per CU) the longest one
+    // counts: one pass of eight planes, or equal shares.  Else what they do together: whole passes, and
+    // two at least where there are workgroups enough (64 to 512 planes of 64 x 128 to 512 x 1024,
+    // strides 2 and 4).
+    const int64_t at_once = 768;
+    const int64_t chunks = std::max<int64_t>(8, std::min<int64_t>(planes / 16, 1024 / spans) / 8 * 8);
+    int64_t per = 8;
+    if (spans * ceil_div(planes, 8) > at_once)
+      per = spans * chunks <= at_once
+                ? ceil_div(planes, chunks)
+                : std::max<int64_t>(spans >= 256 ? 16 : 8, (planes / chunks + 5) / 8 * 8);
+    const int64_t grid = 8 * ceil_div(spans * ceil_div(planes, per), 8);
     if (grid < ((int64_t)1 << 31)) {
       launch(unpool_spans_kernel, dim3((unsigned)grid), dim3(kUnpoolSpan), stream, gout,
              (const int*)l.offset, (const int*)l.count, (const int*)l.src, (const float*)l.co, gin,
-             HW, M, (int)planes, (int)spans, (int)chunks, (float)K);
+             HW, M, (int)planes, (int)spans, (int)per, (float)K);
       SDK_LAUNCH_CHECK("mapped_avg_unpool(lists, spans)");
       return SDK_OK;
     }

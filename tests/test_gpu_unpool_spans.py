@@ -17,6 +17,12 @@ SIZES = [
     (3, 43, 40, 1000, 20, 500, "strided"), (1, 67, 16, 2400, 8, 1200, "strided"),
     (4, 48, 48, 100, 24, 50, "repeated"), (1, 70, 64, 120, 32, 60, "scrambled"),
     (2, 40, 64, 120, 32, 60, "one spot"), (1, 64, 80, 6000, 40, 3000, "scrambled"),
+    # lists of more than the kept entries in a span that goes to memory
+    (1, 64, 80, 6000, 40, 3000, "repeated, scrambled"),
+    # planes of a workgroup: equal shares of all that are at work at once (13 planes), whole passes of
+    # eight, of sixteen, and two passes at least where spans are many
+    (1, 104, 128, 256, 64, 128, "strided"), (1, 67, 160, 320, 80, 160, "strided"),
+    (1, 88, 160, 320, 80, 160, "strided"), (1, 67, 256, 513, 128, 256, "strided"),
 ]
 
 
@@ -29,11 +35,11 @@ def test_against_the_oracle(oracle, tc, interp):
     y, x, k = np.meshgrid(np.arange(OH), np.arange(OW), np.arange(4), indexing="ij")
     m = np.stack([x * 2.0 + k % 2, y * 2.0 + k // 2], -1)
     m += rng.integers(-1, 2, m.shape) * 0.5
-    if kind == "repeated":      # a dozen pooled pixels on each element
+    if kind.startswith("repeated"):   # a dozen pooled pixels on each element
         m[..., 0] = m[..., 0] // 12 * 12 + rng.integers(0, 2, m.shape[:-1])
-    elif kind == "scrambled":
+    if kind.endswith("scrambled"):
         m = rng.permutation(m.reshape(-1, 2)).reshape(m.shape)
-    elif kind == "one spot":    # a list of hundreds of entries
+    if kind == "one spot":      # a list of hundreds of entries
         m[rng.random((OH, OW)) < 0.3] = (7.5, 3.0)
     m = m.astype(np.float32)
     g = rng.integers(-4, 5, (B, C, OH, OW)).astype(np.float32)
