@@ -213,8 +213,9 @@ int sdk_resample_to_uv_maps_planned(const void* input, const int64_t* quad_idx, 
  *  src/cpp/voting_resample_layer.cpp:8-37).
  * workspace (required): at least sdk_voting_resample_workspace_bytes() bytes, 16-byte aligned:
  * the vote histogram of one batch element, 4 bytes per (channel, output pixel, candidate), rounded
- * up to 256, and 256 bytes more (without which a call takes the histogram where LDS would do); a
- * workspace n times that size lets n batch elements be processed per pass.
+ * up to 256, and, with one channel, a sixteenth more or the 66 KB or so that counting in LDS needs
+ * (accepted without them: then the votes are counted in memory alone); a workspace n times that size
+ * lets n batch elements be processed per pass.
  * ------------------------------------------------------------------------- */
 size_t sdk_voting_resample_workspace_bytes(int64_t channels, int64_t out_height,
                                            int64_t out_width, int64_t num_candidates);

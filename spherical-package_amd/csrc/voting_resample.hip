@@ -25,14 +25,18 @@ constexpr int kVoteBlock = 256;
 // vote_tile_kernel owns a tile of output cells, finds the input tiles whose box meets it, counts
 // their votes in LDS and writes the winners.  Every label is read about once, every histogram
 // counter stays in LDS: 4 x 512 x 1024 labels, 13 classes, halved: clear 12 + votes 35 + argmax 10
-// us (27 MB of counters cleared, added to by atomics and scanned) -> boxes 6 + cells 10.  A cell tile
-// that more than kVoteMeet input tiles vote into says so in a flag, and the histogram kernels, launched
-// behind it on that flag, do the whole pass again; they cost 2 us each where they have nothing
-// to do (57 -> 27 us a call; a scrambled map, which pays for both, 103 -> 114).
-// ---------------------------------------------------------------------------------------------
+// us (27 MB of counters cleared, added to by atomics and scanned) -> boxes 4 + cells 10.  A cell tile
+// that more than kVoteMeet input tiles vote into is crowded: its workgroup clears its counters in memory
+// instead and marks it, and the histogram kernels, launched behind, cast and count the votes of crowded
+// cell tiles alone; they cost 2 us each where there is none.  A call, with the histogram alone, with one
+// flag that had everything done again in memory, and so: 57, 18.5, 16 us; the upper half of the map in
+// random order 81, 88, 65; a pixel in 256 voting for one far cell 65, 98, 69; all of it in random order
+// 103, 113, 111 (60 classes 160, 180, 185: what finding out costs).
 constexpr int kVoteTile = 16;        // input tile side
 constexpr int kVoteMeet = 64;        // input tiles (16384 pixels) a workgroup takes on
+constexpr int kVoteWide = 8;         // ... of which one with a box of more than 16 cell squares is as many
 constexpr int kVoteTiles = 8192;     // input tiles: every workgroup looks through all boxes (64 KB)
+constexpr size_t kVoteBoxBytes = (size_t)kVoteTiles * sizeof(ushort4);
 constexpr int kVoteCounters = 4096;  // LDS counters of a workgroup
 // Histograms of fewer bytes than this in all stay in memory: the caches hold them, and five launches
 // cost more than three.  (4 x 101 x 314 labels halved, 25 classes, 3.1 MB: 11.2 us there, 12.6 here;
@@ -40,26 +44,30 @@ constexpr int kVoteCounters = 4096;  // LDS counters of a workgroup
 constexpr size_t kVoteBytes = (size_t)4 << 20;
 constexpr int kVoteGridX = 256;      // blocks per plane of a launch that may find nothing to do
 
-__global__ __launch_bounds__(kVoteTile * kVoteTile) void vote_boxes_kernel(
+// One wave per input tile, four rows of it a step.
+__global__ __launch_bounds__(kVoteBlock) void vote_boxes_kernel(
     const int64_t* __restrict__ map, ushort4* __restrict__ boxes, int* __restrict__ flag, int IH,
-    int IW, int tiles_x, int OH, int OW) {
-  __shared__ int box[4];
-  const int tid = threadIdx.x;
-  if (blockIdx.x == 0 && tid == 0) *flag = 0;
-  if (tid < 4) box[tid] = tid < 2 ? 0xffff : 0;
-  __syncthreads();
-  const int iy = (blockIdx.x / tiles_x) * kVoteTile + tid / kVoteTile;
-  const int ix = (blockIdx.x % tiles_x) * kVoteTile + tid % kVoteTile;
+    int IW, int tiles, int tiles_x, int OH, int OW) {
+  const int lane = threadIdx.x & 63;
+  const int tile = blockIdx.x * (kVoteBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+  if (tile >= tiles) return;
+  const int ix = (tile % tiles_x) * kVoteTile + lane % kVoteTile;
+  const int iy0 = (tile / tiles_x) * kVoteTile + lane / kVoteTile;
+  longlong2 t[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    t[r] = reinterpret_cast<const longlong2*>(map)[(size_t)min(iy0 + 4 * r, IH - 1) * IW +
+                                                   min(ix, IW - 1)];
   int x0 = 0xffff, y0 = 0xffff, x1 = 0, y1 = 0;   // (x1, y1: one past the last)
-  if (iy < IH && ix < IW) {
-    const longlong2 t = reinterpret_cast<const longlong2*>(map)[(size_t)iy * IW + ix];
-    if (t.x >= 0 && t.x < OW && t.y >= 0 && t.y < OH) {
-      x0 = (int)t.x;
-      y0 = (int)t.y;
-      x1 = x0 + 1;
-      y1 = y0 + 1;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)   // (past the edge: the last pixel again)
+    if (t[r].x >= 0 && t[r].x < OW && t[r].y >= 0 && t[r].y < OH) {
+      x0 = min(x0, (int)t[r].x);
+      y0 = min(y0, (int)t[r].y);
+      x1 = max(x1, (int)t[r].x + 1);
+      y1 = max(y1, (int)t[r].y + 1);
     }
-  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     x0 = min(x0, __shfl_xor(x0, o));
@@ -67,51 +75,65 @@ __global__ __launch_bounds__(kVoteTile * kVoteTile) void vote_boxes_kernel(
     x1 = max(x1, __shfl_xor(x1, o));
     y1 = max(y1, __shfl_xor(y1, o));
   }
-  if ((tid & 63) == 0) {
-    atomicMin(&box[0], x0);
-    atomicMin(&box[1], y0);
-    atomicMax(&box[2], x1);
-    atomicMax(&box[3], y1);
-  }
-  __syncthreads();
-  if (tid == 0)
-    boxes[blockIdx.x] = make_ushort4((unsigned short)box[0], (unsigned short)box[1],
-                                     (unsigned short)box[2], (unsigned short)box[3]);
+  if (lane == 0)
+    boxes[tile] = make_ushort4((unsigned short)x0, (unsigned short)y0, (unsigned short)x1,
+                               (unsigned short)y1);
 }
 
 // Workgroup: 2^cell_shift x 2^cell_shift output cells (at most one a thread) of batch element
-// blockIdx.y.
+// blockIdx.y of this pass.  crowded: a mark for each tile of cells, written by the first element's workgroups;
+// hist: the elements' histograms, element_stride counters apart.
 __global__ __launch_bounds__(kVoteBlock) void vote_tile_kernel(
     const int64_t* __restrict__ labels, const int64_t* __restrict__ map,
-    const ushort4* __restrict__ boxes, int* __restrict__ flag, int64_t* __restrict__ out, int IH,
-    int IW, int tiles, int tiles_x, int OH, int OW, int cells_x, int cell_shift, int candidates) {
+    const ushort4* __restrict__ boxes, int* __restrict__ flag, unsigned char* __restrict__ crowded,
+    unsigned* __restrict__ hist, size_t element_stride, int64_t* __restrict__ out, int IH, int IW,
+    int tiles, int tiles_x, int OH, int OW, int cells_x, int cell_shift, int candidates) {
   __shared__ unsigned votes[kVoteCounters];
   __shared__ int meet[kVoteMeet];
-  __shared__ int n_meet;
+  __shared__ int n_meet, n_wide;
   const int tid = threadIdx.x, side = 1 << cell_shift, cells = side << cell_shift;
   const int ox0 = (blockIdx.x % cells_x) << cell_shift, oy0 = (blockIdx.x / cells_x) << cell_shift;
   const int ox1 = min(ox0 + side, OW), oy1 = min(oy0 + side, OH);
-  if (tid == 0) n_meet = 0;
-  for (int i = tid; i < cells * candidates; i += kVoteBlock) votes[i] = 0;
+  if (tid == 0) n_meet = n_wide = 0;
   __syncthreads();
-  for (int t0 = tid; t0 < tiles; t0 += 8 * kVoteBlock) {   // (eight reads in flight)
-    ushort4 b[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) b[u] = boxes[min(t0 + u * kVoteBlock, tiles - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int t = t0 + u * kVoteBlock;
-      if (t < tiles && b[u].x < ox0 + side && b[u].z > ox0 && b[u].y < oy0 + side && b[u].w > oy0) {
-        const int at = atomicAdd(&n_meet, 1);
-        if (at < kVoteMeet) meet[at] = t;
-      }
+  auto look = [&](const ushort4& b, int t) {
+    const bool meets =
+        t < tiles && b.x < ox0 + side && b.z > ox0 && b.y < oy0 + side && b.w > oy0;
+    const unsigned long long all = __ballot(meets);
+    if (all == 0) return;
+    const unsigned long long wide = __ballot(meets && (b.z - b.x) * (b.w - b.y) > 16 * cells);
+    int at = 0;
+    if ((tid & 63) == 0) {
+      at = atomicAdd(&n_meet, __popcll(all));
+      if (wide != 0) atomicAdd(&n_wide, __popcll(wide));
     }
+    at = __builtin_amdgcn_readfirstlane(at) + __popcll(all & ((1ull << (tid & 63)) - 1));
+    if (meets && at < kVoteMeet) meet[at] = t;
+  };
+  bool crowd = false;
+  for (int seen = 0; seen < tiles && !crowd; seen += 8 * kVoteBlock) {
+    ushort4 b[8];   // (eight reads in flight)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = boxes[min(seen + tid + u * kVoteBlock, tiles - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) look(b[u], seen + tid + u * kVoteBlock);
+    __syncthreads();
+    crowd = n_meet + (kVoteWide - 1) * n_wide > kVoteMeet;
+    if (seen + 8 * kVoteBlock < tiles) __syncthreads();   // (read by all before the next are counted)
   }
-  __syncthreads();
-  if (n_meet > kVoteMeet) {
+  if (tid == 0 && blockIdx.y == 0) crowded[blockIdx.x] = crowd ? 1 : 0;
+  if (crowd) {
     if (tid == 0) *flag = 1;   // (every writer writes the same)
+    const int run = (ox1 - ox0) * candidates;
+    for (int y = oy0 + (tid >> 6); y < oy1; y += kVoteBlock / 64) {
+      unsigned* row =
+          hist + blockIdx.y * element_stride + ((size_t)y * OW + ox0) * (size_t)candidates;
+      for (int i = tid & 63; i < run; i += 64) row[i] = 0;
+    }
     return;
   }
+  for (int i = tid; i < cells * candidates; i += kVoteBlock) votes[i] = 0;
+  __syncthreads();
   const int64_t* plane = labels + (size_t)blockIdx.y * IH * IW;
   const int py = tid / kVoteTile, px = tid % kVoteTile;
   constexpr int U = 4;   // input tiles whose pixels are requested together
@@ -154,14 +176,23 @@ __global__ __launch_bounds__(kVoteBlock) void vote_tile_kernel(
   }
 }
 
-// flag (optional): the kernel runs only if *flag != 0.
-__global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restrict__ p, size_t n16,
-                                                                const int* __restrict__ flag) {
-  if (flag != nullptr && *flag == 0) return;
+__global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restrict__ p, size_t n16) {
   const size_t stride = (size_t)gridDim.x * kVoteBlock;
   for (size_t i = (size_t)blockIdx.x * kVoteBlock + threadIdx.x; i < n16; i += stride)
     p[i] = make_uint4(0, 0, 0, 0);
 }
+
+// The cell tiles that the histogram kernels are for: those marked, if there are any (*flag != 0); all of
+// them where there are no marks (flag == nullptr).
+struct VoteCrowd {
+  const int* flag;
+  const unsigned char* marks;
+  int cells_x, shift;
+  __device__ bool none() const { return flag != nullptr && *flag == 0; }
+  __device__ bool at(int x, int y) const {
+    return flag == nullptr || marks[(y >> shift) * cells_x + (x >> shift)] != 0;
+  }
+};
 
 // One thread per input pixel (and grid width), grid.y over (batch element of this pass, channel): the plane
 // arithmetic is per workgroup, and the pixel's target (16 bytes of the map) and its label are
@@ -172,8 +203,8 @@ __global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restric
 __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
     const int64_t* __restrict__ labels, const int64_t* __restrict__ map,
     unsigned* __restrict__ votes, int in_pixels, int channels, int OH, int OW, int candidates,
-    size_t element_stride, const int* __restrict__ flag) {
-  if (flag != nullptr && *flag == 0) return;
+    size_t element_stride, VoteCrowd crowd) {
+  if (crowd.none()) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
   for (long long first = (long long)blockIdx.x * kVoteBlock; first < in_pixels;
@@ -183,7 +214,7 @@ __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
     const long long x = map[(size_t)at * 2], y = map[(size_t)at * 2 + 1];
     const long long label = labels[(size_t)plane * in_pixels + at];
     const bool ok = pix < in_pixels && x >= 0 && x <= OW - 1 && y >= 0 && y <= OH - 1 &&
-                    label >= 0 && label < candidates;
+                    label >= 0 && label < candidates && crowd.at((int)x, (int)y);
     // channel offset in histogram elements as the reference has it (common/resample.h:127-129):
     // c * OH * OW, not c whole histograms, so the histograms of several channels overlap
     const long long cell = ok ? (long long)(e * element_stride + (size_t)c * OH * OW +
@@ -200,13 +231,14 @@ __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
 // the first largest count.  The counts are read eight at a time, all eight requested before
 // the first is compared.
 __global__ __launch_bounds__(kVoteBlock) void vote_argmax_kernel(
-    const unsigned* __restrict__ votes, int64_t* __restrict__ out, int out_pixels, int channels,
-    int candidates, size_t element_stride, const int* __restrict__ flag) {
-  if (flag != nullptr && *flag == 0) return;
+    const unsigned* __restrict__ votes, int64_t* __restrict__ out, int out_pixels, int OW,
+    int channels, int candidates, size_t element_stride, VoteCrowd crowd) {
+  if (crowd.none()) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
   for (long long pix = (long long)blockIdx.x * kVoteBlock + threadIdx.x; pix < out_pixels;
        pix += (long long)gridDim.x * kVoteBlock) {
+    if (!crowd.at((int)pix % OW, (int)pix / OW)) continue;
     const unsigned* v =
         votes + e * element_stride + ((size_t)c * out_pixels + pix) * (size_t)candidates;
     unsigned best = 0;
@@ -232,6 +264,23 @@ static size_t vote_bytes(int64_t channels, int64_t oh, int64_t ow, int64_t candi
 }
 constexpr size_t kVoteFlagBytes = 256;
 
+// Side (a power of two, as its exponent) of a workgroup's tile of cells: as many as its counters allow,
+// 0 where they allow less than 4 x 4.
+static int vote_cell_shift(int64_t candidates) {
+  for (int shift = 4; shift >= 2; --shift)
+    if ((candidates << (2 * shift)) <= kVoteCounters) return shift;
+  return 0;
+}
+
+// What the LDS kernels need beside the histograms: the flag, the boxes, a mark for each tile of cells.  0 where
+// they do not run: several channels (whose histograms overlap), coordinates past 16 bits, many classes.
+static size_t vote_tile_bytes(int64_t channels, int64_t oh, int64_t ow, int64_t candidates) {
+  const int shift = vote_cell_shift(candidates);
+  if (channels != 1 || oh >= 0xffff || ow >= 0xffff || shift == 0) return 0;
+  const size_t marks = (size_t)ceil_div(oh, 1 << shift) * ceil_div(ow, 1 << shift);
+  return kVoteFlagBytes + kVoteBoxBytes + ((marks + 255) & ~(size_t)255);
+}
+
 }  // namespace sdk
 
 using namespace sdk;
@@ -241,7 +290,10 @@ extern "C" {
 size_t sdk_voting_resample_workspace_bytes(int64_t channels, int64_t out_height,
                                            int64_t out_width, int64_t num_candidates) {
   if (channels < 1 || out_height < 1 || out_width < 1 || num_candidates < 1) return 0;
-  return vote_bytes(channels, out_height, out_width, num_candidates) + kVoteFlagBytes;
+  // (small histograms, of which such a call has a batch of 4 MB in all, bring the room together)
+  const size_t need = vote_bytes(channels, out_height, out_width, num_candidates);
+  return need + std::min(vote_tile_bytes(channels, out_height, out_width, num_candidates),
+                         (need / 16 + 255) & ~(size_t)255);
 }
 
 int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, int64_t* out,
@@ -270,52 +322,60 @@ int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, 
   const size_t n_in = (size_t)channels * in_pixels;
   const size_t n_out = (size_t)channels * out_height * out_width;
   SDK_REQUIRE(channels <= 65535, "voting_resample_to_map: more than 65535 channels");
-  // as many batch elements per pass as the workspace holds histograms (and grid.y planes)
-  const int64_t per_pass = std::min<int64_t>(
-      std::min<int64_t>(batch, (int64_t)(workspace_bytes / need)), 65535 / channels);
-  // The LDS kernels: one channel (several share cells), boxes of 16-bit coordinates, few enough
-  // input tiles and counters; the boxes lie where the histogram would, the flag behind it (a
-  // workspace without room for it: the histogram).  A workgroup's cells are as many as its counters allow.
+  // The LDS kernels: few enough input tiles, histograms worth it, and a workspace with room for what
+  // they need behind at least one (else: the histograms alone).
   const int tiles_x = (int)ceil_div(in_width, kVoteTile);
   const int64_t tiles = (int64_t)tiles_x * ceil_div(in_height, kVoteTile);
-  int shift = 4;
-  while (shift > 2 && (num_candidates << (2 * shift)) > kVoteCounters) --shift;
-  const int* flag = nullptr;
-  if (channels == 1 && out_height < 0xffff && out_width < 0xffff && tiles <= kVoteTiles &&
-      need * (size_t)batch >= kVoteBytes && batch <= 65535 &&
-      (num_candidates << (2 * shift)) <= kVoteCounters &&
-      tiles * sizeof(ushort4) <= need * (size_t)per_pass && (uintptr_t)sample_map % 16 == 0 &&
-      workspace_bytes >= need * (size_t)per_pass + kVoteFlagBytes) {
-    ushort4* boxes = static_cast<ushort4*>(workspace);
-    int* raised = reinterpret_cast<int*>(static_cast<char*>(workspace) + need * (size_t)per_pass);
-    launch(vote_boxes_kernel, dim3((unsigned)tiles), dim3(kVoteTile * kVoteTile), s, sample_map,
-           boxes, raised, (int)in_height, (int)in_width, tiles_x, (int)out_height, (int)out_width);
-    const int64_t cells_x = ceil_div(out_width, 1 << shift);
-    launch(vote_tile_kernel,
-           dim3((unsigned)(cells_x * ceil_div(out_height, 1 << shift)), (unsigned)batch),
-           dim3(kVoteBlock), s, input, sample_map, (const ushort4*)boxes, raised, out,
-           (int)in_height, (int)in_width, (int)tiles, tiles_x, (int)out_height, (int)out_width,
-           (int)cells_x, shift, (int)num_candidates);
-    flag = raised;
+  const size_t beside = vote_tile_bytes(channels, out_height, out_width, num_candidates);
+  const bool by_tile = beside != 0 && tiles <= kVoteTiles && need * (size_t)batch >= kVoteBytes &&
+                       (uintptr_t)sample_map % 16 == 0 && workspace_bytes >= need + beside;
+  // as many batch elements per pass as the workspace holds histograms (and grid.y planes)
+  const int64_t per_pass = std::min<int64_t>(
+      std::min<int64_t>(batch, (int64_t)((workspace_bytes - (by_tile ? beside : 0)) / need)),
+      65535 / channels);
+  VoteCrowd crowd = {nullptr, nullptr, 0, 0};
+  int* flag = nullptr;
+  ushort4* boxes = nullptr;
+  unsigned char* marks = nullptr;
+  unsigned cell_tiles = 0;
+  if (by_tile) {
+    char* p = static_cast<char*>(workspace) + need * (size_t)per_pass;
+    flag = reinterpret_cast<int*>(p);
+    boxes = reinterpret_cast<ushort4*>(p + kVoteFlagBytes);
+    marks = reinterpret_cast<unsigned char*>(p + kVoteFlagBytes + kVoteBoxBytes);
+    crowd.flag = flag;
+    crowd.marks = marks;
+    crowd.shift = vote_cell_shift(num_candidates);
+    crowd.cells_x = (int)ceil_div(out_width, 1 << crowd.shift);
+    cell_tiles = (unsigned)(crowd.cells_x * ceil_div(out_height, 1 << crowd.shift));
+    launch(vote_boxes_kernel, dim3((unsigned)ceil_div(tiles, kVoteBlock / 64)), dim3(kVoteBlock), s,
+           sample_map, boxes, flag, (int)in_height, (int)in_width, (int)tiles, tiles_x,
+           (int)out_height, (int)out_width);
   }
+  // (behind the LDS kernels: narrow grids, whose blocks are quick to find nothing to do)
+  const int64_t most = by_tile ? kVoteGridX : ((int64_t)1 << 31) - 1;
   for (int64_t b = 0; b < batch; b += per_pass) {
     const int64_t nb = std::min<int64_t>(per_pass, batch - b);
-    const size_t n16 = need / 16 * (size_t)nb;
-    // (behind a flag: narrow grids, whose blocks are quick to find nothing to do)
-    const int64_t most = flag != nullptr ? kVoteGridX : ((int64_t)1 << 31) - 1;
-    const int64_t clear_blocks =
-        std::min<int64_t>(ceil_div((int64_t)n16, kVoteBlock), flag != nullptr ? kVoteGridX : 4096);
-    launch(vote_clear_kernel, dim3((unsigned)clear_blocks), dim3(kVoteBlock), s, (uint4*)workspace,
-           n16, flag);
+    if (by_tile) {
+      launch(vote_tile_kernel, dim3(cell_tiles, (unsigned)nb), dim3(kVoteBlock), s,
+             input + (size_t)b * n_in, sample_map, (const ushort4*)boxes, flag, marks, votes,
+             need / sizeof(unsigned), out + (size_t)b * n_out, (int)in_height, (int)in_width,
+             (int)tiles, tiles_x, (int)out_height, (int)out_width, crowd.cells_x, crowd.shift,
+             (int)num_candidates);
+    } else {
+      const size_t n16 = need / 16 * (size_t)nb;
+      const int clear_blocks = (int)std::min<int64_t>(ceil_div((int64_t)n16, kVoteBlock), 4096);
+      launch(vote_clear_kernel, dim3(clear_blocks), dim3(kVoteBlock), s, (uint4*)workspace, n16);
+    }
     const unsigned planes = (unsigned)(nb * channels);
     launch(vote_kernel, dim3((unsigned)std::min(ceil_div(in_pixels, kVoteBlock), most), planes),
            dim3(kVoteBlock), s, input + (size_t)b * n_in, sample_map, votes, in_pixels,
            (int)channels, (int)out_height, (int)out_width, (int)num_candidates,
-           need / sizeof(unsigned), flag);
+           need / sizeof(unsigned), crowd);
     launch(vote_argmax_kernel,
            dim3((unsigned)std::min(ceil_div(out_pixels, kVoteBlock), most), planes),
            dim3(kVoteBlock), s, (const unsigned*)votes, out + (size_t)b * n_out, out_pixels,
-           (int)channels, (int)num_candidates, need / sizeof(unsigned), flag);
+           (int)out_width, (int)channels, (int)num_candidates, need / sizeof(unsigned), crowd);
   }
   SDK_LAUNCH_CHECK("voting_resample_to_map");
   return SDK_OK;

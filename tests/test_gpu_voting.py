@@ -79,3 +79,28 @@ def test_maps_that_raise_the_flag(oracle, kind, nc):
         vmap[:, iw // 2:] = (0, 0)
     assert np.array_equal(_call(labels, vmap, oh, ow, nc),
                           oracle.voting_resample_to_map(labels, vmap, oh, ow, nc))
+
+
+@pytest.mark.parametrize("nc", [4, 40])
+@pytest.mark.parametrize("kind", ["coherent", "half scrambled", "one far cell", "scrambled", "folded"])
+def test_crowded_and_other_cells_side_by_side(oracle, kind, nc):
+    """Cells of crowded squares are counted in memory, the others in LDS, with room for one, three and
+    all of the elements' histograms, in memory that is not clear."""
+    ih, iw, oh, ow = 160, 208, 40, 52
+    if kind == "folded":    # squares of 16 x 16 cells that 81 tiles and more vote into, side by side
+        ih, iw, oh, ow = 320, 640, 34, 68
+    hist = _hist(oh, ow, nc)
+    B = _enough(oh, ow, nc)
+    rng = np.random.default_rng(nc)
+    labels = rng.integers(-1, nc + 1, (B, 1, ih, iw))
+    vmap = _coherent(ih, iw, oh, ow)
+    if kind == "half scrambled":
+        vmap[:80] = rng.permutation(vmap[:80].reshape(-1, 2)).reshape(80, iw, 2)
+    elif kind == "one far cell":
+        vmap[::16, ::16] = (1, 2)
+    elif kind == "scrambled":
+        vmap = rng.permutation(vmap.reshape(-1, 2)).reshape(vmap.shape)
+    want = oracle.voting_resample_to_map(labels, vmap, oh, ow, nc)
+    for n in (1, 3, B):   # (and 128 KB for what the LDS kernels need beside the histograms)
+        assert np.array_equal(_call(labels, vmap, oh, ow, nc, n * hist + (1 << 17)), want)
+    assert np.array_equal(_call(labels, vmap, oh, ow, nc), want)
