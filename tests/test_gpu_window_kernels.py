@@ -79,6 +79,35 @@ def test_exact_values(oracle, tile_kernels, tc, mode):
         assert np.array_equal(have.cpu().numpy(), want)
 
 
+# Batches so large that a workgroup of the weight gradient takes two or three tiles of the list after one
+# another (one of eight groups a batch element; 20, 15 and 9 tiles, the last ones of fewer pixels and with
+# windows of another size): four waves and two, eight waves (ten samples, big tiles), every remainder of
+# K by 4, one row a sample and four
+TURNS = [
+    (64, 5, 40, 40, 60, 40, 60, 9, 1, 0), (64, 5, 40, 40, 60, 40, 60, 7, 0, 0),
+    (64, 6, 66, 24, 72, 24, 72, 9, 1, 0), (64, 5, 66, 40, 60, 40, 60, 7, 0, 0),
+    (64, 5, 66, 24, 72, 24, 72, 6, 2, 0), (64, 5, 33, 24, 72, 24, 72, 8, 1, 0),
+    (64, 5, 70, 40, 60, 40, 60, 10, 0, 0), (64, 5, 66, 24, 72, 24, 72, 10, 1, 0),
+    (64, 5, 33, 40, 60, 40, 60, 10, 1, 0), (64, 5, 66, 96, 192, 24, 48, 9, 1, 0),
+    (64, 5, 40, 96, 192, 24, 48, 7, 0, 0), (64, 5, 66, 96, 192, 24, 48, 10, 0, 0),
+    (64, 5, 40, 96, 192, 24, 48, 10, 1, 0),
+]
+
+
+@pytest.mark.parametrize("tc", TURNS, ids=lambda t: "x".join(map(str, t)))
+def test_weight_gradient_over_several_tiles(oracle, tile_kernels, tc):
+    import _spherical_distortion_ext._ops as ops
+    K, interp = tc[7], tc[8]
+    m, _, x, w, b, g = _arrays(tc)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    want = oracle.mapped_conv_backward(g, m, x, w, b, K, interp, None)[1]
+    for mode in ("native", "split", "bf16"):
+        with ops.conv_compute(mode):
+            gw = ops.ops.mapped_conv_backward_select(t(g), t(m), None, t(x), t(w), K, interp, False,
+                                                     False, True)[1]
+        assert np.array_equal(gw.cpu().numpy(), want), mode
+
+
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
 def test_values_that_are_not_finite_stay_where_they_are(tile_kernels, mode):
     """An infinite pixel reaches the outputs and weights that read it and no others (padding of
