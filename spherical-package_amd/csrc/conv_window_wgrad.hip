@@ -68,6 +68,16 @@ WwGrid ww_grid(const ConvGeom& g, int tiles, bool big) {
   // for the big windows)
   const int64_t want = std::max<int64_t>(8, ceil_div(ceil_div(big ? 256 : 512, w.kinds), 8) * 8);
   w.groups = (int)std::min<int64_t>(ceil_div(tiles, 8) * 8, want);
+  // ten samples: one workgroup per CU (conv_window_wgrad_quarter.hpp), and what the last ones leave idle
+  // counts: the runs of which up to three rounds of 256 workgroups take the fewest tiles one after
+  // another (2 x 177 -> 209 channels, 172 x 346 pixels, one row a sample, float32: 24 runs of 21 tiles
+  // in three rounds of which the last is a quarter full 2197 us, 32 runs of 16 in three full ones
+  // 1683; four waves that built their own columns 1789)
+  if (!big && g.K == 10) {
+    auto in_turn = [&](int64_t n) { return ceil_div(n * w.kinds, 256) * ceil_div(tiles, n); };
+    for (int64_t n = 8; n * w.kinds <= 768 && n <= ceil_div(tiles, 8) * 8; n += 8)
+      if (in_turn(n) < in_turn(w.groups)) w.groups = (int)n;
+  }
   w.slots = (int64_t)w.groups * w.kinds;
   w.nreg = g.K * 16;
   return w;
