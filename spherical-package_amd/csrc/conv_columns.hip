@@ -165,15 +165,14 @@ __global__ __launch_bounds__(kClThreads) void columns_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kGk = 32;
 constexpr int kGld = 36;
-// bf16 operands (CONV) are formed on the way to LDS, once per workgroup: a wave that forms its own from
+// CONV: bf16 operands are formed on the way to LDS, once per workgroup: a wave that forms its own from
 // float32 rows repeats what the neighbour of the same rows does, and six vector instructions an element
 // weigh as much as the products.  A row then holds 64 bytes a piece (one, or the three of the split)
 // and 16 of skew.  6 x 25 x 50 pixels, 96 -> 160, split, weight gradient 41.7 -> 39.0 us; 325 x 648, batch 2,
-// 16 -> 29, bf16, map and forward 251 -> 232.  Two groups on split operands keep float32 rows: two
-// workgroups would no longer share a CU.
-constexpr bool columns_conv(int mm, int ks) { return mm == kMmBf16 || (mm == kMmSplit && ks == 1); }
-constexpr int columns_row_bytes(int mm, int ks) {
-  return !columns_conv(mm, ks) ? kGld * 4 : (mm == kMmBf16 ? 64 : 192) + 16;
+// 16 -> 29, bf16, map and forward 251 -> 232.  Split operands take three workgroups to a CU so instead of
+// four: where the products are short (gemm below) and with two groups of waves they stay float32 rows.
+constexpr int columns_row_bytes(int mm, bool conv) {
+  return !conv ? kGld * 4 : (mm == kMmBf16 ? 64 : 192) + 16;
 }
 // A split of the weight gradient's reduction is hundreds of pixels; added up one after the other they
 // lose twice the bits of the tile kernels' sums (6 x 25 x 50 pixels, 96 -> 160: 4.5e-7 of the float64
@@ -205,24 +204,31 @@ struct GemmArgs {
   int red;                  // reduction length
   int lda, ldb;
   size_t ldc;
-  size_t batch_b, batch_c;  // strides of grid.y (TN: batch_c of the split)
-  int split;                // TN: reduction elements of one split (grid.y)
+  size_t batch_b, batch_c;  // strides of a batch element (TN: batch_c of the split)
+  int split;                // TN: reduction elements of one split
+  int spread;               // TN: splits and tiles dealt to the XCDs together
   int tiles_a, tiles_b;
 };
 
-template <int MM, bool TN, int KS>
+template <int MM, bool TN, int KS, bool CONV>
 __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs g) {
   constexpr int BM = 64, BN = 64;
   constexpr int LA = BM / 32, LB = BN / 32;   // 16-byte pieces per thread and step
-  constexpr bool CONV = columns_conv(MM, KS);
-  constexpr int RB = columns_row_bytes(MM, KS);
+  static_assert(CONV ? MM != kMmF32 : MM != kMmBf16, "bf16 operands are formed early, float32 never");
+  constexpr int RB = columns_row_bytes(MM, CONV);
   __shared__ __attribute__((aligned(16))) char lds[KS][2][(BM + BN) * RB];
   __shared__ float s_bias[BM];
-  // consecutive slots of one XCD share the tile of the larger operand (workgroup ids go
-  // round-robin over the 8 XCDs)
+  // consecutive slots of one XCD share the tile of the larger operand, or (spread) the rows of one
+  // split (workgroup ids go round-robin over the 8 XCDs)
   const int total = g.tiles_a * g.tiles_b;
-  const int slot = (blockIdx.x & 7) * ((total + 7) / 8) + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= (total + 7) / 8 || slot >= total) return;
+  int slot = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), z = blockIdx.y;
+  if (TN && g.spread) {
+    z = slot / total;
+    if (z * g.split >= g.red) return;
+    slot -= z * total;
+  } else {
+    if (slot >= total) return;
+  }
   const int ta = slot % g.tiles_a, tb = slot / g.tiles_a;
   const int i0 = ta * BM, n0 = tb * BN;
   const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kClThreads);
@@ -231,9 +237,9 @@ __global__ __launch_bounds__(KS * kClThreads) void columns_gemm_kernel(GemmArgs 
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   char* As[2] = {lds[group][0], lds[group][1]};
   char* Bs[2] = {lds[group][0] + BM * RB, lds[group][1] + BM * RB};
-  const float* B = TN ? g.B : g.B + (size_t)blockIdx.y * g.batch_b;
-  float* C = g.C + (size_t)blockIdx.y * g.batch_c;
-  const int r_begin = TN ? (int)blockIdx.y * g.split : 0;
+  const float* B = TN ? g.B : g.B + (size_t)z * g.batch_b;
+  float* C = g.C + (size_t)z * g.batch_c;
+  const int r_begin = TN ? z * g.split : 0;
   const int r_end = TN ? min(r_begin + g.split, g.red) : g.red;
 
   const int kb = tid & 7, rb = tid >> 3;   // reduction quad, row (TN: quad of columns)
@@ -560,25 +566,42 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
   a.tiles_a = (int)ceil_div(a.rows_a, 64);
   a.tiles_b = (int)ceil_div(a.rows_b, 64);
   const int64_t total = (int64_t)a.tiles_a * a.tiles_b;
-  const dim3 grid((unsigned)((total + 7) / 8 * 8), (unsigned)batches);
+  // Tiles of a weight gradient that leave more than an eighth of the XCDs' shares empty are dealt together
+  // with the splits: one tile in 450 splits is not one XCD's.  (32 x 32 in runs of 256 of 115200 pixels, split,
+  // the product alone 74 -> 13.5 us, 8 x 720 in runs of 672 40.3 -> 38.2; with 40 tiles, 200 x 600 in runs
+  // of 256, 16.6 -> 20.2, so not there.)
+  const int64_t padded = (total + 7) / 8 * 8;
+  a.spread = TN && 8 * total < 7 * padded;
+  const dim3 grid((unsigned)(a.spread ? (total * batches + 7) / 8 * 8 : padded),
+                  (unsigned)(a.spread ? 1 : batches));
   // Two groups of waves per tile where the tiles alone leave the SIMDs with a wave or two and the
   // reduction is long enough to share (whole forward: 6 x 25 x 50, 96 -> 160, split 65 -> 55 us;
   // 3 x 45 x 91, 200 -> 37, bf16 86 -> 67 us).  With fp32 MFMAs two waves of 512 tiles keep a SIMD
   // busy as it is (1 x 128 x 256, 64 -> 64: 62 -> 67 us), and so do the splits of the weight
   // gradient (57 -> 66 us).
   const bool shared = !TN && total * batches <= (mm == kMmF32 ? 256 : 1024) && a.red >= 4 * kGk;
-#define CG(MMv)                                                                                   \
-  do {                                                                                            \
-    if constexpr (!TN) {                                                                          \
-      if (shared) {                                                                               \
-        launch((columns_gemm_kernel<MMv, false, 2>), grid, dim3(2 * kClThreads), stream, a);      \
-        break;                                                                                    \
-      }                                                                                           \
-    }                                                                                             \
-    launch((columns_gemm_kernel<MMv, TN, 1>), grid, dim3(kClThreads), stream, a);                 \
-  } while (0)
-  if (mm == kMmBf16) CG(kMmBf16); else if (mm == kMmSplit) CG(kMmSplit); else CG(kMmF32);
-#undef CG
+  // Split operands are formed early by the weight gradient, where a reduction is longer than two steps, and by a
+  // forward of so few tiles that all are at work at once either way.  (The product alone, us late and
+  // early: weight gradient 200 x 200 in runs of 416 pixels 24.0 and 20.1, 32 x 32 in runs of 256 14.9 and 13.5;
+  // forward 160 x 28800 x 288 37.1 and 34.2, 64 x 28800 x 64 7.8 and 6.6, 64 x 51200 x 8 10.4 and 11.5, 240 x
+  // 115200 x 8 46 and 52; columns' gradient 12800 x 32 x 32 6.3 and 7.2, 115200 x 72 x 8 26.8 and 28.1.)
+  const bool early = TN || a.red > 2 * kGk || (a.rows_a <= a.rows_b && total * batches <= 768);
+#define CG2(MMv, KSv, CONVv) \
+  launch((columns_gemm_kernel<MMv, TN, KSv, CONVv>), grid, dim3(KSv * kClThreads), stream, a)
+  if constexpr (!TN) {
+    if (shared) {
+      if (mm == kMmBf16) CG2(kMmBf16, 2, true);
+      else if (mm == kMmSplit) CG2(kMmSplit, 2, false);
+      else CG2(kMmF32, 2, false);
+    }
+  }
+  if (!shared) {
+    if (mm == kMmBf16) CG2(kMmBf16, 1, true);
+    else if (mm == kMmF32) CG2(kMmF32, 1, false);
+    else if (early) CG2(kMmSplit, 1, true);
+    else CG2(kMmSplit, 1, false);
+  }
+#undef CG2
   SDK_LAUNCH_CHECK("mapped_conv(columns product)");
   return SDK_OK;
 }

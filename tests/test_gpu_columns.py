@@ -341,3 +341,27 @@ def test_weight_gradient_keeps_the_bits_of_its_sums(ops, mode):
     d = lambda a: t(a).double()  # noqa: E731
     want = ops.ops.mapped_conv_backward(d(g), d(m), None, d(x), d(w), d(b), 9, 1)[1]
     assert _rel(gw.cpu().numpy(), want.cpu().numpy()) <= 2.6e-7
+
+
+@pytest.mark.parametrize("tc", [
+    # reductions of two steps and fewer (operands split late, or by a small forward early), in few tiles and
+    # in more than are at work at once, and of more steps; weight gradients in runs of 64 pixels and of 128
+    (1, 8, 8, 16, 31, 1), (1, 64, 8, 20, 40, 1), (1, 8, 70, 24, 40, 9), (4, 8, 9, 112, 113, 1),
+    (2, 7, 65, 50, 100, 3), (1, 65, 72, 30, 61, 1),
+], ids=lambda t: "x".join(map(str, t)))
+def test_split_products_early_and_late_are_exact(ops, oracle, tc):
+    """Integers of four bits and samples at halves: every product and sum is a float32 number."""
+    B, Cin, Cout, H, W, K = tc
+    assert runs_by_columns(B, Cin, Cout, H, W, H, W, K, 0, 1)
+    rng = np.random.default_rng(sum(tc))
+    y, x, k = np.meshgrid(np.arange(H), np.arange(W), np.arange(K), indexing="ij")
+    m = np.stack([x + k % 3 * 0.5 - 0.5, y + k // 3 * 0.5 - 0.5], -1).astype(np.float32)
+    f = lambda *s: rng.integers(-4, 5, s).astype(np.float32)  # noqa: E731
+    img, w, b, g = f(B, Cin, H, W), f(Cout, Cin, K), f(Cout), f(B, Cout, H, W)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    with ops.conv_compute("split"):
+        out = ops.ops.mapped_conv_forward(t(img), t(m), None, t(w), t(b), K, 1)
+        grads = ops.ops.mapped_conv_backward(t(g), t(m), None, t(img), t(w), t(b), K, 1)
+    assert np.array_equal(out.cpu().numpy(), oracle.mapped_conv_forward(img, m, w, b, K, 1))
+    for have, want in zip(grads, oracle.mapped_conv_backward(g, m, img, w, b, K, 1)):
+        assert np.array_equal(have.cpu().numpy(), want)
