@@ -182,15 +182,14 @@ __global__ __launch_bounds__(kVoteBlock) void vote_clear_kernel(uint4* __restric
     p[i] = make_uint4(0, 0, 0, 0);
 }
 
-// The cell tiles that the histogram kernels are for: those marked, if there are any (*flag != 0); all of
-// them where there are no marks (flag == nullptr).
+// The cell tiles that the histogram kernels are for behind the LDS kernels (CROWD): those marked, if there
+// are any (*flag != 0).
 struct VoteCrowd {
   const int* flag;
   const unsigned char* marks;
   int cells_x, shift;
-  __device__ bool none() const { return flag != nullptr && *flag == 0; }
   __device__ bool at(int x, int y) const {
-    return flag == nullptr || marks[(y >> shift) * cells_x + (x >> shift)] != 0;
+    return marks[(y >> shift) * cells_x + (x >> shift)] != 0;
   }
 };
 
@@ -200,11 +199,12 @@ struct VoteCrowd {
 // write outside its histogram).  Neighbouring lanes often vote for the same cell (pixels of a
 // label image that share a target): a run of them casts its votes with one atomic, from its
 // last lane.
+template <bool CROWD>
 __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
     const int64_t* __restrict__ labels, const int64_t* __restrict__ map,
     unsigned* __restrict__ votes, int in_pixels, int channels, int OH, int OW, int candidates,
     size_t element_stride, VoteCrowd crowd) {
-  if (crowd.none()) return;
+  if (CROWD && *crowd.flag == 0) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
   for (long long first = (long long)blockIdx.x * kVoteBlock; first < in_pixels;
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
     const long long x = map[(size_t)at * 2], y = map[(size_t)at * 2 + 1];
     const long long label = labels[(size_t)plane * in_pixels + at];
     const bool ok = pix < in_pixels && x >= 0 && x <= OW - 1 && y >= 0 && y <= OH - 1 &&
-                    label >= 0 && label < candidates && crowd.at((int)x, (int)y);
+                    label >= 0 && label < candidates && (!CROWD || crowd.at((int)x, (int)y));
     // channel offset in histogram elements as the reference has it (common/resample.h:127-129):
     // c * OH * OW, not c whole histograms, so the histograms of several channels overlap
     const long long cell = ok ? (long long)(e * element_stride + (size_t)c * OH * OW +
@@ -230,15 +230,16 @@ __global__ __launch_bounds__(kVoteBlock) void vote_kernel(
 // One thread per output pixel, grid.y over (batch element of this pass, channel): index of
 // the first largest count.  The counts are read eight at a time, all eight requested before
 // the first is compared.
+template <bool CROWD>
 __global__ __launch_bounds__(kVoteBlock) void vote_argmax_kernel(
     const unsigned* __restrict__ votes, int64_t* __restrict__ out, int out_pixels, int OW,
     int channels, int candidates, size_t element_stride, VoteCrowd crowd) {
-  if (crowd.none()) return;
+  if (CROWD && *crowd.flag == 0) return;
   const unsigned plane = blockIdx.y;
   const unsigned e = plane / (unsigned)channels, c = plane - e * (unsigned)channels;
   for (long long pix = (long long)blockIdx.x * kVoteBlock + threadIdx.x; pix < out_pixels;
        pix += (long long)gridDim.x * kVoteBlock) {
-    if (!crowd.at((int)pix % OW, (int)pix / OW)) continue;
+    if (CROWD && !crowd.at((int)pix % OW, (int)pix / OW)) continue;
     const unsigned* v =
         votes + e * element_stride + ((size_t)c * out_pixels + pix) * (size_t)candidates;
     unsigned best = 0;
@@ -368,14 +369,20 @@ int sdk_voting_resample_to_map(const int64_t* input, const int64_t* sample_map, 
       launch(vote_clear_kernel, dim3(clear_blocks), dim3(kVoteBlock), s, (uint4*)workspace, n16);
     }
     const unsigned planes = (unsigned)(nb * channels);
-    launch(vote_kernel, dim3((unsigned)std::min(ceil_div(in_pixels, kVoteBlock), most), planes),
-           dim3(kVoteBlock), s, input + (size_t)b * n_in, sample_map, votes, in_pixels,
-           (int)channels, (int)out_height, (int)out_width, (int)num_candidates,
-           need / sizeof(unsigned), crowd);
-    launch(vote_argmax_kernel,
-           dim3((unsigned)std::min(ceil_div(out_pixels, kVoteBlock), most), planes),
-           dim3(kVoteBlock), s, (const unsigned*)votes, out + (size_t)b * n_out, out_pixels,
-           (int)out_width, (int)channels, (int)num_candidates, need / sizeof(unsigned), crowd);
+#define VOTES(CROWDv)                                                                              \
+  do {                                                                                             \
+    launch(vote_kernel<CROWDv>,                                                                    \
+           dim3((unsigned)std::min(ceil_div(in_pixels, kVoteBlock), most), planes),                \
+           dim3(kVoteBlock), s, input + (size_t)b * n_in, sample_map, votes, in_pixels,            \
+           (int)channels, (int)out_height, (int)out_width, (int)num_candidates,                    \
+           need / sizeof(unsigned), crowd);                                                        \
+    launch(vote_argmax_kernel<CROWDv>,                                                             \
+           dim3((unsigned)std::min(ceil_div(out_pixels, kVoteBlock), most), planes),               \
+           dim3(kVoteBlock), s, (const unsigned*)votes, out + (size_t)b * n_out, out_pixels,       \
+           (int)out_width, (int)channels, (int)num_candidates, need / sizeof(unsigned), crowd);    \
+  } while (0)
+    if (by_tile) VOTES(true); else VOTES(false);
+#undef VOTES
   }
   SDK_LAUNCH_CHECK("voting_resample_to_map");
   return SDK_OK;
