@@ -2474,7 +2474,7 @@ __device__ __forceinline__ void unpool_from_lds(
 #pragma unroll
       for (int j = 0; j < PG; ++j) acc[j] += i < n ? c[i] * v[j] : 0.0f;
     }
-    for (int i = kUnpoolKept; i < n; ++i) {
+    for (int i = kUnpoolKept; i < n; ++i) {   // (four reads at a time: 5 to 20 in a hundred slower)
       const vecp v = g[src[beg + i] - m0];
       const float ci = co[beg + i];
 #pragma unroll
@@ -2688,14 +2688,29 @@ static int build_unpool_lists(const float* map, const float* wts, void* lists, i
   return SDK_OK;
 }
 
+// Whether the sources go to LDS (unpool_spans_kernel): maps of at most half the image's pixels and planes to
+// take the staging and the lists for; not where an element has hardly an entry to read, nor where so many
+// that most are read again for each eight planes.  points: samples of a pooled pixel.  (us from memory and so:
+//   one sample, stride 2, 96 planes of 256 x 512 17.6 and 18.7, 192 of 512 x 1024 195 and 149; stride 3, 64 of
+//   256 x 512 11.9 and 14.0, 192 of 512 x 1024 164 and 138;
+//   5 x 5 samples, stride 2 (25 products an element before they are merged), 96 of 128 x 256 49 and 66, of 256 x
+//   512 152 and 168, of 512 x 1024 633 and 611, 192 of 256 x 512 295 and 227;
+//   7 x 7, stride 2 (49), 96 of 128 x 256 113 and 159, 192 197 and 179, of 512 x 1024 3385 and 3710, 96 of 64 x
+//   128 81 and 19; stride 3 (22), 96 of 256 x 512 163 and 131.)
+static bool unpool_in_lds(int64_t planes, int64_t HW, int64_t M, int64_t points) {
+  if (planes < 64 || 2 * M > HW) return false;
+  if (points == 1) return planes >= 192 && HW >= (1 << 18);
+  const int64_t products = M * points * 4 / HW;
+  if (products <= 24 || HW <= (1 << 14)) return true;
+  return products <= 32 ? planes >= 192 || HW >= (1 << 19) : planes >= 192 && HW <= (1 << 17);
+}
+
 static int launch_unpool_lists(const float* gout, float* gin, const void* lists, int64_t planes,
                                int H, int W, int M, int K, int P, int interp, hipStream_t stream) {
   const Col2imLists l = col2im_lists_at(const_cast<void*>(lists), H, W, M, K, P, interp);
   const int HW = H * W;
-  // From LDS where the map has half the image's pixels or fewer and there are planes to take the staging
-  // and the lists for (both sides at unpool_spans_kernel).
   const int64_t spans = ceil_div(HW, kUnpoolSpan);
-  if (planes >= 64 && 2 * (int64_t)M <= HW) {
+  if (unpool_in_lds(planes, HW, M, (int64_t)K * std::max(P, 1))) {
     // Planes of a workgroup.  Where all workgroups are at work at once (three per CU) the longest one
     // counts: one pass of eight planes, or equal shares.  Else what they do together: whole passes, and
     // two at least where there are workgroups enough (64 to 512 planes of 64 x 128 to 512 x 1024,
