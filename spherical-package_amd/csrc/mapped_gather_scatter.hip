@@ -596,10 +596,9 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
   const int lo0 = offset[t], hi0 = offset[t + 1];
   const int per = (hi0 - lo0 + (int)gridDim.z - 1) / (int)gridDim.z;
   const int lo = lo0 + (int)blockIdx.z * per, hi = min(hi0, lo + per);
-  for (int i = threadIdx.x; i < PL * THW; i += threads) acc[i] = ACC(0);
-  __syncthreads();
   constexpr int N = PointTaps<T, INTERP>::N;
-  // this round's pixel, point and values are loaded during the round before
+  // this round's pixel, point and values are loaded during the round before, the first round's while
+  // the sums are cleared
   int e = lo + (int)threadIdx.x;
   int pix = e < hi ? list[e] : 0;
   T pu = uv[(size_t)pix * 2], pv = uv[(size_t)pix * 2 + 1];
@@ -607,6 +606,9 @@ __global__ __launch_bounds__(kUvBlock) void uv_texture_scatter_kernel(
 #pragma unroll
   for (int j = 0; j < PL; ++j) val[j] = in[(size_t)(plane0 + (j < np ? j : 0)) * MP + pix];
   int pix_next = e + threads < hi ? list[e + threads] : 0;
+  __builtin_amdgcn_sched_barrier(0);
+  for (int i = threadIdx.x; i < PL * THW; i += threads) acc[i] = ACC(0);
+  __syncthreads();
   for (int base = lo; base < hi; base += threads) {   // uniform trip count over the workgroup
     const bool live = e < hi;
     PointTaps<T, INTERP> taps;
@@ -1680,9 +1682,9 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
     }
     const dim3 grid((unsigned)NT, (unsigned)ceil_div(planes, pl), (unsigned)split);
     // (short buckets of one large texture: three workgroups of 512 share a CU where two of 1024 would.
-    // 64 planes, 320 textures of 80 x 80, 256 x 512 pixels: 207 -> 178 us)
+    // 30 planes, 320 textures of 81 x 81, 52 x 105 pixels: 73 -> 49 us)
     const bool halves = !uv_ordered(NT, MP) && pl == 1 && groups >= 1536 &&
-                        3 * THW * sum <= (size_t)150 * 1024;
+                        3 * THW * sum <= (size_t)160 * 1024;
     const int threads = halves ? kUvBlock / 2 : kUvBlock;
     const int* order = uv_ordered(NT, MP) ? reinterpret_cast<const int*>(ws + off[0]) : nullptr;
 #define UVS(PLv, ACCv)                                                                        \
