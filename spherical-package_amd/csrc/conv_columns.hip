@@ -179,18 +179,10 @@ constexpr int columns_row_bytes(int mm, bool conv) {
 // norm against 2.1e-7), so two steps at a time are summed apart and then added: 1.7e-7, for 2 us of the
 // layer's 174.
 
-// (as split_bf16x8)
 __device__ __forceinline__ void split_bf16x4(const vec4& f, uint2 (&piece)[3]) {
   unsigned u[3][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float r = f[i];
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      u[p][i] = __float_as_uint(r) & 0xffff0000u;
-      r -= __uint_as_float(u[p][i]);
-    }
-  }
+  for (int i = 0; i < 4; ++i) split_bf16(f[i], u[0][i], u[1][i], u[2][i]);
 #pragma unroll
   for (int p = 0; p < 3; ++p)
     piece[p] = make_uint2((u[p][0] >> 16) | u[p][1], (u[p][2] >> 16) | u[p][3]);

@@ -795,7 +795,7 @@ static int wgrad_from_plan(const ConvGeom& g, int mm, const Plan& plan, const fl
     float* wp = reinterpret_cast<float*>(base + t.window_partial);
     rc = window_wgrad_narrow(g, mm, plan, tl, pix, img, gW, wp, stream);
     if (rc) return rc;
-    if (window_wgrad_big_supported(g, mm) && plan.big_lut != nullptr) {
+    if (window_wgrad_big_supported(g) && plan.big_lut != nullptr) {
       rc = window_wgrad(g, mm, plan, tl, pix, img, gW, wp, stream, true);
       if (rc) return rc;
       return planned_wgrad(g, mm, plan, pix, img, gW, wgrad_partial(g, workspace), stream,

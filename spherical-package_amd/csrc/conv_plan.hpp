@@ -151,7 +151,7 @@ int planned_wgrad(const ConvGeom& g, int mm, const Plan& plan, const float* pix,
 bool window_wgrad_supported(const ConvGeom& g, int mm);
 // ... for the big tiles alone (window_wgrad(..., big = true)): also the layers whose other tiles
 // window_wgrad_narrow takes.
-bool window_wgrad_big_supported(const ConvGeom& g, int mm);
+bool window_wgrad_big_supported(const ConvGeom& g);
 // ... and for layers of at most 64 pixel-side channels with nearest taps and no interpolation
 // weights (mm: the matrix arithmetic): the tiles of tl.inside; partial:
 // window_wgrad_narrow_partial_bytes(g), which window_wgrad_partial_bytes(g) returns for them.

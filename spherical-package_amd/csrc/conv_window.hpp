@@ -18,6 +18,10 @@
 
 namespace sdk {
 
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t Rsrc;   // a buffer descriptor
+
 constexpr int kCC = 32;          // channels staged per region chunk
 constexpr int kRegionCap = 288;  // region elements per channel (kCC * 289 * 4 B = 36 KB)
 // A plan's header: kHdrStride ints per tile.  [0..3] window origin and size (row, column,

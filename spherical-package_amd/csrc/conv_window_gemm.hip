@@ -52,11 +52,8 @@ namespace {
 constexpr int kWgThreads = 256;
 constexpr int kWE = 36;   // floats per window element: 32 channels + 4 of skew
 
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Reads at uniform base + lane offset + uniform offset, both in bytes: no vector address arithmetic.
-typedef __amdgpu_buffer_rsrc_t Rsrc;
 __device__ __forceinline__ Rsrc rsrc_of(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }
@@ -335,7 +332,6 @@ __global__ __launch_bounds__(kWgThreads) void inverse_plan_kernel(
 //   lists[4 tiles .. 5 tiles)    small_cap > 0: the tiles of the first list whose window has at
 //                                most small_cap elements, count[4]
 //   lists[5 tiles .. 6 tiles)    ... and the others of the first list, count[5]
-//   lists[6 tiles .. 7 tiles)    every tile that is not in the third list, count[6]
 // max_rows > 0: a tile with a sample of more rows is neither inside nor big.
 __global__ __launch_bounds__(1024) void tile_lists_kernel(const int* __restrict__ hdr, int tiles,
                                                           int* __restrict__ lists,
@@ -921,7 +917,8 @@ bool window_gemm_supported(const ConvGeom& g) {
 size_t window_gemm_weight_bytes(const ConvGeom& g) {
   const size_t blks = (size_t)(g.Cp + 127) / 128 * 4;
   const size_t chunks = (size_t)(g.Cg + kCC - 1) / kCC;
-  return (size_t)g.K * chunks * blks * kPieces<kMmSplit> * 1024;   // (the largest arithmetic)
+  // (the largest arithmetic: a workspace asked for with one serves a call with another)
+  return (size_t)g.K * chunks * blks * kPieces<kMmSplit> * 1024;
 }
 
 size_t tile_lists_bytes(const ConvGeom& g) {

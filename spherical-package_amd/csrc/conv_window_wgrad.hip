@@ -84,8 +84,7 @@ WwGrid ww_grid(const ConvGeom& g, int tiles, bool big) {
 }
 }  // namespace
 
-bool window_wgrad_big_supported(const ConvGeom& g, int mm) {
-  (void)mm;   // every matrix arithmetic
+bool window_wgrad_big_supported(const ConvGeom& g) {
   // (32-bit byte offsets over 32 planes of the image)
   return planned_wgrad_supported(g) && g.K >= 1 && g.K <= 10 && g.Cp >= 1 &&
          (int64_t)g.H * g.W <= ((int64_t)1 << 24);
@@ -97,7 +96,7 @@ bool window_wgrad_supported(const ConvGeom& g, int mm) {
   // the slower one down to 8 rows and 8 channels.  9 samples, 256 x 512, batch 8, weight gradient in
   // us, there and here: 64 -> 64 float32 1627 / 953, split 1558 / 853, bf16 1248 / 508;
   // 128 -> 32 float32 2773 / 1800; 8 -> 16 float32 658 / 460; 220 x 440, batch 1, 48 -> 40 252 / 135)
-  return window_wgrad_big_supported(g, mm) && (g.Cp > 64 || !window_wgrad_narrow_supported(g, mm));
+  return window_wgrad_big_supported(g) && (g.Cp > 64 || !window_wgrad_narrow_supported(g, mm));
 }
 
 size_t window_wgrad_partial_bytes(const ConvGeom& g) {
@@ -105,7 +104,7 @@ size_t window_wgrad_partial_bytes(const ConvGeom& g) {
   // (one buffer serves whichever window kernels the call runs, one after the other)
   const size_t narrow =
       window_wgrad_narrow_supported(g, kMmF32) ? window_wgrad_narrow_partial_bytes(g) : 0;
-  if (!window_wgrad_big_supported(g, kMmF32)) return narrow;
+  if (!window_wgrad_big_supported(g)) return narrow;
   const PixelTiling pt = plan_tiling(g.M / g.OW, g.OW);
   const int tiles = pt.tiles_x * pt.tiles_y;
   const WwGrid w = ww_grid(g, tiles, false), wb = ww_grid(g, tiles, true);

@@ -57,10 +57,7 @@ constexpr int kWvE = 36;     // floats per window element: 32 channels + 4 of sk
 // bytes of one sample's column tile of a quarter: 32 pixels x 32 channels
 constexpr int col_bytes(int mm) { return mm == kMmBf16 ? 2048 : 4096; }
 
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __amdgpu_buffer_rsrc_t Rsrc;
 
 // Byte of 16-byte piece q (8 channels) of pixel p in a column tile.  The pieces of each four
 // pixels change places in a way of their own, so that equal pieces of the pixels that are written

@@ -1694,7 +1694,7 @@ static int launch_uv_scatter(const T* in, const int64_t* quad, const T* uv, T* t
                                         textures, (int)planes, NT, TH, TW, MP)))
     if (direct) {
       if (pl == 4) UVS(4, double); else if (pl == 2) UVS(2, double); else UVS(1, double);
-    } else {   // (such a texture takes half of kUvLdsBytes or more)
+    } else if constexpr (sizeof(T) < sizeof(double)) {   // (such a texture takes half of kUvLdsBytes or more)
       UVS(1, T);
     }
 #undef UVS

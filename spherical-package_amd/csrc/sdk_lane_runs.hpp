@@ -16,16 +16,6 @@ struct LaneRuns {
     dist = lane - (63 - __clzll((long long)upto));
     tail = lane == 63 || (((heads >> 1) >> lane) & 1ull);
   }
-  // inclusive sum of v over the lanes of the run up to this one
-  template <typename T>
-  __device__ __forceinline__ T sum(T v) const {
-    for (int d = 1; d < 64; d <<= 1) {
-      if (!__any(dist >= d)) break;
-      const T below = __shfl_up(v, d);
-      if (dist >= d) v += below;
-    }
-    return v;
-  }
 };
 
 // v of the lane D below in the same row of 16 lanes (0 past its start): a vector instruction, where

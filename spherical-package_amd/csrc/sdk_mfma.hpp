@@ -45,16 +45,19 @@ struct Bf16Split {
   Bf16Frag hi, mid, lo;
 };
 
+// One float's pieces, each in the upper half of a word.
+__device__ __forceinline__ void split_bf16(float f, unsigned& h, unsigned& m, unsigned& l) {
+  h = __float_as_uint(f) & 0xffff0000u;
+  const float r = f - __uint_as_float(h);
+  m = __float_as_uint(r) & 0xffff0000u;
+  const float r2 = r - __uint_as_float(m);
+  l = __float_as_uint(r2) & 0xffff0000u;
+}
+
 __device__ __forceinline__ Bf16Split split_bf16x8(const float (&f)[8]) {
   unsigned h[8], m[8], l[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    h[i] = __float_as_uint(f[i]) & 0xffff0000u;
-    const float r = f[i] - __uint_as_float(h[i]);
-    m[i] = __float_as_uint(r) & 0xffff0000u;
-    const float r2 = r - __uint_as_float(m[i]);
-    l[i] = __float_as_uint(r2) & 0xffff0000u;
-  }
+  for (int i = 0; i < 8; ++i) split_bf16(f[i], h[i], m[i], l[i]);
   Bf16Split s;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
