@@ -425,17 +425,14 @@ window_gemm_kernel(const float* __restrict__ img, const int* __restrict__ hdr,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, h = lane >> 5;
   const int pw = wave & 3, group = wave >> 2;
-  const int cnt = *count;
-  const int per = (cnt + 7) >> 3;
-  const int wg = blockIdx.x / n_tiles;
-  const int slot = (wg & 7) * per + (wg >> 3);
-  if ((wg >> 3) >= per || slot >= cnt) return;
-  const int tile = list[slot];
-  const int nt = blockIdx.x % n_tiles, n0 = nt * TN;
+  const ListShare share(*count, n_tiles);
+  if (share.none) return;
+  const int tile = list[share.slot];
+  const int nt = share.nt, n0 = nt * TN;
   const int ty0 = (tile / pt.tiles_x) * pt.TY(), tx0 = (tile % pt.tiles_x) << pt.tx_shift;
   const int M = pt.OH * pt.OW;
   const size_t HW = (size_t)H * W;
-  const float* img_b = img + (size_t)blockIdx.y * Cg * HW;
+  const float* img_b = img + (size_t)share.batch * Cg * HW;
 
   const int p_local = 32 * pw + lane_pixel(j);
   // the window elements this lane stages (the same for every chunk): lane, lane + 64, ...
@@ -678,7 +675,7 @@ window_gemm_kernel(const float* __restrict__ img, const int* __restrict__ hdr,
   }
   const int oy = ty0 + (p_local >> pt.tx_shift), ox = tx0 + (p_local & (pt.TX() - 1));
   if (oy < pt.OH && ox < pt.OW) {
-    float* out = pix + (size_t)blockIdx.y * Cp * M + (size_t)oy * pt.OW + ox;
+    float* out = pix + (size_t)share.batch * Cp * M + (size_t)oy * pt.OW + ox;
 #pragma unroll
     for (int a = 0; a < NB; ++a)
 #pragma unroll
@@ -734,18 +731,15 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int j = lane & 31, h = lane >> 5;
-  const int cnt = *count;
-  const int per = (cnt + 7) >> 3;
-  const int wg = blockIdx.x / n_tiles;
-  const int slot = (wg & 7) * per + (wg >> 3);
-  if ((wg >> 3) >= per || slot >= cnt) return;
-  const int tile = list[slot];
+  const ListShare share(*count, n_tiles);
+  if (share.none) return;
+  const int tile = list[share.slot];
   constexpr int TN = 64 * NBP, HN = TN / 2;   // channels per workgroup, per wave pair / thread
-  const int n0 = (blockIdx.x % n_tiles) * TN;
+  const int n0 = share.nt * TN;
   const int ty0 = (tile / pt.tiles_x) * pt.TY(), tx0 = (tile % pt.tiles_x) << pt.tx_shift;
   const int M = pt.OH * pt.OW;
   const size_t HW = (size_t)H * W;
-  const float* img_b = img + (size_t)blockIdx.y * Cg * HW;
+  const float* img_b = img + (size_t)share.batch * Cg * HW;
 
   const int RS = min(hdr[tile * kHdrStride + 2] * hdr[tile * kHdrStride + 3], kProductCap);
   load_region_lut(hdr + (size_t)tile * kHdrStride, RS, src);
@@ -897,7 +891,7 @@ __global__ __launch_bounds__(kWgThreads, CH <= 4 ? 2 : 1) void window_product_ke
   // ---- store
   const int oy = ty0 + (p_local >> pt.tx_shift), ox = tx0 + (p_local & (pt.TX() - 1));
   if (oy < pt.OH && ox < pt.OW) {
-    float* out = pix + (size_t)blockIdx.y * Cp * M + (size_t)oy * pt.OW + ox;
+    float* out = pix + (size_t)share.batch * Cp * M + (size_t)oy * pt.OW + ox;
 #pragma unroll
     for (int i = 0; i < HN; ++i) {
       const int n = n0 + HN * hh + i;
