@@ -261,7 +261,9 @@ __device__ __forceinline__ int set_rank(const WindowSet& ws, int n, int off) {
 // the 8 XCDs) takes entries x * per .. of the list, of one batch element (grid.y) after the other, the
 // channel tiles of an entry side by side.  The workgroups that find nothing to do are the last of the launch: between
 // the others they leave some CUs a workgroup more than they need, others one less (4 x 96 x 192, 128 -> 128, float32
-// forward, 504 of 576: 319 -> 253 us; 277 where only two workgroups fitted a CU).  grid.x: a multiple of 8.
+// forward, 504 of 576: 318 -> 255 us; 277 where only two workgroups fitted a CU).  Against that, tiles of unlike cost
+// no longer meet the same tile of the next batch element on a CU, and the last few of a launch can crowd on one
+// (4 x 128 x 256, bilinear, backward of the input 64 -> 128, 896 workgroups: 272 -> 305).  grid.x: a multiple of 8.
 struct ListShare {
   int slot = 0, batch = 0, nt = 0;   // entry of the list, batch element, channel tile
   bool none = true;

@@ -108,6 +108,30 @@ def test_weight_gradient_over_several_tiles(oracle, tile_kernels, tc):
         assert np.array_equal(gw.cpu().numpy(), want), mode
 
 
+# several batch elements and channel tiles over lists that are shorter than their launch and no multiple
+# of 8: windows of every form (contraction with wide, 64 and 32 rows, product form in the strided ones)
+SHARES = [
+    (3, 20, 257, 40, 72, 40, 72, 9, 1, 0),
+    (5, 257, 33, 17, 33, 17, 33, 9, 1, 0),
+    (3, 130, 64, 48, 96, 24, 48, 9, 1, 0),
+    (7, 9, 130, 9, 16, 9, 16, 4, 0, 0),
+]
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", SHARES, ids=lambda t: "x".join(map(str, t)))
+def test_every_tile_of_every_batch_element_is_written_once(oracle, tile_kernels, tc, mode):
+    import _spherical_distortion_ext._ops as ops
+    K, interp = tc[7], tc[8]
+    m, _, x, w, b, g = _arrays(tc)
+    tx, tm, tw, tb, tg = (torch.from_numpy(a).to(DEV) for a in (x, m, w, b, g))
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(tx, tm, None, tw, tb, K, interp)
+        gi = ops.ops.mapped_conv_backward(tg, tm, None, tx, tw, tb, K, interp)[0]
+    np.testing.assert_array_equal(y.cpu().numpy(), oracle.mapped_conv_forward(x, m, w, b, K, interp))
+    np.testing.assert_array_equal(gi.cpu().numpy(), oracle.mapped_conv_backward(g, m, x, w, b, K, interp)[0])
+
+
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
 def test_values_that_are_not_finite_stay_where_they_are(tile_kernels, mode):
     """An infinite pixel reaches the outputs and weights that read it and no others (padding of
