@@ -31,7 +31,7 @@ constexpr int kVoteBlock = 256;
 // cell tiles alone; they cost 2 us each where there is none.  A call, with the histogram alone, with one
 // flag that had everything done again in memory, and so: 57, 18.5, 16 us; the upper half of the map in
 // random order 81, 88, 65; a pixel in 256 voting for one far cell 65, 98, 69; all of it in random order
-// 103, 113, 111 (60 classes 160, 180, 185: what finding out costs).
+// 103, 113, 111 (60 classes 163, 180, 175; one picture 30, 39, 38: what finding out costs).
 constexpr int kVoteTile = 16;        // input tile side
 constexpr int kVoteMeet = 64;        // input tiles (16384 pixels) a workgroup takes on
 constexpr int kVoteWide = 8;         // ... of which one with a box of more than 16 cell squares is as many
