@@ -34,7 +34,6 @@ namespace {
 constexpr int kClThreads = 256;
 typedef float vec4 __attribute__((ext_vector_type(4)));
 
-int pad8(int c) { return (c + 7) & ~7; }
 
 // dst[b][n][c] = src[b][c][n], c padded to Cp8 with zeros.  grid (tiles of 64 n, tiles of 32 c,
 // batch): the tile goes through LDS, reads run along n, writes along c.
@@ -42,27 +41,7 @@ __global__ __launch_bounds__(kClThreads) void channels_last_kernel(
     const float* __restrict__ src, float* __restrict__ dst, int C, int Cp8, int N) {
   __shared__ float tile[32][65];
   const int n0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
-  const float* s = src + (size_t)blockIdx.z * C * N;
-  float* d = dst + (size_t)blockIdx.z * N * Cp8;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int c = c0 + w + 4 * i, n = n0 + lane;
-    tile[w + 4 * i][lane] = (c < C && n < N) ? s[(size_t)c * N + n] : 0.0f;
-  }
-  __syncthreads();
-  // 64 n x 8 channel quads
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int item = threadIdx.x + kClThreads * i;
-    const int n = item >> 3, q = item & 7;
-    if (n0 + n < N && c0 + 4 * q < Cp8) {
-      vec4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = tile[4 * q + e][n];
-      *reinterpret_cast<vec4*>(d + (size_t)(n0 + n) * Cp8 + c0 + 4 * q) = v;
-    }
-  }
+  channels_last_tile(src + (size_t)blockIdx.z * C * N, dst + (size_t)blockIdx.z * N * Cp8, C, Cp8, N, n0, c0, tile);
 }
 
 // REDUCTION_N = false: W[n][k][c]; true: W[k][c][n].  c and n padded to multiples of eight.
@@ -517,9 +496,9 @@ ColumnsLayout columns_layout(const ConvGeom& g) {
     return here;
   };
   l.pix_rows = take((size_t)g.B * g.M * Cpp);
-  l.img_rows = take((size_t)g.B * g.H * g.W * Cgp);
+  l.img_rows = take(((size_t)g.B * g.H * g.W + 1) * Cgp);   // (and a row of zeros)
   l.col = take(column_values(g));
-  l.weights = take((size_t)g.K * Cgp * Cpp);
+  l.weights = take(std::max((size_t)g.K * Cgp * Cpp, columns_operand_bytes(g) / sizeof(float)));
   // the weight gradient's reduction (all pixels of the batch) in splits: about two
   // workgroups per CU, at least 64 pixels each
   const int64_t tiles = ceil_div(g.Cp, 64) * ceil_div((int64_t)g.K * Cgp, 64);
@@ -643,6 +622,8 @@ int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float
   float* rows = reinterpret_cast<float*>(ws + l.img_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
   float* w = reinterpret_cast<float*>(ws + l.weights);
+  if (columns_direct(g))
+    return columns_direct_forward(g, mm, img, map, wts, Wm, bias, pix, rows, w, reinterpret_cast<float*>(ws + l.col), stream);
   const int Cgp = pad8(g.Cg), R = g.K * Cgp;
   int rc = to_rows(img, rows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
   if (rc) return rc;

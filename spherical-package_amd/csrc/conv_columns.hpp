@@ -7,6 +7,42 @@
 
 namespace sdk {
 
+inline int pad8(int c) { return (c + 7) & ~7; }
+
+// One 64-element x 32-channel tile of src[C][N] into dst[N][Cp8] (256 threads; channels C .. Cp8 - 1 are
+// zeros): through LDS, reads along n, 16-byte writes along c.
+__device__ __forceinline__ void channels_last_tile(const float* __restrict__ src, float* __restrict__ dst, int C,
+                                                   int Cp8, int N, int n0, int c0, float (*tile)[65]) {
+  typedef float vec4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = c0 + w + 4 * i, n = n0 + lane;
+    const float v = src[(size_t)min(c, C - 1) * N + min(n, N - 1)];
+    tile[w + 4 * i][lane] = (c < C && n < N) ? v : 0.0f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {   // 64 n x 8 channel quads
+    const int item = threadIdx.x + 256 * i;
+    const int n = item >> 3, q = item & 7;
+    if (n0 + n < N && c0 + 4 * q < Cp8) {
+      vec4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile[4 * q + e][n];
+      *reinterpret_cast<vec4*>(dst + (size_t)(n0 + n) * Cp8 + c0 + 4 * q) = v;
+    }
+  }
+}
+
+// The forward without a column matrix (conv_columns_forward.hip), for calls of the route that
+// columns_direct() takes.  rows: B * H * W + 1 rows of pad8(Cg) floats, operands: columns_operand_bytes().
+bool columns_direct(const ConvGeom& g);
+size_t columns_operand_bytes(const ConvGeom& g);
+int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
+                           const float* Wm, const float* bias, float* pix, float* rows, void* operands,
+                           float* partial, hipStream_t stream);
+
 // Maps whose kept plan holds the inverted lists the route's scatter reads (H, W, M, K, P and
 // interp of g).
 bool columns_map(const ConvGeom& g);

@@ -1,0 +1,86 @@
+"""The forward of small calls that blends its columns on the way to LDS
+(csrc/conv_columns_forward.hip), against the oracle."""
+import pytest
+import torch
+
+import test_gpu_columns as columns
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import _spherical_distortion_ext._ops as o
+    return o
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from oracle import oracle as o
+    return o
+
+
+# (batch, Cin, Cout, H, W, OH, OW, K, P, interp), as in test_gpu_columns: every number of channel
+# blocks a tile may have and one over (32 .. 161 channels), tiles of one pixel and one over 32
+# pixels, one and several groups and splits of the reduction (K * Cin of 32 steps and more on few
+# tiles), runs of samples that share no table of taps (25 samples, weighted samples of up to 16
+# taps, channel counts whose steps of 32 straddle samples), calls with more tiles than XCDs' shares
+SIZES = [
+    (1, 8, 32, 6, 9, 3, 11, 9, 0, 1),
+    (1, 40, 33, 6, 9, 3, 11, 9, 0, 2),
+    (2, 24, 96, 9, 14, 7, 13, 9, 0, 1),
+    (1, 33, 97, 9, 14, 8, 8, 9, 0, 0),
+    (1, 16, 160, 9, 14, 8, 9, 4, 0, 1),
+    (1, 16, 161, 9, 14, 8, 9, 4, 0, 0),
+    (1, 72, 64, 9, 14, 4, 8, 25, 0, 1),
+    (2, 130, 40, 9, 14, 5, 7, 25, 0, 2),
+    (1, 64, 128, 9, 14, 5, 7, 25, 0, 0),
+    (1, 8, 16, 9, 14, 5, 7, 25, 4, 1),
+    (2, 40, 24, 9, 14, 5, 7, 9, 4, 2),
+    (1, 21, 24, 9, 14, 5, 7, 25, 3, 0),
+    (1, 96, 48, 9, 14, 5, 7, 25, 2, 1),
+    (3, 12, 20, 40, 80, 40, 80, 9, 0, 1),
+    (1, 16, 64, 64, 128, 64, 128, 9, 4, 1),
+]
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
+def test_forward_matches_the_oracle(ops, oracle, tc, mode):
+    from _spherical_distortion_ext import _capi
+    B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
+    assert _capi.load().sdk_mapped_conv_by_columns(B, Cin, Cout, H, W, OH, OW, K, P, interp,
+                                                   _capi.SDK_F32, 0, 0) == 1
+    m, iw, x, w, b, _, _ = columns._arrays(tc)
+    t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
+    odd = torch.empty(m.size + 1, device=DEV)[1:].view(m.shape).copy_(t(m))   # 4 bytes off a pair's place
+    want = oracle.mapped_conv_forward(x, m, w, b, K, interp, iw)
+    # float32: sums of at most K * Cin terms of random signs, eps * sqrt(n) < 5e-6; bf16 operands: 2^-9 each
+    tol = 4e-3 if mode == "bf16" else 5e-6
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(t(x), t(m), t(iw), t(w), t(b), K, interp)
+        again = ops.ops.mapped_conv_forward(t(x), odd, t(iw), t(w), t(b), K, interp)
+    assert columns._rel(y.cpu().numpy(), want) <= tol
+    assert torch.equal(y, again)
+
+
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+def test_values_no_tap_reads_stay_out(ops, mode):
+    """An infinite pixel without a tap, and an infinite weight of a channel beside the others."""
+    tc = (1, 12, 40, 9, 14, 5, 7, 9, 0, 0)
+    m, _, x, w, b, _, _ = columns._arrays(tc)
+    m[..., 0] = m[..., 0].clip(0, 12)
+    x[0, :, :, 13] = float("inf")
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    with ops.conv_compute(mode):
+        y = ops.ops.mapped_conv_forward(t(x), t(m), None, t(w), t(b), 9, 0)
+        clean = x.copy()
+        clean[0, :, :, 13] = 0
+        want = ops.ops.mapped_conv_forward(t(clean), t(m), None, t(w), t(b), 9, 0)
+        assert torch.equal(y, want)
+        w[7, 3, 2] = float("inf")
+        y = ops.ops.mapped_conv_forward(t(clean), t(m), None, t(w), t(b), 9, 0)
+    rest = [n for n in range(40) if n != 7]
+    assert torch.equal(y[:, rest], want[:, rest])
+    assert not torch.isfinite(y[:, 7]).all()
