@@ -6,6 +6,7 @@
 
 #include <mutex>
 
+#include "conv_columns.hpp"
 #include "conv_fused.hpp"
 #include "conv_small.hpp"
 #include "conv_internal.hpp"
@@ -379,8 +380,15 @@ static int impl_mapped_conv_backward(const void* grad_output, const void* sample
     shared.cleared = true;
     shared.bias_sum = static_cast<float*>(grad_bias);   // summed by the weight-gradient kernel
   }
+  // Calls of the columns route lay grad_output and input out once for both contractions, and the
+  // sums of the weight gradient's pixels come from there.
+  if (grad_weight != nullptr && dtype == SDK_F32 && compute != SDK_COMPUTE_UNFUSED && batch > 0 &&
+      fused_supported(g) && columns_first(g)) {
+    shared.wgrad_img = static_cast<const float*>(input);
+    if (columns_sums_bias(g)) shared.columns_bias = static_cast<float*>(grad_bias);
+  }
   hipEvent_t joined = nullptr;
-  if (!shared.cleared && grad_bias != nullptr)
+  if (!shared.cleared && shared.columns_bias == nullptr && grad_bias != nullptr)
     rc = fork_side((hipStream_t)stream, &joined, side_worth(batch, out_channels, M, dtype),
                    [&](hipStream_t s) {
       return bias_grad(grad_output, grad_bias, batch, out_channels, M, dtype, s,

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "conv_columns.hpp"
 #include "conv_product.hpp"
@@ -392,83 +393,93 @@ __global__ __launch_bounds__(kClThreads) void columns_wgrad_sum_kernel(
 }
 
 // img[b][c][u] = bias[c] + sum over the entries of u's list of coefficient * col[b][sample][c].
-// A workgroup owns 16 image elements x 64 channels of one batch element, a thread one element
-// and four channels: the 16 lanes of an element read an entry's 64 products as one run, eight
-// entries in flight, and the sums leave through LDS as runs along the image.  grid (blocks of 16
+// A workgroup owns 256 / (L S) image elements x 4 L channels of one batch element, L S lanes an element:
+// L lanes read an entry's products as one run, S such groups share the list, eight entries of it in
+// flight, and the sums leave through LDS as runs along the image.  L is what the channels fill: with 16
+// lanes of which two have channels (8 -> 56, 6 x 100 x 200, 5 x 5) 154 us, with L = 2 and S = 4 84; 64 channels
+// 24 us with S = 1, 22 with S = 2; 96 channels 17 us in two chunks of 64, 15 in three of 32.  grid (blocks of
 // elements, channel chunks, batch).
 // A list of more than kClLong entries (a map that sends many samples to one image element, invalid ones
-// for instance) is the whole workgroup's: eight entries in turn for each group of 16 lanes, whose
+// for instance) is the whole workgroup's: sixteen entries in turn for each group of L lanes, whose
 // sums are added in their order.  (64 channels, 1 x 128 x 256, a tenth of 295 thousand samples on
-// one spot, forward + backward: 4184 us with one group per list, 660 now; 241 without the spot.)
-constexpr int kClTargets = 16;
+// one spot, backward: 365 us with eight entries, 288 now; 124 without the spot.)
 constexpr int kClLong = 256;
+template <int L, int S>
 __global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
     const float* __restrict__ col, const int* __restrict__ offset, const int* __restrict__ src,
     const float* __restrict__ co, const float* __restrict__ bias, float* __restrict__ img, int Cg,
     int C4, int HW, int samples) {
-  __shared__ float tile[64][kClTargets + 1];
-  __shared__ vec4 parts[kClTargets][16];
-  const int q = threadIdx.x & 15, t = threadIdx.x >> 4;
-  const int u0 = blockIdx.x * kClTargets, c0 = blockIdx.y * 64;
+  constexpr int T = kClThreads / (L * S);
+  __shared__ float tile[4 * L][T + 1];
+  __shared__ vec4 parts[T][L * S];
+  const int ql = threadIdx.x % (L * S), q = ql % L, share = ql / L, t = threadIdx.x / (L * S);
+  const int u0 = blockIdx.x * T, c0 = blockIdx.y * (4 * L);
   const vec4* col_b = reinterpret_cast<const vec4*>(col) + (size_t)blockIdx.z * samples * C4 +
                       min(c0 / 4 + q, C4 - 1);
   vec4 acc = {0.f, 0.f, 0.f, 0.f};
-  // acc += entries beg .. beg + 7, beg + step .. beg + step + 7, ... of those before end (> 0); those
-  // of the next step are named before this one's products are here
-  auto add = [&](int beg, int end, int step) {
-    int s[8];
-    float w[8];
+  // acc += this lane's shares (U entries of each S * U) of the entries from beg on, S * U and then `step`
+  // further each turn, before end (> 0); those of the next turn are named before this one's products are here
+  auto add = [&](auto count, int beg, int end, int step) {
+    constexpr int U = decltype(count)::value;
+    int s[U];
+    float w[U];
     auto name = [&](int e) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < U; ++i) {
         const int at = min(e + i, end - 1);
         w[i] = co[at];
         s[i] = src[at];
       }
     };
+    beg += share * U;
     if (beg < end) name(beg);
     for (int e = beg; e < end; e += step) {
-      vec4 v[8];
-      float here[8];
+      vec4 v[U];
+      float here[U];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < U; ++i) {
         v[i] = col_b[(size_t)s[i] * C4];
         here[i] = w[i];
       }
       if (e + step < end) name(e + step);
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < U; ++i)
         if (e + i < end) acc += here[i] * v[i];
     }
   };
+  constexpr int kShort = 8 / S, kLong = 16;   // entries of a lane in flight
   const int u = min(u0 + t, HW - 1);
   const int beg = offset[u], end = offset[u + 1];
-  if (end - beg <= kClLong) add(beg, end, 8);
-  const int u_last = min(u0 + kClTargets, HW);   // (uniform from here on)
-  if (offset[u_last] - offset[u0] > kClLong) {
+  if (end - beg <= kClLong) add(std::integral_constant<int, kShort>(), beg, end, 8);
+  if (__syncthreads_or(end - beg > kClLong)) {
+    const int u_last = min(u0 + T, HW);
     for (int x = u0; x < u_last; ++x) {
       const int b = offset[x], e = offset[x + 1];
       if (e - b <= kClLong) continue;
       const vec4 own = acc;
       acc = vec4{0.f, 0.f, 0.f, 0.f};
-      add(b + 8 * t, e, 8 * kClTargets);
-      parts[t][q] = acc;
+      add(std::integral_constant<int, kLong>(), b + kLong * S * t, e, kLong * S * T);
+      parts[t][ql] = acc;
       acc = own;
       __syncthreads();
       if (t == x - u0) {
-        acc = parts[0][q];
-        for (int p = 1; p < kClTargets; ++p) acc += parts[p][q];
+        acc = parts[0][ql];
+        for (int p = 1; p < T; ++p) acc += parts[p][ql];
       }
       __syncthreads();
     }
   }
 #pragma unroll
-  for (int x = 0; x < 4; ++x) tile[4 * q + x][t] = acc[x];
+  for (int x = 0; x < 4; ++x) {
+#pragma unroll
+    for (int d = L; d < L * S; d *= 2) acc[x] += __shfl_xor(acc[x], d, 64);
+    tile[4 * q + x][t] = acc[x];   // (equal in the lanes that share a place)
+  }
   __syncthreads();
   float* img_b = img + (size_t)blockIdx.z * Cg * HW;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = (threadIdx.x >> 4) + 16 * i, n = threadIdx.x & 15;
+  for (int i = 0; i < 4 / S; ++i) {
+    const int item = threadIdx.x + kClThreads * i, c = item / T, n = item % T;
     if (c0 + c < Cg && u0 + n < HW)
       img_b[(size_t)(c0 + c) * HW + u0 + n] = tile[c][n] + (bias != nullptr ? bias[c0 + c] : 0.0f);
   }
@@ -480,7 +491,7 @@ __global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct ColumnsLayout {
-  size_t pix_rows, img_rows, col, weights, partial, lists, total;
+  size_t pix_rows, pix_cols, img_rows, col, weights, partial, strip_sums, lists, total;
   int splits, split_len;
 };
 
@@ -488,28 +499,42 @@ size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(
 
 ColumnsLayout columns_layout(const ConvGeom& g) {
   const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp);
-  ColumnsLayout l;
+  ColumnsLayout l{};
   size_t at = 0;
-  auto take = [&](size_t values) {
+  auto take = [&](size_t bytes) {
     const size_t here = at;
-    at += up256(values * sizeof(float));
+    at += up256(bytes);
     return here;
   };
-  l.pix_rows = take((size_t)g.B * g.M * Cpp);
-  l.img_rows = take(((size_t)g.B * g.H * g.W + 1) * Cgp);   // (and a row of zeros)
-  l.col = take(column_values(g));
-  l.weights = take(std::max((size_t)g.K * Cgp * Cpp, columns_operand_bytes(g) / sizeof(float)));
-  // the weight gradient's reduction (all pixels of the batch) in splits: about two
-  // workgroups per CU, at least 64 pixels each
-  const int64_t tiles = ceil_div(g.Cp, 64) * ceil_div((int64_t)g.K * Cgp, 64);
-  const int64_t pixels = g.B * (int64_t)g.M;
-  int64_t splits = std::max<int64_t>(1, std::min<int64_t>(ceil_div(512, tiles), ceil_div(pixels, 64)));
-  l.split_len = (int)(ceil_div(ceil_div(pixels, splits), kGk) * kGk);
-  l.splits = (int)ceil_div(pixels, l.split_len);
-  l.partial = take((size_t)l.splits * g.Cp * g.K * Cgp);
+  l.img_rows = take(sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp);   // (and a row of zeros)
+  l.col = take(sizeof(float) * column_values(g));
+  if (columns_direct(g)) {
+    l.weights = take(columns_weight_bytes(g));
+    l.pix_rows = take(columns_pixel_bytes(g));
+    l.pix_cols = take(columns_pixel_bytes(g));
+    l.strip_sums = take(columns_strip_bytes(g));
+    l.partial = take(columns_partial_bytes(g));
+  } else {
+    l.weights = take(sizeof(float) * g.K * Cgp * Cpp);
+    l.pix_rows = take(sizeof(float) * g.B * g.M * Cpp);
+    // the weight gradient's reduction (all pixels of the batch) in splits: about two
+    // workgroups per CU, at least 64 pixels each
+    const int64_t tiles = ceil_div(g.Cp, 64) * ceil_div((int64_t)g.K * Cgp, 64);
+    const int64_t pixels = g.B * (int64_t)g.M;
+    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(ceil_div(512, tiles), ceil_div(pixels, 64)));
+    l.split_len = (int)(ceil_div(ceil_div(pixels, splits), kGk) * kGk);
+    l.splits = (int)ceil_div(pixels, l.split_len);
+    l.partial = take(sizeof(float) * l.splits * g.Cp * g.K * Cgp);
+  }
   l.lists = at;
   l.total = at + up256(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp));
   return l;
+}
+
+ColumnsScratch columns_scratch(const ColumnsLayout& l, char* ws) {
+  return ColumnsScratch{reinterpret_cast<float*>(ws + l.img_rows), ws + l.weights, ws + l.pix_rows, ws + l.pix_cols,
+                        reinterpret_cast<float*>(ws + l.strip_sums), reinterpret_cast<float*>(ws + l.col),
+                        reinterpret_cast<float*>(ws + l.partial)};
 }
 
 int to_rows(const float* src, float* dst, int64_t B, int C, int64_t N, hipStream_t stream) {
@@ -610,6 +635,9 @@ bool columns_route(const ConvGeom& g) {
          (size_t)pad8(g.Cp) * g.K * pad8(g.Cg) < ((size_t)1 << 31);
 }
 
+// (a wave adds up a channel's strips)
+bool columns_sums_bias(const ConvGeom& g) { return columns_direct(g) && g.B * ceil_div(g.M, 64) <= 4096; }
+
 size_t columns_workspace_bytes(const ConvGeom& g) {
   return columns_route(g) ? columns_layout(g).total : 0;
 }
@@ -623,7 +651,7 @@ int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float
   float* col = reinterpret_cast<float*>(ws + l.col);
   float* w = reinterpret_cast<float*>(ws + l.weights);
   if (columns_direct(g))
-    return columns_direct_forward(g, mm, img, map, wts, Wm, bias, pix, rows, w, reinterpret_cast<float*>(ws + l.col), stream);
+    return columns_direct_forward(g, mm, img, map, wts, Wm, bias, pix, columns_scratch(l, ws), stream);
   const int Cgp = pad8(g.Cg), R = g.K * Cgp;
   int rc = to_rows(img, rows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
   if (rc) return rc;
@@ -650,7 +678,8 @@ int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float
 
 int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* Wm, const float* bias, float* img,
-                         void* workspace, hipStream_t stream, const void* lists) {
+                         void* workspace, hipStream_t stream, const void* lists,
+                         const float* wgrad_img, bool bias_sum) {
   const ColumnsLayout l = columns_layout(g);
   char* ws = static_cast<char*>(workspace);
   float* rows = reinterpret_cast<float*>(ws + l.pix_rows);
@@ -663,46 +692,60 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
     if (rc) return rc;
     lists = ws + l.lists;
   }
-  rc = to_rows(pix, rows, g.B, g.Cp, g.M, stream);
-  if (rc) return rc;
-  const int total = R * Cpp;
-  launch(columns_weight_kernel<true>, dim3((unsigned)ceil_div(total, kClThreads)),
-         dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, Cpp, total);
-  SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
-  // all pixels of the batch are the rows of one product
-  GemmArgs a{};
-  a.A = rows;
-  a.B = w;
-  a.C = col;
-  a.rows_a = (int)(g.B * g.M);
-  a.rows_b = R;
-  a.red = Cpp;
-  a.lda = a.ldb = Cpp;
-  a.ldc = (size_t)R;
-  rc = gemm<false>(mm, a, 1, stream);
-  if (rc) return rc;
+  if (columns_direct(g)) {
+    rc = columns_direct_product(g, mm, pix, Wm, wgrad_img, bias_sum, columns_scratch(l, ws), stream);
+    if (rc) return rc;
+  } else {
+    rc = to_rows(pix, rows, g.B, g.Cp, g.M, stream);
+    if (rc) return rc;
+    const int total = R * Cpp;
+    launch(columns_weight_kernel<true>, dim3((unsigned)ceil_div(total, kClThreads)),
+           dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, Cpp, total);
+    SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
+    // all pixels of the batch are the rows of one product
+    GemmArgs a{};
+    a.A = rows;
+    a.B = w;
+    a.C = col;
+    a.rows_a = (int)(g.B * g.M);
+    a.rows_b = R;
+    a.red = Cpp;
+    a.lda = a.ldb = Cpp;
+    a.ldc = (size_t)R;
+    rc = gemm<false>(mm, a, 1, stream);
+    if (rc) return rc;
+  }
   const Col2imView v = col2im_lists_view(lists, g.H, g.W, g.M, g.K, g.P, g.interp);
   const int HW = g.H * g.W;
-  launch(columns_col2im_kernel,
-         dim3((unsigned)ceil_div(HW, kClTargets), (unsigned)ceil_div(g.Cg, 64), (unsigned)g.B),
-         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, img, g.Cg,
-         Cgp / 4, HW, g.M * g.K);
+  // as many lanes an element as its channels fill
+  const int C4 = Cgp / 4;
+#define CI(Lv, Sv)                                                                                          \
+  launch((columns_col2im_kernel<Lv, Sv>),                                                                   \
+         dim3((unsigned)ceil_div(HW, kClThreads / (Lv * Sv)), (unsigned)ceil_div(C4, Lv), (unsigned)g.B),   \
+         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, img, g.Cg, C4, HW, g.M * g.K)
+  if (C4 <= 2) CI(2, 4);
+  else if (C4 <= 4) CI(4, 4);
+  else if (ceil_div(C4, 16) * 2 > ceil_div(C4, 8)) CI(8, 2);
+  else CI(16, 2);
+#undef CI
   SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
   return SDK_OK;
 }
 
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,
-                         hipStream_t stream, bool pix_ready) {
+                         hipStream_t stream, bool prepared, float* gb) {
   const ColumnsLayout l = columns_layout(g);
   char* ws = static_cast<char*>(workspace);
+  if (columns_direct(g))
+    return columns_direct_wgrad(g, mm, pix, map, wts, img, gW, columns_scratch(l, ws), prepared, gb, stream);
   float* prows = reinterpret_cast<float*>(ws + l.pix_rows);
   float* irows = reinterpret_cast<float*>(ws + l.img_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
   float* partial = reinterpret_cast<float*>(ws + l.partial);
   const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp), R = g.K * Cgp;
   int rc = SDK_OK;
-  if (!pix_ready) rc = to_rows(pix, prows, g.B, g.Cp, g.M, stream);
+  if (!prepared) rc = to_rows(pix, prows, g.B, g.Cp, g.M, stream);
   if (rc) return rc;
   rc = to_rows(img, irows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
   if (rc) return rc;

@@ -35,13 +35,32 @@ __device__ __forceinline__ void channels_last_tile(const float* __restrict__ src
   }
 }
 
-// The forward without a column matrix (conv_columns_forward.hip), for calls of the route that
-// columns_direct() takes.  rows: B * H * W + 1 rows of pad8(Cg) floats, operands: columns_operand_bytes().
+// The contractions without a column matrix in front of them (conv_columns_direct.hip), for calls of the
+// route that columns_direct() takes.
+struct ColumnsScratch {
+  float* img_rows;      // B * H * W + 1 rows of pad8(Cg) floats
+  void* weights;        // columns_weight_bytes()
+  void *pix_rows, *pix_cols;   // columns_pixel_bytes() each
+  float* strip_sums;    // columns_strip_bytes()
+  float* col;           // the products of a scatter, or a forward's sums
+  float* partial;       // columns_partial_bytes()
+};
 bool columns_direct(const ConvGeom& g);
-size_t columns_operand_bytes(const ConvGeom& g);
+size_t columns_weight_bytes(const ConvGeom& g);
+size_t columns_pixel_bytes(const ConvGeom& g);
+size_t columns_partial_bytes(const ConvGeom& g);
+size_t columns_strip_bytes(const ConvGeom& g);
 int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
-                           const float* Wm, const float* bias, float* pix, float* rows, void* operands,
-                           float* partial, hipStream_t stream);
+                           const float* Wm, const float* bias, float* pix, const ColumnsScratch& s,
+                           hipStream_t stream);
+// s.col[b][m][(k, c)] = sum over n of pix * Wm.  wgrad_img: that of a columns_direct_wgrad of the same call that
+// follows, laid out by the same launch; strip_sums: ... which is asked for the bias gradient.
+int columns_direct_product(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
+                           bool strip_sums, const ColumnsScratch& s, hipStream_t stream);
+// gb: also gb[n] = sum of pix[b][n][m] (optional).
+int columns_direct_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map, const float* wts,
+                         const float* img, float* gW, const ColumnsScratch& s, bool prepared, float* gb,
+                         hipStream_t stream);
 
 // Maps whose kept plan holds the inverted lists the route's scatter reads (H, W, M, K, P and
 // interp of g).
@@ -55,14 +74,18 @@ int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float
                         const float* wts, const float* Wm, const float* bias, float* pix,
                         void* workspace, hipStream_t stream);
 // img[b] = bias + col2im(Wm^T x pix[b]); every element of img is written.  lists: the inverted
-// map of a kept plan, or nullptr: built in the workspace.
+// map of a kept plan, or nullptr: built in the workspace.  wgrad_img (optional): the image of a
+// columns_gather_wgrad of the same call that follows with `prepared`; bias_sum: it is asked for the bias gradient.
 int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* Wm, const float* bias, float* img,
-                         void* workspace, hipStream_t stream, const void* lists);
-// gW = sum_b pix[b] x im2col(img[b])^T; every element of gW is written.  pix_ready: the
-// workspace still holds the channels-last copy of pix a columns_gemm_scatter of the same g left.
+                         void* workspace, hipStream_t stream, const void* lists,
+                         const float* wgrad_img, bool bias_sum);
+// gW = sum_b pix[b] x im2col(img[b])^T; every element of gW is written.  prepared: the workspace
+// still holds what a columns_gemm_scatter of the same g laid out for it.  gb (columns_sums_bias): also
+// gb[n] = sum of pix[b][n][m].
+bool columns_sums_bias(const ConvGeom& g);
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,
-                         hipStream_t stream, bool pix_ready);
+                         hipStream_t stream, bool prepared, float* gb);
 
 }  // namespace sdk

@@ -1153,10 +1153,12 @@ int fused_gemm_scatter(const ConvGeom& g, int compute, const float* pix, const f
   if (columns_first(g)) {
     if (shared != nullptr) {
       shared->valid = false;
-      shared->pix_rows = true;
+      shared->columns_prepared = true;
     }
     return columns_gemm_scatter(g, matrix_mode(compute), pix, map, wts, Wm, bias, img, workspace,
-                                stream, cached != nullptr ? cached->columns_lists : nullptr);
+                                stream, cached != nullptr ? cached->columns_lists : nullptr,
+                                shared != nullptr ? shared->wgrad_img : nullptr,
+                                shared != nullptr && shared->columns_bias != nullptr);
   }
   const bool planned_fb = planned_scatter_supported(g);
   const int* generic_gate = nullptr;   // gate of the atomic scatter kernel at the end
@@ -1292,7 +1294,8 @@ int fused_gather_wgrad(const ConvGeom& g, int compute, const float* pix, const f
   const bool bf16 = compute == SDK_COMPUTE_BF16;
   if (g.B > 0 && !small_wgrad_supported(g) && columns_first(g))
     return columns_gather_wgrad(g, matrix_mode(compute), pix, map, wts, img, gW, workspace, stream,
-                                shared != nullptr && shared->pix_rows);
+                                shared != nullptr && shared->columns_prepared,
+                                shared != nullptr ? shared->columns_bias : nullptr);
   const bool cleared = shared != nullptr && shared->cleared && small_wgrad_supported(g);
   int rc = cleared ? SDK_OK : zero_fill(gW, sizeof(float) * (size_t)g.Cp * g.Cg * g.K, stream);
   if (rc) return rc;

@@ -18,8 +18,12 @@ struct SharedPlan {
   // ... and wants the bias gradient (the sum of the weight gradient's pixel-side operand over
   // batch and pixels) from the weight-gradient kernel, into this cleared buffer.
   float* bias_sum = nullptr;
-  // The workspace holds the channels-last pixel-side tensor the columns route's scatter left.
-  bool pix_rows = false;
+  // Calls of the columns route.  The caller names the image of the weight gradient it will ask for,
+  // and the buffer that one writes the bias gradient to; the scatter says that it has laid out in the
+  // workspace what the weight gradient reads.
+  const float* wgrad_img = nullptr;
+  float* columns_bias = nullptr;
+  bool columns_prepared = false;
 };
 
 // Everything the fused kernels derive from the sample map alone, built once into a

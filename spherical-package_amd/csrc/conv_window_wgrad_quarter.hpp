@@ -57,7 +57,6 @@ constexpr int kWvE = 36;     // floats per window element: 32 channels + 4 of sk
 // bytes of one sample's column tile of a quarter: 32 pixels x 32 channels
 constexpr int col_bytes(int mm) { return mm == kMmBf16 ? 2048 : 4096; }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // Byte of 16-byte piece q (8 channels) of pixel p in a column tile.  The pieces of each four
 // pixels change places in a way of their own, so that equal pieces of the pixels that are written
@@ -70,19 +69,6 @@ __device__ __forceinline__ unsigned col_at(int p, int q) {
 // lie side by side, in different halves of the banks.
 __device__ __forceinline__ unsigned col32_at(int p, int q) {
   return (unsigned)(((p & 16) | ((p & 7) << 1) | ((p >> 3) & 1)) * 128 + ((q ^ (p & 7)) << 4));
-}
-
-__device__ __forceinline__ Bf16Frag tr_frag(const char* lo, const char* hi) {
-  typedef __attribute__((address_space(3))) s16x4* Lds;
-  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(lo));
-  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(hi));
-  const u32x2 ua = __builtin_bit_cast(u32x2, a), ub = __builtin_bit_cast(u32x2, b);
-  Bf16Frag r;
-  r.u[0] = ua.x;
-  r.u[1] = ua.y;
-  r.u[2] = ub.x;
-  r.u[3] = ub.y;
-  return r;
 }
 
 // CAP: kRegionCap: the tiles of `list` lie inside their window; kBigCap: big tiles.

@@ -83,6 +83,24 @@ __device__ __forceinline__ floatx16 mfma_split(const Bf16Split& a, const Bf16Spl
   return mfma_bf16(a.hi, b.hi, c);
 }
 
+// Operand of eight reduction elements from two transposing LDS reads, four each: lane l names the 8 bytes of
+// elements 8 (l / 32) + (l % 16) / 4 (`hi`: four further on), columns 16 ((l / 16) % 2) + 4 (l % 4) .. + 3,
+// and gets column l % 32 of the four elements its group of 16 lanes names.
+__device__ __forceinline__ Bf16Frag tr_frag(const char* lo, const char* hi) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) s16x4* Lds;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(lo));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)(hi));
+  const u32x2_t ua = __builtin_bit_cast(u32x2_t, a), ub = __builtin_bit_cast(u32x2_t, b);
+  Bf16Frag r;
+  r.u[0] = ua.x;
+  r.u[1] = ua.y;
+  r.u[2] = ub.x;
+  r.u[3] = ub.y;
+  return r;
+}
+
 // Matrix arithmetic of a fused kernel: fp32 MFMA, operands rounded to bf16, or fp32 operands
 // split into bf16 pieces (fp32 accuracy on the bf16 matrix unit).
 constexpr int kMmF32 = 0, kMmBf16 = 1, kMmSplit = 2;

@@ -1,5 +1,5 @@
-"""The forward of small calls that blends its columns on the way to LDS
-(csrc/conv_columns_forward.hip), against the oracle."""
+"""Small calls whose columns are blended on the way to LDS (csrc/conv_columns_direct.hip), against the
+oracle."""
 import pytest
 import torch
 
@@ -25,7 +25,8 @@ def oracle():
 # blocks a tile may have and one over (32 .. 161 channels), tiles of one pixel and one over 32
 # pixels, one and several groups and splits of the reduction (K * Cin of 32 steps and more on few
 # tiles), runs of samples that share no table of taps (25 samples, weighted samples of up to 16
-# taps, channel counts whose steps of 32 straddle samples), calls with more tiles than XCDs' shares
+# taps, channel counts whose steps and tiles of 32 straddle samples), calls with more tiles than XCDs'
+# shares, and one with more strips of pixels than a wave of the weight gradient's sums adds up
 SIZES = [
     (1, 8, 32, 6, 9, 3, 11, 9, 0, 1),
     (1, 40, 33, 6, 9, 3, 11, 9, 0, 2),
@@ -42,17 +43,19 @@ SIZES = [
     (1, 96, 48, 9, 14, 5, 7, 25, 2, 1),
     (3, 12, 20, 40, 80, 40, 80, 9, 0, 1),
     (1, 16, 64, 64, 128, 64, 128, 9, 4, 1),
+    (4100, 8, 8, 4, 4, 2, 2, 1, 0, 1),
+    (5, 24, 70, 20, 31, 17, 31, 9, 2, 2),
 ]
 
 
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
 @pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
-def test_forward_matches_the_oracle(ops, oracle, tc, mode):
+def test_contractions_match_the_oracle(ops, oracle, tc, mode):
     from _spherical_distortion_ext import _capi
     B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
     assert _capi.load().sdk_mapped_conv_by_columns(B, Cin, Cout, H, W, OH, OW, K, P, interp,
                                                    _capi.SDK_F32, 0, 0) == 1
-    m, iw, x, w, b, _, _ = columns._arrays(tc)
+    m, iw, x, w, b, g, _ = columns._arrays(tc)
     t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
     odd = torch.empty(m.size + 1, device=DEV)[1:].view(m.shape).copy_(t(m))   # 4 bytes off a pair's place
     want = oracle.mapped_conv_forward(x, m, w, b, K, interp, iw)
@@ -61,8 +64,16 @@ def test_forward_matches_the_oracle(ops, oracle, tc, mode):
     with ops.conv_compute(mode):
         y = ops.ops.mapped_conv_forward(t(x), t(m), t(iw), t(w), t(b), K, interp)
         again = ops.ops.mapped_conv_forward(t(x), odd, t(iw), t(w), t(b), K, interp)
+        grads = ops.ops.mapped_conv_backward(t(g), t(m), t(iw), t(x), t(w), t(b), K, interp)
+        weights_alone = ops.ops.mapped_conv_backward_select(t(g), t(m), t(iw), t(x), t(w), K, interp,
+                                                            False, False, True)
     assert columns._rel(y.cpu().numpy(), want) <= tol
     assert torch.equal(y, again)
+    for have, want in zip(grads, oracle.mapped_conv_backward(g, m, x, w, b, K, interp, iw)):
+        assert columns._rel(have.cpu().numpy(), want) <= tol
+    assert torch.equal(weights_alone[1], grads[1])
+    # (a bias gradient of many strips is added up by atomics, in any order)
+    assert columns._rel(weights_alone[2].cpu().numpy(), grads[2].cpu().numpy()) <= 5e-6
 
 
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
