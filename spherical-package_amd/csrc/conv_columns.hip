@@ -400,12 +400,12 @@ __global__ __launch_bounds__(kClThreads) void columns_wgrad_sum_kernel(
 // 24 us with S = 1, 22 with S = 2; 96 channels 17 us in two chunks of 64, 15 in three of 32.  grid (blocks of
 // elements, channel chunks, batch).
 // A list of more than kClLong entries (a map that sends many samples to one image element, invalid ones
-// for instance) is the whole workgroup's: sixteen entries in turn for each group of L lanes, whose
+// for instance) is the whole workgroup's: eight entries in turn for each group of L lanes, whose
 // sums are added in their order.  (64 channels, 1 x 128 x 256, a tenth of 295 thousand samples on
-// one spot, backward: 365 us with eight entries, 288 now; 124 without the spot.)
+// one spot, backward: 365 us with 16 lanes, 219 with 8; 117 without the spot.)
 constexpr int kClLong = 256;
 template <int L, int S>
-__global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
+__global__ __launch_bounds__(kClThreads, 6) void columns_col2im_kernel(
     const float* __restrict__ col, const int* __restrict__ offset, const int* __restrict__ src,
     const float* __restrict__ co, const float* __restrict__ bias, float* __restrict__ img, int Cg,
     int C4, int HW, int samples) {
@@ -417,6 +417,7 @@ __global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
   const vec4* col_b = reinterpret_cast<const vec4*>(col) + (size_t)blockIdx.z * samples * C4 +
                       min(c0 / 4 + q, C4 - 1);
   vec4 acc = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kShort = 8 / S, kLong = 8;   // entries of a lane in flight
   // acc += this lane's shares (U entries of each S * U) of the entries from beg on, S * U and then `step`
   // further each turn, before end (> 0); those of the next turn are named before this one's products are here
   auto add = [&](auto count, int beg, int end, int step) {
@@ -447,7 +448,6 @@ __global__ __launch_bounds__(kClThreads) void columns_col2im_kernel(
         if (e + i < end) acc += here[i] * v[i];
     }
   };
-  constexpr int kShort = 8 / S, kLong = 16;   // entries of a lane in flight
   const int u = min(u0 + t, HW - 1);
   const int beg = offset[u], end = offset[u + 1];
   if (end - beg <= kClLong) add(std::integral_constant<int, kShort>(), beg, end, 8);
@@ -725,8 +725,7 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
          dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, img, g.Cg, C4, HW, g.M * g.K)
   if (C4 <= 2) CI(2, 4);
   else if (C4 <= 4) CI(4, 4);
-  else if (ceil_div(C4, 16) * 2 > ceil_div(C4, 8)) CI(8, 2);
-  else CI(16, 2);
+  else CI(8, 2);   // (sixteen lanes: 22 us instead of 23 for 64 channels, a long list half as fast)
 #undef CI
   SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
   return SDK_OK;

@@ -18,7 +18,7 @@
 // 60 -> 47; 96 -> 160, 6 x 50 x 100, stride 2, split 52 -> 37; 104 -> 37, 2 x 41 x 83, float32 46 -> 23; 200 -> 37,
 // 3 x 45 x 91, split 82 -> 47; 256 -> 256, 5 x 5, 2 x 24 x 48, stride 2, split 149 -> 45; 24 -> 32, 2 x 115 x 231,
 // float32 50 -> 27.  Forward and backward of the same:
-// 206 -> 166, 170 -> 127, 130 -> 118 (host), 251 -> 176, 264 -> 126, 177 -> 119 (host).
+// 206 -> 156, 170 -> 124, 130 -> 87, 251 -> 171, 264 -> 125, 177 -> 114.
 // What bounds it: in float32 the MFMAs (half of the forward at 64 -> 64) and the vector
 // instructions of the blend, which do not overlap them; in the others the blend, and the reads of operands and
 // taps by too few waves.
@@ -65,7 +65,7 @@ struct DirectArgs {
 };
 
 template <bool WGRAD, int MM, int RA, int G, int NT>
-__global__ __launch_bounds__(64 * RA * G, (RA > 3 || (RA > 1 && MM != kMmSplit) ? 3 : 2)) void columns_direct_kernel(DirectArgs g) {
+__global__ __launch_bounds__(64 * RA * G, (RA > 1 && (MM != kMmSplit || (RA > 3 && !WGRAD)) ? 3 : 2)) void columns_direct_kernel(DirectArgs g) {
   constexpr int BN = kDirectPixels, GT = 64 * RA, NI = (8 * BN + GT - 1) / GT, RB = row_bytes(MM);
   constexpr int kThreads = GT * G;
   // steps on their way: one hides behind the float32 MFMAs; two of four samples a thread would not fit the registers
@@ -154,9 +154,14 @@ __global__ __launch_bounds__(64 * RA * G, (RA > 3 || (RA > 1 && MM != kMmSplit) 
   if (NT == 4 && g.P != 0 && threadIdx.x == 0) s_most = 0;
 
   // Forward: the even and the odd turns of a single group are summed apart, as two groups' are (864 products a
-  // sum, 96 -> 160: 3.2e-7 off float64 in the norm so, 4.5e-7 in one chain).  Weight gradient: two turns at a
-  // time are summed apart and then added, sum[1] the sums: its reduction is hundreds of pixels.
+  // sum, 96 -> 160: 3.2e-7 off float64 in the norm so, 4.5e-7 in one chain).  Weight gradient: its reduction is
+  // hundreds of pixels, so one turn at a time (split operands: two) is summed apart and then added, sum[1] the sums.
+  // Distance from float64, 1e-7 of the norm, with 1, 2, 4 turns and all of a split in a chain: 96 -> 160, 7500 pixels,
+  // float32 1.6, 1.7, 2.2, 5.5, split 1.9, 1.8, 2.0, 4.9; 8 -> 8, 86 thousand pixels, float32 1.6, 1.9, 2.3, 2.3,
+  // split 4.0, 3.2, 3.2, 3.2.
+  constexpr int kAlone = MM == kMmSplit ? 2 : 1;
   constexpr bool kTwo = WGRAD || G == 1;
+  int done = 0;
   floatx16 sum[kTwo ? 2 : 1] = {};
 
   const int quad = tid & 7, px0 = tid >> 3;
@@ -172,7 +177,8 @@ __global__ __launch_bounds__(64 * RA * G, (RA > 3 || (RA > 1 && MM != kMmSplit) 
     // ---- a run: steps t0 .. t1 - 1, samples k0 .. k0 + samples - 1
     const int samples = g.cap / each;
     const int k0 = WGRAD ? 0 : t0 * kDirectStep / g.Cgp;
-    const int t1 = WGRAD ? min(t_end, t0 + max(1, samples / nk))
+    const int run = max(1, samples / nk);   // (whole turns where there are any)
+    const int t1 = WGRAD ? min(t_end, t0 + (run > G ? run - run % G : run))
                          : min(t_end, k0 + samples >= g.K ? g.steps : max(t0 + 1, (k0 + samples) * g.Cgp / kDirectStep));
     __syncthreads();   // the run before is done with the table
     const int held = WGRAD ? min(samples, (t1 - t0) * nk) : min(samples, g.K - k0);
@@ -281,32 +287,44 @@ __global__ __launch_bounds__(64 * RA * G, (RA > 3 || (RA > 1 && MM != kMmSplit) 
     };
     auto stash = [&](int st, int buf) {
       char* dst = lds + tile0 + buf * BN * RB;
+      vec4 blend[NI];
+      auto place_of = [&](int i) { return NI * GT == 8 * BN ? px0 + i * kRowStep : min(px0 + i * kRowStep, BN - 1); };
+      if constexpr (NT == 4) {
+        auto add = [&](int e, bool first) {
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const vec4 w = *reinterpret_cast<const vec4*>(s_co + (e * BN + place_of(i)) * 4);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              float f = first ? w[0] * v[st][i][0][x] : __builtin_fmaf(w[0], v[st][i][0][x], blend[i][x]);
+              f = __builtin_fmaf(w[1], v[st][i][1][x], f);
+              f = __builtin_fmaf(w[2], v[st][i][2][x], f);
+              blend[i][x] = __builtin_fmaf(w[3], v[st][i][3][x], f);
+            }
+          }
+        };
+        add(at_e[st], true);
+        for (int q = 1; q < each; ++q) {   // (more taps than four: read here, those of all samples together)
+          const int e = min(at_e[st] + q, g.cap);
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const ivec4 o = *reinterpret_cast<const ivec4*>(s_off + (e * BN + place_of(i)) * 4);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              v[st][i][x] = *reinterpret_cast<const vec4*>(rows_b + (unsigned)(o[x] + at_c[st]));
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          add(e, false);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) blend[i] = v[st][i][0];
+      }
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int px = px0 + i * kRowStep;
         if (NI * GT != 8 * BN && px >= BN) break;
-        vec4 s;
-        if constexpr (NT == 4) {
-          const vec4 w = *reinterpret_cast<const vec4*>(s_co + (at_e[st] * BN + px) * 4);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            s[x] = w[0] * v[st][i][0][x];
-            s[x] = __builtin_fmaf(w[1], v[st][i][1][x], s[x]);
-            s[x] = __builtin_fmaf(w[2], v[st][i][2][x], s[x]);
-            s[x] = __builtin_fmaf(w[3], v[st][i][3][x], s[x]);
-          }
-          for (int q = 1; q < each; ++q)
-#pragma unroll
-            for (int y = 0; y < 4; ++y) {
-              const int at = (min(at_e[st] + q, g.cap) * BN + px) * 4 + y;
-              const float w = s_co[at];
-              const vec4 r = *reinterpret_cast<const vec4*>(rows_b + (unsigned)(s_off[at] + at_c[st]));
-#pragma unroll
-              for (int x = 0; x < 4; ++x) s[x] = __builtin_fmaf(w, r[x], s[x]);
-            }
-        } else {
-          s = v[st][i][0];
-        }
+        const vec4 s = blend[i];
         char* row = dst + px * RB;
         if constexpr (MM == kMmF32) {
           *reinterpret_cast<vec4*>(row + 16 * quad) = s;
@@ -355,9 +373,9 @@ __global__ __launch_bounds__(64 * RA * G, (RA > 3 || (RA > 1 && MM != kMmSplit) 
       fetch(kNext);
       __builtin_amdgcn_sched_barrier(0);
       const char* src = lds + tile0 + kBuf * BN * RB;
-      floatx16& acc = sum[!WGRAD && G == 1 ? kBuf : 0];
-      if constexpr (WGRAD && kBuf == 0) {
-        sum[1] += acc;
+      floatx16& acc = sum[kTwo && !WGRAD ? kBuf : 0];
+      if (WGRAD && done++ % kAlone == 0) {
+        sum[kTwo ? 1 : 0] += acc;
         acc = floatx16{};
       }
       if (now < t1) {   // (the last turn of a run may have no step left for this group)
@@ -765,7 +783,7 @@ DirectShape direct_shape(const ConvGeom& g) {
 
 // The weight gradient's: tiles of 32 columns (k, c) and of at most five blocks of 32 channels, the pixels in
 // splits of at least four turns.  Its kernel alone, us, with 1024, 2048 and 4096 waves: 160 rows (one tile of five
-// blocks, a workgroup a CU), 6 x 25 x 50, 96 -> 160, split 31, 35, 42; 64 rows, 128 x 256, 64 -> 64, float32 68, 61,
+// blocks: one workgroup a CU; 1536, where some CUs have two, 54), 6 x 25 x 50, 96 -> 160, split 31, 35, 42; 64 rows, 128 x 256, 64 -> 64, float32 68, 61,
 // 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55, 45, 42; 32 rows, 2 x 115 x 231,
 // 24 -> 32, float32 42, 26, 31.
 struct WgradShape {
@@ -782,8 +800,8 @@ WgradShape wgrad_shape(const ConvGeom& g) {
   t.samples = pad8(g.Cg) % 32 == 0 ? 1 : std::min(g.K, pad8(g.Cg) == 8 ? 4 : 2);
   t.steps = (int)(g.B * t.strips);
   const int64_t waves = (int64_t)t.tiles_a * t.tiles_r * t.ra * t.groups;
-  const int64_t wanted = t.ra == 5 ? 1024 : (t.ra == 1 ? 2048 : 4096);
-  const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(ceil_div(wanted, waves), t.steps / (4 * t.groups)));
+  const int64_t wanted = t.ra == 5 ? 256 / ((int64_t)t.tiles_a * t.tiles_r) : ceil_div(t.ra == 1 ? 2048 : 4096, waves);
+  const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(wanted, t.steps / (4 * t.groups)));
   t.split_steps = (int)ceil_div(t.steps, splits);
   t.splits = (int)ceil_div(t.steps, t.split_steps);
   return t;
@@ -846,14 +864,14 @@ int direct(const ConvGeom& g, int mm, DirectArgs a, int ra, int groups, int samp
   // touch, if each has four taps a point
   const size_t rows = (size_t)groups * 2 * kDirectPixels * row_bytes(mm);
   const size_t entry = (size_t)kDirectPixels * (single ? 1 : 4) * 8;
-  const int fit = (int)((65536 - 1024 - rows) / entry) - 1;   // 64 KB of LDS
+  const int fit = (int)((80 * 1024 - 1024 - rows) / entry) - 1;   // half a CU's LDS
   a.cap = std::min(WGRAD ? std::min(40, std::max(4, a.split_steps * samples)) : std::min(g.K, 9), std::max(fit, 9));
   if (g.P != 0) a.cap = std::max(a.cap, (WGRAD ? 4 : 5) * (int)ceil_div((int64_t)g.P * (blended ? 4 : 1), 4));
   const size_t tiles = rows + (a.cap + 1) * entry;
   const size_t sums = (size_t)(groups - 1) * 16 * 64 * ra * 4;
   const size_t smem = std::max(tiles, sums);
   const dim3 block((unsigned)(64 * ra * groups));
-  hipError_t reserved = hipSuccess;   // (weighted samples of up to sixteen taps, four groups of split operands: 74 KB)
+  hipError_t reserved = hipSuccess;   
 #define CF3(MMv, RAv, Gv, NTv)                                                                                \
   do {                                                                                                        \
     const auto kernel = columns_direct_kernel<WGRAD, MMv, RAv, Gv, NTv>;                                      \
@@ -917,7 +935,9 @@ DirectArgs direct_args(const ConvGeom& g, const float* rows, const float* map, c
 
 }  // namespace
 
-// (Maps with more points a sample would need a larger table of taps.)
+// (With more points a sample its taps are too many to be read turn by turn: 64 -> 64, 128 x 256, bilinear points,
+// forward and backward of the other kernels and of these, us: two points 222 and 238, four 302 and 338, six 361 and
+// 484, eight 470 and 648, split; with the four taps that four weighted pixels have 180 and 133, bf16.)
 bool columns_direct(const ConvGeom& g) { return pts(g.P) <= 4; }
 
 // (six bytes a value: the split's pieces, the largest form)
