@@ -497,6 +497,15 @@ struct ColumnsLayout {
 
 size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(g.Cg); }
 
+// The columns of a scatter go through in slices of this many batch elements, so that a slice is still in the 256 MB
+// memory-side cache when it is read back (4 x 128 x 256, 64 -> 64, backward: 474 us in one piece of 288 MB, 442 in
+// two, 421 in four).
+constexpr size_t kSliceBytes = (size_t)128 << 20;
+size_t slice_elements(const ConvGeom& g) {
+  const size_t one = sizeof(float) * column_values(g) / g.B;
+  return std::max<size_t>(1, std::min<size_t>((size_t)g.B, kSliceBytes / one));
+}
+
 ColumnsLayout columns_layout(const ConvGeom& g) {
   const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp);
   ColumnsLayout l{};
@@ -507,14 +516,15 @@ ColumnsLayout columns_layout(const ConvGeom& g) {
     return here;
   };
   l.img_rows = take(sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp);   // (and a row of zeros)
-  l.col = take(sizeof(float) * column_values(g));
   if (columns_direct(g)) {
+    l.col = take(std::max(sizeof(float) * slice_elements(g) * (column_values(g) / g.B), columns_forward_sum_bytes(g)));
     l.weights = take(columns_weight_bytes(g));
     l.pix_rows = take(columns_pixel_bytes(g));
     l.pix_cols = take(columns_pixel_bytes(g));
     l.strip_sums = take(columns_strip_bytes(g));
     l.partial = take(columns_partial_bytes(g));
   } else {
+    l.col = take(sizeof(float) * column_values(g));
     l.weights = take(sizeof(float) * g.K * Cgp * Cpp);
     l.pix_rows = take(sizeof(float) * g.B * g.M * Cpp);
     // the weight gradient's reduction (all pixels of the batch) in splits: about two
@@ -602,19 +612,36 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
   return SDK_OK;
 }
 
-// Column matrices of at most this many bytes take the route.  Measured against the fused kernels,
-// forward + backward of one layer on a kept plan, 3 x 3 kernels (before -> columns):
-//   25 MB  6 x 50 x 100, stride 2, 96 -> 160, split   899 -> 190 us
-//   36 MB  2 x 64 x 128, 64 -> 64, float32            327 -> 160 us
-//   72 MB  1 x 128 x 256, 64 -> 64, float32 / bf16    347 -> 235 / 271 -> 195 us
-//   84 MB  3 x 45 x 91, 200 -> 37, split              570 -> 275 us
-//  144 MB  8 x 64 x 128, 64 -> 128, float32 / bf16    621 -> 585 / 396 -> 470 us: no gain left, the
-//          tiles fill the GPU by then
-// Nearest taps cost the fused kernels least, their line lies lower: 4 x 128 x 256, 32 -> 32
-// (144 MB) 250 -> 380 us.
-constexpr size_t kColumnsBytes = (size_t)100 << 20, kColumnsNearestBytes = (size_t)36 << 20;
-size_t column_limit(const ConvGeom& g) {
-  return g.interp == 0 && g.P == 0 ? kColumnsNearestBytes : kColumnsBytes;
+// Calls whose column matrix has at most this many bytes take the route (a scatter holds a slice of it, the others
+// none of it).  Forward + backward on a kept plan, 3 x 3 kernels, us of the tile kernels and of these, float32 /
+// bf16 / split:
+//   126 MB  4 x 120 x 240, 32 -> 32            275 / 199 / 241 and 228 / 179 / 224
+//   131 MB  2 x 100 x 200, 96 -> 160           992 / 379 / 688 and 617 / 251 / 460
+//   142 MB  4 x 90 x 180, 64 -> 64             373 / 242 / 307 and 293 / 188 / 274
+//   175 MB  4 x 200 x 400, 16 -> 16            444 / 276 / 367 and 384 / 306 / 403
+//   288 MB  4 x 128 x 256, 64 -> 64            513 / 284 / 400 and 558 / 344 / 530
+// nearest taps
+//    72 MB  2 x 128 x 256, 32 -> 32            183 / 174 / 173 and 119 / 116 / 119
+//   108 MB  4 x 64 x 128, 96 -> 96             515 / 249 / 390 and 285 / 123 / 217
+//   144 MB  2 x 256 x 512, 12 -> 24            290 / 196 / 244 and 241 / 167 / 244
+//   288 MB  4 x 128 x 256, 64 -> 64            460 / 247 / 356 and 480 / 253 / 415
+// Above ten samples the tile kernels' weight gradient is another, and there is no such line, 5 x 5:
+//   400 MB  2 x 128 x 256, 64 -> 64            1814 / 1399 / 1646 and 751 / 477 / 706
+//   693 MB  8 x 169 x 336, 16 -> 56            4048 / 2940 / 3520 and 1697 / 1169 / 1640
+//   793 MB  1 x 200 x 400, 104 -> 88           4324 / 2405 / 3269 and 2537 / 1597 / 2155
+// Weighted samples stop at the line their calls had when the columns went through memory, for those whose
+// samples have more than four taps.
+constexpr size_t kColumnsBytes = (size_t)150 << 20, kColumnsWeightedBytes = (size_t)100 << 20;
+constexpr int kTileSamples = 10;
+// ... and the tensors laid out for them (32-bit byte offsets into the image's rows)
+constexpr size_t kColumnsTensorBytes = (size_t)1 << 30, kColumnsElementBytes = (size_t)2 << 30;
+bool columns_fit(const ConvGeom& g) {
+  const size_t image = sizeof(float) * g.B * g.H * g.W * pad8(g.Cg), pixels = sizeof(float) * g.B * g.M * pad8(g.Cp);
+  const size_t columns = sizeof(float) * column_values(g);
+  if (g.K > kTileSamples && columns_direct(g))
+    return columns / g.B <= kColumnsElementBytes && image <= kColumnsTensorBytes && pixels <= kColumnsTensorBytes;
+  const size_t limit = g.P == 0 ? kColumnsBytes : kColumnsWeightedBytes;
+  return columns <= limit && image <= 2 * limit && pixels <= 2 * limit;
 }
 
 thread_local bool t_columns = true;
@@ -622,16 +649,14 @@ thread_local bool t_columns = true;
 }  // namespace
 
 bool columns_map(const ConvGeom& g) {
-  return g.M >= 1 && g.K >= 1 && (int64_t)g.M * g.K <= ((int64_t)1 << 20) && pts(g.P) <= 8 &&
+  // (the lists of the inverted map: 32 bytes a sample of four taps)
+  const int64_t most = !columns_direct(g) ? (int64_t)1 << 20 : (g.K > kTileSamples ? (int64_t)1 << 24 : (int64_t)1 << 21);
+  return g.M >= 1 && g.K >= 1 && (int64_t)g.M * g.K <= most && pts(g.P) <= 8 &&
          col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp) != 0;
 }
 
 bool columns_route(const ConvGeom& g) {
-  const size_t limit = column_limit(g);
-  return t_columns && g.B >= 1 && g.B <= 65535 && g.Cg >= 5 && columns_map(g) &&
-         column_values(g) * sizeof(float) <= limit &&
-         (size_t)g.B * g.H * g.W * pad8(g.Cg) * sizeof(float) <= 2 * limit &&
-         (size_t)g.B * g.M * pad8(g.Cp) * sizeof(float) <= 2 * limit &&
+  return t_columns && g.B >= 1 && g.B <= 65535 && g.Cg >= 5 && columns_map(g) && columns_fit(g) &&
          (size_t)pad8(g.Cp) * g.K * pad8(g.Cg) < ((size_t)1 << 31);
 }
 
@@ -692,43 +717,54 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
     if (rc) return rc;
     lists = ws + l.lists;
   }
-  if (columns_direct(g)) {
-    rc = columns_direct_product(g, mm, pix, Wm, wgrad_img, bias_sum, columns_scratch(l, ws), stream);
-    if (rc) return rc;
-  } else {
-    rc = to_rows(pix, rows, g.B, g.Cp, g.M, stream);
-    if (rc) return rc;
-    const int total = R * Cpp;
-    launch(columns_weight_kernel<true>, dim3((unsigned)ceil_div(total, kClThreads)),
-           dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, Cpp, total);
-    SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
-    // all pixels of the batch are the rows of one product
-    GemmArgs a{};
-    a.A = rows;
-    a.B = w;
-    a.C = col;
-    a.rows_a = (int)(g.B * g.M);
-    a.rows_b = R;
-    a.red = Cpp;
-    a.lda = a.ldb = Cpp;
-    a.ldc = (size_t)R;
-    rc = gemm<false>(mm, a, 1, stream);
-    if (rc) return rc;
-  }
   const Col2imView v = col2im_lists_view(lists, g.H, g.W, g.M, g.K, g.P, g.interp);
-  const int HW = g.H * g.W;
-  // as many lanes an element as its channels fill
-  const int C4 = Cgp / 4;
-#define CI(Lv, Sv)                                                                                          \
-  launch((columns_col2im_kernel<Lv, Sv>),                                                                   \
-         dim3((unsigned)ceil_div(HW, kClThreads / (Lv * Sv)), (unsigned)ceil_div(C4, Lv), (unsigned)g.B),   \
-         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, img, g.Cg, C4, HW, g.M * g.K)
-  if (C4 <= 2) CI(2, 4);
-  else if (C4 <= 4) CI(4, 4);
-  else CI(8, 2);   // (sixteen lanes: 22 us instead of 23 for 64 channels, a long list half as fast)
+  const int HW = g.H * g.W, C4 = Cgp / 4;
+  auto col2im = [&](int64_t first, int64_t elements) -> int {
+    float* out = img + (size_t)first * g.Cg * HW;
+    // as many lanes an element as its channels fill
+#define CI(Lv, Sv)                                                                                            \
+  launch((columns_col2im_kernel<Lv, Sv>),                                                                     \
+         dim3((unsigned)ceil_div(HW, kClThreads / (Lv * Sv)), (unsigned)ceil_div(C4, Lv), (unsigned)elements), \
+         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, out, g.Cg, C4, HW, g.M * g.K)
+    if (C4 <= 2) CI(2, 4);
+    else if (C4 <= 4) CI(4, 4);
+    else CI(8, 2);   // (sixteen lanes: 22 us instead of 23 for 64 channels, a long list half as fast)
 #undef CI
-  SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
-  return SDK_OK;
+    SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
+    return SDK_OK;
+  };
+  if (columns_direct(g)) {
+    const ColumnsScratch s = columns_scratch(l, ws);
+    rc = columns_direct_prepare(g, mm, pix, Wm, wgrad_img, bias_sum, s, stream);
+    if (rc) return rc;
+    const int64_t slice = (int64_t)slice_elements(g);
+    for (int64_t b0 = 0; b0 < g.B; b0 += slice) {
+      const int64_t elements = std::min<int64_t>(slice, g.B - b0);
+      rc = columns_direct_product(g, mm, b0, elements, s, stream);
+      if (rc == SDK_OK) rc = col2im(b0, elements);
+      if (rc) return rc;
+    }
+    return SDK_OK;
+  }
+  rc = to_rows(pix, rows, g.B, g.Cp, g.M, stream);
+  if (rc) return rc;
+  const int total = R * Cpp;
+  launch(columns_weight_kernel<true>, dim3((unsigned)ceil_div(total, kClThreads)),
+         dim3(kClThreads), stream, Wm, w, g.Cg, Cgp, g.K, g.Cp, Cpp, total);
+  SDK_LAUNCH_CHECK("mapped_conv(columns weights)");
+  // all pixels of the batch are the rows of one product
+  GemmArgs a{};
+  a.A = rows;
+  a.B = w;
+  a.C = col;
+  a.rows_a = (int)(g.B * g.M);
+  a.rows_b = R;
+  a.red = Cpp;
+  a.lda = a.ldb = Cpp;
+  a.ldc = (size_t)R;
+  rc = gemm<false>(mm, a, 1, stream);
+  if (rc) return rc;
+  return col2im(0, g.B);
 }
 
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,

@@ -47,16 +47,20 @@ struct ColumnsScratch {
 };
 bool columns_direct(const ConvGeom& g);
 size_t columns_weight_bytes(const ConvGeom& g);
+size_t columns_forward_sum_bytes(const ConvGeom& g);
 size_t columns_pixel_bytes(const ConvGeom& g);
 size_t columns_partial_bytes(const ConvGeom& g);
 size_t columns_strip_bytes(const ConvGeom& g);
 int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
                            const float* Wm, const float* bias, float* pix, const ColumnsScratch& s,
                            hipStream_t stream);
-// s.col[b][m][(k, c)] = sum over n of pix * Wm.  wgrad_img: that of a columns_direct_wgrad of the same call that
+// Lays out what columns_direct_product reads.  wgrad_img: that of a columns_direct_wgrad of the same call that
 // follows, laid out by the same launch; strip_sums: ... which is asked for the bias gradient.
-int columns_direct_product(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
+int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
                            bool strip_sums, const ColumnsScratch& s, hipStream_t stream);
+// s.col[b][m][(k, c)] = sum over n of pix * Wm, of batch elements first .. first + elements - 1.
+int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, const ColumnsScratch& s,
+                           hipStream_t stream);
 // gb: also gb[n] = sum of pix[b][n][m] (optional).
 int columns_direct_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map, const float* wts,
                          const float* img, float* gW, const ColumnsScratch& s, bool prepared, float* gb,

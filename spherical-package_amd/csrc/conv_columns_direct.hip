@@ -770,8 +770,7 @@ DirectShape direct_shape(const ConvGeom& g) {
   const int64_t tiles = (int64_t)t.tiles_a * t.tiles_m * g.B, waves = tiles * t.ra;
   int64_t splits = 1;
   if (tiles < 192 && t.steps >= 32) splits = std::min<int64_t>(384 / tiles, t.steps / 8);
-  // (the sums take the place of the column matrix in the workspace)
-  splits = std::max<int64_t>(1, std::min<int64_t>(splits, (int64_t)g.K * pad8(g.Cg) / g.Cp));
+  splits = std::max<int64_t>(1, splits);
   t.split_steps = (int)ceil_div(t.steps, splits);
   t.splits = (int)ceil_div(t.steps, t.split_steps);
   t.groups = waves >= 1024 || t.splits > 1 ? 1 : (waves >= 512 ? 2 : 4);
@@ -947,6 +946,10 @@ size_t columns_weight_bytes(const ConvGeom& g) {
   const int64_t product = ceil_div((int64_t)g.K * pad8(g.Cg), 32) * 2 * pixel_chunks(g);
   return (size_t)std::max(forward, product) * 64 * 16 * 3;
 }
+size_t columns_forward_sum_bytes(const ConvGeom& g) {
+  const DirectShape t = direct_shape(g);
+  return t.splits > 1 ? sizeof(float) * t.splits * g.B * g.Cp * g.M : 0;
+}
 size_t columns_pixel_bytes(const ConvGeom& g) {
   const WgradShape t = wgrad_shape(g);
   return (size_t)t.tiles_a * t.ra * t.steps * 2 * 64 * 16 * 3;
@@ -986,27 +989,31 @@ int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const fl
   return SDK_OK;
 }
 
-int columns_direct_product(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
+int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
                            bool strip_sums, const ColumnsScratch& s, hipStream_t stream) {
-  const int R = g.K * pad8(g.Cg), chunks = (int)pixel_chunks(g);
   PrepareArgs p = prepare_args(g);
   if (wgrad_img != nullptr) prepare_image(p, wgrad_img, s.img_rows);
-  prepare_weights(p, Wm, s.weights, true, (int)ceil_div(R, 32), 2 * chunks);
+  prepare_weights(p, Wm, s.weights, true, (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32), 2 * (int)pixel_chunks(g));
   prepare_pixels(p, pix, wgrad_img != nullptr ? s.pix_rows : nullptr, s.pix_cols, strip_sums ? s.strip_sums : nullptr);
-  int rc = prepare(mm, p, stream);
-  if (rc) return rc;
+  return prepare(mm, p, stream);
+}
+
+int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, const ColumnsScratch& s,
+                           hipStream_t stream) {
+  const int R = g.K * pad8(g.Cg);
   ProductArgs a{};
-  a.pixels = static_cast<const char*>(s.pix_cols);
   a.weights = static_cast<const char*>(s.weights);
   a.col = s.col;
   a.M = g.M;
   a.R = R;
   a.strips = (int)ceil_div(g.M, 32);
   a.tiles_r = (int)ceil_div(R, 64);
-  const int64_t tiles = (int64_t)g.B * a.strips * a.tiles_r;
+  const int64_t tiles = elements * a.strips * a.tiles_r;
   a.tiles = (int)tiles;
   a.steps = (int)ceil_div(g.Cp, 16);
-  a.stride = 2 * chunks;
+  a.stride = 2 * (int)pixel_chunks(g);
+  const int pieces = mm == kMmF32 ? 2 : (mm == kMmBf16 ? 1 : 3);
+  a.pixels = static_cast<const char*>(s.pix_cols) + (size_t)first * a.strips * a.stride * pieces * 1024;
   // float32: one wave a SIMD.  With two or more, their loads and MFMAs take turns: 64 -> 64, 128 x 256, 33 us with
   // one, 53 with four (21 without the MFMAs, 30 without the loads); MFMAs alone run at
   // 150 TFLOP/s with any number of waves, 16 of them beside six 16-byte loads at 130 with one and 70 with two.  bf16 operands want
