@@ -634,7 +634,7 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
 constexpr size_t kColumnsBytes = (size_t)150 << 20, kColumnsWeightedBytes = (size_t)100 << 20;
 constexpr int kTileSamples = 10;
 // ... and the tensors laid out for them (32-bit byte offsets into the image's rows)
-constexpr size_t kColumnsTensorBytes = (size_t)1 << 30, kColumnsElementBytes = (size_t)2 << 30;
+constexpr size_t kColumnsTensorBytes = (size_t)1 << 30, kColumnsElementBytes = (size_t)1 << 30;
 bool columns_fit(const ConvGeom& g) {
   const size_t image = sizeof(float) * g.B * g.H * g.W * pad8(g.Cg), pixels = sizeof(float) * g.B * g.M * pad8(g.Cp);
   const size_t columns = sizeof(float) * column_values(g);

@@ -695,7 +695,7 @@ bool fused_supported(const ConvGeom& g) {
 }
 
 bool columns_first(const ConvGeom& g) {
-  return !small_conv_supported(g) && !product_route(g) && columns_route(g);
+  return !small_conv_supported(g) && columns_route(g);
 }
 
 static bool inverse_candidate(const ConvGeom& g);
@@ -1143,13 +1143,6 @@ int fused_gemm_scatter(const ConvGeom& g, int compute, const float* pix, const f
     if (shared != nullptr) shared->valid = false;
     return small_scatter(g, pix, map, wts, Wm, img, stream);
   }
-  if (product_route(g)) {
-    // the image is finer than the pixel grid: products at the grid's resolution, then their
-    // splat as a gather (conv_product.hip)
-    if (shared != nullptr) shared->valid = false;
-    return product_gemm_scatter(g, pix, map, wts, Wm, bias, img, workspace, stream,
-                                cached != nullptr ? cached->col2im_lists : nullptr);
-  }
   if (columns_first(g)) {
     if (shared != nullptr) {
       shared->valid = false;
@@ -1159,6 +1152,13 @@ int fused_gemm_scatter(const ConvGeom& g, int compute, const float* pix, const f
                                 stream, cached != nullptr ? cached->columns_lists : nullptr,
                                 shared != nullptr ? shared->wgrad_img : nullptr,
                                 shared != nullptr && shared->columns_bias != nullptr);
+  }
+  if (product_route(g)) {
+    // the image is finer than the pixel grid: products at the grid's resolution, then their
+    // splat as a gather (conv_product.hip)
+    if (shared != nullptr) shared->valid = false;
+    return product_gemm_scatter(g, pix, map, wts, Wm, bias, img, workspace, stream,
+                                cached != nullptr ? cached->col2im_lists : nullptr);
   }
   const bool planned_fb = planned_scatter_supported(g);
   const int* generic_gate = nullptr;   // gate of the atomic scatter kernel at the end

@@ -11,8 +11,10 @@ namespace sdk {
 // product is then read once; a blended sample's would be read by each of its taps), the image
 // with at least twice the pixels of the map's grid.
 bool product_route_map(const ConvGeom& g);
-// Calls that take it: such a map, at least five image channels, 16 to 64 on the pixel side,
-// a column matrix [B, M * K, Cg] below 1 GiB.
+// Calls that take it, unless they run by columns altogether (conv_columns.hpp; level-6 icosphere, 2 x 48
+// channels, up-sampling and 1-ring layer, forward and backward: 488 us with this route for the one and
+// tile kernels for the other, 328 by columns): such a map, at least five image channels, 16 to 64 on the
+// pixel side, a column matrix [B, M * K, Cg] below 1 GiB.
 bool product_route(const ConvGeom& g);
 // Workspace of the route: the column matrix, then the inverted map (0: not taken).
 size_t product_workspace_bytes(const ConvGeom& g);
