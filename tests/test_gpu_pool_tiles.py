@@ -1,0 +1,57 @@
+"""Blended pooling by tiles (csrc/pool_blend.hip) whose boxes cross the image's seam, are as wide as the image,
+narrower than a group of columns or too large for LDS, in rows of one and of several tiles: bit for bit what the
+per-pixel kernels give (one point per sample with weight one), those against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from _spherical_distortion_ext import _ops
+    return _ops
+
+
+# (H, W, OH, OW, K, planes, columns a tap may stray)
+SIZES = [
+    (3, 3, 2, 2, 4, 1, 1), (3, 4, 2, 2, 4, 2, 1), (6, 7, 6, 7, 9, 3, 1), (9, 15, 9, 15, 9, 5, 2),
+    (9, 16, 9, 16, 9, 4, 0), (9, 17, 3, 5, 9, 4, 0), (24, 49, 12, 25, 9, 9, 3), (40, 90, 1, 1, 9, 6, 0),
+    (8, 40, 300, 1, 4, 7, 2), (10, 300, 5, 256, 9, 5, 2), (10, 300, 5, 257, 9, 5, 2), (12, 900, 6, 450, 9, 3, 6),
+    (12, 900, 12, 900, 4, 4, 40), (30, 60, 30, 60, 9, 50, 30), (64, 256, 8, 32, 9, 6, 128),
+    (150, 200, 40, 50, 4, 6, 100), (2, 13311, 1, 6, 9, 2, 9), (2, 13312, 1, 6, 9, 2, 9),
+]
+
+
+@pytest.mark.parametrize("interp", [1, 2])
+@pytest.mark.parametrize("tc", SIZES, ids=lambda t: "x".join(map(str, t)))
+def test_tiles_match_the_per_pixel_kernels(ops, oracle, tc, interp):
+    H, W, OH, OW, K, planes, stray = tc
+    rng = np.random.default_rng(sum(tc) + interp)
+    oy = np.arange(OH)[:, None, None] * (H / OH) + rng.uniform(-1.5, 1.5, (OH, OW, K))
+    ox = np.arange(OW)[None, :, None] * (W / OW) + rng.uniform(-1, 1, (OH, OW, K)) * (stray + 0.5)
+    ox += W / 3                                              # tiles whose box crosses the seam
+    ox[0], oy[-1, ::3] = rng.uniform(0, W, (OW, K)), rng.uniform(-1, H, (len(range(0, OW, 3)), K))
+    ox = np.where(rng.random(ox.shape) < 0.02, np.round(ox), ox)   # taps of weight zero
+    if interp == 1:
+        ox %= W
+    m = np.stack([ox, oy], -1).astype(np.float32)
+    m[-1, -1, 0] = (np.nan, -50)
+    x = rng.standard_normal((1, planes, H, W)).astype(np.float32)
+    x[0, -1, H // 2, W // 2], x[0, 0, 0, 0], x[0, -1, -1, -1] = np.inf, np.nan, -np.inf
+    tx, tm = torch.from_numpy(x).to(DEV), torch.from_numpy(m).to(DEV)
+    points, one = tm[..., None, :].contiguous(), torch.ones(tm.shape[:-1] + (1,), device=DEV)
+    v, i = ops.ops.mapped_max_pool(tx, tm, None, K, interp)
+    a = ops.ops.mapped_avg_pool(tx, tm, None, K, interp)
+    v1, i1 = ops.ops.mapped_max_pool(tx, points, one, K, interp)
+    a1 = ops.ops.mapped_avg_pool(tx, points, one, K, interp)
+    assert torch.equal(i, i1) and torch.equal(v, v1)
+    assert torch.equal(torch.nan_to_num(a, nan=7e9), torch.nan_to_num(a1, nan=7e9))
+    m[-1, -1, 0] = (-50, -50)
+    x = np.nan_to_num(x, nan=1.0, posinf=2.0, neginf=3.0)
+    a = ops.ops.mapped_avg_pool(torch.from_numpy(x).to(DEV), torch.from_numpy(m).to(DEV), None, K, interp)
+    # the same products and sums in the same order; K + 3 roundings where a compiler contracts
+    np.testing.assert_allclose(a.cpu().numpy(), oracle.mapped_avg_pool(x, m, K, interp), rtol=1e-6,
+                               atol=(K + 3) * 2.0 ** -22)
