@@ -1,4 +1,4 @@
-// Mapped convolution with the column matrix in memory, for calls so small that the fused
+// Mapped convolution as columns and matrix products, for calls so small that the fused
 // kernels cannot fill the GPU.
 //
 // The fused kernels (conv_window_gemm.hip, conv_window_wgrad.hip) own 128-pixel tiles and walk
@@ -6,12 +6,16 @@
 // few dozen workgroups on 256 CUs, each a serial chain of hundreds of dependent LDS and memory
 // steps, once per class of tiles.  The same work cut into an im2col, a matrix product and a
 // col2im (the reference's own order, ext_modules/src/cpp/mapped_convolution_layer.cpp:8-60)
-// has thousands of independent pieces per launch, and the column matrix, a few tens of MB,
-// stays in the 256 MB memory-side cache between the launch that writes it and the one that
-// reads it.  No tap plan is needed either: the map is read once per sample.
-// (Measured: 96 -> 160 channels, 6 x 50 x 100, stride 2, split, forward + backward 907 -> 180 us;
-// 64 -> 64 channels on a map not seen before, 1 x 128 x 256, forward 368 -> 62 us, of which 265
-// were its plan.)
+// has thousands of independent pieces per launch.  No tap plan is needed either: the map is read
+// once per sample.
+//
+// Here: which calls take the route, the layout of its workspace, the col2im, and the products of
+// columns that lie in memory, of samples of more than four points.  All others' columns exist only in
+// LDS, or, a scatter's, as the products of a slice of the batch that stays in the 256 MB memory-side
+// cache until the col2im reads them (conv_columns_direct.hip).
+// (Measured, on the fused kernels and so: 96 -> 160 channels, 6 x 50 x 100, stride 2, split,
+// forward + backward 907 -> 122 us; 64 -> 64 channels on a map not seen before, 1 x 128 x 256,
+// forward 368 -> 50 us, of which 265 were its plan.)
 //
 // Everything is channels-last and padded with zeros to a multiple of eight channels, so that
 // every access of these kernels is an aligned 16-byte one:
@@ -34,7 +38,6 @@ namespace {
 
 constexpr int kClThreads = 256;
 typedef float vec4 __attribute__((ext_vector_type(4)));
-
 
 // dst[b][n][c] = src[b][c][n], c padded to Cp8 with zeros.  grid (tiles of 64 n, tiles of 32 c,
 // batch): the tile goes through LDS, reads run along n, writes along c.
