@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kBlendThreads, 3) void pool_blend_kernel(
     int64_t* __restrict__ idx, int planes, int H, int W, int OH, int OW, int R, int P, int tiles_x,
     int tiles_y, int chunks, int lds_floats) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  __shared__ int s_rows[2], s_cols[2], s_ref;
+  __shared__ int s_rows[2], s_cols[2], s_middle;
   const int t = threadIdx.x, M = OH * OW, tiles = tiles_x * tiles_y;
   const int unit = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int tile = unit % tiles, chunk = unit / tiles;
@@ -220,11 +220,11 @@ __global__ __launch_bounds__(kBlendThreads, 3) void pool_blend_kernel(
   if (t == 0) {
     s_rows[0] = s_cols[0] = INT_MAX;
     s_rows[1] = s_cols[1] = -1;
-    s_ref = (int)fminf(fmaxf(at[K / 2].x, 0.0f), (float)(W - 1));
+    s_middle = (int)fminf(fmaxf(at[K / 2].x, 0.0f), (float)(W - 1));
   }
   __syncthreads();
   // columns are counted from half the image's width before the first pixel's
-  int start = s_ref - W / 2;
+  int start = s_middle - W / 2;
   start += start < 0 ? W : 0;
   int rmin = INT_MAX, rmax = -1, cmin = INT_MAX, cmax = -1;
 #pragma unroll
