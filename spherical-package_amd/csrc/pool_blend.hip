@@ -11,7 +11,7 @@
 // Per pass the box of four planes goes to LDS interleaved, [element][plane], so that one
 // 16-byte LDS read serves a tap of four planes; the next pass's first groups are read while this
 // one is blended.  A box too large for four planes (at a pole it is as wide as the image) takes two or
-// one per pass, past that its taps come from global memory; the choice is made per workgroup.
+// one per pass, past that its taps come from global memory (blend_apart); the choice is made per workgroup.
 // Results are the per-pixel kernels' bit for bit: the same products, summed in the same order.
 // (Measured, us, average / maximum, per-pixel kernels or whole rows of the image in LDS -> so: 4 x 48 planes of
 // 190 x 378, stride 2, 51 / 54 -> 31 / 33; 8 x 64 of 256 x 512, stride 2, 120 / 132 -> 96 / 108; 4 x 32 of
@@ -192,6 +192,36 @@ __device__ __forceinline__ void run_blend(const float* __restrict__ in, float* _
   }
 }
 
+// A pooled pixel whose taps come from global memory, PC planes side by side, S samples of them in flight: a tap's
+// two neighbours of a row in one read.  Bound by the lines that the caches hold: planes that are no larger than
+// kBlendNear go four at a time, others alone.  (Uniformly random samples, average, us, an element a read and one
+// plane / four planes at a time -> pairs, one / two / four planes: 64 planes of 128 x 256, stride 2, 53 / 44 -> 46 /
+// 42 / 43; 4 x 48 of 190 x 378 370 / 300 -> 301 / 275 / 282; 8 x 64 of 256 x 512 1496 / 2207 -> 1473 / 2146 / 2248;
+// 64 of 300 x 600 600 / 459 -> 308 / 363 / 474; 128 of 512 x 1024 4498 / 4416 -> 3796 / 4563 / 4570.)
+constexpr size_t kBlendNear = 384 * 1024;
+template <bool AVG, int INTERP, int K, int PC, int S>
+__device__ __forceinline__ void blend_apart(const float* __restrict__ in, const float* __restrict__ map,
+                                            float* __restrict__ out, int64_t* __restrict__ idx, int pix,
+                                            int p_begin, int p_end, int H, int W, int M) {
+  const float* coords = map + (size_t)pix * K * 2;
+  for (int p = p_begin; p < p_end; p += PC) {
+    const int np = min(PC, p_end - p);
+    const float* base = in + (size_t)p * H * W;
+    BlendOp<AVG, K> op[PC];
+#pragma unroll S
+    for (int k = 0; k < K; ++k) {
+      float v[PC];
+      if (W >= 2) gather_pairs<float, INTERP, PC>(base, (size_t)H * W, np, coords[2 * k], coords[2 * k + 1], H, W, v);
+      else gather_sample<float, INTERP, false, PC>(base, (size_t)H * W, np, coords + 2 * k, nullptr, 0, H, W, v);
+#pragma unroll
+      for (int g = 0; g < PC; ++g) op[g].take(v[g], k);
+    }
+#pragma unroll
+    for (int g = 0; g < PC; ++g)
+      if (g < np) op[g].store(out, idx, (size_t)(p + g) * M + pix, pix);
+  }
+}
+
 // An XCD takes an eighth of the tiles of all plane chunks in turn, so whole chunks or parts of one:
 // the image elements neighbouring tiles share are read through one L2.  Tile rows from both poles
 // towards the equator: the widest boxes first.
@@ -291,22 +321,9 @@ __global__ __launch_bounds__(kBlendThreads, 3) void pool_blend_kernel(
     else
       run_blend<AVG, K, 1>(in, out, idx, lds, taps, pix, on, p_begin, p_end, HW, W, M, b);
   } else if (on) {
-    for (int p = p_begin; p < p_end; p += 4) {
-      BlendOp<AVG, K> op[4];
-#pragma unroll 1   // (a sample of four planes at a time: more in flight and the planes leave the caches, 300 -> 430 us)
-      for (int k = 0; k < K; ++k) {
-        PointTaps<float, INTERP> tp;
-        tp.set(coords[k].x, coords[k].y, H, W);
-        float v[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) v[g] = tp.gather(in + (size_t)min(p + g, p_end - 1) * HW);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) op[g].take(v[g], k);
-      }
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        if (p + g < p_end) op[g].store(out, idx, (size_t)(p + g) * M + pix, pix);
-    }
+    if (HW * sizeof(float) <= kBlendNear)
+      blend_apart<AVG, INTERP, K, 4, 1>(in, map, out, idx, pix, p_begin, p_end, H, W, M);
+    else blend_apart<AVG, INTERP, K, 1, 3>(in, map, out, idx, pix, p_begin, p_end, H, W, M);
   }
 }
 
