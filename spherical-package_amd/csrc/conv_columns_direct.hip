@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void columns_gradient_sum_kernel(const float* 
   if ((int)blockIdx.x >= weight_blocks) {
     const int n = ((int)blockIdx.x - weight_blocks) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (n >= Cp) return;
-    float sum = 0.f;
+    double sum = 0.0;   // (up to 64 strips a lane: in float32 1.8e-7 off float64 with 4096 strips, so 0.7e-7)
     for (int s = lane; s < strips; s += 256) {
       float v[4];
 #pragma unroll
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256) void columns_gradient_sum_kernel(const float* 
       for (int x = 0; x < 4; ++x) sum += s + 64 * x < strips ? v[x] : 0.0f;
     }
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
-    if (lane == 0) gb[n] = sum;
+    if (lane == 0) gb[n] = (float)sum;
     return;
   }
   const int e = blockIdx.x * 256 + threadIdx.x;   // (n, k, c), c fastest

@@ -1,9 +1,11 @@
 """Small calls whose columns are blended on the way to LDS (csrc/conv_columns_direct.hip), against the
 oracle."""
+import numpy as np
 import pytest
 import torch
 
 import test_gpu_columns as columns
+from conftest import runs_by_columns
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -74,6 +76,19 @@ def test_contractions_match_the_oracle(ops, oracle, tc, mode):
     assert torch.equal(weights_alone[1], grads[1])
     # (a bias gradient of many strips is added up by atomics, in any order)
     assert columns._rel(weights_alone[2].cpu().numpy(), grads[2].cpu().numpy()) <= 5e-6
+
+
+@pytest.mark.parametrize("height", [64, 128])
+def test_bias_gradient_keeps_the_bits_of_its_sums(ops, height):
+    """8 x 512 strips of 64 pixels a channel, the most that are added up here: in a float32 chain they were 1.8e-7
+    from float64 in the norm, the sums of before 1.4e-7.  A strip is a tree of six float32 additions and the result is
+    rounded once: 2^-24 * sqrt(7 / 3) = 0.9e-7 for random signs, on 128 channels within a fifth."""
+    tc = (8, 8, 128, 8, 16, height, 256, 1, 0, 1)
+    assert runs_by_columns(*tc)
+    m, _, x, w, b, g, _ = columns._arrays(tc)
+    t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    gb = ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 1, 1)[2]
+    assert columns._rel(gb.cpu().numpy(), g.astype(np.float64).sum((0, 2, 3))) <= 1.1e-7
 
 
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
