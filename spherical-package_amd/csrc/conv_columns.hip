@@ -11,8 +11,9 @@
 //
 // Here: which calls take the route, the layout of its workspace, the col2im, and the products of
 // columns that lie in memory, of samples of more than four points.  All others' columns exist only in
-// LDS, or, a scatter's, as the products of a slice of the batch that stays in the 256 MB memory-side
-// cache until the col2im reads them (conv_columns_direct.hip).
+// LDS, or, a scatter's, as the products of a slice of the batch or of its channels that, where 32 channels
+// of one element have no more, stays in the 256 MB memory-side cache until the col2im reads them
+// (conv_columns_direct.hip).
 // (Measured, on the fused kernels and so: 96 -> 160 channels, 6 x 50 x 100, stride 2, split,
 // forward + backward 907 -> 122 us; 64 -> 64 channels on a map not seen before, 1 x 128 x 256,
 // forward 368 -> 50 us, of which 265 were its plan.)
@@ -493,23 +494,52 @@ __global__ __launch_bounds__(kClThreads, 6) void columns_col2im_kernel(
 // ---------------------------------------------------------------------------
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// What a call's contractions take at a time.
+struct Slices {
+  bool both;
+  int64_t scatter, wgrad;   // elements of the batch
+  int channels;
+};
+
 struct ColumnsLayout {
   size_t pix_rows, pix_cols, img_rows, col, weights, partial, strip_sums, lists, total;
   int splits, split_len;
+  Slices slices;
 };
 
 size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(g.Cg); }
 
-// The columns of a scatter go through in slices of this many batch elements, so that a slice is still in the 256 MB
+// The products of a scatter go through in slices of so many batch elements that a slice is still in the 256 MB
 // memory-side cache when it is read back (4 x 128 x 256, 64 -> 64, backward: 474 us in one piece of 288 MB, 442 in
-// two, 421 in four).
-constexpr size_t kSliceBytes = (size_t)128 << 20;
-size_t slice_elements(const ConvGeom& g) {
-  const size_t one = sizeof(float) * column_values(g) / g.B;
-  return std::max<size_t>(1, std::min<size_t>((size_t)g.B, kSliceBytes / one));
+// two, 421 in four), at least one; an element that alone has more than that cache in chunks of so many channels, at
+// least 32, a run of 128 bytes (backward, float32 / bf16, us, whole and so: 793 MB, 104 -> 88, 200 x 400, 5 x 5 1973 /
+// 1363 and 1799 / 1138; 381 MB, 200 -> 160, 100 x 200 1636 / 801 and 1592 / 688; but 200 MB, 8 x 128 x 256, 64 -> 256,
+// whose pixels are as large, 6143 / 2624 and 6404 / 2713).
+// Both forms of the pixels' operands are laid out in one launch where they take no more than 128 MB; beyond that
+// each contraction lays out its own, one after the other in the same place, of elements of up to 128 MB (8 x 256 x
+// 512, 64 -> 64, 5 x 5, workspace 1938 -> 554 MB, backward 9864 -> 10041 us).
+constexpr size_t kSliceBytes = (size_t)128 << 20, kOperandBytes = (size_t)128 << 20, kCacheBytes = (size_t)256 << 20;
+Slices slices_of(const ConvGeom& g, int mm) {
+  const size_t samples = sizeof(float) * g.M * g.K;
+  const size_t rows = columns_pixel_row_bytes(g, mm, 1), cols = columns_pixel_column_bytes(g, mm, 1);
+  auto elements = [&](size_t most, size_t one) { return std::max<int64_t>(1, std::min<int64_t>(g.B, most / one)); };
+  Slices s;
+  s.both = g.B * (rows + cols) <= kOperandBytes;
+  s.wgrad = s.both ? g.B : elements(kOperandBytes, rows);
+  s.channels = pad8(g.Cg);
+  if (samples * s.channels > kCacheBytes && s.channels > 32) {
+    const int64_t most = std::max<int64_t>(1, kSliceBytes / (32 * samples));   // chunks of 32, shared out evenly
+    s.channels = std::min(s.channels, (int)(32 * ceil_div(s.channels, 32 * ceil_div(s.channels, 32 * most))));
+    s.scatter = 1;
+  } else {
+    s.scatter = elements(kSliceBytes, samples * s.channels);
+  }
+  if (!s.both) s.scatter = std::min(s.scatter, elements(kOperandBytes, cols));
+  return s;
 }
 
-ColumnsLayout columns_layout(const ConvGeom& g) {
+// mm: of the calls without a column matrix.
+ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
   const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp);
   ColumnsLayout l{};
   size_t at = 0;
@@ -518,15 +548,24 @@ ColumnsLayout columns_layout(const ConvGeom& g) {
     at += up256(bytes);
     return here;
   };
-  l.img_rows = take(sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp);   // (and a row of zeros)
+  const size_t image = sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp;   // (and a row of zeros)
   if (columns_direct(g)) {
-    l.col = take(std::max(sizeof(float) * slice_elements(g) * (column_values(g) / g.B), columns_forward_sum_bytes(g)));
+    const Slices& t = l.slices = slices_of(g, mm);
+    const size_t products = sizeof(float) * t.scatter * g.M * g.K * t.channels;
+    const size_t partial = std::max(columns_partial_bytes(g, t.wgrad), columns_forward_sum_bytes(g));
     l.weights = take(columns_weight_bytes(g));
-    l.pix_rows = take(columns_pixel_bytes(g));
-    l.pix_cols = take(columns_pixel_bytes(g));
     l.strip_sums = take(columns_strip_bytes(g));
-    l.partial = take(columns_partial_bytes(g));
+    const size_t base = at;
+    l.pix_cols = take(columns_pixel_column_bytes(g, mm, t.both ? g.B : t.scatter));
+    l.col = take(products);
+    const size_t end = at;
+    if (!t.both) at = base;
+    l.img_rows = take(image);
+    l.pix_rows = take(columns_pixel_row_bytes(g, mm, t.wgrad));
+    l.partial = take(partial);   // (not in the products' place: calls of a few us take 5 longer so)
+    at = std::max(at, end);
   } else {
+    l.img_rows = take(image);
     l.col = take(sizeof(float) * column_values(g));
     l.weights = take(sizeof(float) * g.K * Cgp * Cpp);
     l.pix_rows = take(sizeof(float) * g.B * g.M * Cpp);
@@ -653,7 +692,7 @@ thread_local bool t_columns = true;
 
 bool columns_map(const ConvGeom& g) {
   // (the lists of the inverted map: 32 bytes a sample of four taps)
-  const int64_t most = !columns_direct(g) ? (int64_t)1 << 20 : (g.K > kTileSamples ? (int64_t)1 << 24 : (int64_t)1 << 21);
+  const int64_t most = (int64_t)1 << (!columns_direct(g) ? 20 : (g.K > kTileSamples ? 24 : 21));
   return g.M >= 1 && g.K >= 1 && (int64_t)g.M * g.K <= most && pts(g.P) <= 8 &&
          col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp) != 0;
 }
@@ -666,14 +705,18 @@ bool columns_route(const ConvGeom& g) {
 // (a wave adds up a channel's strips)
 bool columns_sums_bias(const ConvGeom& g) { return columns_direct(g) && g.B * ceil_div(g.M, 64) <= 4096; }
 
+// (one size for every arithmetic)
 size_t columns_workspace_bytes(const ConvGeom& g) {
-  return columns_route(g) ? columns_layout(g).total : 0;
+  if (!columns_route(g)) return 0;
+  size_t most = 0;
+  for (int mm : {kMmF32, kMmBf16, kMmSplit}) most = std::max(most, columns_layout(g, mm).total);
+  return most;
 }
 
 int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float* map,
                         const float* wts, const float* Wm, const float* bias, float* pix,
                         void* workspace, hipStream_t stream) {
-  const ColumnsLayout l = columns_layout(g);
+  const ColumnsLayout l = columns_layout(g, mm);
   char* ws = static_cast<char*>(workspace);
   float* rows = reinterpret_cast<float*>(ws + l.img_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
@@ -708,7 +751,7 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
                          const float* wts, const float* Wm, const float* bias, float* img,
                          void* workspace, hipStream_t stream, const void* lists,
                          const float* wgrad_img, bool bias_sum) {
-  const ColumnsLayout l = columns_layout(g);
+  const ColumnsLayout l = columns_layout(g, mm);
   char* ws = static_cast<char*>(workspace);
   float* rows = reinterpret_cast<float*>(ws + l.pix_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
@@ -721,14 +764,17 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
     lists = ws + l.lists;
   }
   const Col2imView v = col2im_lists_view(lists, g.H, g.W, g.M, g.K, g.P, g.interp);
-  const int HW = g.H * g.W, C4 = Cgp / 4;
-  auto col2im = [&](int64_t first, int64_t elements) -> int {
-    float* out = img + (size_t)first * g.Cg * HW;
+  const int HW = g.H * g.W;
+  // channels c0 .. of so many batch elements, of one where they are not all
+  auto col2im = [&](int64_t first, int64_t elements, int c0, int padded) -> int {
+    float* out = img + ((size_t)first * g.Cg + c0) * HW;
+    const float* add = bias != nullptr ? bias + c0 : nullptr;
+    const int C4 = padded / 4, channels = std::min(padded, g.Cg - c0);
     // as many lanes an element as its channels fill
 #define CI(Lv, Sv)                                                                                            \
   launch((columns_col2im_kernel<Lv, Sv>),                                                                     \
          dim3((unsigned)ceil_div(HW, kClThreads / (Lv * Sv)), (unsigned)ceil_div(C4, Lv), (unsigned)elements), \
-         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, bias, out, g.Cg, C4, HW, g.M * g.K)
+         dim3(kClThreads), stream, (const float*)col, v.offset, v.src, v.co, add, out, channels, C4, HW, g.M * g.K)
     if (C4 <= 2) CI(2, 4);
     else if (C4 <= 4) CI(4, 4);
     else CI(8, 2);   // (sixteen lanes: 22 us instead of 23 for 64 channels, a long list half as fast)
@@ -738,13 +784,18 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
   };
   if (columns_direct(g)) {
     const ColumnsScratch s = columns_scratch(l, ws);
-    rc = columns_direct_prepare(g, mm, pix, Wm, wgrad_img, bias_sum, s, stream);
-    if (rc) return rc;
-    const int64_t slice = (int64_t)slice_elements(g);
-    for (int64_t b0 = 0; b0 < g.B; b0 += slice) {
-      const int64_t elements = std::min<int64_t>(slice, g.B - b0);
-      rc = columns_direct_product(g, mm, b0, elements, s, stream);
-      if (rc == SDK_OK) rc = col2im(b0, elements);
+    const Slices& t = l.slices;
+    const bool rows_too = t.both && wgrad_img != nullptr;
+    for (int64_t first = 0; first < g.B; first += t.scatter) {
+      const int64_t elements = std::min<int64_t>(t.scatter, g.B - first);
+      if (first == 0 || !t.both)
+        rc = columns_direct_prepare(g, mm, pix, first, t.both ? g.B : elements, rows_too, true, rows_too && bias_sum,
+                                    first == 0 ? Wm : nullptr, t.channels, rows_too ? wgrad_img : nullptr, s, stream);
+      for (int c0 = 0; c0 < Cgp && rc == SDK_OK; c0 += t.channels) {
+        const int channels = std::min(t.channels, Cgp - c0);
+        rc = columns_direct_product(g, mm, t.both ? first : 0, elements, c0, channels, s, stream);
+        if (rc == SDK_OK) rc = col2im(first, elements, c0, channels);
+      }
       if (rc) return rc;
     }
     return SDK_OK;
@@ -767,16 +818,17 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
   a.ldc = (size_t)R;
   rc = gemm<false>(mm, a, 1, stream);
   if (rc) return rc;
-  return col2im(0, g.B);
+  return col2im(0, g.B, 0, Cgp);
 }
 
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,
                          hipStream_t stream, bool prepared, float* gb) {
-  const ColumnsLayout l = columns_layout(g);
+  const ColumnsLayout l = columns_layout(g, mm);
   char* ws = static_cast<char*>(workspace);
   if (columns_direct(g))
-    return columns_direct_wgrad(g, mm, pix, map, wts, img, gW, columns_scratch(l, ws), prepared, gb, stream);
+    return columns_direct_wgrad(g, mm, pix, map, wts, img, gW, l.slices.wgrad, columns_scratch(l, ws),
+                                prepared && l.slices.both, gb, stream);
   float* prows = reinterpret_cast<float*>(ws + l.pix_rows);
   float* irows = reinterpret_cast<float*>(ws + l.img_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);

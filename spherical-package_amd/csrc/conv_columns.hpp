@@ -40,30 +40,35 @@ __device__ __forceinline__ void channels_last_tile(const float* __restrict__ src
 struct ColumnsScratch {
   float* img_rows;      // B * H * W + 1 rows of pad8(Cg) floats
   void* weights;        // columns_weight_bytes()
-  void *pix_rows, *pix_cols;   // columns_pixel_bytes() each
+  void *pix_rows, *pix_cols;   // columns_pixel_row_bytes(), columns_pixel_column_bytes()
   float* strip_sums;    // columns_strip_bytes()
-  float* col;           // the products of a scatter, or a forward's sums
-  float* partial;       // columns_partial_bytes()
+  float* col;           // the products of a scatter
+  float* partial;       // columns_partial_bytes(), or columns_forward_sum_bytes()
 };
 bool columns_direct(const ConvGeom& g);
 size_t columns_weight_bytes(const ConvGeom& g);
 size_t columns_forward_sum_bytes(const ConvGeom& g);
-size_t columns_pixel_bytes(const ConvGeom& g);
-size_t columns_partial_bytes(const ConvGeom& g);
+size_t columns_pixel_row_bytes(const ConvGeom& g, int mm, int64_t elements);
+size_t columns_pixel_column_bytes(const ConvGeom& g, int mm, int64_t elements);
+size_t columns_partial_bytes(const ConvGeom& g, int64_t elements);
 size_t columns_strip_bytes(const ConvGeom& g);
 int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
                            const float* Wm, const float* bias, float* pix, const ColumnsScratch& s,
                            hipStream_t stream);
-// Lays out what columns_direct_product reads.  wgrad_img: that of a columns_direct_wgrad of the same call that
-// follows, laid out by the same launch; strip_sums: ... which is asked for the bias gradient.
-int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
-                           bool strip_sums, const ColumnsScratch& s, hipStream_t stream);
-// s.col[b][m][(k, c)] = sum over n of pix * Wm, of batch elements first .. first + elements - 1.
-int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, const ColumnsScratch& s,
-                           hipStream_t stream);
-// gb: also gb[n] = sum of pix[b][n][m] (optional).
+// Lays out, in one launch, the pixels of batch elements first .. first + elements - 1 as operands of the weight
+// gradient (rows) and of the scatter's product (cols), the sums of their strips, and, where they are given, the
+// product's weights, in chunks of so many channels (multiples of 32, or all of them), and the whole image.
+int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, int64_t first, int64_t elements, bool rows,
+                           bool cols, bool strip_sums, const float* Wm, int channels, const float* img,
+                           const ColumnsScratch& s, hipStream_t stream);
+// s.col[b][m][(k, c)] = sum over n of pix * Wm, of elements first .. first + elements - 1 of those whose cols are laid
+// out and of the chunk of channels c0 .. c0 + channels - 1.
+int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, int c0, int channels,
+                           const ColumnsScratch& s, hipStream_t stream);
+// `slice` batch elements at a time.  prepared: image, rows of the whole batch, one slice, and the sums of its strips
+// are laid out.  gb: also gb[n] = sum of pix[b][n][m] (optional).
 int columns_direct_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map, const float* wts,
-                         const float* img, float* gW, const ColumnsScratch& s, bool prepared, float* gb,
+                         const float* img, float* gW, int64_t slice, const ColumnsScratch& s, bool prepared, float* gb,
                          hipStream_t stream);
 
 // Maps whose kept plan holds the inverted lists the route's scatter reads (H, W, M, K, P and
@@ -85,8 +90,8 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
                          void* workspace, hipStream_t stream, const void* lists,
                          const float* wgrad_img, bool bias_sum);
 // gW = sum_b pix[b] x im2col(img[b])^T; every element of gW is written.  prepared: the workspace
-// still holds what a columns_gemm_scatter of the same g laid out for it.  gb (columns_sums_bias): also
-// gb[n] = sum of pix[b][n][m].
+// still holds what a columns_gemm_scatter of the same g and mm may have laid out for it.  gb
+// (columns_sums_bias): also gb[n] = sum of pix[b][n][m].
 bool columns_sums_bias(const ConvGeom& g);
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,

@@ -483,13 +483,13 @@ __global__ __launch_bounds__(256) void columns_forward_sum_kernel(const float* _
   out[e] = sum;
 }
 
-// gW[n][c][k] = sum over the splits of partial[split][n][k][c]; the last blocks, four channels each, sum the
-// bias gradient gb[n] = sum of strip_sums[n][strip].
+// gW[n][c][k] = (or, `add`, +=) sum over the splits of partial[split][n][k][c]; the last blocks, four channels each,
+// sum the bias gradient gb[n] = sum of strip_sums[n][strip].
 __global__ __launch_bounds__(256) void columns_gradient_sum_kernel(const float* __restrict__ partial,
                                                                    float* __restrict__ gW, int splits, int Cg, int Cgp,
                                                                    int K, int Cp, int total, int weight_blocks,
                                                                    const float* __restrict__ strip_sums,
-                                                                   float* __restrict__ gb, int strips) {
+                                                                   float* __restrict__ gb, int strips, int add) {
   if ((int)blockIdx.x >= weight_blocks) {
     const int n = ((int)blockIdx.x - weight_blocks) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (n >= Cp) return;
@@ -518,7 +518,8 @@ __global__ __launch_bounds__(256) void columns_gradient_sum_kernel(const float* 
     for (int x = 0; x < 8; ++x) v[x] = s + x < splits ? v[x] : 0.0f;
     sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
-  gW[((size_t)n * Cg + c) * K + k] = sum;
+  float* out = gW + ((size_t)n * Cg + c) * K + k;
+  *out = add ? *out + sum : sum;
 }
 
 // col[b][m][r] = sum over n of pix[b][n][m] * W[n][r], r = (k, c): a wave makes 32 pixels x 64 columns from operands
@@ -527,7 +528,7 @@ __global__ __launch_bounds__(256) void columns_gradient_sum_kernel(const float* 
 struct ProductArgs {
   const char *pixels, *weights;   // operands: [block of 32 pixels][n / 16], [block of 32 columns][n / 16]
   float* col;
-  int M, R, strips, tiles_r, tiles, steps, stride;   // strips, stride: blocks of an element, steps of a block
+  int M, R, strips, tiles_r, tiles, steps;   // strips, steps: blocks of an element, steps of a block
 };
 template <int MM, bool LONG>
 __global__ __launch_bounds__(256, 2) void columns_product_kernel(ProductArgs g) {
@@ -538,7 +539,7 @@ __global__ __launch_bounds__(256, 2) void columns_product_kernel(ProductArgs g) 
   int tile = first + (blockIdx.x >> 3) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (tile >= last) return;
   const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
-  const size_t block = (size_t)g.stride * kFrag * 1024;
+  const size_t block = (size_t)g.steps * kFrag * 1024;
   uint4 a[kFrag], w[2][kFrag];
   auto fetch = [&](int tile, int s) {
     const int tr = tile % g.tiles_r, tm = tile / g.tiles_r;
@@ -623,8 +624,8 @@ __global__ __launch_bounds__(256, 2) void columns_product_kernel(ProductArgs g) 
 // ---------------------------------------------------------------------------
 // What a call lays out before its products, in one launch.
 //   image   [b][u][c], and a row of zeros behind the last
-//   weights as operands: of the forward [block of 32 n][step of 32 (k, c)][s], of the product
-//           [block of 32 (k, c)][step of 16 n]
+//   weights as operands: of the forward [block of 32 n][step of 32 (k, c)][s], of the product, one chunk of channels
+//           after the other, [block of 32 (k, c)][step of 16 n]
 //   pixels  as operands: of the weight gradient [block of 32 n][step of 32 pixels][s], of the product
 //           [block of 32 pixels][step of 16 n], and their sums over each 64 pixels of a channel
 // An operand of 16 reduction elements is [piece][lane][16 bytes], lane l holding row (or column) l % 32 and elements
@@ -636,8 +637,9 @@ struct PrepareArgs {
   uint4 *weights, *pix_rows, *pix_cols;   // pix_rows: of the weight gradient; pix_cols: of the product
   float* strip_sums;
   int B, Cg, Cgp, HW, K, Cp, M;
+  int pix_B, pix_first;                   // elements of the batch whose pixels are laid out, and the first
   int steps;                              // of the weights' blocks
-  int product_weights;                    // which weights
+  int product_weights;                    // channels of a chunk of the product's weights; 0: the forward's
   int img_strips, img_chunks, img_blocks;      // 64 pixels, 32 channels
   int pix_strips, pix_chunks, pix_blocks;
   int total;                              // operands of the weights times 64 lanes
@@ -677,7 +679,7 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
   if (block < g.pix_blocks) {
     // 32 channels of 64 pixels
     const int strip = block % g.pix_strips, q = block / g.pix_strips, chunk = q % g.pix_chunks, b = q / g.pix_chunks;
-    const float* src = g.pix + (size_t)b * g.Cp * g.M;
+    const float* src = g.pix + (size_t)(g.pix_first + b) * g.Cp * g.M;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int n = 32 * chunk + wave + 4 * i, m = 64 * strip + lane;
@@ -692,7 +694,7 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) f[i] = tile[j][16 * wave + 8 * h + i];
       if (g.pix_rows != nullptr && step < steps)
-        put_operand<MM>(g.pix_rows, (((size_t)chunk * g.B + b) * steps + step) * 2 + (wave & 1), lane, f);
+        put_operand<MM>(g.pix_rows, (((size_t)chunk * g.pix_B + b) * steps + step) * 2 + (wave & 1), lane, f);
       if (g.strip_sums != nullptr)
         part[j][2 * wave + h] = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
     }
@@ -700,15 +702,15 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
       const int at = 2 * strip + (wave >> 1);
 #pragma unroll
       for (int i = 0; i < 8; ++i) f[i] = tile[16 * (wave & 1) + 8 * h + i][32 * (wave >> 1) + j];
-      if (at < steps)
-        put_operand<MM>(g.pix_cols, ((size_t)b * steps + at) * 2 * g.pix_chunks + 2 * chunk + (wave & 1), lane, f);
+      const int of = (g.Cp + 15) / 16, n16 = 2 * chunk + (wave & 1);
+      if (at < steps && n16 < of) put_operand<MM>(g.pix_cols, ((size_t)b * steps + at) * of + n16, lane, f);
     }
     if (g.strip_sums != nullptr) {
       __syncthreads();
       const int n = 32 * chunk + (int)threadIdx.x;
       if (threadIdx.x < 32 && n < g.Cp) {
         const float* p = part[threadIdx.x];
-        g.strip_sums[((size_t)n * g.B + b) * g.pix_strips + strip] =
+        g.strip_sums[((size_t)n * g.B + g.pix_first + b) * g.pix_strips + strip] =
             ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       }
     }
@@ -725,7 +727,9 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
   float f[8];
   if (g.product_weights) {
     const int s = e / 64 % g.steps, r = e / 64 / g.steps * 32 + j, n0 = 16 * s + 8 * h;
-    const int k = r / g.Cgp, c = r - k * g.Cgp;
+    const int chunk = min(r / (g.K * g.product_weights), (g.Cgp - 1) / g.product_weights);
+    const int c0 = chunk * g.product_weights, width = min(g.product_weights, g.Cgp - c0);
+    const int k = (r - g.K * c0) / width, c = c0 + (r - g.K * c0) - k * width;
     const float* w = g.Wm + (size_t)min(c, g.Cg - 1) * g.K + min(k, g.K - 1);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -786,9 +790,9 @@ DirectShape direct_shape(const ConvGeom& g) {
 // 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55, 45, 42; 32 rows, 2 x 115 x 231,
 // 24 -> 32, float32 42, 26, 31.
 struct WgradShape {
-  int ra, groups, tiles_a, tiles_r, strips, steps, splits, split_steps, samples;   // samples: most of a tile
+  int ra, groups, tiles_a, tiles_r, strips, steps, most, splits, split_steps, samples;   // samples: most of a tile
 };
-WgradShape wgrad_shape(const ConvGeom& g) {
+WgradShape wgrad_shape(const ConvGeom& g, int64_t elements) {   // (most: splits of this many elements or fewer)
   WgradShape t;
   const int64_t blocks = ceil_div(g.Cp, 32);
   t.tiles_a = (int)ceil_div(blocks, 5);
@@ -797,17 +801,19 @@ WgradShape wgrad_shape(const ConvGeom& g) {
   t.tiles_r = (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32);
   t.strips = (int)ceil_div(g.M, 32);
   t.samples = pad8(g.Cg) % 32 == 0 ? 1 : std::min(g.K, pad8(g.Cg) == 8 ? 4 : 2);
-  t.steps = (int)(g.B * t.strips);
+  t.steps = (int)(elements * t.strips);
   const int64_t waves = (int64_t)t.tiles_a * t.tiles_r * t.ra * t.groups;
   const int64_t wanted = t.ra == 5 ? 256 / ((int64_t)t.tiles_a * t.tiles_r) : ceil_div(t.ra == 1 ? 2048 : 4096, waves);
   const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(wanted, t.steps / (4 * t.groups)));
+  t.most = (int)splits;
   t.split_steps = (int)ceil_div(t.steps, splits);
   t.splits = (int)ceil_div(t.steps, t.split_steps);
   return t;
 }
 
-// 32-channel chunks, 64-pixel strips and 16-byte operands of the pixel-side tensor
-int64_t pixel_chunks(const ConvGeom& g) { return ceil_div(g.Cp, 32); }
+// 16-byte pieces of an operand
+int operand_pieces(int mm) { return mm == kMmF32 ? 2 : (mm == kMmBf16 ? 1 : 3); }
+// 64-pixel strips of the pixel-side tensor
 int64_t pixel_strips(const ConvGeom& g) { return ceil_div(g.M, 64); }
 
 PrepareArgs prepare_args(const ConvGeom& g) {
@@ -828,21 +834,24 @@ void prepare_image(PrepareArgs& p, const float* img, float* rows) {
   p.img_chunks = (int)ceil_div(p.Cgp, 32);
   p.img_blocks = p.img_strips * p.img_chunks * p.B;
 }
-void prepare_weights(PrepareArgs& p, const float* Wm, void* weights, bool product, int blocks, int steps) {
+void prepare_weights(PrepareArgs& p, const float* Wm, void* weights, int product, int blocks, int steps) {
   p.Wm = Wm;
   p.weights = static_cast<uint4*>(weights);
   p.product_weights = product;
   p.steps = steps;
   p.total = blocks * steps * (product ? 64 : 128);
 }
-void prepare_pixels(PrepareArgs& p, const float* pix, void* rows, void* cols, float* strip_sums) {
+void prepare_pixels(PrepareArgs& p, const float* pix, int64_t first, int64_t elements, void* rows, void* cols,
+                    float* strip_sums) {
   p.pix = pix;
+  p.pix_first = (int)first;
+  p.pix_B = (int)elements;
   p.pix_rows = static_cast<uint4*>(rows);
   p.pix_cols = static_cast<uint4*>(cols);
   p.strip_sums = strip_sums;
   p.pix_strips = (int)ceil_div(p.M, 64);
   p.pix_chunks = (int)ceil_div(p.Cp, 32);
-  p.pix_blocks = p.pix_strips * p.pix_chunks * p.B;
+  p.pix_blocks = p.pix_strips * p.pix_chunks * p.pix_B;
 }
 int prepare(int mm, const PrepareArgs& p, hipStream_t stream) {
   const dim3 grid((unsigned)(p.img_blocks + p.pix_blocks + 1 + ceil_div(p.total, 256)));
@@ -943,19 +952,22 @@ bool columns_direct(const ConvGeom& g) { return pts(g.P) <= 4; }
 size_t columns_weight_bytes(const ConvGeom& g) {
   const DirectShape t = direct_shape(g);
   const int64_t forward = (int64_t)t.tiles_a * t.ra * t.steps * 2;
-  const int64_t product = ceil_div((int64_t)g.K * pad8(g.Cg), 32) * 2 * pixel_chunks(g);
+  const int64_t product = ceil_div((int64_t)g.K * pad8(g.Cg), 32) * ceil_div(g.Cp, 16);
   return (size_t)std::max(forward, product) * 64 * 16 * 3;
 }
 size_t columns_forward_sum_bytes(const ConvGeom& g) {
   const DirectShape t = direct_shape(g);
   return t.splits > 1 ? sizeof(float) * t.splits * g.B * g.Cp * g.M : 0;
 }
-size_t columns_pixel_bytes(const ConvGeom& g) {
-  const WgradShape t = wgrad_shape(g);
-  return (size_t)t.tiles_a * t.ra * t.steps * 2 * 64 * 16 * 3;
+size_t columns_pixel_row_bytes(const ConvGeom& g, int mm, int64_t elements) {
+  const WgradShape t = wgrad_shape(g, elements);
+  return (size_t)t.tiles_a * t.ra * t.steps * 2 * 64 * 16 * operand_pieces(mm);
 }
-size_t columns_partial_bytes(const ConvGeom& g) {
-  return (size_t)wgrad_shape(g).splits * g.Cp * g.K * pad8(g.Cg) * sizeof(float);
+size_t columns_pixel_column_bytes(const ConvGeom& g, int mm, int64_t elements) {
+  return (size_t)(elements * ceil_div(g.M, 32) * ceil_div(g.Cp, 16)) * 64 * 16 * operand_pieces(mm);
+}
+size_t columns_partial_bytes(const ConvGeom& g, int64_t elements) {
+  return (size_t)wgrad_shape(g, elements).most * g.Cp * g.K * pad8(g.Cg) * sizeof(float);
 }
 size_t columns_strip_bytes(const ConvGeom& g) { return (size_t)g.B * pixel_strips(g) * g.Cp * sizeof(float); }
 
@@ -965,7 +977,7 @@ int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const fl
   const DirectShape t = direct_shape(g);
   PrepareArgs p = prepare_args(g);
   prepare_image(p, img, s.img_rows);
-  prepare_weights(p, Wm, s.weights, false, t.tiles_a * t.ra, t.steps);
+  prepare_weights(p, Wm, s.weights, 0, t.tiles_a * t.ra, t.steps);
   int rc = prepare(mm, p, stream);
   if (rc) return rc;
   DirectArgs a = direct_args(g, s.img_rows, map, wts, s.weights);
@@ -976,33 +988,37 @@ int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const fl
   a.tiles_n = t.tiles_m;
   a.splits = t.splits;
   a.split_steps = t.split_steps;
-  a.partial = t.splits > 1 ? s.col : nullptr;
+  a.partial = t.splits > 1 ? s.partial : nullptr;
   const dim3 grid((unsigned)(((int64_t)t.tiles_a * t.tiles_m * g.B + 7) / 8 * 8), (unsigned)t.splits);
   rc = direct<false>(g, mm, a, t.ra, t.groups, 1, grid, stream);
   if (rc) return rc;
   if (t.splits > 1) {
     const int total = (int)(g.B * g.Cp * g.M);
     launch(columns_forward_sum_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), stream,
-           (const float*)s.col, bias, pix, t.splits, g.Cp, g.M, total);
+           (const float*)s.partial, bias, pix, t.splits, g.Cp, g.M, total);
     SDK_LAUNCH_CHECK("mapped_conv(columns forward sums)");
   }
   return SDK_OK;
 }
 
-int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, const float* Wm, const float* wgrad_img,
-                           bool strip_sums, const ColumnsScratch& s, hipStream_t stream) {
+int columns_direct_prepare(const ConvGeom& g, int mm, const float* pix, int64_t first, int64_t elements, bool rows,
+                           bool cols, bool strip_sums, const float* Wm, int channels, const float* img,
+                           const ColumnsScratch& s, hipStream_t stream) {
   PrepareArgs p = prepare_args(g);
-  if (wgrad_img != nullptr) prepare_image(p, wgrad_img, s.img_rows);
-  prepare_weights(p, Wm, s.weights, true, (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32), 2 * (int)pixel_chunks(g));
-  prepare_pixels(p, pix, wgrad_img != nullptr ? s.pix_rows : nullptr, s.pix_cols, strip_sums ? s.strip_sums : nullptr);
+  if (img != nullptr) prepare_image(p, img, s.img_rows);
+  if (Wm != nullptr)
+    prepare_weights(p, Wm, s.weights, channels, (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32), (int)ceil_div(g.Cp, 16));
+  prepare_pixels(p, pix, first, elements, rows ? s.pix_rows : nullptr, cols ? s.pix_cols : nullptr,
+                 strip_sums ? s.strip_sums : nullptr);
   return prepare(mm, p, stream);
 }
 
-int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, const ColumnsScratch& s,
-                           hipStream_t stream) {
-  const int R = g.K * pad8(g.Cg);
+int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t elements, int c0, int channels,
+                           const ColumnsScratch& s, hipStream_t stream) {
+  const int R = g.K * channels;
+  const int pieces = operand_pieces(mm), steps = (int)ceil_div(g.Cp, 16);
   ProductArgs a{};
-  a.weights = static_cast<const char*>(s.weights);
+  a.weights = static_cast<const char*>(s.weights) + (size_t)c0 * g.K / 32 * steps * pieces * 1024;
   a.col = s.col;
   a.M = g.M;
   a.R = R;
@@ -1010,10 +1026,8 @@ int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t ele
   a.tiles_r = (int)ceil_div(R, 64);
   const int64_t tiles = elements * a.strips * a.tiles_r;
   a.tiles = (int)tiles;
-  a.steps = (int)ceil_div(g.Cp, 16);
-  a.stride = 2 * (int)pixel_chunks(g);
-  const int pieces = mm == kMmF32 ? 2 : (mm == kMmBf16 ? 1 : 3);
-  a.pixels = static_cast<const char*>(s.pix_cols) + (size_t)first * a.strips * a.stride * pieces * 1024;
+  a.steps = steps;
+  a.pixels = static_cast<const char*>(s.pix_cols) + (size_t)first * a.strips * steps * pieces * 1024;
   // float32: one wave a SIMD.  With two or more, their loads and MFMAs take turns: 64 -> 64, 128 x 256, 33 us with
   // one, 53 with four (21 without the MFMAs, 30 without the loads); MFMAs alone run at
   // 150 TFLOP/s with any number of waves, 16 of them beside six 16-byte loads at 130 with one and 70 with two.  bf16 operands want
@@ -1034,31 +1048,35 @@ int columns_direct_product(const ConvGeom& g, int mm, int64_t first, int64_t ele
 }
 
 int columns_direct_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map, const float* wts,
-                         const float* img, float* gW, const ColumnsScratch& s, bool prepared, float* gb,
+                         const float* img, float* gW, int64_t slice, const ColumnsScratch& s, bool prepared, float* gb,
                          hipStream_t stream) {
-  if (!prepared) {
-    PrepareArgs p = prepare_args(g);
-    prepare_image(p, img, s.img_rows);
-    prepare_pixels(p, pix, s.pix_rows, nullptr, gb != nullptr ? s.strip_sums : nullptr);
-    const int rc = prepare(mm, p, stream);
-    if (rc) return rc;
-  }
-  const WgradShape t = wgrad_shape(g);
-  DirectArgs a = direct_args(g, s.img_rows, map, wts, s.pix_rows);
-  a.steps = t.steps;
-  a.tiles_a = t.tiles_a;
-  a.tiles_n = t.tiles_r;
-  a.splits = t.splits;
-  a.split_steps = t.split_steps;
-  a.partial = s.partial;
-  const dim3 grid((unsigned)(((int64_t)t.tiles_a * t.tiles_r * t.splits + 7) / 8 * 8));
-  const int rc = direct<true>(g, mm, a, t.ra, t.groups, t.samples, grid, stream);
-  if (rc) return rc;
   const int Cgp = pad8(g.Cg), total = g.Cp * g.K * Cgp, weight_blocks = (int)ceil_div(total, 256);
-  launch(columns_gradient_sum_kernel, dim3((unsigned)(weight_blocks + (gb != nullptr ? ceil_div(g.Cp, 4) : 0))),
-         dim3(256), stream, (const float*)s.partial, gW, t.splits, g.Cg, Cgp, g.K, g.Cp, total, weight_blocks,
-         (const float*)s.strip_sums, gb, (int)(g.B * pixel_strips(g)));
-  SDK_LAUNCH_CHECK("mapped_conv(columns sums)");
+  for (int64_t first = 0; first < g.B; first += slice) {
+    const int64_t elements = std::min<int64_t>(slice, g.B - first);
+    if (!prepared) {
+      const int rc = columns_direct_prepare(g, mm, pix, first, elements, true, false, gb != nullptr, nullptr,
+                                            0, first == 0 ? img : nullptr, s, stream);
+      if (rc) return rc;
+    }
+    const WgradShape t = wgrad_shape(g, elements);
+    DirectArgs a = direct_args(g, s.img_rows + (size_t)first * g.H * g.W * Cgp, map, wts, s.pix_rows);
+    a.B = (int)(g.B - first);   // (where the row of zeros is)
+    a.steps = t.steps;
+    a.tiles_a = t.tiles_a;
+    a.tiles_n = t.tiles_r;
+    a.splits = t.splits;
+    a.split_steps = t.split_steps;
+    a.partial = s.partial;
+    const dim3 grid((unsigned)(((int64_t)t.tiles_a * t.tiles_r * t.splits + 7) / 8 * 8));
+    const int rc = direct<true>(g, mm, a, t.ra, t.groups, t.samples, grid, stream);
+    if (rc) return rc;
+    // (the strips of all slices are there with the last)
+    const int bias_blocks = gb != nullptr && first + elements == g.B ? (int)ceil_div(g.Cp, 4) : 0;
+    launch(columns_gradient_sum_kernel, dim3((unsigned)(weight_blocks + bias_blocks)), dim3(256), stream,
+           (const float*)s.partial, gW, t.splits, g.Cg, Cgp, g.K, g.Cp, total, weight_blocks,
+           (const float*)s.strip_sums, gb, (int)(g.B * pixel_strips(g)), first > 0 ? 1 : 0);
+    SDK_LAUNCH_CHECK("mapped_conv(columns sums)");
+  }
   return SDK_OK;
 }
 

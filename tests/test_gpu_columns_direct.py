@@ -91,6 +91,56 @@ def test_bias_gradient_keeps_the_bits_of_its_sums(ops, height):
     assert columns._rel(gb.cpu().numpy(), g.astype(np.float64).sum((0, 2, 3))) <= 1.1e-7
 
 
+def _gradients(ops, tc, arrays, mode):
+    m, _, x, w, b, g, _ = arrays
+    with ops.conv_compute(mode):
+        return ops.ops.mapped_conv_backward(g, m, None, x, w, b, tc[7], tc[9])
+
+
+def _on_gpu(tc):
+    return [None if a is None else torch.from_numpy(a).to(DEV) for a in columns._arrays(tc)]
+
+
+# (..., as above) whose scatter has slices of two elements and one; slices of one, in three chunks of channels, the
+# last of six; whose pixels' operands are laid out by each contraction (float32 and split), those of the weight
+# gradient in two slices (split)
+LARGE = [
+    (3, 32, 8, 40, 80, 100, 200, 25, 0, 1),
+    (2, 70, 8, 40, 80, 144, 288, 25, 0, 1),
+    (30, 8, 96, 64, 128, 64, 128, 1, 0, 1),
+    (2, 40, 208, 40, 80, 144, 288, 11, 0, 0),
+]
+
+
+@pytest.mark.parametrize("kept", [True, False], ids=["plan", "no-plan"])
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+@pytest.mark.parametrize("tc", LARGE, ids=lambda t: "x".join(map(str, t)))
+def test_calls_in_slices(ops, tc, mode, kept):
+    B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
+    assert runs_by_columns(*tc)
+    arrays = m, _, x, w, b, g, bt = _on_gpu(tc)
+    ops.set_conv_plan_cache(kept)
+    try:
+        gi, gw, gb = _gradients(ops, tc, arrays, mode)
+        # a call of one element, and of one chunk of channels, whose sums are the same ones
+        for at in (0, B - 1):
+            one = (m, None, x[at:at + 1].contiguous(), w, b, g[at:at + 1].contiguous(), None)
+            assert torch.equal(gi[at:at + 1], _gradients(ops, tc, one, mode)[0])
+        if Cin == 70:
+            with ops.conv_compute(mode):
+                up = ops.ops.mapped_transposed_conv_forward(g, m, None, w, x.new_ones(Cin), H, W, K, interp)
+            for c in (slice(0, 32), slice(32, 64), slice(64, 70)):
+                part = (m, None, x[:, c].contiguous(), w[:, c].contiguous(), b, g, None)
+                assert torch.equal(gi[:, c], _gradients(ops, tc, part, mode)[0])
+                assert torch.equal(gi[:, c] + 1, up[:, c])
+    finally:
+        ops.set_conv_plan_cache(True)
+    want = _gradients(ops, tc, [None if a is None else a.double() for a in arrays], "native")
+    # float32 sums: eps * sqrt(n) / 2, apart by 64 channels or 32 pixels; bf16 operands: 2^-9 each
+    for have, ref in zip((gi, gw, gb), want):
+        assert columns._rel(have.cpu().numpy(), ref.cpu().numpy()) <= (4e-3 if mode == "bf16" else 2e-6)
+
+
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
 def test_values_no_tap_reads_stay_out(ops, mode):
     """An infinite pixel without a tap, and an infinite weight of a channel beside the others."""

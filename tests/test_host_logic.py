@@ -337,3 +337,20 @@ def test_window_weight_gradient_has_no_limit_of_output_pixels():
         at_limit, past = (_capi.load().sdk_mapped_conv_workspace_bytes(
             1, 32, cout, 512, 512, 4096, w, 9, 0, 1, _capi.SDK_F32, compute) for w in (4096, 4097))
         assert past >= at_limit > 0
+
+
+@pytest.mark.parametrize("call, most", [
+    # a map of 25 samples: one element's products 200 and 839 MB, of the transposed layer 800
+    ((8, 64, 256, 128, 256, 128, 256, 25), 600), ((8, 64, 64, 256, 512, 256, 512, 25), 600),
+    ((1, 256, 256, 128, 256, 128, 256, 25), 300),
+    # pixels padded to 32 channels, and pictures of one pixel to 32
+    ((64, 8, 8, 64, 128, 64, 128, 1), 140), ((4096, 64, 256, 4, 8, 1, 1, 1), 250),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "%dMB" % v)
+def test_workspace_of_convolutions_by_columns(call, most):
+    """The operands and products of large calls take turns in the workspace, which had 1286, 1938, 982, 225 and
+    437 MB with all of them side by side; one size for every arithmetic."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    assert lib.sdk_mapped_conv_by_columns(*call, 0, 1, _capi.SDK_F32, 0, 0) == 1
+    need = {lib.sdk_mapped_conv_workspace_bytes(*call, 0, 1, _capi.SDK_F32, compute) for compute in (0, 1, 3)}
+    assert len(need) == 1 and need.pop() <= most << 20
