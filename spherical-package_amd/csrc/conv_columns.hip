@@ -552,8 +552,8 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
   if (columns_direct(g)) {
     const Slices& t = l.slices = slices_of(g, mm);
     const size_t products = sizeof(float) * t.scatter * g.M * g.K * t.channels;
-    const size_t partial = std::max(columns_partial_bytes(g, t.wgrad), columns_forward_sum_bytes(g));
-    l.weights = take(columns_weight_bytes(g));
+    const size_t partial = std::max(columns_partial_bytes(g, mm, t.wgrad), columns_forward_sum_bytes(g, mm));
+    l.weights = take(columns_weight_bytes(g, mm));
     l.strip_sums = take(columns_strip_bytes(g));
     const size_t base = at;
     l.pix_cols = take(columns_pixel_column_bytes(g, mm, t.both ? g.B : t.scatter));

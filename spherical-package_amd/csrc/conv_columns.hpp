@@ -46,11 +46,11 @@ struct ColumnsScratch {
   float* partial;       // columns_partial_bytes(), or columns_forward_sum_bytes()
 };
 bool columns_direct(const ConvGeom& g);
-size_t columns_weight_bytes(const ConvGeom& g);
-size_t columns_forward_sum_bytes(const ConvGeom& g);
+size_t columns_weight_bytes(const ConvGeom& g, int mm);
+size_t columns_forward_sum_bytes(const ConvGeom& g, int mm);
 size_t columns_pixel_row_bytes(const ConvGeom& g, int mm, int64_t elements);
 size_t columns_pixel_column_bytes(const ConvGeom& g, int mm, int64_t elements);
-size_t columns_partial_bytes(const ConvGeom& g, int64_t elements);
+size_t columns_partial_bytes(const ConvGeom& g, int mm, int64_t elements);
 size_t columns_strip_bytes(const ConvGeom& g);
 int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
                            const float* Wm, const float* bias, float* pix, const ColumnsScratch& s,

@@ -751,9 +751,15 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
 }
 
 // Shape of a call.  Measured, us of the whole forward, on either side of each line:
-//   blocks of 32 channels share a tile (the columns are blended once for all of them) up to five: 160 channels
+//   blocks of 32 channels share a tile (the columns are blended once for all of them), up to five: 160 channels
 //     of 6 x 25 x 50 pixels, split, 50 as 96 + 64, 37 as one tile; 256 channels of 60 x 120, nearest, bf16, 31 as
-//     one tile of eight, 22 as two of four;
+//     one tile of eight, 22 as two of four.  More are tiles of four, the last perhaps of padding: three or five waves
+//     share four SIMDs badly.  Forward alone, us, float32 / bf16 / split, as equal tiles of three or five and so:
+//     19 -> 176 channels, 188 x 376 106 / 56 / 102 and 109 / 50 / 80 (float32 as three of two 90; 176 -> 176,
+//     4 x 24 x 49 78, 75 and 52 so); 32 -> 264, 3 x 62 x 125 87 / 40 / 74 and 72 / 33 / 53; 32 -> 291, 136 x 272
+//     126 / 57 / 118 and 106 / 45 / 77; 72 -> 264, 62 x 125 54 / 23 / 49 and 55 / 25 / 42.  Five blocks whose columns
+//     are quickly multiplied are two tiles of four where they are split: 48 -> 160, 2 x 54 x 108 36 and 30, 24 -> 160,
+//     7 x 60 x 121 75 and 62; 96 -> 160 above 33 and 33, 216 -> 152, 2 x 56 x 112 112 and 123;
 //   groups where the tiles leave SIMDs without a wave: 216 tiles of two blocks (104 -> 37 channels, 2 x 41 x 83)
 //     39, 26 and 24 with 1, 2, 4; 384 of two (200 -> 37, 3 x 45 x 91, split) 60 and 47; 638 of three (8 -> 96,
 //     101 x 202) 18.5 and 21.5; 1024 of two (64 -> 64, 128 x 256, bf16) 36, 41 and 55;
@@ -764,14 +770,16 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
 struct DirectShape {
   int ra, groups, tiles_a, tiles_m, steps, splits, split_steps;
 };
-DirectShape direct_shape(const ConvGeom& g) {
+DirectShape direct_shape(const ConvGeom& g, int mm) {
   DirectShape t;
   const int64_t blocks = ceil_div(g.Cp, 32);
-  t.tiles_a = (int)ceil_div(blocks, 5);
-  t.ra = (int)ceil_div(blocks, t.tiles_a);
   t.tiles_m = (int)ceil_div(g.M, kDirectPixels);
   t.steps = (int)ceil_div((int64_t)g.K * pad8(g.Cg), kDirectStep);
-  const int64_t tiles = (int64_t)t.tiles_a * t.tiles_m * g.B, waves = tiles * t.ra;
+  if (blocks <= 4 || (blocks == 5 && (mm != kMmSplit || t.steps >= 24))) t.ra = (int)blocks;
+  else t.ra = blocks == 6 && mm == kMmF32 ? 2 : 4;
+  t.tiles_a = (int)ceil_div(blocks, t.ra);
+  // (splits by the columns' tiles of up to five blocks: the sums' chains do not grow with the tiles of four)
+  const int64_t waves = (int64_t)t.tiles_a * t.tiles_m * g.B * t.ra, tiles = ceil_div(blocks, 5) * t.tiles_m * g.B;
   int64_t splits = 1;
   if (tiles < 192 && t.steps >= 32) splits = std::min<int64_t>(384 / tiles, t.steps / 8);
   splits = std::max<int64_t>(1, splits);
@@ -783,22 +791,27 @@ DirectShape direct_shape(const ConvGeom& g) {
   return t;
 }
 
-
 // The weight gradient's: tiles of 32 columns (k, c) and of at most five blocks of 32 channels, the pixels in
 // splits of at least four turns.  Its kernel alone, us, with 1024, 2048 and 4096 waves: 160 rows (one tile of five
-// blocks: one workgroup a CU; 1536, where some CUs have two, 54), 6 x 25 x 50, 96 -> 160, split 31, 35, 42; 64 rows, 128 x 256, 64 -> 64, float32 68, 61,
-// 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55, 45, 42; 32 rows, 2 x 115 x 231,
-// 24 -> 32, float32 42, 26, 31.
+// blocks: one workgroup a CU; 1536, where some CUs have two, 54), 6 x 25 x 50, 96 -> 160, split 31, 35, 42; 64 rows,
+// 128 x 256, 64 -> 64, float32 68, 61, 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55,
+// 45, 42; 32 rows, 2 x 115 x 231, 24 -> 32, float32 42, 26, 31.
+// More than five blocks are tiles of four, the last perhaps of padding; nine and ten of bf16 operands two of five where
+// there are few columns and so several splits.  Whole backward, float32 / bf16 / split, as equal tiles of three or
+// five and of four: 176 -> 176, 4 x 24 x 49 141 / 86 / 113 and 127 / 69 / 105; 128 -> 184, 3 x 45 x 91 226 / 121 / 173
+// and 206 / 92 / 163; 32 -> 291, 136 x 272 265 / 113 / 212 and 251 / 107 / 222; 56 -> 264, 49 x 99 85 / 49 / 63 and
+// 85 / 51 / 69; 211 -> 272, 5 x 5, 2 x 19 x 36 245 / 122 / 185 and 180 / 99 / 148.
 struct WgradShape {
   int ra, groups, tiles_a, tiles_r, strips, steps, most, splits, split_steps, samples;   // samples: most of a tile
 };
-WgradShape wgrad_shape(const ConvGeom& g, int64_t elements) {   // (most: splits of this many elements or fewer)
+WgradShape wgrad_shape(const ConvGeom& g, int mm, int64_t elements) {   // (most: splits of so many or fewer)
   WgradShape t;
   const int64_t blocks = ceil_div(g.Cp, 32);
-  t.tiles_a = (int)ceil_div(blocks, 5);
-  t.ra = (int)ceil_div(blocks, t.tiles_a);
-  t.groups = t.ra == 1 ? 4 : (t.ra <= 3 ? 2 : 1);
   t.tiles_r = (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32);
+  if (blocks <= 5) t.ra = (int)blocks;
+  else t.ra = (blocks == 9 || blocks == 10) && mm != kMmF32 && t.tiles_r <= 64 ? 5 : 4;
+  t.tiles_a = (int)ceil_div(blocks, t.ra);
+  t.groups = t.ra == 1 ? 4 : (t.ra <= 3 ? 2 : 1);
   t.strips = (int)ceil_div(g.M, 32);
   t.samples = pad8(g.Cg) % 32 == 0 ? 1 : std::min(g.K, pad8(g.Cg) == 8 ? 4 : 2);
   t.steps = (int)(elements * t.strips);
@@ -948,33 +961,32 @@ DirectArgs direct_args(const ConvGeom& g, const float* rows, const float* map, c
 // 484, eight 470 and 648, split; with the four taps that four weighted pixels have 180 and 133, bf16.)
 bool columns_direct(const ConvGeom& g) { return pts(g.P) <= 4; }
 
-// (six bytes a value: the split's pieces, the largest form)
-size_t columns_weight_bytes(const ConvGeom& g) {
-  const DirectShape t = direct_shape(g);
+size_t columns_weight_bytes(const ConvGeom& g, int mm) {
+  const DirectShape t = direct_shape(g, mm);
   const int64_t forward = (int64_t)t.tiles_a * t.ra * t.steps * 2;
   const int64_t product = ceil_div((int64_t)g.K * pad8(g.Cg), 32) * ceil_div(g.Cp, 16);
-  return (size_t)std::max(forward, product) * 64 * 16 * 3;
+  return (size_t)std::max(forward, product) * 64 * 16 * operand_pieces(mm);
 }
-size_t columns_forward_sum_bytes(const ConvGeom& g) {
-  const DirectShape t = direct_shape(g);
+size_t columns_forward_sum_bytes(const ConvGeom& g, int mm) {
+  const DirectShape t = direct_shape(g, mm);
   return t.splits > 1 ? sizeof(float) * t.splits * g.B * g.Cp * g.M : 0;
 }
 size_t columns_pixel_row_bytes(const ConvGeom& g, int mm, int64_t elements) {
-  const WgradShape t = wgrad_shape(g, elements);
+  const WgradShape t = wgrad_shape(g, mm, elements);
   return (size_t)t.tiles_a * t.ra * t.steps * 2 * 64 * 16 * operand_pieces(mm);
 }
 size_t columns_pixel_column_bytes(const ConvGeom& g, int mm, int64_t elements) {
   return (size_t)(elements * ceil_div(g.M, 32) * ceil_div(g.Cp, 16)) * 64 * 16 * operand_pieces(mm);
 }
-size_t columns_partial_bytes(const ConvGeom& g, int64_t elements) {
-  return (size_t)wgrad_shape(g, elements).most * g.Cp * g.K * pad8(g.Cg) * sizeof(float);
+size_t columns_partial_bytes(const ConvGeom& g, int mm, int64_t elements) {
+  return (size_t)wgrad_shape(g, mm, elements).most * g.Cp * g.K * pad8(g.Cg) * sizeof(float);
 }
 size_t columns_strip_bytes(const ConvGeom& g) { return (size_t)g.B * pixel_strips(g) * g.Cp * sizeof(float); }
 
 int columns_direct_forward(const ConvGeom& g, int mm, const float* img, const float* map, const float* wts,
                            const float* Wm, const float* bias, float* pix, const ColumnsScratch& s,
                            hipStream_t stream) {
-  const DirectShape t = direct_shape(g);
+  const DirectShape t = direct_shape(g, mm);
   PrepareArgs p = prepare_args(g);
   prepare_image(p, img, s.img_rows);
   prepare_weights(p, Wm, s.weights, 0, t.tiles_a * t.ra, t.steps);
@@ -1058,7 +1070,7 @@ int columns_direct_wgrad(const ConvGeom& g, int mm, const float* pix, const floa
                                             0, first == 0 ? img : nullptr, s, stream);
       if (rc) return rc;
     }
-    const WgradShape t = wgrad_shape(g, elements);
+    const WgradShape t = wgrad_shape(g, mm, elements);
     DirectArgs a = direct_args(g, s.img_rows + (size_t)first * g.H * g.W * Cgp, map, wts, s.pix_rows);
     a.B = (int)(g.B - first);   // (where the row of zeros is)
     a.steps = t.steps;

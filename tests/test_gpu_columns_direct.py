@@ -47,6 +47,15 @@ SIZES = [
     (1, 16, 64, 64, 128, 64, 128, 9, 4, 1),
     (4100, 8, 8, 4, 4, 2, 2, 1, 0, 1),
     (5, 24, 70, 20, 31, 17, 31, 9, 2, 2),
+    # ... six to eleven blocks, nine with few columns and with many; five of fewer steps than 24 and of as many
+    (1, 16, 192, 9, 14, 8, 9, 9, 0, 1),
+    (2, 16, 200, 9, 14, 8, 9, 9, 0, 2),
+    (1, 24, 288, 9, 14, 8, 9, 9, 0, 1),
+    (1, 96, 257, 9, 14, 8, 9, 25, 0, 1),
+    (1, 24, 290, 9, 14, 8, 9, 9, 4, 1),
+    (1, 24, 330, 9, 14, 8, 9, 9, 0, 0),
+    (1, 88, 160, 9, 14, 8, 9, 9, 0, 2),
+    (1, 80, 131, 9, 14, 8, 9, 9, 0, 1),
 ]
 
 
