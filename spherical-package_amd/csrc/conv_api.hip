@@ -385,7 +385,7 @@ static int impl_mapped_conv_backward(const void* grad_output, const void* sample
   if (grad_weight != nullptr && dtype == SDK_F32 && compute != SDK_COMPUTE_UNFUSED && batch > 0 &&
       fused_supported(g) && columns_first(g)) {
     shared.wgrad_img = static_cast<const float*>(input);
-    if (columns_sums_bias(g)) shared.columns_bias = static_cast<float*>(grad_bias);
+    if (columns_sums_bias(g, matrix_mode(compute))) shared.columns_bias = static_cast<float*>(grad_bias);
   }
   hipEvent_t joined = nullptr;
   if (!shared.cleared && shared.columns_bias == nullptr && grad_bias != nullptr)

@@ -10,7 +10,8 @@
 // once per sample.
 //
 // Here: which calls take the route, the layout of its workspace, the col2im, and the products of
-// columns that lie in memory, of samples of more than four points.  All others' columns exist only in
+// columns that lie in memory: of samples of more than four points, and of wide layers of few columns.
+// All others' columns exist only in
 // LDS, or, a scatter's, as the products of a slice of the batch or of its channels that, where 32 channels
 // of one element have no more, stays in the 256 MB memory-side cache until the col2im reads them
 // (conv_columns_direct.hip).
@@ -538,8 +539,8 @@ Slices slices_of(const ConvGeom& g, int mm) {
   return s;
 }
 
-// mm: of the calls without a column matrix.
-ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
+// Of a forward, or of both gradients.
+ColumnsLayout columns_layout(const ConvGeom& g, int mm, bool backward) {
   const int Cgp = pad8(g.Cg), Cpp = pad8(g.Cp);
   ColumnsLayout l{};
   size_t at = 0;
@@ -549,10 +550,13 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
     return here;
   };
   const size_t image = sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp;   // (and a row of zeros)
-  if (columns_direct(g)) {
+  if (!backward && columns_direct_gather(g, mm)) {
+    l.weights = take(columns_weight_bytes(g, mm));
+    l.img_rows = take(image);
+    l.partial = take(columns_forward_sum_bytes(g, mm));
+  } else if (backward && columns_direct_backward(g, mm)) {
     const Slices& t = l.slices = slices_of(g, mm);
     const size_t products = sizeof(float) * t.scatter * g.M * g.K * t.channels;
-    const size_t partial = std::max(columns_partial_bytes(g, mm, t.wgrad), columns_forward_sum_bytes(g, mm));
     l.weights = take(columns_weight_bytes(g, mm));
     l.strip_sums = take(columns_strip_bytes(g));
     const size_t base = at;
@@ -562,7 +566,7 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
     if (!t.both) at = base;
     l.img_rows = take(image);
     l.pix_rows = take(columns_pixel_row_bytes(g, mm, t.wgrad));
-    l.partial = take(partial);   // (not in the products' place: calls of a few us take 5 longer so)
+    l.partial = take(columns_partial_bytes(g, mm, t.wgrad));   // (not in the products' place: calls of a few us take 5 longer so)
     at = std::max(at, end);
   } else {
     l.img_rows = take(image);
@@ -579,7 +583,7 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm) {
     l.partial = take(sizeof(float) * l.splits * g.Cp * g.K * Cgp);
   }
   l.lists = at;
-  l.total = at + up256(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp));
+  l.total = at + (backward ? up256(col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp)) : 0);
   return l;
 }
 
@@ -703,25 +707,28 @@ bool columns_route(const ConvGeom& g) {
 }
 
 // (a wave adds up a channel's strips)
-bool columns_sums_bias(const ConvGeom& g) { return columns_direct(g) && g.B * ceil_div(g.M, 64) <= 4096; }
+bool columns_sums_bias(const ConvGeom& g, int mm) {
+  return columns_direct_backward(g, mm) && g.B * ceil_div(g.M, 64) <= 4096;
+}
 
-// (one size for every arithmetic)
+// (one size for every arithmetic and direction)
 size_t columns_workspace_bytes(const ConvGeom& g) {
   if (!columns_route(g)) return 0;
   size_t most = 0;
-  for (int mm : {kMmF32, kMmBf16, kMmSplit}) most = std::max(most, columns_layout(g, mm).total);
+  for (int mm : {kMmF32, kMmBf16, kMmSplit})
+    for (bool backward : {false, true}) most = std::max(most, columns_layout(g, mm, backward).total);
   return most;
 }
 
 int columns_gather_gemm(const ConvGeom& g, int mm, const float* img, const float* map,
                         const float* wts, const float* Wm, const float* bias, float* pix,
                         void* workspace, hipStream_t stream) {
-  const ColumnsLayout l = columns_layout(g, mm);
+  const ColumnsLayout l = columns_layout(g, mm, false);
   char* ws = static_cast<char*>(workspace);
   float* rows = reinterpret_cast<float*>(ws + l.img_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
   float* w = reinterpret_cast<float*>(ws + l.weights);
-  if (columns_direct(g))
+  if (columns_direct_gather(g, mm))
     return columns_direct_forward(g, mm, img, map, wts, Wm, bias, pix, columns_scratch(l, ws), stream);
   const int Cgp = pad8(g.Cg), R = g.K * Cgp;
   int rc = to_rows(img, rows, g.B, g.Cg, (int64_t)g.H * g.W, stream);
@@ -751,7 +758,7 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
                          const float* wts, const float* Wm, const float* bias, float* img,
                          void* workspace, hipStream_t stream, const void* lists,
                          const float* wgrad_img, bool bias_sum) {
-  const ColumnsLayout l = columns_layout(g, mm);
+  const ColumnsLayout l = columns_layout(g, mm, true);
   char* ws = static_cast<char*>(workspace);
   float* rows = reinterpret_cast<float*>(ws + l.pix_rows);
   float* col = reinterpret_cast<float*>(ws + l.col);
@@ -782,7 +789,7 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
     SDK_LAUNCH_CHECK("mapped_conv(columns col2im)");
     return SDK_OK;
   };
-  if (columns_direct(g)) {
+  if (columns_direct_backward(g, mm)) {
     const ColumnsScratch s = columns_scratch(l, ws);
     const Slices& t = l.slices;
     const bool rows_too = t.both && wgrad_img != nullptr;
@@ -824,9 +831,9 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,
                          hipStream_t stream, bool prepared, float* gb) {
-  const ColumnsLayout l = columns_layout(g, mm);
+  const ColumnsLayout l = columns_layout(g, mm, true);
   char* ws = static_cast<char*>(workspace);
-  if (columns_direct(g))
+  if (columns_direct_backward(g, mm))
     return columns_direct_wgrad(g, mm, pix, map, wts, img, gW, l.slices.wgrad, columns_scratch(l, ws),
                                 prepared && l.slices.both, gb, stream);
   float* prows = reinterpret_cast<float*>(ws + l.pix_rows);

@@ -35,8 +35,8 @@ __device__ __forceinline__ void channels_last_tile(const float* __restrict__ src
   }
 }
 
-// The contractions without a column matrix in front of them (conv_columns_direct.hip), for calls of the
-// route that columns_direct() takes.
+// The contractions without a column matrix in front of them (conv_columns_direct.hip): of the calls of the
+// route on maps that columns_direct() takes, the forwards and the backwards that ..._gather and ..._backward do.
 struct ColumnsScratch {
   float* img_rows;      // B * H * W + 1 rows of pad8(Cg) floats
   void* weights;        // columns_weight_bytes()
@@ -46,6 +46,8 @@ struct ColumnsScratch {
   float* partial;       // columns_partial_bytes(), or columns_forward_sum_bytes()
 };
 bool columns_direct(const ConvGeom& g);
+bool columns_direct_gather(const ConvGeom& g, int mm);
+bool columns_direct_backward(const ConvGeom& g, int mm);
 size_t columns_weight_bytes(const ConvGeom& g, int mm);
 size_t columns_forward_sum_bytes(const ConvGeom& g, int mm);
 size_t columns_pixel_row_bytes(const ConvGeom& g, int mm, int64_t elements);
@@ -92,7 +94,7 @@ int columns_gemm_scatter(const ConvGeom& g, int mm, const float* pix, const floa
 // gW = sum_b pix[b] x im2col(img[b])^T; every element of gW is written.  prepared: the workspace
 // still holds what a columns_gemm_scatter of the same g and mm may have laid out for it.  gb
 // (columns_sums_bias): also gb[n] = sum of pix[b][n][m].
-bool columns_sums_bias(const ConvGeom& g);
+bool columns_sums_bias(const ConvGeom& g, int mm);
 int columns_gather_wgrad(const ConvGeom& g, int mm, const float* pix, const float* map,
                          const float* wts, const float* img, float* gW, void* workspace,
                          hipStream_t stream, bool prepared, float* gb);

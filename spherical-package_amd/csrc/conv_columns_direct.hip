@@ -797,7 +797,7 @@ DirectShape direct_shape(const ConvGeom& g, int mm) {
 // 128 x 256, 64 -> 64, float32 68, 61, 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55,
 // 45, 42; 32 rows, 2 x 115 x 231, 24 -> 32, float32 42, 26, 31.
 // More than five blocks are tiles of four, the last perhaps of padding; nine and ten of bf16 operands two of five where
-// there are few columns and so several splits.  Whole backward, float32 / bf16 / split, as equal tiles of three or
+// there are few columns and so several splits, float32 ones of a sample (32 -> 280, 3 x 88 x 177 103 and 112).  Whole backward, float32 / bf16 / split, as equal tiles of three or
 // five and of four: 176 -> 176, 4 x 24 x 49 141 / 86 / 113 and 127 / 69 / 105; 128 -> 184, 3 x 45 x 91 226 / 121 / 173
 // and 206 / 92 / 163; 32 -> 291, 136 x 272 265 / 113 / 212 and 251 / 107 / 222; 56 -> 264, 49 x 99 85 / 49 / 63 and
 // 85 / 51 / 69; 211 -> 272, 5 x 5, 2 x 19 x 36 245 / 122 / 185 and 180 / 99 / 148.
@@ -809,7 +809,7 @@ WgradShape wgrad_shape(const ConvGeom& g, int mm, int64_t elements) {   // (most
   const int64_t blocks = ceil_div(g.Cp, 32);
   t.tiles_r = (int)ceil_div((int64_t)g.K * pad8(g.Cg), 32);
   if (blocks <= 5) t.ra = (int)blocks;
-  else t.ra = (blocks == 9 || blocks == 10) && mm != kMmF32 && t.tiles_r <= 64 ? 5 : 4;
+  else t.ra = (blocks == 9 || blocks == 10) && t.tiles_r <= (mm == kMmF32 ? 2 : 64) ? 5 : 4;
   t.tiles_a = (int)ceil_div(blocks, t.ra);
   t.groups = t.ra == 1 ? 4 : (t.ra <= 3 ? 2 : 1);
   t.strips = (int)ceil_div(g.M, 32);
@@ -960,6 +960,28 @@ DirectArgs direct_args(const ConvGeom& g, const float* rows, const float* map, c
 // forward and backward of the other kernels and of these, us: two points 222 and 238, four 302 and 338, six 361 and
 // 484, eight 470 and 648, split; with the four taps that four weighted pixels have 180 and 133, bf16.)
 bool columns_direct(const ConvGeom& g) { return pts(g.P) <= 4; }
+
+// One sample of few channels at many pixels of a wide layer: a tile of the forward is over after a step or two, and
+// the pixels, laid out twice at four or six bytes a value, are most of the backward.  us, columns in memory and so,
+// float32 / bf16 / split:
+//   forward   8 -> 64   50 / 32 / 42 and 42 / 40 / 53      48 -> 64   78 / 64 / 72 and 64 / 57 / 73    4 x 181 x 363
+//             8 -> 128  46 / 28 / 39 and 38 / 30 / 39      32 -> 128  55 / 39 / 48 and 42 / 35 / 44    2 x 181 x 363
+//             8 -> 232  52 / 29 / 42 and 44 / 34 / 44      40 -> 232  60 / 38 / 51 and 60 / 41 / 56    2 x 147 x 290
+//   backward 16 -> 64  189 / 165 / 178 and 197 / 159 / 230  96 -> 64  376 / 342 / 359 and 365 / 298 / 388
+//            24 -> 128 152 / 130 / 144 and 170 / 119 / 182  64 -> 232 170 / 146 / 163 and 190 / 121 / 207
+// With a quarter of the pixels (17 MB) all of these are the faster ones.
+static bool one_sample_of_wide_pixels(const ConvGeom& g, int most_channels, size_t pixel_bytes) {
+  return g.K == 1 && pad8(g.Cg) <= most_channels && g.Cp >= 64 && sizeof(float) * g.B * g.M * g.Cp >= pixel_bytes;
+}
+bool columns_direct_gather(const ConvGeom& g, int mm) {
+  const bool four = ceil_div(g.Cp, 32) == 4;   // (a wave a SIMD: 32 -> 128, split, 48 and 44)
+  const int most = mm == kMmF32 ? 0 : (mm == kMmSplit ? (four ? 8 : 48) : std::min(48, (g.Cp - 1) / 4));
+  return columns_direct(g) && !one_sample_of_wide_pixels(g, most, (size_t)32 << 20);
+}
+bool columns_direct_backward(const ConvGeom& g, int mm) {
+  const int most = mm == kMmF32 ? 64 : (mm == kMmSplit ? 96 : 0);
+  return columns_direct(g) && !one_sample_of_wide_pixels(g, most, (size_t)54 << 20);
+}
 
 size_t columns_weight_bytes(const ConvGeom& g, int mm) {
   const DirectShape t = direct_shape(g, mm);

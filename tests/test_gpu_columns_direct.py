@@ -92,11 +92,11 @@ def test_bias_gradient_keeps_the_bits_of_its_sums(ops, height):
     """8 x 512 strips of 64 pixels a channel, the most that are added up here: in a float32 chain they were 1.8e-7
     from float64 in the norm, the sums of before 1.4e-7.  A strip is a tree of six float32 additions and the result is
     rounded once: 2^-24 * sqrt(7 / 3) = 0.9e-7 for random signs, on 128 channels within a fifth."""
-    tc = (8, 8, 128, 8, 16, height, 256, 1, 0, 1)
+    tc = (8, 8, 128, 8, 16, height, 256, 2, 0, 1)
     assert runs_by_columns(*tc)
     m, _, x, w, b, g, _ = columns._arrays(tc)
     t = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
-    gb = ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 1, 1)[2]
+    gb = ops.ops.mapped_conv_backward(t(g), t(m), None, t(x), t(w), t(b), 2, 1)[2]
     assert columns._rel(gb.cpu().numpy(), g.astype(np.float64).sum((0, 2, 3))) <= 1.1e-7
 
 
@@ -116,7 +116,7 @@ def _on_gpu(tc):
 LARGE = [
     (3, 32, 8, 40, 80, 100, 200, 25, 0, 1),
     (2, 70, 8, 40, 80, 144, 288, 25, 0, 1),
-    (30, 8, 96, 64, 128, 64, 128, 1, 0, 1),
+    (30, 8, 96, 64, 128, 64, 128, 7, 0, 1),
     (2, 40, 208, 40, 80, 144, 288, 11, 0, 0),
 ]
 
@@ -148,6 +148,23 @@ def test_calls_in_slices(ops, tc, mode, kept):
     # float32 sums: eps * sqrt(n) / 2, apart by 64 channels or 32 pixels; bf16 operands: 2^-9 each
     for have, ref in zip((gi, gw, gb), want):
         assert columns._rel(have.cpu().numpy(), ref.cpu().numpy()) <= (4e-3 if mode == "bf16" else 2e-6)
+
+
+@pytest.mark.parametrize("Cin", [8, 48, 64, 96, 97])
+@pytest.mark.parametrize("Cout", [64, 66, 112])
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+def test_wide_layers_of_one_sample(ops, mode, Cout, Cin):
+    """31.5, 32.5 and 55 MB of pixels: forwards (up to 48 channels, from 32 MB) and backwards (up to 96, from 54) with
+    their columns in memory and without."""
+    tc = (15, Cin, Cout, 12, 24, 67, 128, 1, 0, 1)
+    assert runs_by_columns(*tc)
+    arrays = m, _, x, w, b, g, bt = _on_gpu(tc)
+    with ops.conv_compute(mode):
+        have = [ops.ops.mapped_conv_forward(x, m, None, w, b, 1, 1), *_gradients(ops, tc, arrays, mode)]
+    m, x, w, b, g = (a.double() for a in (m, x, w, b, g))
+    want = [ops.ops.mapped_conv_forward(x, m, None, w, b, 1, 1), *ops.ops.mapped_conv_backward(g, m, None, x, w, b, 1, 1)]
+    for h, ref in zip(have, want):
+        assert columns._rel(h.cpu().numpy(), ref.cpu().numpy()) <= (4e-3 if mode == "bf16" else 2e-6)
 
 
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])
