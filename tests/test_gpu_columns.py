@@ -72,11 +72,11 @@ def _rel(a, b):
 def test_columns_route_matches_the_oracle(ops, oracle, tc, mode):
     from _spherical_distortion_ext import _capi
     B, Cin, Cout, H, W, OH, OW, K, P, interp = tc
-    for transposed in (0, 1) if Cout >= 5 else (0,):   # (nearest up-sampling layers: products)
+    for transposed in (0, 1) if Cout >= 5 else (0,):
         taken = _capi.load().sdk_mapped_conv_by_columns(
             B, Cout if transposed else Cin, Cin if transposed else Cout, H, W, OH, OW, K, P,
             interp, _capi.SDK_F32, 0, transposed)
-        assert taken == 1 or (interp == 0 and P == 0)
+        assert taken == 1
     m, iw, x, w, b, g, bt = _arrays(tc)
     t = lambda a: None if a is None else torch.from_numpy(a).to(DEV)  # noqa: E731
     with ops.conv_compute(mode):

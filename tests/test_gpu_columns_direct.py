@@ -150,6 +150,37 @@ def test_calls_in_slices(ops, tc, mode, kept):
         assert columns._rel(have.cpu().numpy(), ref.cpu().numpy()) <= (4e-3 if mode == "bf16" else 2e-6)
 
 
+@pytest.mark.parametrize("mode", ["native", "split", "bf16"])
+def test_gradients_of_values_no_tap_reads_stay_out(ops, mode):
+    """An infinite pixel of the image without a tap, an infinite value of the gradient and an infinite weight reach
+    what is summed from them and nothing else."""
+    tc = (1, 12, 40, 9, 14, 5, 7, 9, 0, 0)
+    arrays = m, _, x, w, b, g, _ = _on_gpu(tc)
+    m[..., 0].clamp_(0, 12)
+    x[0, :, :, 13] = 0
+    gi, gw, gb = _gradients(ops, tc, arrays, mode)
+    x[0, :, :, 13] = float("inf")
+    for have, want in zip(_gradients(ops, tc, arrays, mode), (gi, gw, gb)):
+        assert torch.equal(have, want)
+    x[0, :, :, 13] = 0
+    kept, g[0, 7, 2, 3] = g[0, 7, 2, 3].item(), float("inf")
+    hi, hw, hb = _gradients(ops, tc, arrays, mode)
+    rest = [n for n in range(40) if n != 7]
+    assert torch.equal(hw[rest], gw[rest]) and torch.equal(hb[rest], gb[rest])
+    assert not torch.isfinite(hb[7]) and not torch.isfinite(hw[7]).all()
+    at = (m[2, 3] + 0.5).floor().long()     # (the samples' pixels; no coordinate is a half)
+    at = at[(at[:, 1] >= 0) & (at[:, 1] < 9)]
+    reached = torch.zeros(9, 14, dtype=torch.bool, device=DEV)
+    reached[at[:, 1], at[:, 0]] = True
+    assert torch.equal(hi[0][:, ~reached], gi[0][:, ~reached])
+    assert not torch.isfinite(hi[0][:, reached]).any()
+    g[0, 7, 2, 3], w[7, 3, 2] = kept, float("inf")
+    hi, hw, hb = _gradients(ops, tc, arrays, mode)
+    assert torch.equal(hw, gw) and torch.equal(hb, gb)
+    rest = [c for c in range(12) if c != 3]
+    assert torch.equal(hi[:, rest], gi[:, rest]) and not torch.isfinite(hi[:, 3]).all()
+
+
 @pytest.mark.parametrize("Cin", [8, 48, 64, 96, 97])
 @pytest.mark.parametrize("Cout", [64, 66, 112])
 @pytest.mark.parametrize("mode", ["native", "split", "bf16"])

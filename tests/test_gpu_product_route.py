@@ -4,13 +4,14 @@ resolution, then a gather of the products over the inverted map.  Against the or
 float32 backward tolerance (1e-4 of the largest value), on shapes that cut the kernels' tiles
 (pixel counts, columns (k, c), channel counts on either side), maps with taps outside the image,
 image elements no tap reaches, and elements that collect hundreds of taps; planned against
-plain calls and call against call bit for bit (sums in list order, no atomics).
+plain calls and call against call bit for bit (sums in list order, no atomics).  Calls of these sizes
+run by columns; the route is theirs with the columns off, and the cases run both ways.
 """
 import numpy as np
 import pytest
 import torch
 
-from conftest import relerr
+from conftest import relerr, runs_by_columns
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -58,8 +59,14 @@ CASES = [
 
 
 @pytest.mark.parametrize("tc", CASES, ids=lambda t: "x".join(map(str, t)))
-def test_products_then_gather_match_the_oracle(ops, oracle, tc):
+def test_products_then_gather_match_the_oracle(ops, oracle, conv_route, tc):
+    from _spherical_distortion_ext import _capi
     Cg, Cp, H, W, OH, OW, K, B, kind = tc
+    for transposed, channels in ((0, (Cg, Cp)), (1, (Cp, Cg))):
+        assert runs_by_columns(B, *channels, H, W, OH, OW, K, 0, 0, transposed) == (conv_route == "columns")
+        # (4: the inverted map, which the products' gather reads)
+        assert conv_route == "columns" or _capi.load().sdk_mapped_conv_plan_parts(
+            B, *channels, H, W, OH, OW, K, 0, 0, _capi.SDK_F32, 0, transposed, 0, 0, 1) == 4
     rng = np.random.default_rng(sum(tc[:8]))
     m = _map(rng, OH, OW, K, H, W, kind)
     tm = _t(m)
