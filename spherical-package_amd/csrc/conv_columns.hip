@@ -566,7 +566,8 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm, bool backward) {
     if (!t.both) at = base;
     l.img_rows = take(image);
     l.pix_rows = take(columns_pixel_row_bytes(g, mm, t.wgrad));
-    l.partial = take(columns_partial_bytes(g, mm, t.wgrad));   // (not in the products' place: calls of a few us take 5 longer so)
+    // (not in the products' place: 256 x 4 x 6 pixels, 64 -> 128, bf16, backward 52 us, 57 so)
+    l.partial = take(columns_partial_bytes(g, mm, t.wgrad));
     at = std::max(at, end);
   } else {
     l.img_rows = take(image);
@@ -626,17 +627,16 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
   a.spread = TN && 8 * total < 7 * padded;
   const dim3 grid((unsigned)(a.spread ? (total * batches + 7) / 8 * 8 : padded),
                   (unsigned)(a.spread ? 1 : batches));
-  // Two groups of waves per tile where the tiles alone leave the SIMDs with a wave or two and the
-  // reduction is long enough to share (whole forward: 6 x 25 x 50, 96 -> 160, split 65 -> 55 us;
-  // 3 x 45 x 91, 200 -> 37, bf16 86 -> 67 us).  With fp32 MFMAs two waves of 512 tiles keep a SIMD
-  // busy as it is (1 x 128 x 256, 64 -> 64: 62 -> 67 us), and so do the splits of the weight
-  // gradient (57 -> 66 us).
+  // Two groups of waves per tile, each with every other step of a reduction that is long enough to share, where the
+  // tiles alone leave the SIMDs with a wave or two.  (Whole forward of eight points a sample, float32 / bf16 / split,
+  // one group and two: 1 x 20 x 40, 256 -> 200 125 / 96 / 121 and 123 / 92 / 118 us; 2 x 24 x 48, 128 -> 96, nearest
+  // 54 / 40 / 52 and 54 / 38 / 50; of many more tiles no faster: five points, 1 x 128 x 256, 64 -> 64 99 / 86 / 94 and
+  // 99 / 87 / 99; but the chains of the sums are half as long.)
   const bool shared = !TN && total * batches <= (mm == kMmF32 ? 256 : 1024) && a.red >= 4 * kGk;
   // Split operands are formed early by the weight gradient, where a reduction is longer than two steps, and by a
-  // forward of so few tiles that all are at work at once either way.  (The product alone, us late and
-  // early: weight gradient 200 x 200 in runs of 416 pixels 24.0 and 20.1, 32 x 32 in runs of 256 14.9 and 13.5;
-  // forward 160 x 28800 x 288 37.1 and 34.2, 64 x 28800 x 64 7.8 and 6.6, 64 x 51200 x 8 10.4 and 11.5, 240 x
-  // 115200 x 8 46 and 52; columns' gradient 12800 x 32 x 32 6.3 and 7.2, 115200 x 72 x 8 26.8 and 28.1.)
+  // forward of so few tiles that all are at work at once either way.  (us late and early: backward of one sample,
+  // 40 -> 232, 2 x 147 x 290 159 and 150, 64 -> 232 172 and 164; forward 40 -> 232 51 and 54, 24 -> 83, 3 x 156 x 312
+  // 46 and 50, 8 -> 64, 4 x 181 x 363 43 and 45; eight points, 6 x 50 x 100, stride 2, 96 -> 160, backward 185 and 181.)
   const bool early = TN || a.red > 2 * kGk || (a.rows_a <= a.rows_b && total * batches <= 768);
 #define CG2(MMv, KSv, CONVv) \
   launch((columns_gemm_kernel<MMv, TN, KSv, CONVv>), grid, dim3(KSv * kClThreads), stream, a)
@@ -659,22 +659,37 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
 }
 
 // Calls whose column matrix has at most this many bytes take the route (a scatter holds a slice of it, the others
-// none of it).  Forward + backward on a kept plan, 3 x 3 kernels, us of the tile kernels and of these, float32 /
-// bf16 / split:
-//   126 MB  4 x 120 x 240, 32 -> 32            275 / 199 / 241 and 228 / 179 / 224
-//   131 MB  2 x 100 x 200, 96 -> 160           992 / 379 / 688 and 617 / 251 / 460
-//   142 MB  4 x 90 x 180, 64 -> 64             373 / 242 / 307 and 293 / 188 / 274
-//   175 MB  4 x 200 x 400, 16 -> 16            444 / 276 / 367 and 384 / 306 / 403
-//   288 MB  4 x 128 x 256, 64 -> 64            513 / 284 / 400 and 558 / 344 / 530
+// none of it).  On a kept plan, 3 x 3 kernels, us of the tile kernels and of these, float32 / bf16 / split, forward
+// and backward, and the forward alone:
+//   112 MB  4 x 160 x 320, 16 -> 16   350 / 231 / 294 and 213 / 181 / 221    72 /  46 /  59 and  59 /  44 /  60
+//   122 MB  6 x 96 x 192, 32 -> 32    304 / 210 / 266 and 217 / 168 / 216    46 /  34 /  41 and  59 /  42 /  58
+//   122 MB  8 x 96 x 192, 24 -> 24    274 / 194 / 238 and 246 / 196 / 243    54 /  37 /  46 and  60 /  44 /  54
+//   126 MB  4 x 120 x 240, 32 -> 32   271 / 194 / 238 and 219 / 173 / 216    55 /  38 /  48 and  59 /  44 /  58
+//   131 MB  2 x 100 x 200, 96 -> 160  990 / 377 / 690 and 618 / 254 / 472   259 /  81 / 173 and 181 /  60 / 136
+//   142 MB  4 x 90 x 180, 64 -> 64    371 / 236 / 304 and 300 / 190 / 288    92 /  49 /  70 and  71 /  45 /  69
+//   175 MB  4 x 200 x 400, 16 -> 16   444 / 276 / 367 and 384 / 306 / 403
+//   288 MB  4 x 128 x 256, 64 -> 64   513 / 284 / 400 and 558 / 344 / 530
 // nearest taps
-//    72 MB  2 x 128 x 256, 32 -> 32            183 / 174 / 173 and 119 / 116 / 119
-//   108 MB  4 x 64 x 128, 96 -> 96             515 / 249 / 390 and 285 / 123 / 217
-//   144 MB  2 x 256 x 512, 12 -> 24            290 / 196 / 244 and 241 / 167 / 244
-//   288 MB  4 x 128 x 256, 64 -> 64            460 / 247 / 356 and 480 / 253 / 415
-// Above ten samples the tile kernels' weight gradient is another, and there is no such line, 5 x 5:
-//   400 MB  2 x 128 x 256, 64 -> 64            1814 / 1399 / 1646 and 751 / 477 / 706
-//   693 MB  8 x 169 x 336, 16 -> 56            4048 / 2940 / 3520 and 1697 / 1169 / 1640
-//   793 MB  1 x 200 x 400, 104 -> 88           4324 / 2405 / 3269 and 2537 / 1597 / 2155
+//    72 MB  2 x 128 x 256, 32 -> 32   177 / 138 / 162 and 107 /  78 / 106    37 /  27 /  33 and  25 /  18 /  23
+//   108 MB  4 x 64 x 128, 96 -> 96    513 / 246 / 387 and 284 / 119 / 219   147 /  58 / 103 and  78 /  30 /  64
+//   122 MB  8 x 96 x 192, 24 -> 24    215 / 155 / 187 and 176 / 121 / 180    48 /  33 /  41 and  50 /  28 /  41
+//   144 MB  2 x 256 x 512, 12 -> 24   289 / 192 / 240 and 231 / 153 / 239    70 /  42 /  54 and  56 /  33 /  50
+//   288 MB  4 x 128 x 256, 64 -> 64   460 / 247 / 356 and 480 / 253 / 415
+// (A forward of 24 or 32 channels that is called again and again on one map is faster by the tile kernels from 100 MB
+// on; the first call on a map, which builds their plan for 200 to 300 us, is not, nor is a training step.)
+// Above ten samples the tile kernels' weight gradient is another, 5 x 5:
+//   400 MB  2 x 128 x 256, 64 -> 64  1815 / 1403 / 1657 and 737 / 475 / 694   492 / 335 / 430 and 164 / 92 / 159
+//   693 MB  8 x 169 x 336, 16 -> 56  4043 / 2935 / 3529 and 1676 / 1169 / 1600   734 / 371 / 544 and 317 / 190 / 308
+//   793 MB  1 x 200 x 400, 104 -> 88  4320 / 2396 / 3274 and 2358 / 1367 / 1945   1417 / 597 / 982 and 554 / 222 / 412
+//   800 MB  4 x 128 x 256, 64 -> 64, nearest  1616 / 926 / 1301 and 1188 / 616 / 996
+//           309 / 106 / 224 and 325 / 92 / 215
+//   1.6 GB  8 x 128 x 256, 64 -> 256  11929 / 7004 / 9174 and 8576 / 3450 / 6460
+//           2137 / 742 / 1457 and 2235 / 709 / 1615
+//   3.2 GB  8 x 256 x 512, 32 -> 32  6085 / 4988 / 5805 and 5166 / 4197 / 5132   912 / 555 / 755 and 877 / 568 / 846
+//   6.4 GB  8 x 256 x 512, 64 -> 64  13310 / 8850 / 11446 and 12557 / 8334 / 11489
+//           2399 / 1039 / 1796 and 2429 / 1226 / 2176
+// No training step up there is slower by columns; forwards alone are even from about 1.5 GB on and behind, where split
+// or bf16, by up to a fifth at the end.  What ends the route are the 1 GB below.
 // Weighted samples stop at the line their calls had when the columns went through memory, for those whose
 // samples have more than four taps.
 constexpr size_t kColumnsBytes = (size_t)150 << 20, kColumnsWeightedBytes = (size_t)100 << 20;

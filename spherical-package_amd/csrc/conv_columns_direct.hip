@@ -39,7 +39,7 @@ namespace {
 // 32 channels x all pixels of the tile.  Per step a thread blends up to four channels of NI
 // samples (NT taps each, offsets and coefficients from a table in LDS) and leaves them in LDS in
 // the form the MFMAs read; the weights come from memory as the operands they are
-// (columns_operand_kernel).  The reads of a step are made before the MFMAs of the step before it.
+// (columns_prepare_kernel).  The reads of a step are made before the MFMAs of the step before it.
 //
 // The taps of `cap` samples of every pixel of the tile fit the table at a time; the reduction is
 // walked in runs of steps whose samples do.  Unused slots and steps past the end point at a row
@@ -158,7 +158,9 @@ __global__ __launch_bounds__(64 * RA * G, (RA > 1 && (MM != kMmSplit || (RA > 3 
   // hundreds of pixels, so one turn at a time (split operands: two) is summed apart and then added, sum[1] the sums.
   // Distance from float64, 1e-7 of the norm, with 1, 2, 4 turns and all of a split in a chain: 96 -> 160, 7500 pixels,
   // float32 1.6, 1.7, 2.2, 5.5, split 1.9, 1.8, 2.0, 4.9; 8 -> 8, 86 thousand pixels, float32 1.6, 1.9, 2.3, 2.3,
-  // split 4.0, 3.2, 3.2, 3.2.
+  // split 4.0, 3.2, 3.2, 3.2.  Wide layers of few splits have longer chains of turns, and the tile kernels longer ones
+  // yet (their distance in brackets): 5 x 5, 200 -> 160, 100 x 200, one split of 625 turns, float32 4.6 (6.4), split
+  // 3.7 (6.0); 256 -> 160, 128 x 256, 1024 turns, 5.9 (8.2), 4.6 (8.1); 32 -> 32, 8 x 256 x 512, 3.8 (6.8), 9.4 (19).
   constexpr int kAlone = MM == kMmSplit ? 2 : 1;
   constexpr bool kTwo = WGRAD || G == 1;
   int done = 0;
@@ -795,12 +797,15 @@ DirectShape direct_shape(const ConvGeom& g, int mm) {
 // splits of at least four turns.  Its kernel alone, us, with 1024, 2048 and 4096 waves: 160 rows (one tile of five
 // blocks: one workgroup a CU; 1536, where some CUs have two, 54), 6 x 25 x 50, 96 -> 160, split 31, 35, 42; 64 rows,
 // 128 x 256, 64 -> 64, float32 68, 61, 47; 37 rows, 3 x 45 x 91, split 67, 65, 51; 128 rows, 4 x 40 x 80, split 55,
-// 45, 42; 32 rows, 2 x 115 x 231, 24 -> 32, float32 42, 26, 31.
+// 45, 42; 32 rows, 2 x 115 x 231, 24 -> 32, float32 42, 26, 31.  One tile of five blocks for each of 129 to 255 column
+// tiles is one split, and leaves CUs idle: 5 x 5, 256 -> 160, 48 x 96 (200), backward, float32 / bf16 / split, 405 / 177
+// / 297 (tile kernels 1182 / 600 / 861); 512 -> 160, 3 x 3, 2 x 40 x 80 (144) 468 / 189 / 327 (549 / 264 / 422).
 // More than five blocks are tiles of four, the last perhaps of padding; nine and ten of bf16 operands two of five where
-// there are few columns and so several splits, float32 ones of a sample (32 -> 280, 3 x 88 x 177 103 and 112).  Whole backward, float32 / bf16 / split, as equal tiles of three or
-// five and of four: 176 -> 176, 4 x 24 x 49 141 / 86 / 113 and 127 / 69 / 105; 128 -> 184, 3 x 45 x 91 226 / 121 / 173
-// and 206 / 92 / 163; 32 -> 291, 136 x 272 265 / 113 / 212 and 251 / 107 / 222; 56 -> 264, 49 x 99 85 / 49 / 63 and
-// 85 / 51 / 69; 211 -> 272, 5 x 5, 2 x 19 x 36 245 / 122 / 185 and 180 / 99 / 148.
+// there are few columns and so several splits, float32 ones of a sample (32 -> 280, 3 x 88 x 177 103 and 112).  Whole
+// backward, float32 / bf16 / split, as equal tiles of three or five and of four: 176 -> 176, 4 x 24 x 49 141 / 86 / 113
+// and 127 / 69 / 105; 128 -> 184, 3 x 45 x 91 226 / 121 / 173 and 206 / 92 / 163; 32 -> 291, 136 x 272 265 / 113 / 212
+// and 251 / 107 / 222; 56 -> 264, 49 x 99 85 / 49 / 63 and 85 / 51 / 69; 211 -> 272, 5 x 5, 2 x 19 x 36 245 / 122 / 185
+// and 180 / 99 / 148.
 struct WgradShape {
   int ra, groups, tiles_a, tiles_r, strips, steps, most, splits, split_steps, samples;   // samples: most of a tile
 };
@@ -892,7 +897,7 @@ int direct(const ConvGeom& g, int mm, DirectArgs a, int ra, int groups, int samp
   const size_t sums = (size_t)(groups - 1) * 16 * 64 * ra * 4;
   const size_t smem = std::max(tiles, sums);
   const dim3 block((unsigned)(64 * ra * groups));
-  hipError_t reserved = hipSuccess;   
+  hipError_t reserved = hipSuccess;
 #define CF3(MMv, RAv, Gv, NTv)                                                                                \
   do {                                                                                                        \
     const auto kernel = columns_direct_kernel<WGRAD, MMv, RAv, Gv, NTv>;                                      \
@@ -956,9 +961,18 @@ DirectArgs direct_args(const ConvGeom& g, const float* rows, const float* map, c
 
 }  // namespace
 
-// (With more points a sample its taps are too many to be read turn by turn: 64 -> 64, 128 x 256, bilinear points,
-// forward and backward of the other kernels and of these, us: two points 222 and 238, four 302 and 338, six 361 and
-// 484, eight 470 and 648, split; with the four taps that four weighted pixels have 180 and 133, bf16.)
+// Samples of several points.  The line is drawn for points on pixels, a tap each: the four nearest pixels with weights
+// of their own, and vertices.  Between pixels a blended point has four, of which the first of a sample are read ahead and
+// the others turn by turn; the host cannot tell the two.  us of the columns in memory and of these, float32 / bf16 /
+// split, forward and backward:
+//   1 x 128 x 256, 64 -> 64   four pixels 217 / 180 / 206 and 174 / 124 / 166   two points between 241 / 204 / 235 and
+//                             219 / 176 / 222   four between 313 / 276 / 300 and 303 / 262 / 315   six, split, 361 and
+//                             484   eight 470 and 648
+//   2 x 48 x 96, 96 -> 96     four pixels 176 / 127 / 154 and 150 / 106 / 138   two between 193 / 145 / 172 and
+//                             191 / 159 / 186   four between 234 / 186 / 213 and 252 / 227 / 255
+// Over 180 drawn calls each, median: forward 0.72 / 0.70 / 0.71 on pixels, 0.90 / 0.98 / 0.92 with two points between,
+// 1.00 / 1.12 / 1.07 with four; backward 0.77 / 0.70 / 0.78, 0.85 / 0.79 / 0.86, 0.89 / 0.87 / 0.94.  (The worst are
+// forwards of eight channels: twice the time with four points between pixels.)
 bool columns_direct(const ConvGeom& g) { return pts(g.P) <= 4; }
 
 // One sample of few channels at many pixels of a wide layer: a tile of the forward is over after a step or two, and
