@@ -516,16 +516,18 @@ size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(
 // least 32, a run of 128 bytes (backward, float32 / bf16, us, whole and so: 793 MB, 104 -> 88, 200 x 400, 5 x 5 1973 /
 // 1363 and 1799 / 1138; 381 MB, 200 -> 160, 100 x 200 1636 / 801 and 1592 / 688; but 200 MB, 8 x 128 x 256, 64 -> 256,
 // whose pixels are as large, 6143 / 2624 and 6404 / 2713).
-// Both forms of the pixels' operands are laid out in one launch where they take no more than 128 MB; beyond that
-// each contraction lays out its own, one after the other in the same place, of elements of up to 128 MB (8 x 256 x
-// 512, 64 -> 64, 5 x 5, workspace 1938 -> 554 MB, backward 9864 -> 10041 us).
-constexpr size_t kSliceBytes = (size_t)128 << 20, kOperandBytes = (size_t)128 << 20, kCacheBytes = (size_t)256 << 20;
+// Both forms of the pixels' operands are laid out in one launch, side by side, where they take less than 256 MB; beyond
+// that each contraction lays out its own, one after the other in the same place, of elements of up to 256 MB (both always
+// and so, float32: 8 x 256 x 512, 64 -> 64, 5 x 5 1938 and 626 MB of workspace, backward 9857 and 10035 us; 8 x 128 x
+// 256, 64 -> 256 1286 and 521, 6100 and 6331; apart from 128 MB on 16 -> 194, 3 x 302 x 605, stride 2 487 and 520 us).
+constexpr size_t kSliceBytes = (size_t)128 << 20, kCacheBytes = (size_t)256 << 20;
+constexpr size_t kOperandBytes = (size_t)256 << 20;
 Slices slices_of(const ConvGeom& g, int mm) {
   const size_t samples = sizeof(float) * g.M * g.K;
   const size_t rows = columns_pixel_row_bytes(g, mm, 1), cols = columns_pixel_column_bytes(g, mm, 1);
   auto elements = [&](size_t most, size_t one) { return std::max<int64_t>(1, std::min<int64_t>(g.B, most / one)); };
   Slices s;
-  s.both = g.B * (rows + cols) <= kOperandBytes;
+  s.both = g.B * (rows + cols) < kOperandBytes;
   s.wgrad = s.both ? g.B : elements(kOperandBytes, rows);
   s.channels = pad8(g.Cg);
   if (samples * s.channels > kCacheBytes && s.channels > 32) {
@@ -550,25 +552,26 @@ ColumnsLayout columns_layout(const ConvGeom& g, int mm, bool backward) {
     return here;
   };
   const size_t image = sizeof(float) * ((size_t)g.B * g.H * g.W + 1) * Cgp;   // (and a row of zeros)
+  // The image first, always: the gather and the weight gradient of a transposed layer's backward lay out the same one,
+  // and a second copy beside the first pushes both out of the memory-side cache (84 MB, icosphere level 7, 128
+  // channels: weight gradient 34 us in one place, 51 in two).
   if (!backward && columns_direct_gather(g, mm)) {
-    l.weights = take(columns_weight_bytes(g, mm));
     l.img_rows = take(image);
+    l.weights = take(columns_weight_bytes(g, mm));
     l.partial = take(columns_forward_sum_bytes(g, mm));
   } else if (backward && columns_direct_backward(g, mm)) {
     const Slices& t = l.slices = slices_of(g, mm);
-    const size_t products = sizeof(float) * t.scatter * g.M * g.K * t.channels;
-    l.weights = take(columns_weight_bytes(g, mm));
-    l.strip_sums = take(columns_strip_bytes(g));
-    const size_t base = at;
-    l.pix_cols = take(columns_pixel_column_bytes(g, mm, t.both ? g.B : t.scatter));
-    l.col = take(products);
-    const size_t end = at;
-    if (!t.both) at = base;
     l.img_rows = take(image);
     l.pix_rows = take(columns_pixel_row_bytes(g, mm, t.wgrad));
     // (not in the products' place: 256 x 4 x 6 pixels, 64 -> 128, bf16, backward 52 us, 57 so)
     l.partial = take(columns_partial_bytes(g, mm, t.wgrad));
+    const size_t end = at;
+    if (!t.both) at = 0;
+    l.pix_cols = take(columns_pixel_column_bytes(g, mm, t.both ? g.B : t.scatter));
+    l.col = take(sizeof(float) * t.scatter * g.M * g.K * t.channels);
     at = std::max(at, end);
+    l.weights = take(columns_weight_bytes(g, mm));
+    l.strip_sums = take(columns_strip_bytes(g));
   } else {
     l.img_rows = take(image);
     l.col = take(sizeof(float) * column_values(g));

@@ -116,7 +116,7 @@ def _on_gpu(tc):
 LARGE = [
     (3, 32, 8, 40, 80, 100, 200, 25, 0, 1),
     (2, 70, 8, 40, 80, 144, 288, 25, 0, 1),
-    (30, 8, 96, 64, 128, 64, 128, 7, 0, 1),
+    (32, 8, 192, 64, 128, 64, 128, 7, 0, 1),
     (2, 40, 208, 40, 80, 144, 288, 11, 0, 0),
 ]
 
