@@ -19,6 +19,9 @@
 // 3 x 45 x 91, split 82 -> 47; 256 -> 256, 5 x 5, 2 x 24 x 48, stride 2, split 149 -> 45; 24 -> 32, 2 x 115 x 231,
 // float32 50 -> 27.  Forward and backward of the same:
 // 206 -> 156, 170 -> 124, 130 -> 87, 251 -> 171, 264 -> 125, 177 -> 114.
+// A tile's 32 pixels are of one batch element, so a grid of fewer is padded; it is still the faster way: backward,
+// float32, 4096 x 2 x 2 pixels, 16 -> 16 908 -> 104, 1024 x 2 x 4, 64 -> 64 468 -> 108, 4096 of one pixel, 64 -> 256,
+// nine samples 1704 -> 1152, one sample 1663 -> 259.
 // What bounds it: in float32 the MFMAs (half of the forward at 64 -> 64) and the vector
 // instructions of the blend, which do not overlap them; in the others the blend, and the reads of operands and
 // taps by too few waves.
