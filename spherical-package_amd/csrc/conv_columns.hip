@@ -729,9 +729,18 @@ bool columns_sums_bias(const ConvGeom& g, int mm) {
   return columns_direct_backward(g, mm) && g.B * ceil_div(g.M, 64) <= 4096;
 }
 
-// (one size for every arithmetic and direction)
+// One size for every arithmetic and direction.  Where split operands, the largest, lie side by side, their backward's is
+// it, but for the sums, of which other shapes of tiles, or a forward, may have more.  (Six layouts a query are 300 ns a
+// query more, two or three queries a call.)
 size_t columns_workspace_bytes(const ConvGeom& g) {
   if (!columns_route(g)) return 0;
+  if (g.K > 1 && columns_direct(g)) {
+    const ColumnsLayout l = columns_layout(g, kMmSplit, true);
+    if (l.slices.both) {
+      const size_t split = columns_partial_bytes(g, kMmSplit, g.B), f32 = columns_partial_bytes(g, kMmF32, g.B);
+      return l.total - up256(split) + up256(std::max({split, f32, columns_forward_sum_bytes(g, kMmSplit)}));
+    }
+  }
   size_t most = 0;
   for (int mm : {kMmF32, kMmBf16, kMmSplit})
     for (bool backward : {false, true}) most = std::max(most, columns_layout(g, mm, backward).total);

@@ -762,7 +762,9 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(PrepareArgs g) {
 //     share four SIMDs badly.  Forward alone, us, float32 / bf16 / split, as equal tiles of three or five and so:
 //     19 -> 176 channels, 188 x 376 106 / 56 / 102 and 109 / 50 / 80 (float32 as three of two 90; 176 -> 176,
 //     4 x 24 x 49 78, 75 and 52 so); 32 -> 264, 3 x 62 x 125 87 / 40 / 74 and 72 / 33 / 53; 32 -> 291, 136 x 272
-//     126 / 57 / 118 and 106 / 45 / 77; 72 -> 264, 62 x 125 54 / 23 / 49 and 55 / 25 / 42.  Five blocks whose columns
+//     126 / 57 / 118 and 106 / 45 / 77.  Nine, a third of them padding so, stay two of five and four where the products
+//     are long and not split: 72 -> 264, 62 x 125 54 / 23 / 49 and 55 / 25 / 42; 75 -> 280, 7 x 32 x 65, bf16 27 and 30.
+//     Five blocks whose columns
 //     are quickly multiplied are two tiles of four where they are split: 48 -> 160, 2 x 54 x 108 36 and 30, 24 -> 160,
 //     7 x 60 x 121 75 and 62; 96 -> 160 above 33 and 33, 216 -> 152, 2 x 56 x 112 112 and 123;
 //   groups where the tiles leave SIMDs without a wave: 216 tiles of two blocks (104 -> 37 channels, 2 x 41 x 83)
@@ -781,6 +783,7 @@ DirectShape direct_shape(const ConvGeom& g, int mm) {
   t.tiles_m = (int)ceil_div(g.M, kDirectPixels);
   t.steps = (int)ceil_div((int64_t)g.K * pad8(g.Cg), kDirectStep);
   if (blocks <= 4 || (blocks == 5 && (mm != kMmSplit || t.steps >= 24))) t.ra = (int)blocks;
+  else if (blocks == 9 && mm != kMmSplit && t.steps >= 20) t.ra = 5;
   else t.ra = blocks == 6 && mm == kMmF32 ? 2 : 4;
   t.tiles_a = (int)ceil_div(blocks, t.ra);
   // (splits by the columns' tiles of up to five blocks: the sums' chains do not grow with the tiles of four)
@@ -991,8 +994,10 @@ static bool one_sample_of_wide_pixels(const ConvGeom& g, int most_channels, size
   return g.K == 1 && pad8(g.Cg) <= most_channels && g.Cp >= 64 && sizeof(float) * g.B * g.M * g.Cp >= pixel_bytes;
 }
 bool columns_direct_gather(const ConvGeom& g, int mm) {
-  const bool four = ceil_div(g.Cp, 32) == 4;   // (a wave a SIMD: 32 -> 128, split, 48 and 44)
-  const int most = mm == kMmF32 ? 0 : (mm == kMmSplit ? (four ? 8 : 48) : std::min(48, (g.Cp - 1) / 4));
+  // (whole tiles of four waves, one a SIMD: 32 -> 128, split, 48 and 44; single taps: 16 -> 243, 4 x 159 x 316, nearest,
+  // bf16 / split 56 / 85 and 51 / 72)
+  const bool four = ceil_div(g.Cp, 32) % 4 == 0, single = g.interp == 0 && g.P == 0;
+  const int most = mm == kMmF32 || single ? 0 : (mm == kMmSplit ? (four ? 8 : 48) : std::min(48, (g.Cp - 1) / 4));
   return columns_direct(g) && !one_sample_of_wide_pixels(g, most, (size_t)32 << 20);
 }
 bool columns_direct_backward(const ConvGeom& g, int mm) {
