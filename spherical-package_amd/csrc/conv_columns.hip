@@ -695,8 +695,19 @@ int gemm(int mm, GemmArgs a, int64_t batches, hipStream_t stream) {
 // or bf16, by up to a fifth at the end.  What ends the route are the 1 GB below.
 // Weighted samples stop at the line their calls had when the columns went through memory, for those whose
 // samples have more than four taps.
+// Fewer than seven samples leave the tile kernels' scatter little to sum twice, and pixels and image are most of the
+// traffic: the lines their calls had when the columns went through memory.  us of the tile kernels -> by columns,
+// float32 / bf16 / split:
+//                                                 forward                  backward
+//   nearest, one, 4 x 159 x 316, 64 -> 128    65/ 43/ 57 ->  73/ 51/ 65    173/138/161 -> 271/201/293
+//   nearest, four, 8 x 120 x 240, 32 -> 64    59/ 36/ 48 ->  68/ 36/ 51    161/115/136 -> 200/136/224
+//   nearest, four, 4 x 159 x 316, 16 -> 128   87/ 41/ 64 ->  60/ 35/ 51    237/151/194 -> 225/149/245
+//   bilinear, one, 8 x 200 x 400, 48 -> 64   122/103/127 -> 165/153/187    316/282/308 -> 538/457/578
+//   bilinear, four, 8 x 120 x 240, 32 -> 64   68/ 43/ 59 ->  72/ 51/ 74    203/149/176 -> 224/162/247
+// (the third, few channels into many, is the one kind that float32 loses by it.)
 constexpr size_t kColumnsBytes = (size_t)150 << 20, kColumnsWeightedBytes = (size_t)100 << 20;
-constexpr int kTileSamples = 10;
+constexpr size_t kColumnsFewBytes = (size_t)100 << 20, kColumnsFewNearestBytes = (size_t)36 << 20;
+constexpr int kTileSamples = 10, kFewSamples = 7;
 // ... and the tensors laid out for them (32-bit byte offsets into the image's rows)
 constexpr size_t kColumnsTensorBytes = (size_t)1 << 30, kColumnsElementBytes = (size_t)1 << 30;
 bool columns_fit(const ConvGeom& g) {
@@ -704,7 +715,8 @@ bool columns_fit(const ConvGeom& g) {
   const size_t columns = sizeof(float) * column_values(g);
   if (g.K > kTileSamples && columns_direct(g))
     return columns / g.B <= kColumnsElementBytes && image <= kColumnsTensorBytes && pixels <= kColumnsTensorBytes;
-  const size_t limit = g.P == 0 ? kColumnsBytes : kColumnsWeightedBytes;
+  const size_t few = g.interp == 0 ? kColumnsFewNearestBytes : kColumnsFewBytes;
+  const size_t limit = g.P != 0 ? kColumnsWeightedBytes : (g.K < kFewSamples ? few : kColumnsBytes);
   return columns <= limit && image <= 2 * limit && pixels <= 2 * limit;
 }
 
@@ -714,7 +726,7 @@ thread_local bool t_columns = true;
 
 bool columns_map(const ConvGeom& g) {
   // (the lists of the inverted map: 32 bytes a sample of four taps)
-  const int64_t most = (int64_t)1 << (!columns_direct(g) ? 20 : (g.K > kTileSamples ? 24 : 21));
+  const int64_t most = (int64_t)1 << (!columns_direct(g) || g.K < kFewSamples ? 20 : (g.K > kTileSamples ? 24 : 21));
   return g.M >= 1 && g.K >= 1 && (int64_t)g.M * g.K <= most && pts(g.P) <= 8 &&
          col2im_lists_bytes(g.H, g.W, g.M, g.K, g.P, g.interp) != 0;
 }

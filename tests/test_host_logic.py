@@ -354,3 +354,19 @@ def test_workspace_of_convolutions_by_columns(call, most):
     assert lib.sdk_mapped_conv_by_columns(*call, 0, 1, _capi.SDK_F32, 0, 0) == 1
     need = {lib.sdk_mapped_conv_workspace_bytes(*call, 0, 1, _capi.SDK_F32, compute) for compute in (0, 1, 3)}
     assert len(need) == 1 and need.pop() <= most << 20
+
+
+@pytest.mark.parametrize("B, K, interp, taken", [
+    # 64 channels of 128 x 256 pixels, 8 MB a sample and element: 32, 40 and 96, 104 MB ...
+    (4, 1, 0, 1), (5, 1, 0, 0), (1, 4, 0, 1), (1, 5, 0, 0), (1, 6, 0, 0),
+    (12, 1, 1, 1), (13, 1, 1, 0), (3, 4, 1, 1), (4, 4, 1, 0), (3, 4, 2, 1), (4, 4, 2, 0),
+    # ... and from seven samples 144 and 168, 216 MB
+    (2, 7, 0, 1), (3, 7, 0, 0), (2, 9, 0, 1), (2, 9, 1, 1), (3, 9, 1, 0)])
+def test_convolutions_of_few_samples_by_columns(B, K, interp, taken):
+    """Fewer than seven samples end the columns route at 36 MB (nearest) and 100 MB, not at 150 MB: beyond, the tile
+    kernels had been up to twice as fast; and at maps of 2^20 samples, not of 2^21."""
+    from _spherical_distortion_ext import _capi
+    lib = _capi.load()
+    assert lib.sdk_mapped_conv_by_columns(B, 64, 64, 128, 256, 128, 256, K, 0, interp, _capi.SDK_F32, 0, 0) == taken
+    for samples, rows, fits in ((1, 1024, 1), (1, 1025, 0), (4, 256, 1), (4, 257, 0), (7, 257, 1)):
+        assert lib.sdk_mapped_conv_by_columns(1, 8, 8, 64, 128, rows, 1024, samples, 0, 1, _capi.SDK_F32, 0, 0) == fits
