@@ -519,7 +519,9 @@ size_t column_values(const ConvGeom& g) { return (size_t)g.B * g.M * g.K * pad8(
 // Both forms of the pixels' operands are laid out in one launch, side by side, where they take less than 256 MB; beyond
 // that each contraction lays out its own, one after the other in the same place, of elements of up to 256 MB (both always
 // and so, float32: 8 x 256 x 512, 64 -> 64, 5 x 5 1938 and 626 MB of workspace, backward 9857 and 10035 us; 8 x 128 x
-// 256, 64 -> 256 1286 and 521, 6100 and 6331; apart from 128 MB on 16 -> 194, 3 x 302 x 605, stride 2 487 and 520 us).
+// 256, 64 -> 256 1286 and 586, 6100 and 6331; apart from 128 MB on 16 -> 194, 3 x 302 x 605, stride 2 487 and 520 us).
+// The line gives time for memory: few channels into many lose most beyond it (16 -> 256 there, 280 MB 526 and 574 us;
+// split 16 -> 194, 412 MB 491 and 508); 512 MB would take back those, and add up to 300 MB to such calls' workspace.
 constexpr size_t kSliceBytes = (size_t)128 << 20, kCacheBytes = (size_t)256 << 20;
 constexpr size_t kOperandBytes = (size_t)256 << 20;
 Slices slices_of(const ConvGeom& g, int mm) {
